@@ -412,9 +412,9 @@ def main(argv=None) -> int:
 
     pairs = st["total_neighbor_pairs"]
     fused_ms = statistics.mean(fused)
-    # FP64 work executed inside k_curvelets: the transport cells (F_CELLS per
-    # pair; its sines come precomputed from k_edge_trig / k_pair_trig) and the
-    # growth intersections (3 FLOP per cell per intersection)
+    # FP64 work the reference's formulas take for what k_curvelets does: the
+    # transport cells (F_CELLS per pair; without the sines) and the growth
+    # intersections (3 FLOP per cell per intersection)
     flops = pairs * F_CELLS + st["intersections"] * 63 * 3
     achieved = flops / (fused_ms * 1e-3) / 1e12
     line = {

@@ -17,22 +17,6 @@ struct PairRec {
     double cT0m_DX, sT0m_DY, cT0p_DX, sT0p_DY;
 };
 
-// Per-edge trig slots: rows 0-5 are structure of arrays (stride = number of
-// edges n), then one block of 2 Kt values per edge (edge-major, so the fused
-// kernel reads an anchor's grid angles from one or two cache lines):
-//   row 0 cos(theta)      row 1 sin(theta)
-//   row 2 sin(theta+dt)   row 3 cos(theta+dt)   row 4 sin(theta-dt)   row 5 cos(theta-dt)
-//   [6n + 2(i Kt + j)] = sin(theta_i + off_t[j]),  [6n + 2(i Kt + j) + 1] = cos(theta_i + off_t[j])
-enum {
-    TRIG_COS = 0,
-    TRIG_SIN = 1,
-    TRIG_SIN_P = 2,
-    TRIG_COS_P = 3,
-    TRIG_SIN_M = 4,
-    TRIG_COS_M = 5,
-    TRIG_GRID = 6
-};
-
 // Direction class of a neighbour: 1 when dot(To2Pi(atan2(ny-ay, nx-ax)), theta_a)
 // > 0 (forward run), 2 when < 0 (backward run), 0 otherwise
 // (cpu_curvelet.hpp:459-461, curvelet_utils.hpp:58-69).

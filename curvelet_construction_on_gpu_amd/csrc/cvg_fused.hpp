@@ -1,0 +1,1098 @@
+// The fused bundle + chain-growth kernel of double maps (k_curvelets) and the
+// small kernels that feed it.  Included by cvg_pipeline.hip inside its
+// namespace, after the wave helpers.
+//
+// The reference decides everything by comparing bundle bounds lo < hi
+// (cpu_curvelet.hpp:821-854), each bound a quotient of the transport formulas.
+// Four IEEE divisions are ~270 of the ~430 SIMD cycles one pair's 63 cells take
+// that way (66.8 cycles per wave division against 5 for a multiply, measured),
+// and their per-pair sines another pass over memory.  Here the bounds are first
+// formed approximately, with a proven error bound: sines by rotating the edges'
+// correctly rounded sin/cos, one reciprocal for the three denominators, the
+// result in 32-bit fixed point.  A comparison whose margin exceeds the error
+// bound is decided by it.  An anchor with any closer comparison is done again,
+// and then those comparisons are made on the exact bounds (the reference's
+// operands and rounding points, correctly rounded math, IEEE divisions).  The
+// results are the reference's bit for bit.
+//
+// Measured on the 1080p map (207,326 edges, 2.04M pairs, G = 7): 1,000 us for
+// the kernel on exact bounds and 141 us for its sines pass (345 MB) before; now
+// 530 us, and 83 us for the few anchors left open.
+#ifndef CVG_FUSED_HPP
+#define CVG_FUSED_HPP
+
+// The grid and edges of exact_bounds.
+struct ExactGrid {
+    const double *x, *y, *th;
+    const double *off_x, *off_t;  // delta_x2, delta_t2 (cpu_curvelet.hpp:697-698)
+    double dt, dx, dx2, close_thr, max_k;
+    int kt;
+};
+
+// One bound of a pair's bundle at one grid cell, exactly as
+// compute_curve_bundle leaves it (cpu_curvelet.hpp:636-819): lo, or hi with
+// `upper`.  Angles are below 2^20 here (fused_limits), so the sines need no
+// Payne-Hanek reduction.  (sa, ca) = sin/cos of theta_a, (s2, c2) of
+// T2t = theta_a + delta_t2; ox = delta_x2; b the neighbour.  The two branches
+// (:711-751, :774-806) differ in a factor of two on the curvature fraction and
+// in which of theta_n -+ dt bounds which side.
+__device__ inline double exact_bound(const ExactGrid &E, bool upper, double ax, double ay, double sa, double ca,
+                                     double T2t, double s2, double c2, double ox, int b)
+{
+    const double DX = ax - E.x[b], DY = ay - E.y[b], nt = E.th[b];
+    const double DX2 = DX * DX, DY2 = DY * DY;
+    double v = upper ? E.max_k : -E.max_k;
+    if (DX2 + DY2 < E.close_thr) return v;  // :682
+    const bool branch_a = (DX * ca + DY * sa) < 0;  // :690
+    const double tt = s2 * DX - c2 * DY;
+    const double ttm = tt - ox;
+    const double den = -2.0 * ox * tt + DX2 + DY2 - E.dx2 + ox * ox;
+    const double x = upper ? ttm + E.dx : ttm - E.dx;
+    const double kx = (branch_a ? 2.0 * x : x) / (branch_a ? den : den / 2.0);
+    const double T0 = branch_a == upper ? nt + E.dt : nt - E.dt;
+    double s0, c0;
+    cvg::cr_sincos<false>(T0, c_sincos_tab, &s0, &c0);
+    const double s = cvg::cr_sin<false>(T2t - T0, c_sincos_tab);  // :728-729
+    const double kt = s / (-s * ox + DX * c0 + DY * s0);
+    // the reference's compare-and-assign, which ignores NaN
+    if (upper) {
+        if (v > kx) v = kx;
+        if (v > kt) v = kt;
+    } else {
+        if (v < kx) v = kx;
+        if (v < kt) v = kt;
+    }
+    return v;
+}
+
+// Both bounds at the cell (ox, ot) of anchor a.  Out of line: the exact
+// kernel's few anchors spend their time on instruction fetch, and its callers
+// share this copy.
+__device__ __noinline__ double2 exact_bounds(ExactGrid E, double ax, double ay, double sa, double ca, double T2t,
+                                             double ox, int b)
+{
+    double s2, c2;
+    cvg::cr_sincos<false>(T2t, c_sincos_tab, &s2, &c2);
+    double2 r = make_double2(0.0, 0.0);
+#pragma unroll 1
+    for (int side = 0; side < 2; ++side) {
+        const double v = exact_bound(E, side != 0, ax, ay, sa, ca, T2t, s2, c2, ox, b);
+        r.x = side == 0 ? v : r.x;
+        r.y = side == 0 ? r.y : v;
+    }
+    return r;
+}
+
+// Per edge: (x, y, sin theta, cos theta), the correctly rounded pair.  Block 0
+// also clears the curvelet stage's counters (the graph stage's words are left
+// alone, so this may run before its last host read).
+__global__ __launch_bounds__(kBlock) void k_edge_rec(int n, const double *__restrict__ x, const double *__restrict__ y,
+                                                     const double *__restrict__ th, double4 *__restrict__ rec,
+                                                     unsigned *__restrict__ scal)
+{
+    if (blockIdx.x == 0) {
+        const int t = static_cast<int>(threadIdx.x);
+        if (t == 0) scal[S_VALID] = 0u;
+        if (t == 1) scal[S_COUNT] = 0u;
+        if (t == 2) scal[S_COUNT + 1] = 0u;
+        for (int w = kBucketBase + t; w < kScalarBufWords; w += static_cast<int>(blockDim.x)) scal[w] = 0u;
+    }
+    const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i >= n) return;
+    double s, c;
+    cvg::cr_sincos(th[i], c_sincos_tab, &s, &c);
+    rec[i] = make_double4(x[i], y[i], s, c);
+}
+
+// Anchors in spatial (cell) order in lists by falling degree: first those of
+// more than 64 neighbours (for k_curvelets_exact), then k_curvelets': its waves
+// take entries round robin over those concatenated lists, so each gets its
+// share of long and short anchors, and the kernel's tail consists of the
+// shortest.  The open list is k_curvelets' own.  Anchors without neighbours get
+// their zero count here.  Each entry carries (anchor, CSR base, degree).
+constexpr int kOrderBlock = 1024;  // few workgroups: one list-length atomic each per list
+enum { L_OPEN = 0, L_WIDE = 1, L_FIRST = 2, kLists = 6 };
+
+__device__ __forceinline__ int degree_list(unsigned deg)
+{
+    return deg > 64u ? L_WIDE : deg > 24u ? 2 : deg > 12u ? 3 : deg > 6u ? 4 : 5;
+}
+
+__global__ __launch_bounds__(kOrderBlock) void k_order(int n, const int *__restrict__ sorted,
+                                                       const unsigned *__restrict__ off, int4 *__restrict__ lists,
+                                                       unsigned *__restrict__ acc_count, unsigned *__restrict__ scal)
+{
+    __shared__ unsigned s_count[kLists];
+    __shared__ unsigned s_base[kLists];
+    // a guessed size that did not hold (this may run before the host knows):
+    // the graph is built again
+    if (scal[S_MISS] | scal[S_BAD]) return;
+    const int p = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+    const int lane = threadIdx.x & 63;
+    if (threadIdx.x < kLists) s_count[threadIdx.x] = 0;
+    __syncthreads();
+    int a = -1, b = -1;
+    unsigned o0 = 0, o1 = 0;
+    if (p < n) {
+        a = sorted[p];
+        o0 = off[a];
+        o1 = off[a + 1];
+        const unsigned deg = o1 - o0;
+        if (deg == 0)
+            acc_count[a] = 0u;
+        else
+            b = degree_list(deg);
+    }
+    // per wave and list: the group's leader reserves slots in the block's
+    // count, then one global atomic per block and list
+    unsigned my_off = 0;
+#pragma unroll
+    for (int k = 0; k < kLists; ++k) {
+        const unsigned long long grp = __ballot(b == k);
+        if (grp == 0ULL) continue;
+        const int leader = __ffsll(static_cast<long long>(grp)) - 1;
+        unsigned o = 0;
+        if (lane == leader) o = atomicAdd(&s_count[k], static_cast<unsigned>(__popcll(grp)));
+        o = __shfl(o, leader, 64);
+        if (b == k) my_off = o + static_cast<unsigned>(__popcll(grp & ((1ULL << lane) - 1ULL)));
+    }
+    __syncthreads();
+    if (threadIdx.x < kLists && s_count[threadIdx.x] > 0)
+        s_base[threadIdx.x] = atomicAdd(&scal[kBucketBase + threadIdx.x * kBucketStride], s_count[threadIdx.x]);
+    __syncthreads();
+    if (b >= 0)
+        lists[static_cast<long long>(b) * n + s_base[b] + my_off] =
+            make_int4(a, static_cast<int>(o0), static_cast<int>(o1 - o0), 0);
+}
+
+// Load from a wave-uniform address through the scalar data cache (read only).
+template <typename T>
+__device__ __forceinline__ T uload(const T *p)
+{
+    return *(const __attribute__((address_space(4))) T *)p;
+}
+
+// Fixed point: max_k is 2^30; conversions and differences saturate.  Two
+// approximate bounds whose difference is beyond kFixTol compare as the exact
+// ones do: each is off by at most 8 units from the formulas (fused_limits
+// keeps the denominators where that holds) and 1 from the conversion.
+constexpr int kFixOne = 1 << 30;
+constexpr int kFixTol = 18;
+
+// v_cvt_i32_f64: truncates and saturates (NaN gives 0), where the C++ cast is
+// undefined out of range.
+__device__ __forceinline__ int fix(double v)
+{
+    int r;
+    asm("v_cvt_i32_f64 %0, %1" : "=v"(r) : "v"(v));
+    return r;
+}
+
+__device__ __forceinline__ int sub_sat(int a, int b) { return __builtin_elementwise_sub_sat(a, b); }
+
+__device__ __forceinline__ unsigned long long perm64(int src_lane, unsigned long long v)
+{
+    const int lo = __builtin_amdgcn_ds_bpermute(src_lane << 2, static_cast<int>(v));
+    const int hi = __builtin_amdgcn_ds_bpermute(src_lane << 2, static_cast<int>(v >> 32));
+    return static_cast<unsigned long long>(static_cast<unsigned>(hi)) << 32 | static_cast<unsigned>(lo);
+}
+
+// v with lane `l` (uniform) replaced by the uniform value s.
+__device__ __forceinline__ unsigned long long set_lane64(unsigned long long v, unsigned long long s, int l)
+{
+    const unsigned lo = static_cast<unsigned>(
+        lane_write(static_cast<int>(s), l, static_cast<int>(v)));
+    const unsigned hi = static_cast<unsigned>(
+        lane_write(static_cast<int>(s >> 32), l, static_cast<int>(v >> 32)));
+    return static_cast<unsigned long long>(hi) << 32 | lo;
+}
+
+__device__ __forceinline__ unsigned long long get_lane64(unsigned long long v, int l)
+{
+    const unsigned lo = static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<int>(v), l));
+    const unsigned hi = static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<int>(v >> 32), l));
+    return static_cast<unsigned long long>(hi) << 32 | lo;
+}
+
+// Staged row of an accepted seed: the run's hypotheses as bits over the
+// anchor's neighbour list, the chain as bits over the hypotheses, and this
+// word: the best cell's rank, the direction, whether the masks have four words, and
+// the seed (a hypothesis; its bundle belongs to the running one even when the
+// chain filled up before its turn).  The record forms k_min and k_max.
+__host__ __device__ inline unsigned row_meta(int rank, bool fwd, bool wide, int seed)
+{
+    return static_cast<unsigned>(rank) | (fwd ? 1u << 8 : 0u) | (wide ? 1u << 9 : 0u) |
+           static_cast<unsigned>(seed) << 10;
+}
+
+struct FusedArgs {
+    const double4 *rec;  // per edge (x, y, sin, cos)
+    const double *th;
+    ExactGrid exact;
+    const int *ids;
+    int4 *lists;         // kLists x n entries (anchor, CSR base, degree, -)
+    unsigned *list_len;  // entry counts, kBucketStride words apart (device; k_order's, and the open list's)
+    int n;
+    int K, G;
+    // per cell in rank order: delta_x2, delta_t2, sin and cos of delta_t2,
+    // whether it can be a best cell
+    const double *rank_ox, *rank_ot, *rank_so, *rank_co;
+    const int *rank_elig;
+    int rank_of_cell0;
+    double sin_dt, cos_dt, dx, two_dx, dx2, close_thr, max_k;
+    double scale;                    // kFixOne / max_k
+    double min_den, num_err, den_err;  // fused_limits
+    double min_prod;                 // below it a product of the three denominators may have a small one
+    int slots;                       // bundle slots in LDS; a run's other bundles go to `spill`
+    int2 *spill;
+    size_t spill_stride;             // per wave
+    ulonglong2 *st_mask;             // (hypotheses, chain) per row
+    size_t mask_plane;               // entries between the 64-bit planes of st_mask
+    unsigned *st_meta;
+    unsigned *acc_count;
+    unsigned *partial;               // per wave: valid pairs, then two words of the intersection count
+};
+
+constexpr int kFusedWaves = 4;  // anchor streams (waves) per workgroup
+constexpr int kFusedWavesPerSimd = 4;
+constexpr int kFusedSlots = 14;  // bundle slots at one cell per lane
+constexpr int kPairBatch = 16;  // pair records in LDS at a time
+constexpr int kSmallRun = 8;    // runs up to here grow on cell masks
+
+struct SliceCarve {
+    int bun, rec, pm, bytes;
+};
+
+// One wave's LDS slice: bundle slots (lo, hi per lane), the pair records of
+// one batch (80 B each), and the mask matrix of a small run.
+__host__ __device__ inline SliceCarve slice_carve(int slots, int cpl)
+{
+    SliceCarve c{};
+    c.bun = 0;
+    c.rec = c.bun + slots * cpl * 64 * 8;
+    c.pm = c.rec + kPairBatch * 80;
+    c.bytes = c.pm + 64 * cpl * 8;
+    return c;
+}
+
+// A lane's cells: lanes without one repeat the first.
+template <int CPL>
+struct WaveCells {
+    double ox[CPL], m2ox[CPL], ox2[CPL], oxp[CPL], so[CPL], co[CPL];
+    unsigned long long emask[CPL];  // cells that can be a best one
+};
+
+// LDS and device memory, told apart by type: one pointer for both would make
+// every bundle access a flat one.
+template <typename T>
+using lds_ptr = __attribute__((address_space(3))) T *;
+template <typename T>
+using mem_ptr = __attribute__((address_space(1))) T *;
+
+// f(0), f(1), ... as constants, until one returns false.
+template <class F, int... I>
+__device__ __forceinline__ void each(F &f, std::integer_sequence<int, I...>)
+{
+    (void)(f(std::integral_constant<int, I>{}) && ...);
+}
+
+struct alignas(8) Bounds {
+    int lo, hi;
+};
+
+// One anchor on one wave.  EXACT = false returns true, with nothing counted,
+// when some comparison is closer than the approximate bounds can decide;
+// EXACT = true makes such comparisons on the exact bounds.
+//
+// Lane = neighbour forms the pairs' direction class, flags and
+// cell-independent terms (16 records in LDS at a time, in run order).  Then,
+// lane = bundle cell in "rank" order (cells sorted by (ox^2 + ot^2, index), so
+// that fill_curvelet_info's cell, cpu_curvelet.hpp:202-219, is the lowest
+// valid one; CPL cells per lane), each run's bundles: forward neighbours,
+// backward, neither (validity only, for the count).  A valid (or close) pair
+// is a hypothesis and takes the next slot; its cells with hi <= lo are stored
+// as (largest, smallest), so that they compare as invalid from then on.
+//
+// Growth.  A chain's running bundle is max lo, min hi over its members, so it
+// is valid at a cell exactly where every member's lo lies below every member's
+// hi.  For a run of up to 8 hypotheses one 64-bit mask per pair of them says
+// at which cells that holds; the seeds' chains then grow together, lane
+// (j, h) holding the cells where seed j's chain and hypothesis h are
+// compatible: step h is one ballot and two ANDs for all seeds at once.  (A
+// step per seed and hypothesis, lane = cell, is a chain of LDS reads,
+// compares, ballots and branches: 34% of the kernel's wave time before.)
+// Longer runs walk seed by seed.
+//
+// Rows.  Chains are sets of slots, so equal chains are equal masks
+// (check_curvelet_exist, :876-916: the first of equal chains is kept).  The
+// best cell is the lowest eligible bit of the seed's final mask.  k_min and
+// k_max are left to the record, where a lane has a row of its own.
+//
+// NW: 64-bit words of a slot or neighbour mask (64 NW neighbours at most).
+template <int CPL, int NW, bool EXACT>
+__device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CPL> &W, char *sl, int2 *spill, int a,
+                                          unsigned base, int deg, const double4 nb, unsigned &vp_sum,
+                                          unsigned long long &isect_sum)
+{
+    typedef unsigned long long u64;
+    constexpr int NC = NW;  // 64-seed (64-neighbour) chunks
+    const int lane = threadIdx.x & 63;
+    const int G = A.G;
+    const int slots = A.slots;
+    const SliceCarve cv = slice_carve(A.slots, CPL);
+    const lds_ptr<Bounds> bun = (lds_ptr<Bounds>)(sl + cv.bun) + lane;
+    const lds_ptr<double2> rec = (lds_ptr<double2>)(sl + cv.rec);
+    const lds_ptr<u64> pm = (lds_ptr<u64>)(sl + cv.pm);
+    const mem_ptr<Bounds> spl = (mem_ptr<Bounds>)spill + lane;
+    auto get_bundle = [&](int s, int m) -> Bounds {
+        Bounds v;
+        if (s < slots) {
+            v.lo = bun[(s * CPL + m) * 64].lo;
+            v.hi = bun[(s * CPL + m) * 64].hi;
+        } else {
+            v.lo = spl[((s - slots) * CPL + m) * 64].lo;
+            v.hi = spl[((s - slots) * CPL + m) * 64].hi;
+        }
+        return v;
+    };
+    auto load_rec = [&](int c) -> double4 {  // neighbours 64 c + lane
+        double4 v = make_double4(0.0, 0.0, 0.0, 1.0);
+        if (64 * c + lane < deg) v = A.rec[A.ids[base + 64 * c + lane]];
+        return v;
+    };
+    // Each comparison's t = hi - lo: true above kFixTol, false below -kFixTol,
+    // and in between open.  Not EXACT: a lane's smallest t + kFixTol, as
+    // unsigned, says at the end whether any of its comparisons was open.
+    unsigned closest = ~0u;
+    auto note = [&](int t) { closest = min(closest, static_cast<unsigned>(t + kFixTol)); };
+    auto is_open = [&](int t) -> u64 {
+        return __builtin_amdgcn_ballot_w64(static_cast<unsigned>(t + kFixTol) <= 2u * kFixTol);
+    };
+    u64 open = 0ULL;
+
+    const double *ar = reinterpret_cast<const double *>(A.rec + a);
+    const double ax = uload(ar), ay = uload(ar + 1), sa = uload(ar + 2), ca = uload(ar + 3);
+    // sin/cos of theta_a + delta_t2 by rotation
+    double sT[CPL], cT[CPL];
+#pragma unroll
+    for (int m = 0; m < CPL; ++m) {
+        sT[m] = __builtin_fma(sa, W.co[m], ca * W.so[m]);
+        cT[m] = __builtin_fma(ca, W.co[m], -(sa * W.so[m]));
+    }
+
+    // EXACT: the exact bounds of neighbour b at this lane's cell of group m
+    auto exact_cell = [&](int m, int b, double &lo, double &hi) {
+        const int rho = lane + 64 * m < A.K ? lane + 64 * m : 0;
+        const double2 v = exact_bounds(A.exact, ax, ay, sa, ca, A.th[a] + A.rank_ot[rho], A.rank_ox[rho], b);
+        lo = v.x;
+        hi = v.y;
+    };
+
+    // direction classes (:459-461), lane = neighbour; a neighbour's place in
+    // run order (forward, backward, neither; CSR order within)
+    int pos[NC];
+    u64 closep[NC];  // close pairs, as bits over the places
+    int n1 = 0, n2 = 0;
+    {
+        int cls[NC];
+        bool cl[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            cls[c] = 3;
+            cl[c] = false;
+            if (NC > 1 && 64 * c >= deg) continue;
+            const double4 q = c > 0 ? load_rec(c) : nb;
+            const bool in = 64 * c + lane < deg;
+            const double vx = q.x - ax, vy = q.y - ay;
+            cl[c] = in && vx * vx + vy * vy < A.close_thr;  // :682 (DX^2 + DY^2, the same squares)
+            int k;
+            if constexpr (EXACT) {
+                k = in ? cvg::direction_class(ax, ay, ca, sa, q.x, q.y, c_sincos_tab, c_atan_tab) : 3;
+            } else {
+                // (direction_class's projection and a bound at least as strict)
+                const double p = vx * ca + vy * sa;
+                open |= __ballot(in && !(fabs(p) > 1e-12 * (fabs(vx) + fabs(vy))));
+                k = p > 0 ? 1 : 2;
+            }
+            cls[c] = in ? k : 3;
+            n1 += __popcll(__ballot(cls[c] == 1));
+            if (EXACT) n2 += __popcll(__ballot(cls[c] == 2));
+        }
+        if (!EXACT) n2 = deg - n1;
+        int b1 = 0, b2 = n1, b0 = n1 + n2;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            auto below = [&](u64 m) {
+                return static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                    static_cast<unsigned>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m), 0u)));
+            };
+            const u64 m1 = __ballot(cls[c] == 1);
+            if constexpr (EXACT) {
+                const u64 m2 = __ballot(cls[c] == 2), m0 = __ballot(cls[c] == 0);
+                pos[c] = cls[c] == 1 ? b1 + below(m1) : cls[c] == 2 ? b2 + below(m2) : b0 + below(m0);
+                b2 += __popcll(m2);
+                b0 += __popcll(m0);
+            } else {
+                const int f = below(m1);  // (no third class without exact directions)
+                pos[c] = cls[c] == 1 ? b1 + f : b2 + lane - f;
+                b2 += 64 - __popcll(m1);
+            }
+            pos[c] = cls[c] == 3 ? -1 : pos[c];
+            b1 += __popcll(m1);
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c) closep[c] = 0ULL;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            for (u64 m = __ballot(cl[c]); m != 0ULL; m &= m - 1ULL) {  // (few: within 2 dx)
+                const int at = __builtin_amdgcn_readlane(pos[c], __builtin_ctzll(m));
+#pragma unroll
+                for (int w = 0; w < NC; ++w)
+                    if (NC == 1 || (at >> 6) == w) closep[w] |= 1ULL << (at & 63);
+            }
+    }
+
+    // the pair records of batch b (places 16 b .. 16 b + 15) into LDS: DX, DY,
+    // DX^2 + DY^2 - dx^2, and for the lower and the upper orientation
+    // constraint (theta_n -+ dt, by branch, :736, :799) the sine and cosine of
+    // the angle and DX cos + DY sin
+    auto fill_batch = [&](int b) {
+        wave_sync();  // the last batch's reads are done
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            if (NC > 1 && 64 * c >= deg) continue;
+            const double4 q = c > 0 ? load_rec(c) : nb;
+            const double DX = ax - q.x, DY = ay - q.y;
+            const bool branch_a = (DX * ca + DY * sa) < 0;  // :690
+            const double sd = branch_a ? -A.sin_dt : A.sin_dt;
+            const double s0 = __builtin_fma(q.z, A.cos_dt, q.w * sd), c0 = __builtin_fma(q.w, A.cos_dt, -(q.z * sd));
+            const double s1 = __builtin_fma(q.z, A.cos_dt, -(q.w * sd)), c1 = __builtin_fma(q.w, A.cos_dt, q.z * sd);
+            if (pos[c] >= 0 && (pos[c] >> 4) == b) {
+                const lds_ptr<double2> o = rec + (pos[c] & 15) * 5;
+                o[0].x = DX;
+                o[0].y = DY;
+                o[1].x = __builtin_fma(DX, DX, __builtin_fma(DY, DY, -A.dx2));
+                o[1].y = __builtin_fma(DX, c0, DY * s0);
+                o[2].x = __builtin_fma(DX, c1, DY * s1);
+                o[2].y = s0;
+                o[3].x = c0;
+                o[3].y = s1;
+                o[4].x = c1;
+            }
+        }
+        wave_sync();
+    };
+
+    // EXACT: the edge at place p
+    auto neighbour = [&](int p) -> int {
+        int r = 0;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const u64 m = __ballot(pos[c] == p);
+            if (m != 0ULL) r = 64 * c + __builtin_ctzll(m);
+        }
+        return A.ids[base + r];
+    };
+
+    int batch = -1;
+    unsigned nacc = 0, vp = 0, isect_u = 0;  // isect_u: the wave's, isect: the lane's
+    unsigned isect = 0;
+    for (int run = 0; run < (EXACT ? 3 : 2); ++run) {
+        const int p0 = run == 0 ? 0 : (run == 1 ? n1 : n1 + n2);
+        const int p1 = run == 0 ? n1 : (run == 1 ? n1 + n2 : deg);
+        int R = 0;      // hypotheses of the run
+        u64 place[NW];  // as bits over the places
+#pragma unroll
+        for (int w = 0; w < NW; ++w) place[w] = 0ULL;
+
+        // the run's bundles (compute_curve_bundle, :636-819)
+        lds_ptr<Bounds> bp = bun;  // the next slot
+        for (int p = p0; p < p1;) {
+            if ((p >> 4) != batch) {
+                batch = p >> 4;
+                fill_batch(batch);
+            }
+            const int pe = min(p1, (p | 15) + 1);
+            lds_ptr<double2> q = rec + (p & 15) * 5;
+            for (; p < pe; ++p, q += 5) {
+                bool close = false;
+#pragma unroll
+                for (int c = 0; c < NC; ++c)
+                    if (NC == 1 || (p >> 6) == c) close = (closep[c] >> (p & 63)) & 1ULL;
+                Bounds v[CPL];
+                if (close) {
+                    // the default bundle [-max_k, max_k]
+#pragma unroll
+                    for (int m = 0; m < CPL; ++m) {
+                        v[m].lo = -kFixOne;
+                        v[m].hi = kFixOne;
+                    }
+                } else {
+                    const double DX = q[0].x, DY = q[0].y, r2 = q[1].x, C0 = q[1].y, C1 = q[2].x;
+                    const double s0n = q[2].y, c0n = q[3].x, s1n = q[3].y, c1n = q[4].x;
+                    u64 any = 0ULL;  // cells with hi > lo
+#pragma unroll
+                    for (int m = 0; m < CPL; ++m) {
+                        const double tt = __builtin_fma(sT[m], DX, -(cT[m] * DY));
+                        const double den = __builtin_fma(W.m2ox[m], tt, r2 + W.ox2[m]);
+                        const double x0 = tt - W.oxp[m];  // half of :712's numerator
+                        const double s0 = __builtin_fma(sT[m], c0n, -(cT[m] * s0n));
+                        const double s1 = __builtin_fma(sT[m], c1n, -(cT[m] * s1n));
+                        const double d0 = __builtin_fma(-s0, W.ox[m], C0);
+                        const double d1 = __builtin_fma(-s1, W.ox[m], C1);
+                        // 1 / den, 1 / d0 and 1 / d1 (times scale) from one reciprocal
+                        const double pp = den * d0, ppp = pp * d1;
+                        double y = __builtin_amdgcn_rcp(ppp);
+                        y = __builtin_fma(y, __builtin_fma(-ppp, y, 1.0), y);
+                        y *= A.scale;
+                        const double yd1 = y * pp, w = y * d1;
+                        const double yd0 = w * den, yx = w * (d0 + d0);
+                        const double k0 = x0 * yx, k1 = __builtin_fma(A.two_dx, yx, k0);
+                        int lo = max(fix(k0), fix(s0 * yd0));
+                        int hi = min(fix(k1), fix(s1 * yd1));
+                        const int t = min(sub_sat(hi, lo), min(sub_sat(hi, -kFixOne), sub_sat(kFixOne, lo)));
+                        if (!EXACT) note(t);
+                        bool ok = t > kFixTol;
+                        u64 T = __builtin_amdgcn_ballot_w64(ok);
+                        u64 U = EXACT ? is_open(t) : 0ULL;
+                        // a small denominator (then the product is small as well)
+                        // settles nothing unless its sign is certain and its
+                        // quotients lie well beyond max_k, where they stay either way
+                        if (__builtin_amdgcn_ballot_w64(!(fabs(ppp) >= A.min_prod)) != 0ULL) {
+                            auto weak = [&](double n, double d) {
+                                return !(fabs(d) >= A.min_den) &&
+                                       !(fabs(d) > A.den_err && fabs(n) > 4.0 * A.max_k * fabs(d) + A.num_err);
+                            };
+                            const bool bad = weak(2.0 * x0, den) || weak(2.0 * x0 + 2.0 * A.two_dx, den) ||
+                                             weak(s0, d0) || weak(s1, d1);
+                            if (EXACT)
+                                U |= __builtin_amdgcn_ballot_w64(bad);
+                            else
+                                closest = bad ? 0u : closest;
+                        }
+                        if constexpr (EXACT) {
+                            if (U != 0ULL) {
+                                const int b = neighbour(p);
+                                bool valid = false;
+                                if (__builtin_amdgcn_inverse_ballot_w64(U)) {
+                                    double elo = 0.0, ehi = 0.0;
+                                    exact_cell(m, b, elo, ehi);
+                                    valid = ehi > elo;
+                                    lo = fix(elo * A.scale);
+                                    hi = max(fix(ehi * A.scale), lo + 1);
+                                }
+                                T = (T & ~U) | __ballot(valid);
+                                ok = __builtin_amdgcn_inverse_ballot_w64(T);
+                            }
+                        }
+                        v[m].lo = ok ? lo : INT_MAX;
+                        v[m].hi = ok ? hi : INT_MIN;
+                        any |= T;
+                    }
+                    if (any == 0ULL) continue;  // bundle_valid_check, :821-830
+                }
+                ++vp;
+                if (EXACT && run == 2) continue;
+                if (R < slots) {
+#pragma unroll
+                    for (int m = 0; m < CPL; ++m) {
+                        bp[m * 64].lo = v[m].lo;
+                        bp[m * 64].hi = v[m].hi;
+                    }
+                    bp += CPL * 64;
+                } else {
+#pragma unroll
+                    for (int m = 0; m < CPL; ++m) {
+                        spl[((R - slots) * CPL + m) * 64].lo = v[m].lo;
+                        spl[((R - slots) * CPL + m) * 64].hi = v[m].hi;
+                    }
+                }
+#pragma unroll
+                for (int w = 0; w < NW; ++w)
+                    if (NW == 1 || (p >> 6) == w) place[w] |= 1ULL << (p & 63);
+                ++R;
+            }
+        }
+        // a chain longer than 2 takes two hypotheses and G >= 3
+        if ((EXACT && run == 2) || R < 2 || G < 3) continue;
+
+        u64 hyp[NW];  // the run's hypotheses as bits over the neighbour list
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            u64 word = place[0];
+#pragma unroll
+            for (int w = 1; w < NW; ++w)
+                if ((pos[c] >> 6) == w) word = place[w];
+            hyp[c] = __builtin_amdgcn_ballot_w64(pos[c] >= 0 && ((word >> (pos[c] & 63)) & 1ULL) != 0ULL);
+        }
+        // EXACT: whether the running bundle of the slots in `set` is valid, in
+        // the lanes U of cell group m
+        auto exact_run = [&](int m, u64 U, const u64 (&set)[NW]) -> u64 {
+            double lo = 0.0, hi = 0.0;
+            bool begun = false;
+            int s = 0;
+#pragma unroll 1
+            for (int p = p0; p < p1; ++p) {
+                u64 word = place[0], in = set[0];
+#pragma unroll
+                for (int w = 1; w < NW; ++w) {
+                    word = (p >> 6) == w ? place[w] : word;
+                    in = (s >> 6) == w ? set[w] : in;
+                }
+                if (!((word >> (p & 63)) & 1ULL)) continue;
+                const bool member = (in >> (s & 63)) & 1ULL;
+                ++s;
+                if (!member) continue;
+                const int b = neighbour(p);
+                if (__builtin_amdgcn_inverse_ballot_w64(U)) {
+                    double elo = 0.0, ehi = 0.0;
+                    exact_cell(m, b, elo, ehi);
+                    lo = !begun || lo < elo ? elo : lo;
+                    hi = !begun || hi > ehi ? ehi : hi;
+                }
+                begun = true;
+            }
+            return __ballot(hi > lo) & U;
+        };
+        auto put_row = [&](unsigned rank, const u64 (&chain)[NW], int best, int seed) {
+            const size_t q = static_cast<size_t>(base) + rank;
+#pragma unroll
+            for (int w = 0; w < NW; ++w)
+                if (w == 0 || deg > 64) {
+                    const mem_ptr<ulonglong2> o = (mem_ptr<ulonglong2>)A.st_mask + w * A.mask_plane + q;
+                    o->x = hyp[w];
+                    o->y = chain[w];
+                }
+            ((mem_ptr<unsigned>)A.st_meta)[q] = row_meta(best, run == 0, deg > 64, seed);
+        };
+        auto best_cell = [&](const u64 (&valid)[CPL]) -> int {  // fill_curvelet_info, :202-226
+            int best = -1;
+#pragma unroll
+            for (int m = 0; m < CPL; ++m) {
+                const u64 e = valid[m] & W.emask[m];
+                if (best < 0 && e != 0ULL) best = 64 * m + __builtin_ctzll(e);
+            }
+            return best < 0 ? A.rank_of_cell0 : best;
+        };
+        auto rank_of = [&](u64 acc) -> unsigned {
+            return nacc + static_cast<unsigned>(__builtin_amdgcn_mbcnt_hi(
+                              static_cast<unsigned>(acc >> 32),
+                              __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(acc), 0u)));
+        };
+
+        if (R <= kSmallRun) {
+            // the compatibility masks of every two slots: lane 8 i + k, the
+            // cells where slots i and k are valid together
+            Bounds b[kSmallRun][CPL];
+            u64 P[CPL];
+            u64 redo = 0ULL;  // EXACT: bit 8 i + k: the pair has an open cell
+#pragma unroll
+            for (int i = 0; i < kSmallRun; ++i)
+#pragma unroll
+                for (int m = 0; m < CPL; ++m) {  // (slots >= kSmallRun)
+                    b[i][m].lo = bun[(i * CPL + m) * 64].lo;
+                    b[i][m].hi = bun[(i * CPL + m) * 64].hi;
+                }
+#pragma unroll
+            for (int m = 0; m < CPL; ++m) P[m] = 0ULL;
+#pragma unroll
+            for (int i = 0; i < kSmallRun; ++i) {
+                if (i >= R) break;
+#pragma unroll
+                for (int m = 0; m < CPL; ++m)
+                    P[m] = set_lane64(P[m], __builtin_amdgcn_ballot_w64(b[i][m].hi > b[i][m].lo), 9 * i);
+#pragma unroll
+                for (int k = 0; k < i; ++k) {
+#pragma unroll
+                    for (int m = 0; m < CPL; ++m) {
+                        const int t = min(sub_sat(b[k][m].hi, b[i][m].lo), sub_sat(b[i][m].hi, b[k][m].lo));
+                        if (EXACT)
+                            redo |= is_open(t) != 0ULL ? 1ULL << (8 * i + k) : 0ULL;
+                        else
+                            note(t);
+                        P[m] = set_lane64(P[m], __builtin_amdgcn_ballot_w64(t > kFixTol), 8 * i + k);
+                    }
+                }
+            }
+            if constexpr (EXACT) {
+                for (; redo != 0ULL; redo &= redo - 1ULL) {
+                    const int ik = __builtin_ctzll(redo), i = ik >> 3, k = ik & 7;
+                    u64 set[NW];
+#pragma unroll
+                    for (int w = 0; w < NW; ++w) set[w] = w == 0 ? 1ULL << i | 1ULL << k : 0ULL;
+#pragma unroll
+                    for (int m = 0; m < CPL; ++m) {
+                        const Bounds bi = get_bundle(i, m), bk = get_bundle(k, m);
+                        const int t = min(sub_sat(bk.hi, bi.lo), sub_sat(bi.hi, bk.lo));
+                        const u64 U = is_open(t);
+                        if (U != 0ULL)
+                            P[m] = set_lane64(P[m], (__builtin_amdgcn_ballot_w64(t > kFixTol) & ~U) | exact_run(m, U, set),
+                                              ik);
+                    }
+                }
+            }
+            // the upper triangle, and the rows in LDS
+            u64 C[CPL];
+            wave_sync();  // (the last matrix's reads are done)
+#pragma unroll
+            for (int m = 0; m < CPL; ++m) {
+                C[m] = P[m] | perm64((lane & 7) << 3 | lane >> 3, P[m]);
+                pm[m * 64 + lane] = C[m];
+            }
+            wave_sync();
+            // growth (:479-536): step h offers slot h to every seed's chain.
+            // Lane (j, h'): C = the cells where seed j's running bundle and
+            // slot h' are valid together; taking h leaves of them those where
+            // h is valid with the chain and with h'.
+            const bool limited = R > G - 1;  // a chain can fill up
+            const u64 ones = 0x0101010101010101ULL;
+            u64 count = 0ULL, stop = 0ULL;  // per seed, one byte each
+            u64 chain = 0ULL;               // byte j: seed j's chain, as slots
+            auto step = [&](auto slot) -> bool {
+                constexpr int h = decltype(slot)::value;
+                if (h >= R) return false;
+                u64 nz = 0ULL;
+#pragma unroll
+                for (int m = 0; m < CPL; ++m) nz |= C[m];
+                const u64 okb = __builtin_amdgcn_ballot_w64(
+                    (static_cast<unsigned>(nz) | static_cast<unsigned>(nz >> 32)) != 0u);
+                // the seed joins at its own distance rank (:496-510)
+                u64 rows = ((okb >> h) & ones) | 1ULL << (8 * h);
+                if (limited) rows &= ~stop;
+                const bool take = __builtin_amdgcn_inverse_ballot_w64((rows << 8) - rows);
+#pragma unroll
+                for (int m = 0; m < CPL; ++m) {
+                    // (lane & 56) | h's value: ds_swizzle, within 8 lanes
+                    const unsigned lo = static_cast<unsigned>(
+                        __builtin_amdgcn_ds_swizzle(static_cast<int>(C[m]), h << 5 | 0x18));
+                    const unsigned hi = static_cast<unsigned>(
+                        __builtin_amdgcn_ds_swizzle(static_cast<int>(C[m] >> 32), h << 5 | 0x18));
+                    const u64 n = C[m] & (static_cast<u64>(hi) << 32 | lo) & pm[m * 64 + 8 * h + (lane & 7)];
+                    C[m] = take ? n : C[m];
+                }
+                chain |= rows << h;
+                if (limited) {
+                    count += rows;
+                    stop = ((count + (128ULL - static_cast<u64>(G - 1)) * ones) >> 7) & ones;
+                }
+                return true;
+            };
+            each(step, std::make_integer_sequence<int, kSmallRun>{});
+            // rows, lane 9 j = seed j: kept with more than 2 edges (:549) and
+            // no earlier seed with the same chain (lane 8 j + k compares j's
+            // with k's)
+            const int j = lane >> 3, k = lane & 7;
+            const unsigned cj = static_cast<unsigned>(chain >> (lane & 56)) & 0xffu;
+            const unsigned ck = static_cast<unsigned>(chain >> (8 * k)) & 0xffu;
+            const u64 dup = __builtin_amdgcn_ballot_w64(cj == ck && k < j);
+            const int members = __popc(cj);
+            if (!limited) {
+                isect_u += static_cast<unsigned>(R * (R - 1));  // every seed meets every other hypothesis
+            } else if (j == k && j < R) {
+                // the slots the reference's loop visits, without the seed's own step
+                const int visited = members + 1 >= G ? 32 - __clz(static_cast<int>(cj)) : R;
+                isect += static_cast<unsigned>(visited - (j < visited ? 1 : 0));
+            }
+            const bool keep = j == k && j < R && members >= 2 && ((dup >> (lane & 56)) & 0xffULL) == 0ULL;
+            const u64 acc = __builtin_amdgcn_ballot_w64(keep);
+            if (keep) {
+                u64 row[NW];
+#pragma unroll
+                for (int w = 0; w < NW; ++w) row[w] = w == 0 ? static_cast<u64>(cj) : 0ULL;
+                put_row(rank_of(acc), row, best_cell(C), j);
+            }
+            nacc += static_cast<unsigned>(__popcll(acc));
+            continue;
+        }
+
+        // longer runs: seed by seed, lane = cell: the running bundle over the
+        // hypotheses in CSR order
+        u64 sm[NC][NW];   // lane = seed (of chunk c): the chain's slots
+        u64 sM[NC][CPL];  // and the running bundle's valid cells
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+#pragma unroll
+            for (int w = 0; w < NW; ++w) sm[c][w] = 0ULL;
+#pragma unroll
+            for (int m = 0; m < CPL; ++m) sM[c][m] = 0ULL;
+        }
+        for (int j = 0; j < R; ++j) {
+            Bounds cur[CPL], nx[CPL];
+#pragma unroll
+            for (int m = 0; m < CPL; ++m) {
+                // (clamped at -+max_k)
+                cur[m] = get_bundle(j, m);
+                cur[m].lo = max(cur[m].lo, -kFixOne);
+                cur[m].hi = min(cur[m].hi, kFixOne);
+                nx[m] = get_bundle(0, m);
+            }
+            u64 S[NW];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) S[w] = 0ULL;
+            int len = 1, h = 0;
+            for (; h < R && len < G; ++h) {
+                Bounds n[CPL];
+                u64 T = 0ULL;
+#pragma unroll
+                for (int m = 0; m < CPL; ++m) {
+                    n[m].lo = max(cur[m].lo, nx[m].lo);
+                    n[m].hi = min(cur[m].hi, nx[m].hi);
+                    T |= __builtin_amdgcn_ballot_w64(sub_sat(n[m].hi, n[m].lo) > kFixTol);
+                }
+                const int hn = h + 1 < R ? h + 1 : h;
+#pragma unroll
+                for (int m = 0; m < CPL; ++m) nx[m] = get_bundle(hn, m);
+                if (T == 0ULL && h != j) {
+                    // (a step with a certainly valid cell is settled by it)
+                    if constexpr (EXACT) {
+                        u64 set[NW];
+#pragma unroll
+                        for (int w = 0; w < NW; ++w)
+                            set[w] = S[w] | ((h >> 6) == w ? 1ULL << (h & 63) : 0ULL) |
+                                     ((j >> 6) == w ? 1ULL << (j & 63) : 0ULL);
+#pragma unroll
+                        for (int m = 0; m < CPL; ++m) {
+                            const u64 U = is_open(sub_sat(n[m].hi, n[m].lo));
+                            if (U != 0ULL) T |= exact_run(m, U, set);
+                        }
+                    } else {
+#pragma unroll
+                        for (int m = 0; m < CPL; ++m) note(sub_sat(n[m].hi, n[m].lo));
+                    }
+                }
+                if (h == j || T != 0ULL) {
+#pragma unroll
+                    for (int m = 0; m < CPL; ++m) cur[m] = n[m];
+#pragma unroll
+                    for (int w = 0; w < NW; ++w)
+                        if (NW == 1 || (h >> 6) == w) S[w] |= 1ULL << (h & 63);
+                    ++len;
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < CPL; ++m) {
+                const int t = sub_sat(cur[m].hi, cur[m].lo);
+                u64 T = __builtin_amdgcn_ballot_w64(t > kFixTol);
+                if constexpr (EXACT) {
+                    const u64 U = is_open(t);
+                    if (U != 0ULL) {
+                        u64 set[NW];
+#pragma unroll
+                        for (int w = 0; w < NW; ++w) set[w] = S[w] | ((j >> 6) == w ? 1ULL << (j & 63) : 0ULL);
+                        T = (T & ~U) | exact_run(m, U, set);
+                    }
+                } else {
+                    note(t);
+                }
+#pragma unroll
+                for (int c = 0; c < NC; ++c)
+                    if (NC == 1 || (j >> 6) == c) sM[c][m] = set_lane64(sM[c][m], T, j & 63);
+            }
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int w = 0; w < NW; ++w)
+                    if (NC == 1 || (j >> 6) == c) sm[c][w] = set_lane64(sm[c][w], S[w], j & 63);
+        }
+        // rows, lane = seed (as above)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            if (NC > 1 && 64 * c >= R) break;
+            const int j = 64 * c + lane;
+            const bool in = j < R;
+            int members = 0, top = -1;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                members += __popcll(sm[c][w]);
+                if (sm[c][w] != 0ULL) top = 64 * w + 63 - __clzll(static_cast<long long>(sm[c][w]));
+            }
+            if (in) {
+                const int visited = members + 1 >= G ? top + 1 : R;
+                isect += static_cast<unsigned>(visited - (j < visited ? 1 : 0));
+            }
+            u64 acc = __builtin_amdgcn_ballot_w64(in && members >= 2);
+#pragma unroll
+            for (int cc = 0; cc <= c; ++cc) {
+                const int kend = min(64, R - 64 * cc);
+                for (int k = 0; k < kend; ++k) {
+                    u64 same = cc < c ? ~0ULL : ~1ULL << k;  // the later seeds
+#pragma unroll
+                    for (int w = 0; w < NW; ++w)
+                        same &= __builtin_amdgcn_ballot_w64(get_lane64(sm[cc][w], k) == sm[c][w]);
+                    acc &= ~same;
+                }
+            }
+            if (__builtin_amdgcn_inverse_ballot_w64(acc)) put_row(rank_of(acc), sm[c], best_cell(sM[c]), j);
+            nacc += static_cast<unsigned>(__popcll(acc));
+        }
+    }
+    if (!EXACT && (open | __builtin_amdgcn_ballot_w64(closest <= 2u * kFixTol)) != 0ULL) return true;
+    if (lane == 0) ((mem_ptr<unsigned>)A.acc_count)[a] = nacc;
+    vp_sum += vp;
+    isect_sum += isect + (lane == 0 ? isect_u : 0u);
+    return false;
+}
+
+// One wave's sums into its place (k_row_anchors adds the places up).
+__device__ __forceinline__ void put_sums(unsigned *partial, int g, unsigned vp, unsigned long long isect)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+        isect += static_cast<unsigned long long>(__shfl_xor(static_cast<long long>(isect), o, 64));
+    if ((threadIdx.x & 63) == 0) {
+        partial[3 * g] = vp;
+        partial[3 * g + 1] = static_cast<unsigned>(isect);
+        partial[3 * g + 2] = static_cast<unsigned>(isect >> 32);
+    }
+}
+
+template <int CPL>
+__device__ __forceinline__ WaveCells<CPL> wave_cells(const FusedArgs &A)
+{
+    WaveCells<CPL> W;
+#pragma unroll
+    for (int m = 0; m < CPL; ++m) {
+        const int rho = static_cast<int>(threadIdx.x & 63) + 64 * m;
+        const bool live = rho < A.K;
+        const int r = live ? rho : 0;
+        W.ox[m] = A.rank_ox[r];
+        W.m2ox[m] = -2.0 * W.ox[m];
+        W.ox2[m] = W.ox[m] * W.ox[m];
+        W.oxp[m] = W.ox[m] + A.dx;
+        W.so[m] = A.rank_so[r];
+        W.co[m] = A.rank_co[r];
+        W.emask[m] = __ballot(live && A.rank_elig[r] != 0);
+    }
+    return W;
+}
+
+__device__ __forceinline__ void load_entry(const int4 *p, int &a, unsigned &base, int &deg)
+{
+    const int *e = reinterpret_cast<const int *>(p);
+    a = uload(e);
+    base = static_cast<unsigned>(uload(e + 1));
+    deg = uload(e + 2);
+}
+
+// build_curvelets_greedy (cpu_curvelet.hpp:437-591) plus the
+// form_pairwise_bundles valid-pair count (:305-361), in one pass, for anchors
+// of up to 64 neighbours.
+//
+// Persistent: one wave per anchor (do_anchor), wave g takes entries g,
+// g + waves, ... of the concatenated lists.  The neighbours' records of the
+// next anchor, the ids of the one after it and the list entry of the third are
+// in flight while an anchor is worked on.  Bound by instruction issue: the
+// SIMDs issue about one instruction of any kind per four cycles from start to
+// end (counters; 820 vector, 490 scalar and 90 LDS instructions an anchor), and
+// waves that take entries from a shared counter instead of a fixed share end
+// together but no sooner (741 us against 724 at the time).  Anchors with a comparison too close
+// for the approximate bounds go to the open list.  (Done again here, their
+// code costs the main loop its registers: 1,272 us against 720 on the 1080p
+// map.)
+template <int CPL>
+__global__ __launch_bounds__(64 * kFusedWaves, CPL == 1 ? kFusedWavesPerSimd + 1 : kFusedWavesPerSimd)
+void k_curvelets(FusedArgs A)
+{
+    extern __shared__ double lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int g = static_cast<int>(blockIdx.x) * kFusedWaves + wave;
+    const int streams = static_cast<int>(gridDim.x) * kFusedWaves;
+    unsigned vp = 0;               // valid or close pairs of this wave's anchors
+    unsigned long long isect = 0;  // bundle intersections the reference tests (per lane)
+    char *sl = reinterpret_cast<char *>(lds) + static_cast<size_t>(wave) * slice_carve(A.slots, CPL).bytes;
+    int2 *spill = A.spill + static_cast<size_t>(g) * A.spill_stride;
+    const WaveCells<CPL> W = wave_cells<CPL>(A);
+
+    // the wave's entries: a cursor into the current list
+    int list = L_FIRST - 1, left = 0, at = g;
+    auto next = [&](int &ea, unsigned &eb, int &ed) {
+        ed = -1;
+        while (at >= left) {
+            at -= left;
+            if (list == kLists - 1) return;
+            ++list;
+            left = static_cast<int>(uload(A.list_len + list * kBucketStride));
+        }
+        load_entry(A.lists + static_cast<size_t>(list) * A.n + at, ea, eb, ed);
+        at += streams;
+    };
+    auto load_id = [&](unsigned b0, int d0) -> int { return lane < d0 ? A.ids[b0 + lane] : -1; };
+    auto load_rec = [&](int id) -> double4 {
+        double4 v = make_double4(0.0, 0.0, 0.0, 1.0);
+        if (id >= 0) v = A.rec[id];
+        return v;
+    };
+    int a = 0, deg, na = 0, ndeg = -1;
+    unsigned base = 0, nbase = 0;
+    next(a, base, deg);
+    double4 nb = load_rec(load_id(base, deg));
+    if (deg >= 0) next(na, nbase, ndeg);
+    int nid = load_id(nbase, ndeg);
+    while (deg >= 0) {
+        // start the next anchor's loads
+        const double4 nnb = load_rec(nid);
+        int nna = 0, nndeg = -1;
+        unsigned nnbase = 0;
+        if (ndeg >= 0) next(nna, nnbase, nndeg);
+        const int nnid = load_id(nnbase, nndeg);
+        if (do_anchor<CPL, 1, false>(A, W, sl, spill, a, base, deg, nb, vp, isect)) {
+            if (lane == 0)
+                A.lists[static_cast<size_t>(L_OPEN) * A.n + atomicAdd(A.list_len + L_OPEN * kBucketStride, 1u)] =
+                    make_int4(a, static_cast<int>(base), deg, 0);
+        }
+        a = na;
+        base = nbase;
+        deg = ndeg;
+        nb = nnb;
+        na = nna;
+        nbase = nnbase;
+        ndeg = nndeg;
+        nid = nnid;
+    }
+    put_sums(A.partial, g, vp, isect);
+}
+
+// The anchors of one list, with close comparisons made on the exact bounds:
+// those k_curvelets left open, or those of 65 to 256 neighbours.  One wave per
+// workgroup, at the registers the main kernel leaves on a SIMD, so that the
+// latter run beside it.
+template <int CPL, int NW>
+__global__ __launch_bounds__(64, 4) void k_curvelets_exact(FusedArgs A, int list)
+{
+    extern __shared__ double lds[];
+    const int lane = threadIdx.x & 63;
+    const int g = static_cast<int>(blockIdx.x);
+    const int total = static_cast<int>(uload(A.list_len + list * kBucketStride));
+    unsigned vp = 0;
+    unsigned long long isect = 0;
+    if (g < total) {
+        const WaveCells<CPL> W = wave_cells<CPL>(A);
+        int2 *spill = A.spill + static_cast<size_t>(g) * A.spill_stride;
+        for (int L = g; L < total; L += static_cast<int>(gridDim.x)) {
+            int a, deg;
+            unsigned base;
+            load_entry(A.lists + static_cast<size_t>(list) * A.n + L, a, base, deg);
+            double4 nb = make_double4(0.0, 0.0, 0.0, 1.0);
+            if (lane < deg) nb = A.rec[A.ids[base + lane]];
+            (void)do_anchor<CPL, NW, true>(A, W, reinterpret_cast<char *>(lds), spill, a, base, deg, nb, vp, isect);
+        }
+    }
+    put_sums(A.partial, g, vp, isect);
+}
+
+using FusedKernel = void (*)(FusedArgs);
+using ExactKernel = void (*)(FusedArgs, int);
+
+// by cells per lane
+inline FusedKernel fused_kernel(int cpl)
+{
+    return cpl == 1 ? k_curvelets<1> : (cpl == 2 ? k_curvelets<2> : k_curvelets<4>);
+}
+template <int NW>
+inline ExactKernel exact_kernel(int cpl)
+{
+    return cpl == 1 ? k_curvelets_exact<1, NW> : (cpl == 2 ? k_curvelets_exact<2, NW> : k_curvelets_exact<4, NW>);
+}
+
+#endif

@@ -319,13 +319,14 @@ CVG_HD double sin_or_cos_reduced(double rh, double rl, const double *tab, bool w
     return h3.hi + t;
 }
 
+template <bool LARGE = true>
 CVG_HD double cr_sin(double x, const double *tab)
 {
     const double ax = fabs(x);
     if (!(ax <= 0x1.fffffffffffffp+1023)) return x - x;  // NaN for NaN and infinities
     if (ax < 0x1p-26) return x;
     double rh, rl;
-    const int k = reduce_pio2(x, tab, &rh, &rl);
+    const int k = reduce_pio2<LARGE>(x, tab, &rh, &rl);
     const double v = sin_or_cos_reduced(rh, rl, tab, (k & 1) != 0);
     return (k & 2) ? -v : v;
 }

@@ -19,21 +19,19 @@
 //                             another) it counts the lists itself and finds
 //                             the offsets by a decoupled look-back, in place
 //                             of the counting pass and the scan
-//   curvelets k_edge_trig     per edge: sin/cos of theta, theta+-dt, theta+grid
-//           k_pair_prep       per pair: direction-filter class, close/branch
-//                             flags, the bundle's cell-independent terms
-//           k_pair_trig       per (pair, grid angle): the transport's two sines
-//                             (at Kt = 7 with k_pair_prep's work per pair first;
-//                             queued with k_edge_trig behind the graph stage's
-//                             count read where the pair buffers hold the
-//                             guessed capacity)
-//           k_bucket          anchors binned by their largest run (LDS capacity)
-//           k_curvelets       one wave per anchor, bucket by bucket: bundles
-//                             (lane = cell) into the wave's LDS slice, chain
-//                             growth with ballot validity, dedup, staging rows
+//   curvelets k_edge_rec      per edge: (x, y, sin theta, cos theta)
+//           k_order           anchors into lists by neighbour count (with
+//                             k_edge_rec queued behind the graph stage's count
+//                             read)
+//           k_curvelets       one wave per anchor: bundles (lane = cell) from
+//                             certified approximations, chain growth, dedup,
+//                             staging rows (cvg_fused.hpp)
+//           k_curvelets_exact the same on exact bounds, for anchors whose
+//                             comparisons the approximations leave open and
+//                             those of more than 64 neighbours
 //           scan              per-anchor accepted counts -> output row offsets
-//           k_row_slots       staging slot -> row, and the row count into the
-//                             scalars read back with the stream
+//           k_row_anchors     row -> anchor, and the counts into the scalars
+//                             read back with the stream
 //           k_record          chain rows (1-based) and the 10 info columns
 //
 // The reference path this replaces is cpu_curvelet (preprocess.hpp,
@@ -43,6 +41,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <type_traits>
+#include <utility>
 #include <atomic>
 #include <chrono>
 #include <climits>
@@ -79,6 +78,10 @@ __constant__ double c_atan_tab[2 * CVG_ATAN_ROWS] = CVG_ATAN_TABLE_INIT;
 // hipGetSymbolAddress (scratch_address) and that pointer is what kernels get.
 static __device__ __align__(256) unsigned char scratch[static_cast<size_t>(CVG_NOALLOC_SCRATCH_MIB) << 20];
 
+// v_writelane_b32 (value, lane, old): the compiler has no builtin of it.
+extern "C" __device__ __attribute__((const)) int lane_write(int value, int lane, int old) __asm(
+    "llvm.amdgcn.writelane.i32");
+
 namespace {
 
 constexpr int kBlock = 256;
@@ -112,9 +115,9 @@ struct GridDesc {
 struct cvg_context {
     int device = 0;
     hipStream_t stream = nullptr;
-    // extra streams so the bucket launches of the fused kernel run concurrently
-    hipStream_t aux[3] = {nullptr, nullptr, nullptr};
-    hipEvent_t ev_join[3] = {nullptr, nullptr, nullptr};
+    // an extra stream: the fused stage's widest anchors run beside the others
+    hipStream_t aux = nullptr;
+    hipEvent_t ev_join = nullptr;
     // timing events: ev[0..2] run start, graph end, run end; ev[3..4] around
     // the fused kernel's launches
     hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -123,7 +126,7 @@ struct cvg_context {
     hipEvent_t fused_ev[kFusedRing][2] = {};
     long long fused_runs = 0;
     // events without timing for ordering and host waits: the graph stage's
-    // count read, the fork to the auxiliary streams, the end of an untimed run
+    // count read, the fork to the auxiliary stream, the end of an untimed run
     hipEvent_t ev_read = nullptr, ev_fork = nullptr, ev_end = nullptr;
     // Runs with stats record the timing events (their stage times come from
     // them); runs without stats only while event_timing is set
@@ -133,9 +136,9 @@ struct cvg_context {
     bool timed_run = false;  // the current run records the timing events
     std::string err;
     size_t lds_limit = 65536;
-    // fused-kernel launch shape: buckets whose key is at least coop_min_cap
-    // run one anchor per workgroup of coop_waves waves (cvg_set_tuning, or
-    // CVG_COOP_MIN_CAP / CVG_COOP_WAVES at creation; results never depend on it)
+    // accepted, checked and reported as before (cvg_set_tuning, or
+    // CVG_COOP_MIN_CAP / CVG_COOP_WAVES at creation); no launch depends on them
+    // since every anchor is one wave's
     int coop_min_cap = 8;
     int coop_waves = 4;
     int num_cu = 1;
@@ -168,6 +171,7 @@ struct cvg_context {
     unsigned max_deg = 0;
     unsigned truncated = 0;
     unsigned ambiguous = 0;
+    bool wide_theta = false;  // some |theta| above kWideTheta
     int gx0 = 0, gy0 = 0, gw = 0, gh = 0;
     // d_grid's leading cell counts known to be zero (while d_grid is grid_zero_ptr)
     const void *grid_zero_ptr = nullptr;
@@ -179,10 +183,9 @@ struct cvg_context {
     unsigned to_host_rows = 0;  // rows of the last cvg_run_to_host (its early copy's size)
     unsigned long long rebuilds = 0;  // runs built again in the reference's within-cell order
     // a run's parameters while its graph is built (fused double maps): the
-    // graph stage queues k_edge_trig behind its last host read
-    const cvg_params *early_params = nullptr;
-    bool edge_trig_queued = false;  // k_edge_trig of the current run is queued
-    bool pair_setup_queued = false;  // and its per-pair records and sines
+    // graph stage queues k_edge_rec and k_order behind its last host read
+    bool early_setup = false;
+    bool setup_queued = false;  // k_edge_rec and k_order of the current run are queued
     GridDesc spec_g{};
     unsigned spec_R = 0;
     int spec_fill_cap = 1;
@@ -193,7 +196,7 @@ struct cvg_context {
     const void *tables_ptr = nullptr;
     std::vector<char> tables_blob;
     DevBuf d_edges_up, d_x, d_y, d_th, d_cx, d_cy, d_scal, d_grid, d_tmp_ids, d_sorted, d_sxy, d_scell, d_part, d_deg,
-        d_off, d_tiles, d_cand, d_ids, d_d2, d_pair_anchor;
+        d_off, d_tiles, d_cand, d_ids, d_d2;
     // the last graph's edge array (device) and, once the reference's
     // within-cell order has been replayed for it, each edge's rank in its cell
     const double *last_edges = nullptr;
@@ -220,8 +223,8 @@ struct cvg_context {
     unsigned long long intersections = 0;
     unsigned num_curvelets = 0;
     unsigned width = 0;
-    DevBuf d_trig, d_tdd, d_cls, d_prec, d_psin, d_lists, d_tables, d_st_ids, d_st_meta, d_st_k, d_st_rank, d_acc, d_rowoff, d_rowslot, d_gbundle,
-        d_chains, d_info;
+    DevBuf d_rec, d_lists, d_partial, d_tables, d_st_mask, d_st_ids, d_st_meta, d_st_k, d_acc, d_rowoff, d_rowanchor,
+        d_gbundle, d_chains, d_info;
 
     // diagnostics
     DevBuf d_dbg;
@@ -231,7 +234,6 @@ struct cvg_context {
     // told apart by the launch's epoch
     DevBuf d_fillstat;
     unsigned lookback_spins = kLookbackSpins;  // CVG_LOOKBACK_SPINS at creation
-    int gate_naps = 40;  // the start gate's bound in naps (CVG_GATE_NAPS at creation)
     // the same for the single-pass scans (k_scan_1pass)
     DevBuf d_scanstat;
     const void *scanstat_zero_ptr = nullptr;
@@ -256,13 +258,13 @@ struct cvg_context {
     template <typename F>
     void for_each_pool(F f)
     {
-        DevBuf *bufs[] = {&d_edges_up, &d_x,      &d_y,      &d_th,     &d_cx,     &d_cy,          &d_scal,
-                          &d_grid,     &d_tmp_ids, &d_sorted, &d_sxy,    &d_scell,  &d_part,        &d_deg,
-                          &d_off,      &d_tiles,  &d_cand,   &d_ids,    &d_d2,     &d_pair_anchor, &d_trig,
-                          &d_tdd,      &d_cls,    &d_prec,   &d_psin,   &d_lists,  &d_tables,      &d_st_ids,
-                          &d_st_meta,  &d_st_k,   &d_st_rank, &d_acc,   &d_rowoff, &d_rowslot, &d_gbundle, &d_chains,
-                          &d_info,     &d_dbg,    &d_map,    &d_eoff,   &d_mapbox, &d_maprow,       &d_cellrank,
-                          &d_skey,     &d_sorttmp, &d_fillstat, &d_scanstat};
+        DevBuf *bufs[] = {&d_edges_up, &d_x,       &d_y,      &d_th,       &d_cx,       &d_cy,      &d_scal,
+                          &d_grid,     &d_tmp_ids, &d_sorted, &d_sxy,      &d_scell,    &d_part,    &d_deg,
+                          &d_off,      &d_tiles,   &d_cand,   &d_ids,      &d_d2,       &d_rec,     &d_lists,
+                          &d_partial,  &d_tables,  &d_st_mask, &d_st_ids,  &d_st_meta,  &d_st_k,    &d_acc,
+                          &d_rowoff,   &d_rowanchor, &d_gbundle, &d_chains, &d_info,    &d_dbg,     &d_map,
+                          &d_eoff,     &d_mapbox,  &d_maprow, &d_cellrank, &d_skey,     &d_sorttmp, &d_fillstat,
+                          &d_scanstat};
         for (DevBuf *b : bufs) f(*b);
     }
 };
@@ -737,8 +739,8 @@ struct SparseCells {
 // int), [4] bad-input flag, [5] max degree, [6] truncated anchors,
 // [7] order-ambiguous anchors, [8] valid pairs, [9] anchors needing the
 // std::sort replay, [10..11] the 64-bit count of bundle intersections, [12]
-// CSR pairs, [13] a size guess that did not hold, [14] output rows.  The
-// fused kernel's bucket list lengths follow, one 128-byte line each (atomics
+// CSR pairs, [13] a size guess that did not hold, [14] output rows, [15] some
+// |theta| above kWideTheta.  The fused kernel's list lengths follow, one 128-byte line each (atomics
 // from many workgroups on one line serialize in L2).
 enum {
     S_MINX = 0,
@@ -754,15 +756,18 @@ enum {
     S_COUNT = 10,
     S_PAIRS = 12,
     S_MISS = 13,
-    S_ROWS = 14
+    S_ROWS = 14,
+    S_WIDE = 15
 };
-constexpr int kScalarWords = S_ROWS + 1;  // the words read back to the host
-constexpr int kMaxBuckets = 14;
+constexpr int kScalarWords = S_WIDE + 1;  // the words read back to the host
+constexpr int kMaxLists = 6;
 constexpr int kBucketStride = 32;  // words
-constexpr int kBucketBase = 32;    // bucket b's list length at [kBucketBase + b * kBucketStride]
-// heavy-bucket anchor streams that have started (own 128-byte line)
-constexpr int kStartedWord = kBucketBase + kMaxBuckets * kBucketStride;
-constexpr int kScalarBufWords = kStartedWord + 32;
+constexpr int kBucketBase = 32;    // list b's length at [kBucketBase + b * kBucketStride]
+constexpr int kScalarBufWords = kBucketBase + kMaxLists * kBucketStride;
+
+// Orientations the fused kernel's error bound covers (fused_limits); maps
+// with larger ones take the general kernel.
+constexpr double kWideTheta = 64.0;
 
 // Cells are (lrint(x), lrint(y)) (preprocess.hpp:85-86).  Coordinates must be
 // finite with |x|, |y| < 2^31 - 2^13 (so that every window cell cx +- R of the
@@ -796,6 +801,7 @@ __global__ __launch_bounds__(kBlock) void k_prep_edges(int n, int sz, const doub
         const double tv = e[static_cast<long long>(i) * sz + 2];
         const bool ok = fabs(xv) < kMaxCoord && fabs(yv) < kMaxCoord && fabs(tv) <= DBL_MAX;
         if (!ok) atomicOr(&sbad, 1);
+        if (!(fabs(tv) <= kWideTheta)) atomicOr(&sbad, 2);
         const int ix = ok ? static_cast<int>(rint(xv)) : 0;
         const int iy = ok ? static_cast<int>(rint(yv)) : 0;
         x[i] = xv;
@@ -875,13 +881,14 @@ __global__ __launch_bounds__(1024) void k_bbox_finish(int nparts, const int *__r
         scal[S_MAXX] = static_cast<unsigned>(v[1]);
         scal[S_MINY] = static_cast<unsigned>(v[2]);
         scal[S_MAXY] = static_cast<unsigned>(v[3]);
-        scal[S_BAD] = v[4] ? 1u : 0u;
+        scal[S_BAD] = v[4] & 1 ? 1u : 0u;
+        scal[S_WIDE] = v[4] & 2 ? 1u : 0u;
         if (spec_on) {
             const bool fits = static_cast<long long>(v[0]) - R >= spec.x0 &&
                               static_cast<long long>(v[1]) + R <= static_cast<long long>(spec.x0) + spec.w - 1 &&
                               static_cast<long long>(v[2]) - R >= spec.y0 &&
                               static_cast<long long>(v[3]) + R <= static_cast<long long>(spec.y0) + spec.h - 1;
-            if (!fits || v[4]) scal[S_MISS] = 1u;
+            if (!fits || (v[4] & 1)) scal[S_MISS] = 1u;
         }
     }
 }
@@ -1365,7 +1372,7 @@ __global__ __launch_bounds__(64 * kFillWaves) void k_fill_csr(int n, const doubl
                                                               const double2 *__restrict__ sxy,
                                                               unsigned *__restrict__ off, Cand *__restrict__ cand,
                                                               int *__restrict__ ids, double *__restrict__ d2,
-                                                              int *__restrict__ pair_anchor, int *__restrict__ tie_list,
+                                                              int *__restrict__ tie_list,
                                                               unsigned max_cand, int cap,
                                                               const int *__restrict__ map_of,
                                                               const long long *__restrict__ map_eoff,
@@ -1556,7 +1563,6 @@ __global__ __launch_bounds__(64 * kFillWaves) void k_fill_csr(int n, const doubl
             const int i = lord[r];
             ids[o + r] = lid[i];
             d2[o + r] = ld[i];
-            pair_anchor[o + r] = a;
         }
         const bool any_tie = (__ballot(tie) & segmask) != 0ULL;
         const bool any_shared = (__ballot(shared) & segmask) != 0ULL;
@@ -1597,7 +1603,6 @@ __global__ __launch_bounds__(64 * kFillWaves) void k_fill_csr(int n, const doubl
     const bool any_tie = (__ballot(tie) & segmask) != 0ULL;
     const bool any_shared = (__ballot(shared) & segmask) != 0ULL;
     const bool any_amb = (__ballot(ambiguous) & segmask) != 0ULL;
-    for (int i = sl; i < dg; i += G) pair_anchor[o + i] = a;
     if (any_tie && dg > 16) {
         for (int i = sl; i < dg; i += G) cand[o + i] = Cand{ld[i], lid[i]};  // scan order
         if (sl == 0) tie_list[atomicAdd(&scal[S_TIES], 1u)] = a;
@@ -1639,904 +1644,26 @@ __global__ __launch_bounds__(kBlock) void k_tie_sort(const int *__restrict__ tie
 // Curvelet stage
 // ---------------------------------------------------------------------------
 
-// The rows of trig (cvg_device.hpp), and in tdd the same values as
-// double-doubles for the per-pair sines: tdd[8i .. 8i+7] = sin, cos of
-// theta_i + dt, then of theta_i - dt (hi, lo each); from tdd + 8n, edge i's
-// grid angles, 4 per j: sin hi, sin lo, cos hi, cos lo of theta_i + off_t[j].
-// One thread per (edge i, angle k), k fastest: k < Kt the grid angle j = k,
-// k = Kt theta + dt, Kt + 1 theta - dt, Kt + 2 theta itself.
-__global__ __launch_bounds__(kBlock) void k_edge_trig(int n, const double *__restrict__ th, double dt, int kt,
-                                                      double st, double *__restrict__ trig, double *__restrict__ tdd,
-                                                      unsigned *__restrict__ scal)
-{
-    // the curvelet stage's counters start at zero (block 0 clears them; the
-    // graph stage's words are left alone, so this may run before its last
-    // host read)
-    if (blockIdx.x == 0) {
-        const int t = static_cast<int>(threadIdx.x);
-        if (t == 0) scal[S_VALID] = 0u;
-        if (t == 1) scal[S_COUNT] = 0u;
-        if (t == 2) scal[S_COUNT + 1] = 0u;
-        for (int w = kBucketBase + t; w < kScalarBufWords; w += static_cast<int>(blockDim.x)) scal[w] = 0u;
-    }
-    const unsigned na = static_cast<unsigned>(kt) + 3u;
-    const unsigned g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= static_cast<unsigned>(n) * na) return;
-    const int i = static_cast<int>(g / na);
-    const int k = static_cast<int>(g - static_cast<unsigned>(i) * na);
-    const double t = th[i];
-    // delta_t2 of grid column k (cpu_curvelet.hpp:698), the host table's expression
-    const double off_t = k < kt ? st * (static_cast<double>(k) - (static_cast<double>(kt) - 1.0) / 2.0) : 0.0;
-    const double ang = k < kt ? t + off_t         // T2t = T2 + delta_t2, cpu_curvelet.hpp:702
-                       : k == kt ? t + dt         // T0_p_dt, :655
-                       : k == kt + 1 ? t - dt     // T0_m_dt, :656
-                                     : t;
-    cvg::dd sd, cd;
-    cvg::cr_sincos_dd(ang, c_sincos_tab, &sd, &cd);
-    if (k < kt) {
-        const long long e = static_cast<long long>(i) * kt + k;
-        reinterpret_cast<double2 *>(trig + static_cast<long long>(cvg::TRIG_GRID) * n)[e] = make_double2(sd.hi, cd.hi);
-        reinterpret_cast<double4 *>(tdd + static_cast<long long>(n) * 8)[e] = make_double4(sd.hi, sd.lo, cd.hi, cd.lo);
-    } else if (k < kt + 2) {
-        const bool plus = k == kt;
-        trig[(plus ? cvg::TRIG_SIN_P : cvg::TRIG_SIN_M) * n + i] = sd.hi;
-        trig[(plus ? cvg::TRIG_COS_P : cvg::TRIG_COS_M) * n + i] = cd.hi;
-        reinterpret_cast<double4 *>(tdd)[2 * static_cast<long long>(i) + (plus ? 0 : 1)] =
-            make_double4(sd.hi, sd.lo, cd.hi, cd.lo);
-    } else {
-        trig[cvg::TRIG_COS * n + i] = cd.hi;
-        trig[cvg::TRIG_SIN * n + i] = sd.hi;
-    }
-}
-
-// Per CSR pair q = (a, b): the direction filter (cpu_curvelet.hpp:459-461),
-// and the cell-independent part of compute_curve_bundle (:646-656, 682, 690).
-//   pflag[q] = class | close << 2 | branch_a << 3
-//   prec[8q .. 8q+7] = DX, DY, DX2, DY2, DX cos(T0-dt), DY sin(T0-dt),
-//                      DX cos(T0+dt), DY sin(T0+dt)
-struct PrepArgs {
-    const double *x, *y, *trig;
-    double close_thr;
-    unsigned char *pflag;
-    double *prec;
-};
-
-// Pair q = (a, b)'s flags and record; returns whether the pair is close.
-__device__ __forceinline__ bool pair_prep_one(int q, int n, int a, int b, const PrepArgs &P)
-{
-    const double ax = P.x[a], ay = P.y[a], bx = P.x[b], by = P.y[b];
-    const double cos_at = P.trig[cvg::TRIG_COS * n + a];
-    const double sin_at = P.trig[cvg::TRIG_SIN * n + a];
-    const int k = cvg::direction_class(ax, ay, cos_at, sin_at, bx, by, c_sincos_tab, c_atan_tab);
-    const cvg::PairRec p = cvg::pair_record(ax, ay, bx, by, P.trig[cvg::TRIG_SIN_P * n + b],
-                                            P.trig[cvg::TRIG_COS_P * n + b], P.trig[cvg::TRIG_SIN_M * n + b],
-                                            P.trig[cvg::TRIG_COS_M * n + b]);
-    const bool close = p.DX2 + p.DY2 < P.close_thr;
-    const bool branch_a = (p.DX * cos_at + p.DY * sin_at) < 0;
-    P.pflag[q] = static_cast<unsigned char>(k | (close ? 4 : 0) | (branch_a ? 8 : 0));
-    double2 *o = reinterpret_cast<double2 *>(P.prec + static_cast<long long>(q) * 8);
-    o[0] = make_double2(p.DX, p.DY);
-    o[1] = make_double2(p.DX2, p.DY2);
-    o[2] = make_double2(p.cT0m_DX, p.sT0m_DY);
-    o[3] = make_double2(p.cT0p_DX, p.sT0p_DY);
-    return close;
-}
-
-__global__ __launch_bounds__(kBlock) void k_pair_prep(int pairs, int n, const int *__restrict__ pair_anchor,
-                                                      const int *__restrict__ ids, PrepArgs P)
-{
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= pairs) return;
-    (void)pair_prep_one(q, n, pair_anchor[q], ids[q], P);
-}
-
-// Anchors in spatial (cell) order, binned by max(forward, backward) + neither
-// of their class counts (read from the anchor's run of pair flags): that key
-// bounds every run's slot count and half the degree (the third class is
-// almost always empty), which size the fused kernel's LDS slots and staging.
-// Each list entry carries (anchor, CSR base, degree).
-constexpr int kBucketBlock = 1024;  // few workgroups: one list-length atomic each per bucket
-constexpr int kHeavyCap = 32;       // buckets from this cap start ahead of the light bucket 0
-// Automatic light-bucket grids: kGridAutoMinPct percent of the resident grid
-// plus one percent per kGridAutoEdgesPerPct edges of the run, at most all of
-// it (measured best on single maps from 320x240 to 3840x2160: ~10% at 6k
-// edges, 20-25% at 30-50k, 33% at 90k, 50% at 150k, 50-75% at 200k, 100%
-// from ~350k).
-constexpr long long kGridAutoEdgesPerPct = 4000;
-constexpr int kGridAutoMinPct = 10;
-
-int auto_grid_pct(long long n)
-{
-    return static_cast<int>(std::min<long long>(100, kGridAutoMinPct + n / kGridAutoEdgesPerPct));
-}
-
-__global__ __launch_bounds__(kBucketBlock) void k_bucket(int n, const int *__restrict__ sorted,
-                                                   const unsigned char *__restrict__ pflag,
-                                                   const unsigned *__restrict__ off,
-                                                   int nb, const int *caps, int4 *__restrict__ lists,
-                                                   unsigned *__restrict__ scal)
-{
-    __shared__ unsigned s_count[kMaxBuckets];
-    __shared__ unsigned s_base[kMaxBuckets];
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63;
-    if (threadIdx.x < kMaxBuckets) s_count[threadIdx.x] = 0;
-    __syncthreads();
-    int a = -1, b = -1;
-    unsigned o0 = 0, o1 = 0;
-    if (p < n) {
-        a = sorted[p];
-        o0 = off[a];
-        o1 = off[a + 1];
-        // the anchor's run of flags, four per aligned 32-bit load (the flag
-        // buffer is padded to whole words)
-        unsigned c[3] = {0u, 0u, 0u};
-        for (unsigned q4 = o0 & ~3u; q4 < o1; q4 += 4) {
-            const unsigned w = *reinterpret_cast<const unsigned *>(pflag + q4);
-#pragma unroll
-            for (unsigned k = 0; k < 4; ++k) {
-                const unsigned q = q4 + k;
-                const unsigned f = (w >> (8 * k)) & 3u;
-                const bool in = q >= o0 && q < o1;
-                c[0] += in && f == 0u ? 1u : 0u;
-                c[1] += in && f == 1u ? 1u : 0u;
-                c[2] += in && f == 2u ? 1u : 0u;
-            }
-        }
-        const unsigned m = max(c[1], c[2]) + c[0];
-        b = 0;
-        while (b < nb - 1 && m > static_cast<unsigned>(caps[b])) ++b;
-    }
-    // per wave and bucket: the group's leader reserves slots in the block's
-    // count, then one global atomic per block and bucket
-    unsigned my_off = 0;
-    for (int k = 0; k < nb; ++k) {
-        const unsigned long long grp = __ballot(b == k);
-        if (grp == 0ULL) continue;
-        const int leader = __ffsll(static_cast<long long>(grp)) - 1;
-        unsigned off = 0;
-        if (lane == leader) off = atomicAdd(&s_count[k], static_cast<unsigned>(__popcll(grp)));
-        off = __shfl(off, leader, 64);
-        if (b == k) my_off = off + static_cast<unsigned>(__popcll(grp & ((1ULL << lane) - 1ULL)));
-    }
-    __syncthreads();
-    if (threadIdx.x < nb && s_count[threadIdx.x] > 0)
-        s_base[threadIdx.x] = atomicAdd(&scal[kBucketBase + threadIdx.x * kBucketStride], s_count[threadIdx.x]);
-    __syncthreads();
-    if (b >= 0)
-        lists[static_cast<long long>(b) * n + s_base[b] + my_off] =
-            make_int4(a, static_cast<int>(o0), static_cast<int>(o1 - o0), 0);
-}
-
-// Start gate for the light buckets' first launch: the heavy buckets' few
-// anchors are the fused stage's critical path, and their workgroups need far
-// more LDS than light ones, so they are placed best before light workgroups
-// fill the CUs.  One wave waits (bounded: at most max_naps sleeps of ~3 us)
-// until every heavy-bucket stream with work has started (each counts itself
-// in scal[kStartedWord]); the light launch queued behind it then starts.
-struct GateArgs {
-    int nheavy;
-    int bucket[kMaxBuckets];
-    int streams[kMaxBuckets];
-};
-
-__global__ void k_gate(GateArgs G, const unsigned *__restrict__ scal, int max_naps)
-{
-    if (threadIdx.x != 0) return;
-    unsigned want = 0;
-    for (int i = 0; i < G.nheavy; ++i)
-        want += min(scal[kBucketBase + G.bucket[i] * kBucketStride], static_cast<unsigned>(G.streams[i]));
-    for (int k = 0; k < max_naps; ++k) {
-        if (__hip_atomic_load(scal + kStartedWord, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= want) return;
-        __builtin_amdgcn_s_sleep(127);
-    }
-}
-
-// Per-pair sines of the transport (compute_curve_bundle, cpu_curvelet.hpp:728-729):
-// psin[q*2Kt + 2j] = sin(T2t_j - (theta_n - dt)), psin[q*2Kt + 2j + 1] =
-// sin(T2t_j - (theta_n + dt)) with T2t_j = theta_a + delta_t2[j], for every
-// pair that is not "close" (pair flag bit 2; close pairs keep the default
-// bundle and never read them, and get zeros).  One thread per pair; KT > 0
-// fixes Kt at compile time so that every load is issued before the arithmetic
-// (KT = 0: any Kt up to kPairTrigMaxKt).  Each sine is the correctly rounded
-// sine of the rounded difference, formed from the double-double sin/cos of
-// both angles in tdd by the subtraction formula; the rare lane whose rounding
-// that does not settle evaluates the sine directly.  For Kt up to
-// kPairTrigMaxKt the block's results go through LDS (dynamic, kBlock x Kt
-// double2) so that its output span is written contiguously.  PREP: the
-// thread first forms its pair's flags and record (k_pair_prep's work) and
-// takes the close bit from there instead of reading pflag.  With scal (a
-// launch queued before the host has read the graph's counts, on buffers of
-// the guessed capacity) the pair count comes from the device, and a guess
-// that did not hold (or bad input) leaves the launch with nothing to do.
-constexpr int kPairTrigMaxKt = 16;
-template <int KT, bool PREP>
-__global__ __launch_bounds__(kBlock) void k_pair_trig(int pairs, int n, int kt_rt, const int *__restrict__ pair_anchor,
-                                                      const int *__restrict__ ids,
-                                                      const unsigned char *__restrict__ pflag,
-                                                      const double *__restrict__ th, double st_step, double dt,
-                                                      const double *__restrict__ tdd, double *__restrict__ psin,
-                                                      PrepArgs P, const unsigned *__restrict__ scal)
-{
-    extern __shared__ double2 stage[];
-    if (scal) pairs = (scal[S_MISS] | scal[S_BAD]) ? 0 : static_cast<int>(scal[S_PAIRS]);
-    if (static_cast<int>(blockIdx.x * blockDim.x) >= pairs) return;  // the whole block
-    const int kt = KT > 0 ? KT : kt_rt;
-    // delta_t2 of grid column j (cpu_curvelet.hpp:698), the host table's expression
-    const double half = (static_cast<double>(kt) - 1.0) / 2.0;
-    const bool staged = kt <= kPairTrigMaxKt;
-    const int q0 = blockIdx.x * blockDim.x;
-    const int q = q0 + threadIdx.x;
-    double2 *out = reinterpret_cast<double2 *>(psin) + static_cast<long long>(q0) * kt;
-    double2 *row = (staged ? stage : out) + threadIdx.x * kt;
-    if (q < pairs) {
-        const int a = pair_anchor[q];
-        const int b = ids[q];
-        const bool close = PREP ? pair_prep_one(q, n, a, b, P) : (pflag[q] & 4) != 0;
-        if (close) {  // :682
-            for (int j = 0; j < kt; ++j) row[j] = make_double2(0.0, 0.0);
-        } else {
-            const double ta = th[a];
-            const double nt = th[b];
-            const double tm = nt - dt, tp = nt + dt;
-            const double4 *nr = reinterpret_cast<const double4 *>(tdd) + 2 * static_cast<long long>(b);
-            const double4 p = nr[0], m = nr[1];
-            const cvg::dd sp = {p.x, p.y}, cp = {p.z, p.w}, sm = {m.x, m.y}, cm = {m.z, m.w};
-            const double4 *gr =
-                reinterpret_cast<const double4 *>(tdd + static_cast<long long>(n) * 8) + static_cast<long long>(a) * kt;
-            if (KT > 0) {
-                double4 g[KT > 0 ? KT : 1];
-#pragma unroll
-                for (int j = 0; j < (KT > 0 ? KT : 1); ++j) g[j] = gr[j];
-#pragma unroll
-                for (int j = 0; j < (KT > 0 ? KT : 1); ++j) {
-                    const double T2t = ta + st_step * (static_cast<double>(j) - half);
-                    const cvg::dd st = {g[j].x, g[j].y}, ct = {g[j].z, g[j].w};
-                    double2 v;
-                    v.x = cvg::sin_difference(T2t, tm, st, ct, sm, cm, c_sincos_tab);
-                    v.y = cvg::sin_difference(T2t, tp, st, ct, sp, cp, c_sincos_tab);
-                    row[j] = v;
-                }
-            } else {
-                for (int j = 0; j < kt; ++j) {
-                    const double T2t = ta + st_step * (static_cast<double>(j) - half);
-                    const double4 g = gr[j];
-                    const cvg::dd st = {g.x, g.y}, ct = {g.z, g.w};
-                    double2 v;
-                    v.x = cvg::sin_difference(T2t, tm, st, ct, sm, cm, c_sincos_tab);
-                    v.y = cvg::sin_difference(T2t, tp, st, ct, sp, cp, c_sincos_tab);
-                    row[j] = v;
-                }
-            }
-        }
-    }
-    if (!staged) return;
-    __syncthreads();
-    const int cnt = min(static_cast<int>(blockDim.x), pairs - q0) * kt;
-    for (int e = threadIdx.x; e < cnt; e += blockDim.x) out[e] = stage[e];
-}
-
-// Host-computed per-parameter tables, laid out in one device block.  Lanes of
-// the fused kernel own bundle cells in "rank" order: rank = position of cell
-// c = i*Kt + j when cells are sorted by (ox^2 + ot^2, c), so the cell that
-// fill_curvelet_info picks (smallest distance, first in row-major order,
-// cpu_curvelet.hpp:202-219) is the lowest lane whose cell is valid.
-struct Tables {
-    double *rank_ox;       // [K]
-    int *rank_j;           // [K]
-    int *rank_cell;        // [K]
-    int *rank_elig;        // [K] d < 100 (the initial best distance)
-    double *off_x;         // [Kx]
-    double *off_t;         // [Kt]
-    int *caps;             // [kMaxBuckets]
-};
-
-struct FusedArgs {
-    int n;
-    const double *trig, *psin, *prec;
-    const int *ids;
-    const unsigned char *pflag;
-    const int4 *list;  // (anchor, CSR base, degree, -)
-    const unsigned *list_len;  // the bucket's entry count (device; written by k_bucket)
-    int nb_cap;        // bundle slots per anchor: the bucket's longest run
-    int deg_cap;       // staged neighbour records per anchor
-    int chain_stride;  // ids per seed record: max(G, 1)
-    int st_stride;     // staging ids per row: max(G, 1)
-    double dx, dx2, max_k;
-    int kt, K, G;
-    const double *rank_ox;
-    const int *rank_j, *rank_cell, *rank_elig;
-    int rank_of_cell0;
-    int *st_ids;
-    unsigned *st_meta;
-    double *st_k;
-    int *st_rank;         // per CSR slot: row among the anchor's accepted chains, or -1
-    unsigned *acc_count;
-    unsigned *valid_pairs;
-    unsigned long long *intersections;
-    double *g_bundle;  // global-bundle kernels: nb_cap*K*2 doubles per anchor stream
-    unsigned *started; // heavy buckets: each stream with work counts itself here at its start
-};
-
-// One anchor stream's LDS slice (byte offsets): the staging buffer (the
-// anchor's pair records and sines, copied from the pre-passes' contiguous
-// blocks), the run's bundles by slot (lo, hi; absent
-// when they live in global memory), the seeds' results (length, hash, best
-// cell, chain), the slots' hypothesis flags, a list area for compacting the
-// run's slots and hypotheses (2 x 64 x nch ints) and the anchor's per-seed
-// accept flags (dc ints).
-struct AnchorCarve {
-    size_t stg, stg_bytes, rec, sin, blo, bhi, ski, hyp, lst, acf, bytes;
-};
-
-__host__ __device__ inline AnchorCarve anchor_carve(int nb, int dc, int K, int kt, int cs, bool lds_bundles, int nch)
-{
-    AnchorCarve c{};
-    c.rec = 0;  // within a staging buffer
-    c.sin = static_cast<size_t>(dc) * 8 * sizeof(double);
-    c.stg_bytes = c.sin + static_cast<size_t>(dc) * kt * 2 * sizeof(double);
-    size_t o = 0;
-    c.stg = o;
-    o += c.stg_bytes;
-    c.blo = o;
-    if (lds_bundles) o += static_cast<size_t>(nb) * K * sizeof(double);
-    c.bhi = o;
-    if (lds_bundles) o += static_cast<size_t>(nb) * K * sizeof(double);
-    c.ski = o;
-    o += static_cast<size_t>(nb) * (cs + 3) * sizeof(int);
-    c.hyp = o;
-    o += static_cast<size_t>(nb) * sizeof(int);
-    c.lst = o;
-    o += static_cast<size_t>(2) * 64 * nch * sizeof(int);
-    c.acf = o;
-    o += static_cast<size_t>(dc) * sizeof(int);
-    c.bytes = (o + 15) & ~static_cast<size_t>(15);
-    return c;
-}
-
-// Load from a wave-uniform address through the scalar data cache (read only).
-template <typename T>
-__device__ __forceinline__ T uload(const T *p)
-{
-    return *(const __attribute__((address_space(4))) T *)p;
-}
-
-// Asynchronous copy of cnt 16-byte entries from global memory into LDS
-// (global_load_lds_dwordx4: lane i of a chunk writes M0 + 16 i); waves t of W
-// split the chunks.  Completion: s_waitcnt vmcnt(0), then a barrier.  Issued
-// as inline assembly: through the builtin the compiler cannot tell the
-// staging buffer from the rest of the LDS and adds vmcnt(0) waits before
-// unrelated LDS reads.
-__device__ __forceinline__ void copy_to_lds(const double2 *src, char *dst, int cnt, int t, int W, int lane)
-{
-    for (int c0 = t * 64; c0 < cnt; c0 += W * 64) {
-        const int i = c0 + lane;
-        const unsigned lds = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(
-            reinterpret_cast<size_t>((__attribute__((address_space(3))) char *)(dst + 16 * c0))));
-        if (i < cnt)
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                         :
-                         : "v"(src + i), "s"(lds)
-                         : "memory", "m0");
-    }
-}
-
-// Lane-indexed arrays: entry k of a wave-wide list lives in lane k % 64 of
-// register v[k / 64]; k is wave-uniform.
-template <int NCH>
-__device__ __forceinline__ int lane_get(const int (&v)[NCH], int k)
-{
-    int r = 0;
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-        const int t = __builtin_amdgcn_readlane(v[c], k & 63);
-        if ((k >> 6) == c) r = t;
-    }
-    return r;
-}
-
-template <int NCH>
-__device__ __forceinline__ void lane_set(int (&v)[NCH], int k, int val, int lane)
-{
-#pragma unroll
-    for (int c = 0; c < NCH; ++c)
-        if ((k >> 6) == c && lane == (k & 63)) v[c] = val;
-}
-
-// Lowest remaining index of a multi-word lane mask (uniform), -1 when empty.
-template <int NCH>
-__device__ __forceinline__ int pop_next(unsigned long long (&m)[NCH])
-{
-    int k = -1;
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-        const bool take = k < 0 && m[c] != 0ULL;
-        const int r = __builtin_ctzll(m[c] | (1ULL << 63));
-        k = take ? 64 * c + r : k;
-        m[c] = take ? (m[c] & (m[c] - 1ULL)) : m[c];
-    }
-    return k;
-}
-
-__device__ __forceinline__ unsigned chain_hash(unsigned h, int id)
-{
-    return (h ^ static_cast<unsigned>(id)) * 16777619u;
-}
-
-// build_curvelets_greedy (cpu_curvelet.hpp:437-591) plus the
-// form_pairwise_bundles valid-pair count (:305-361), in one pass.
-//
-// Persistent: the grid holds as many anchor streams as the GPU keeps resident;
-// stream g processes list entries g, g + streams, ...  A stream is one wave
-// (COOP = false, blockDim/64 streams per workgroup) or a whole workgroup whose
-// W = blockDim/64 waves split each anchor's bundles (slot i on wave i % W) and
-// seeds (hypothesis j on wave j % W) (COOP = true).  An anchor's pair records
-// and sines are copied into the stream's LDS staging buffer (global_load_lds)
-// when it starts; its list entry, flags, ids and per-lane trig values were
-// loaded while the previous anchor was processed.  One staging buffer, not
-// two: the copy's latency is covered by the other resident streams, and the
-// smaller slice keeps more streams resident.
-//
-// Per anchor, runs 0 = forward neighbours (class 1), 1 = backward (class 2),
-// 2 = neither (class 0: validity only, for the count).  Phase A: the run's
-// bundles (lane = cell in rank order, CPL cells per lane) into LDS slots in CSR
-// order, with hypothesis flags.  Phase C: each hypothesis seeds a chain grown
-// by intersecting the hypotheses' bundles in CSR order (validity = one
-// ballot); the seed's chain, hash and best cell (fill_curvelet_info,
-// :202-226: the first valid cell in rank order) go to LDS.  Phase D (wave 0):
-// in seed order, a chain longer than 2 is accepted unless an accepted chain of
-// this (anchor, run) is identical (hash match, then element check), and
-// written to the anchor's staging rows.  Control state is wave-uniform;
-// per-neighbour flags and ids, slot ids and accepted hashes are lane-indexed
-// registers.
-template <int CPL, int NCH, bool GB, bool COOP>
-__global__ __launch_bounds__(256) void k_curvelets(FusedArgs A)
-{
-    extern __shared__ double lds[];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int wpb = static_cast<int>(blockDim.x >> 6);
-    const int W = COOP ? wpb : 1;      // waves per anchor
-    const int t = COOP ? wave : 0;     // this wave's rank within its anchor
-    const int grp = COOP ? 0 : wave;   // anchor stream within the workgroup
-    const int apb = COOP ? 1 : wpb;    // anchor streams per workgroup
-    const int streams = static_cast<int>(gridDim.x) * apb;
-    const int g = static_cast<int>(blockIdx.x) * apb + grp;
-    const int len_list = static_cast<int>(uload(A.list_len));
-    if (A.started && g < len_list && lane == 0 && t == 0) atomicAdd(A.started, 1u);
-    if (g >= len_list) return;  // COOP: the whole workgroup (same g)
-
-    const int n = A.n;
-    const int K = A.K;
-    const int kt = A.kt;
-    const int G = A.G;
-    const int CS = A.chain_stride;
-    const int SR = CS + 3;  // ints per seed record
-    const int NB = A.nb_cap;
-    const AnchorCarve cv = anchor_carve(NB, A.deg_cap, K, kt, CS, !GB, NCH);
-    char *sl = reinterpret_cast<char *>(lds) + static_cast<size_t>(grp) * cv.bytes;
-    int *ski = reinterpret_cast<int *>(sl + cv.ski);
-    int *hypf = reinterpret_cast<int *>(sl + cv.hyp);
-    int *lst = reinterpret_cast<int *>(sl + cv.lst);
-    int *accf = reinterpret_cast<int *>(sl + cv.acf);
-    const unsigned long long lt_mask = (1ULL << lane) - 1ULL;
-    double *blo;
-    double *bhi;
-    if constexpr (GB) {
-        blo = A.g_bundle + static_cast<size_t>(g) * NB * K * 2;
-        bhi = blo + static_cast<size_t>(NB) * K;
-    } else {
-        blo = reinterpret_cast<double *>(sl + cv.blo);
-        bhi = reinterpret_cast<double *>(sl + cv.bhi);
-    }
-    auto sync = [&]() {
-        if constexpr (COOP)
-            __syncthreads();
-        else
-            wave_sync();
-    };
-
-    // per-lane cells (rank order): anchor-independent
-    double ox[CPL];
-    int cj[CPL], ccell[CPL], coff[CPL];
-    bool live[CPL], elig[CPL];
-#pragma unroll
-    for (int m = 0; m < CPL; ++m) {
-        const int rho = lane + 64 * m;
-        live[m] = rho < K;
-        const int r = live[m] ? rho : 0;
-        coff[m] = r;
-        ox[m] = A.rank_ox[r];
-        cj[m] = A.rank_j[r];
-        ccell[m] = A.rank_cell[r];
-        elig[m] = live[m] && A.rank_elig[r] != 0;
-    }
-    // the same as wave masks: a validity test is then one compare ballot
-    unsigned long long lmask[CPL], emask[CPL];
-#pragma unroll
-    for (int m = 0; m < CPL; ++m) {
-        lmask[m] = __ballot(live[m]);
-        emask[m] = __ballot(elig[m]);
-    }
-
-    // the pipeline: entry, staging copy and per-lane values of the next anchor
-    const double2 *prec2 = reinterpret_cast<const double2 *>(A.prec);
-    const double2 *psin2 = reinterpret_cast<const double2 *>(A.psin);
-    auto entry = [&](int L, int &ea, unsigned &eb, int &ed) {
-        const int *e = reinterpret_cast<const int *>(A.list + L);
-        ea = uload(e);
-        eb = static_cast<unsigned>(uload(e + 1));
-        ed = uload(e + 2);
-    };
-    auto stage = [&](int buf, unsigned b0, int d0) {
-        char *sb = sl + cv.stg + static_cast<size_t>(buf) * cv.stg_bytes;
-        copy_to_lds(prec2 + static_cast<size_t>(b0) * 4, sb + cv.rec, d0 * 4, t, W, lane);
-        copy_to_lds(psin2 + static_cast<size_t>(b0) * kt, sb + cv.sin, d0 * kt, t, W, lane);
-    };
-    double nsT2t[CPL], ncT2t[CPL];
-    int nnfl[NCH], nnid[NCH];
-    auto lane_vals = [&](int a0, unsigned b0, int d0) {
-#pragma unroll
-        for (int m = 0; m < CPL; ++m) {
-            const double2 sc = reinterpret_cast<const double2 *>(A.trig + static_cast<long long>(cvg::TRIG_GRID) * n)
-                [static_cast<long long>(a0) * kt + cj[m]];
-            nsT2t[m] = sc.x;
-            ncT2t[m] = sc.y;
-        }
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-            const int r = 64 * c + lane;
-            nnfl[c] = r < d0 ? static_cast<int>(A.pflag[b0 + r]) : 3;
-            nnid[c] = r < d0 ? A.ids[b0 + r] : 0;
-        }
-    };
-
-    int L = g;
-    int a, deg;
-    unsigned base;
-    entry(L, a, base, deg);
-    lane_vals(a, base, deg);
-    int Ln = L + streams;
-    int na = 0, ndeg = 0;
-    unsigned nbase = 0;
-    if (Ln < len_list) entry(Ln, na, nbase, ndeg);
-
-    unsigned vpw = 0;     // valid or close pairs computed by this wave
-    unsigned isect = 0;   // intersections tested by this wave
-    while (L < len_list) {
-        const int buf = 0;
-        double sT2t[CPL], cT2t[CPL];
-        int nfl[NCH], nid[NCH];
-#pragma unroll
-        for (int m = 0; m < CPL; ++m) {
-            sT2t[m] = nsT2t[m];
-            cT2t[m] = ncT2t[m];
-        }
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-            nfl[c] = nnfl[c];
-            nid[c] = nnid[c];
-        }
-        sync();  // every reader of the previous anchor's staging is done
-        stage(0, base, deg);
-        __builtin_amdgcn_s_waitcnt(0);  // this anchor's staging copy and values have landed
-        sync();
-        // start the next anchor's loads
-        const int Lnn = Ln + streams;
-        int nna = 0, nndeg = 0;
-        unsigned nnbase = 0;
-        if (Ln < len_list) {
-            lane_vals(na, nbase, ndeg);
-            if (Lnn < len_list) entry(Lnn, nna, nnbase, nndeg);
-        }
-
-        const char *sb = sl + cv.stg + static_cast<size_t>(buf) * cv.stg_bytes;
-        const double2 *srec = reinterpret_cast<const double2 *>(sb + cv.rec);
-        const double2 *ssin = reinterpret_cast<const double2 *>(sb + cv.sin);
-        int nseed = 0;  // hypotheses of the earlier runs (their seeds' slots come first)
-        for (int run = 0; run < 3; ++run) {
-            const int want = run == 0 ? 1 : (run == 1 ? 2 : 0);
-            unsigned long long mk[NCH];
-            int nL = 0;
-#pragma unroll
-            for (int c = 0; c < NCH; ++c) {
-                mk[c] = __ballot((nfl[c] & 3) == want);
-                nL += __popcll(mk[c]);
-            }
-            if (nL == 0) continue;
-
-            // phase A: the run's bundles (compute_curve_bundle, :636-819), slot
-            // i = i-th neighbour of the run in CSR order.  The slots' neighbour
-            // indices are compacted through the list area (every wave writes
-            // the same values) into lane-indexed rr, their ids into rid.
-            {
-                int pb = 0;
-#pragma unroll
-                for (int c = 0; c < NCH; ++c) {
-                    if ((mk[c] >> lane) & 1ULL) lst[pb + __popcll(mk[c] & lt_mask)] = 64 * c + lane;
-                    pb += __popcll(mk[c]);
-                }
-            }
-            wave_sync();
-            int rr[NCH], rid[NCH];
-#pragma unroll
-            for (int c = 0; c < NCH; ++c) rr[c] = 64 * c + lane < nL ? lst[64 * c + lane] : 0;
-#pragma unroll
-            for (int c = 0; c < NCH; ++c) {
-                int v = 0;
-#pragma unroll
-                for (int cc = 0; cc < NCH; ++cc) {
-                    const int g = __shfl(nid[cc], rr[c] & 63, 64);
-                    if ((rr[c] >> 6) == cc) v = g;
-                }
-                rid[c] = v;
-            }
-            for (int i = COOP ? t : 0; i < nL; i += W) {
-                const int r = lane_get<NCH>(rr, i);
-                const int fl = lane_get<NCH>(nfl, r);
-                const double2 *rr = srec + r * 4;
-                const double2 r0 = rr[0], r1 = rr[1], r2 = rr[2], r3 = rr[3];
-                cvg::PairRec q;
-                q.DX = r0.x;
-                q.DY = r0.y;
-                q.DX2 = r1.x;
-                q.DY2 = r1.y;
-                q.cT0m_DX = r2.x;
-                q.sT0m_DY = r2.y;
-                q.cT0p_DX = r3.x;
-                q.sT0p_DY = r3.y;
-                const bool qclose = (fl & 4) != 0;
-                const bool qbr = (fl & 8) != 0;
-                double lo[CPL], hi[CPL];
-                unsigned long long anym = 0ULL;
-#pragma unroll
-                for (int m = 0; m < CPL; ++m) {
-                    lo[m] = -A.max_k;
-                    hi[m] = A.max_k;
-                    if (!qclose) {
-                        const double2 s = ssin[r * kt + cj[m]];
-                        cvg::bundle_cell(q, qbr, ox[m], sT2t[m], cT2t[m], s.x, s.y, A.dx, A.dx2, A.max_k, lo[m],
-                                         hi[m]);
-                    }
-                    anym |= __builtin_amdgcn_ballot_w64(hi[m] > lo[m]) & lmask[m];
-                }
-                const bool hyp = qclose || anym != 0ULL;  // bundle_valid_check, :821-830
-                vpw += hyp ? 1u : 0u;
-                if (run == 2) continue;
-                if (hyp) {
-#pragma unroll
-                    for (int m = 0; m < CPL; ++m) {
-                        if (live[m]) {
-                            blo[static_cast<size_t>(i) * K + coff[m]] = lo[m];
-                            bhi[static_cast<size_t>(i) * K + coff[m]] = hi[m];
-                        }
-                    }
-                }
-                if (lane == 0) hypf[i] = hyp ? 1 : 0;
-            }
-            if (run == 2) continue;
-            sync();
-
-            // phase B: hypotheses = flagged slots, in CSR order; lane h holds
-            // hypothesis h's bundle offset (hso, bytes) and neighbour id (hid)
-            unsigned long long hm[NCH];
-            int nH = 0;
-#pragma unroll
-            for (int c = 0; c < NCH; ++c) {
-                const int i = 64 * c + lane;
-                hm[c] = __ballot(i < nL && hypf[i] != 0);
-                nH += __popcll(hm[c]);
-            }
-            // compacted through the list area like the slots (the barrier above
-            // ends every wave's reads of the slot list)
-            {
-                int pb = 0;
-#pragma unroll
-                for (int c = 0; c < NCH; ++c) {
-                    if ((hm[c] >> lane) & 1ULL) {
-                        const int h = pb + __popcll(hm[c] & lt_mask);
-                        lst[h] = (64 * c + lane) * K * 8;
-                        lst[64 * NCH + h] = rid[c];
-                    }
-                    pb += __popcll(hm[c]);
-                }
-            }
-            wave_sync();
-            int hso[NCH], hid[NCH];
-#pragma unroll
-            for (int c = 0; c < NCH; ++c) {
-                const int h = 64 * c + lane;
-                hso[c] = h < nH ? lst[h] : 0;
-                hid[c] = h < nH ? lst[64 * NCH + h] : 0;
-            }
-
-            if (nH > 0 && G >= 3) {  // no chain longer than 2 when G < 3
-                const char *blo_b = reinterpret_cast<const char *>(blo);
-                const char *bhi_b = reinterpret_cast<const char *>(bhi);
-                // phase C: growth (:479-536), seed j on wave j % W; the walk
-                // visits the hypotheses in CSR order, the seed at its own rank
-                for (int j = t; j < nH; j += W) {
-                    double lo[CPL], hi[CPL];
-                    const int soff = lane_get<NCH>(hso, j);
-#pragma unroll
-                    for (int m = 0; m < CPL; ++m) {
-                        lo[m] = *reinterpret_cast<const double *>(blo_b + soff + coff[m] * 8);
-                        hi[m] = *reinterpret_cast<const double *>(bhi_b + soff + coff[m] * 8);
-                    }
-                    int len = 1;
-                    int cur = lane == 0 ? a : 0;  // chain position l in lane l
-                    unsigned hsh = chain_hash(2166136261u, a);
-                    // The seed joins at its own distance rank (:496-510); its step
-                    // is an intersection with its own bundle, which leaves the
-                    // running bundle (inside the seed's) bit for bit unchanged.
-                    int h = 0;
-                    for (; h < nH && len < G; ++h) {
-                        double bl[CPL], bh[CPL];
-                        const int noff = lane_get<NCH>(hso, h);
-#pragma unroll
-                        for (int m = 0; m < CPL; ++m) {
-                            bl[m] = *reinterpret_cast<const double *>(blo_b + noff + coff[m] * 8);
-                            bh[m] = *reinterpret_cast<const double *>(bhi_b + noff + coff[m] * 8);
-                        }
-                        double nlo[CPL], nhi[CPL];
-                        unsigned long long okm = 0ULL;
-#pragma unroll
-                        for (int m = 0; m < CPL; ++m) {
-                            nlo[m] = (lo[m] < bl[m]) ? bl[m] : lo[m];  // bundle_intersection, :838-841
-                            nhi[m] = (hi[m] > bh[m]) ? bh[m] : hi[m];
-                            okm |= __builtin_amdgcn_ballot_w64(nhi[m] > nlo[m]) & lmask[m];
-                        }
-                        if (h == j || okm != 0ULL) {
-                            const int id = lane_get<NCH>(hid, h);
-                            cur = lane == len ? id : cur;
-                            hsh = chain_hash(hsh, id);
-#pragma unroll
-                            for (int m = 0; m < CPL; ++m) {
-                                lo[m] = nlo[m];
-                                hi[m] = nhi[m];
-                            }
-                            ++len;
-                        }
-                    }
-                    isect += static_cast<unsigned>(h - (j < h ? 1 : 0));  // steps other than the seed's
-                    int *rec = ski + j * SR;
-                    if (lane == 0) rec[0] = len;
-                    if (len <= 2) continue;  // :549
-                    // best cell of the running bundle (fill_curvelet_info, :202-226)
-                    int best = -1;
-#pragma unroll
-                    for (int m = 0; m < CPL; ++m) {
-                        const unsigned long long mask = __builtin_amdgcn_ballot_w64(hi[m] > lo[m]) & emask[m];
-                        if (best < 0 && mask != 0ULL) best = 64 * m + __builtin_ctzll(mask);
-                    }
-                    if (best < 0) best = A.rank_of_cell0;
-                    const int bm = best >> 6;
-                    const int bl = best & 63;
-                    double kmax = 0.0, kmin = 0.0;
-                    int best_cell = 0;
-#pragma unroll
-                    for (int m = 0; m < CPL; ++m) {
-                        if (m == bm) {
-                            kmax = bcast(hi[m], bl);
-                            kmin = bcast(lo[m], bl);
-                            best_cell = bcast(ccell[m], bl);
-                        }
-                    }
-                    if (lane < len) rec[3 + lane] = cur;
-                    if (lane == 0) {
-                        rec[1] = static_cast<int>(hsh);
-                        rec[2] = best_cell;
-                    }
-                    // the seed's row, staged at its own slot of the anchor; it is
-                    // kept unless an earlier seed has the same chain
-                    const long long q = static_cast<long long>(base) + nseed + j;
-                    if (lane < len) A.st_ids[q * A.st_stride + lane] = cur;
-                    if (lane == 0) {
-                        A.st_meta[q] = static_cast<unsigned>(len) | (run == 0 ? 0x8000u : 0u) |
-                                       (static_cast<unsigned>(best_cell) << 16);
-                        A.st_k[2 * q] = kmax;
-                        A.st_k[2 * q + 1] = kmin;
-                    }
-                }
-                sync();
-
-                // dedup (:546-560, 876-916), seed j on wave j % W: seed j is
-                // dropped when an earlier seed j' (length > 2) has the identical
-                // chain; the first of equal chains is the one the reference
-                // accepted, so "identical to an earlier accepted chain" and
-                // "identical to an earlier seed's chain" coincide.  Earlier seeds
-                // with the same length and hash are found in one ballot (lane =
-                // seed), then their chains compared element by element.
-                {
-                    int slen[NCH], shash[NCH];
-#pragma unroll
-                    for (int c = 0; c < NCH; ++c) {
-                        const int jj = 64 * c + lane;
-                        slen[c] = jj < nH ? ski[jj * SR] : 0;
-                        shash[c] = (jj < nH && slen[c] > 2) ? ski[jj * SR + 1] : 0;
-                    }
-                    for (int j = t; j < nH; j += W) {
-                        const int lj = lane_get<NCH>(slen, j);
-                        bool accept = lj > 2;
-                        if (accept) {
-                            const int hj = lane_get<NCH>(shash, j);
-#pragma unroll
-                            for (int c = 0; c < NCH; ++c) {
-                                unsigned long long cm =
-                                    __ballot(64 * c + lane < j && slen[c] == lj && shash[c] == hj);
-                                while (accept && cm != 0ULL) {
-                                    const int jp = 64 * c + __builtin_ctzll(cm);
-                                    cm &= cm - 1ULL;
-                                    const bool ne = lane < lj && ski[j * SR + 3 + lane] != ski[jp * SR + 3 + lane];
-                                    if (__ballot(ne) == 0ULL) accept = false;
-                                }
-                            }
-                        }
-                        if (lane == 0) accf[nseed + j] = accept ? 1 : 0;
-                    }
-                }
-            }
-            sync();  // the next run reuses the slots and seed records
-            nseed += nH;
-        }
-        // every slot of the anchor: its row among the anchor's accepted chains
-        // (run-0 seeds, then run-1 seeds, each in seed order), or -1
-        if (t == 0) {
-            int accn = 0;
-#pragma unroll
-            for (int c = 0; c < NCH; ++c) {
-                const int k = 64 * c + lane;
-                const bool ac = G >= 3 && k < nseed && accf[k] != 0;
-                const unsigned long long am = __ballot(ac);
-                if (k < deg) A.st_rank[base + k] = ac ? accn + __popcll(am & lt_mask) : -1;
-                accn += __popcll(am);
-            }
-            if (lane == 0) A.acc_count[a] = static_cast<unsigned>(accn);
-        }
-
-        // advance the pipeline
-        L = Ln;
-        a = na;
-        base = nbase;
-        deg = ndeg;
-        Ln = Lnn;
-        na = nna;
-        nbase = nnbase;
-        ndeg = nndeg;
-    }
-    if (lane == 0) {
-        if (vpw) atomicAdd(A.valid_pairs, vpw);
-        if (isect) atomicAdd(A.intersections, static_cast<unsigned long long>(isect));
-    }
-}
-
-using FusedKernel = void (*)(FusedArgs);
-
-// k_curvelets<CPL, NCH, GB, COOP> by (cells per lane, 64-neighbour chunks,
-// bundles in global memory, waves sharing one anchor)
-FusedKernel fused_kernel(int cpl, int nch, bool gb, bool coop)
-{
-#define CVG_FK(C, N)                                                                                         \
-    if (cpl == C && nch == N)                                                                                \
-        return gb ? k_curvelets<C, N, true, false> : (coop ? k_curvelets<C, N, false, true>                  \
-                                                           : k_curvelets<C, N, false, false>);
-    CVG_FK(1, 1) CVG_FK(1, 2) CVG_FK(1, 4)
-    CVG_FK(2, 1) CVG_FK(2, 2) CVG_FK(2, 4)
-    CVG_FK(4, 1) CVG_FK(4, 2) CVG_FK(4, 4)
-#undef CVG_FK
-    return nullptr;
-}
+#include "cvg_fused.hpp"
 
 struct RecordArgs {
-    int pairs;
+    int n;
     const double *x, *y, *th;
-    const int *pair_anchor;
     const int *map_of;        // per edge: its map (batches), or null
     const long long *map_eoff;  // per map: first edge id
-    const unsigned *row_off;
-    const int *st_rank;
-    const int *st_ids;
+    const unsigned *row_off;    // per anchor: its first row
+    const unsigned *off;        // per anchor: its first staging slot (CSR offset); its rows are the first ones
+    const int *ids;             // CSR neighbour ids
     const unsigned *st_meta;
+    // fused kernel's rows (row_meta): (hypotheses, chain) masks
+    const ulonglong2 *st_mask;
+    size_t mask_plane;
+    const double4 *rec;  // per edge (x, y, sin, cos)
+    const int *rank_cell;
+    ExactGrid exact;
+    double sin_dt, cos_dt, min_den;
+    // general kernel's rows: the chain's ids, k_max and k_min
+    const int *st_ids;
     const double *st_k;
     int st_stride;
     int G, kt;
@@ -2552,55 +1679,34 @@ struct RecordArgs {
     float nrad_f;
 };
 
-// record_curvelet_chain + fill_curvelet_info (cpu_curvelet.hpp:197-280) for
-// every accepted staging row, written at its compacted position
-// (compact_curvelet_output, :282-303).  One thread per staging slot q (one per
-// seed of the anchor, the rest unused): an accepted row carries its rank among
-// the anchor's accepted rows.  Chain ids are written 1-based and relative to
-// the anchor's map (batches concatenate maps).  F32: the float instantiation
-// (R.f32); each kernel instantiation holds only its own arithmetic.
 constexpr int kRecordChunk = 8;  // chain ids (and their coordinates) loaded together
 
-template <bool F32>
-__device__ inline void record_row(const RecordArgs &R, unsigned o, int q)
-{
-    using T = typename std::conditional<F32, float, double>::type;
-    const int a = R.pair_anchor[q];
-    const int id0 = R.map_of ? static_cast<int>(R.map_eoff[R.map_of[a]]) : 0;
-    const double ax = R.x[a], ay = R.y[a], at = R.th[a];
-    const int W = R.G + 1;
-    const unsigned meta = R.st_meta[q];
-    const int len = static_cast<int>(meta & 0x7fffu);
-    const bool fwd = (meta >> 15) & 1u;
-    const int c = static_cast<int>(meta >> 16);
-    const int *chain = R.st_ids + static_cast<long long>(q) * R.st_stride;
-    unsigned *row = R.chains + static_cast<long long>(o) * W;
-    row[0] = static_cast<unsigned>(a - id0) + 1;
-    // The chain row, and the chain's length: the distances between
-    // consecutive members in chain order (:231-240, sqrt in T).  Ids and
-    // coordinates come kRecordChunk at a time, so their loads overlap.
-    T length = 0;
-    T x1 = 0, y1 = 0;
-    for (int l0 = 0; l0 < R.G; l0 += kRecordChunk) {
-        int id[kRecordChunk];
-#pragma unroll
-        for (int u = 0; u < kRecordChunk; ++u) id[u] = l0 + u < len ? chain[l0 + u] : 0;
-#pragma unroll
-        for (int u = 0; u < kRecordChunk; ++u)
-            if (l0 + u < R.G) row[l0 + u + 1] = l0 + u < len ? static_cast<unsigned>(id[u] - id0) + 1 : 0u;
+// The running part of a row: the chain's ids into the row, its length the
+// distances between consecutive members in chain order (:231-240, sqrt in
+// T).  Ids and coordinates come kRecordChunk at a time, so that their loads
+// overlap.
+template <typename T>
+struct RowWalk {
+    const RecordArgs &R;
+    unsigned *row;
+    int id0;
+    int l = 0;
+    T length = 0, x1 = 0, y1 = 0;
+    __device__ void take(const int (&id)[kRecordChunk], int cnt)
+    {
         T xs[kRecordChunk], ys[kRecordChunk];
 #pragma unroll
         for (int u = 0; u < kRecordChunk; ++u) {
-            xs[u] = l0 + u < len ? static_cast<T>(R.x[id[u]]) : T(0);
-            ys[u] = l0 + u < len ? static_cast<T>(R.y[id[u]]) : T(0);
+            xs[u] = u < cnt ? static_cast<T>(R.x[id[u]]) : T(0);
+            ys[u] = u < cnt ? static_cast<T>(R.y[id[u]]) : T(0);
         }
 #pragma unroll
         for (int u = 0; u < kRecordChunk; ++u) {
-            const int l = l0 + u;
-            if (l >= len) continue;
-            if (l > 0) {
+            if (u >= cnt) continue;
+            row[l + u + 1] = static_cast<unsigned>(id[u] - id0) + 1;
+            if (l + u > 0) {
                 const T d2 = (x1 - xs[u]) * (x1 - xs[u]) + (y1 - ys[u]) * (y1 - ys[u]);
-                if constexpr (F32)
+                if constexpr (std::is_same<T, float>::value)
                     length += cvg::sqrt_f(d2);
                 else
                     length += sqrt(d2);
@@ -2608,87 +1714,326 @@ __device__ inline void record_row(const RecordArgs &R, unsigned o, int q)
             x1 = xs[u];
             y1 = ys[u];
         }
+        l += cnt;
     }
+};
 
+// The rest of fill_curvelet_info (:242-256) for best cell c.
+__device__ inline void write_info(const RecordArgs &R, unsigned o, double ax, double ay, double at, bool fwd, int c,
+                                  double k_max, double k_min, double length, int len)
+{
     double *inf = R.info + static_cast<long long>(o) * kInfoWidth;
-    if constexpr (F32) {
-        // fill_curvelet_info<float> (:197-256): every value a float, std::sin,
-        // std::cos and std::sqrt the float functions
-        const float fx = static_cast<float>(ax), fy = static_cast<float>(ay), ft = static_cast<float>(at);
-        const float ox = R.inf_x[c / R.kt];
-        const float ot = R.inf_t[c % R.kt];
-        const float k_max = static_cast<float>(R.st_k[2 * static_cast<long long>(q)]);
-        const float k_min = static_cast<float>(R.st_k[2 * static_cast<long long>(q) + 1]);
-        const float kk = (k_max + k_min) / 2.0f;
-        const float theta = cvg::wrap_two_pi_f(ft + ot);
-        float s, cth;
-        cvg::cr_sincosf<false>(theta, c_sincos_tab, &s, &cth);  // theta in [0, 2 pi)
-        const float px = fx - ox * s;
-        const float py = fy + ox * cth;
-        const float quality = (length > 0.0f && len > 0)
-                                  ? 2.0f / (1.0f * R.nrad_f / length + 1.0f * length / static_cast<float>(len))
-                                  : 0.0f;
-        inf[0] = fwd ? 1.0 : 0.0;
-        inf[1] = k_max;
-        inf[2] = k_min;
-        inf[3] = ft;
-        inf[4] = px;
-        inf[5] = py;
-        inf[6] = theta;
-        inf[7] = kk;
-        inf[8] = length;
-        inf[9] = quality;
-    } else {
-        const double ox = R.off_x[c / R.kt];
-        const double ot = R.off_t[c % R.kt];
-        const double k_max = R.st_k[2 * static_cast<long long>(q)];
-        const double k_min = R.st_k[2 * static_cast<long long>(q) + 1];
-        const double kk = (k_max + k_min) / 2.0;
-        const double theta = cvg::wrap_two_pi(at + ot);
-        double s, cth;
-        cvg::cr_sincos<false>(theta, c_sincos_tab, &s, &cth);  // theta in [0, 2 pi)
-        const double px = ax - ox * s;
-        const double py = ay + ox * cth;
-        const double quality = (length > 0.0 && len > 0) ? 2.0 / (R.nrad / length + length / double(len)) : 0.0;
-        inf[0] = fwd ? 1.0 : 0.0;
-        inf[1] = k_max;
-        inf[2] = k_min;
-        inf[3] = at;
-        inf[4] = px;
-        inf[5] = py;
-        inf[6] = theta;
-        inf[7] = kk;
-        inf[8] = length;
-        inf[9] = quality;
+    const double ox = R.off_x[c / R.kt];
+    const double ot = R.off_t[c % R.kt];
+    const double kk = (k_max + k_min) / 2.0;
+    const double theta = cvg::wrap_two_pi(at + ot);
+    double s, cth;
+    cvg::cr_sincos<false>(theta, c_sincos_tab, &s, &cth);  // theta in [0, 2 pi)
+    const double px = ax - ox * s;
+    const double py = ay + ox * cth;
+    const double quality = (length > 0.0 && len > 0) ? 2.0 / (R.nrad / length + length / double(len)) : 0.0;
+    inf[0] = fwd ? 1.0 : 0.0;
+    inf[1] = k_max;
+    inf[2] = k_min;
+    inf[3] = at;
+    inf[4] = px;
+    inf[5] = py;
+    inf[6] = theta;
+    inf[7] = kk;
+    inf[8] = length;
+    inf[9] = quality;
+}
+
+// The same in float (fill_curvelet_info<float>): every value a float,
+// std::sin, std::cos and std::sqrt the float functions.
+__device__ inline void write_info_f(const RecordArgs &R, unsigned o, float fx, float fy, float ft, bool fwd, int c,
+                                    float k_max, float k_min, float length, int len)
+{
+    double *inf = R.info + static_cast<long long>(o) * kInfoWidth;
+    const float ox = R.inf_x[c / R.kt];
+    const float ot = R.inf_t[c % R.kt];
+    const float kk = (k_max + k_min) / 2.0f;
+    const float theta = cvg::wrap_two_pi_f(ft + ot);
+    float s, cth;
+    cvg::cr_sincosf<false>(theta, c_sincos_tab, &s, &cth);  // theta in [0, 2 pi)
+    const float px = fx - ox * s;
+    const float py = fy + ox * cth;
+    const float quality = (length > 0.0f && len > 0)
+                              ? 2.0f / (1.0f * R.nrad_f / length + 1.0f * length / static_cast<float>(len))
+                              : 0.0f;
+    inf[0] = fwd ? 1.0 : 0.0;
+    inf[1] = k_max;
+    inf[2] = k_min;
+    inf[3] = ft;
+    inf[4] = px;
+    inf[5] = py;
+    inf[6] = theta;
+    inf[7] = kk;
+    inf[8] = length;
+    inf[9] = quality;
+}
+
+// record_curvelet_chain + fill_curvelet_info (cpu_curvelet.hpp:197-280) for
+// row o of anchor a.  Chain ids are written 1-based and relative to the
+// anchor's map (batches concatenate maps).  From the general kernel's rows;
+// F32: the float instantiation.
+template <bool F32>
+__device__ inline void record_row(const RecordArgs &R, unsigned o, int a)
+{
+    using T = typename std::conditional<F32, float, double>::type;
+    const long long q = static_cast<long long>(R.off[a]) + (o - R.row_off[a]);
+    const int id0 = R.map_of ? static_cast<int>(R.map_eoff[R.map_of[a]]) : 0;
+    const double ax = R.x[a], ay = R.y[a], at = R.th[a];
+    const unsigned meta = R.st_meta[q];
+    const int len = static_cast<int>(meta & 0x7fffu);
+    const bool fwd = (meta >> 15) & 1u;
+    const int c = static_cast<int>(meta >> 16);
+    const int *chain = R.st_ids + q * R.st_stride;
+    RowWalk<T> walk{R, R.chains + static_cast<long long>(o) * (R.G + 1), id0};
+    walk.row[0] = static_cast<unsigned>(a - id0) + 1;
+    for (int l0 = 0; l0 < len; l0 += kRecordChunk) {
+        int id[kRecordChunk];
+#pragma unroll
+        for (int u = 0; u < kRecordChunk; ++u) id[u] = l0 + u < len ? chain[l0 + u] : 0;
+        walk.take(id, min(kRecordChunk, len - l0));
     }
+    for (int l = walk.l; l < R.G; ++l) walk.row[l + 1] = 0u;
+    if constexpr (F32)
+        write_info_f(R, o, static_cast<float>(ax), static_cast<float>(ay), static_cast<float>(at), fwd, c,
+                     static_cast<float>(R.st_k[2 * q]), static_cast<float>(R.st_k[2 * q + 1]), walk.length, len);
+    else
+        write_info(R, o, ax, ay, at, fwd, c, R.st_k[2 * q], R.st_k[2 * q + 1], walk.length, len);
+}
+
+// The same from the fused kernel's rows.  The chain's members are the marked
+// hypotheses; k_max and k_min are the smallest hi and largest lo over their
+// (and the seed's) bundles at the best cell.  Approximate bounds (do_anchor's
+// formulas in doubles) say which member sets each, and only that one's exact
+// bound is formed; where two are closer than the approximation can tell, or
+// one lies at the clamp, every member's.
+__device__ inline void record_row_fused(const RecordArgs &R, unsigned o, int a)
+{
+    const unsigned base = R.off[a];
+    const size_t q = static_cast<size_t>(base) + (o - R.row_off[a]);
+    const int id0 = R.map_of ? static_cast<int>(R.map_eoff[R.map_of[a]]) : 0;
+    const double4 ra = R.rec[a];
+    const double ax = ra.x, ay = ra.y, sa = ra.z, ca = ra.w, at = R.th[a];
+    const unsigned meta = R.st_meta[q];
+    const int c = R.rank_cell[meta & 0xffu];
+    const int words = (meta >> 9) & 1u ? 4 : 1;
+    const int seed = static_cast<int>(meta >> 10);
+    const ExactGrid &E = R.exact;
+    const double ox = E.off_x[c / R.kt];
+    const double T2t = at + E.off_t[c % R.kt];
+    double s2, c2;
+    cvg::cr_sincos<false>(T2t, c_sincos_tab, &s2, &c2);
+
+    // the hypotheses in order, four loads at a time
+    struct Slots {
+        const RecordArgs &R;
+        size_t q;
+        int words, w, s;
+        unsigned long long hyp, chain;
+        __device__ Slots(const RecordArgs &r, size_t q_, int words_) : R(r), q(q_), words(words_) { restart(); }
+        __device__ void restart()
+        {
+            const ulonglong2 m = R.st_mask[q];
+            w = s = 0;
+            hyp = m.x;
+            chain = m.y;
+        }
+        // the next hypothesis that is a member or the seed: its place in the
+        // neighbour list, or -1
+        __device__ int next(int seed, bool &member)
+        {
+            while (true) {
+                while (hyp == 0ULL) {
+                    if (++w >= words) return -1;
+                    hyp = R.st_mask[w * R.mask_plane + q].x;
+                }
+                const int r = 64 * w + __builtin_ctzll(hyp);
+                hyp &= hyp - 1ULL;
+                if ((s & 63) == 0 && s > 0) chain = R.st_mask[(s >> 6) * R.mask_plane + q].y;
+                member = chain & 1ULL;
+                chain >>= 1;
+                if (s++ == seed || member) return r;
+            }
+        }
+    };
+    constexpr int kChunk = 4;
+    unsigned *row = R.chains + static_cast<long long>(o) * (R.G + 1);
+    row[0] = static_cast<unsigned>(a - id0) + 1;
+    row[1] = row[0];  // the chain starts with the anchor
+    int len = 1;
+    double length = 0.0, x1 = ax, y1 = ay;
+    const double inf = __builtin_inf();
+    double lo1 = -inf, lo2 = -inf, hi1 = inf, hi2 = inf;
+    int lo_id = -1, hi_id = -1;
+    bool vague = false;
+    {
+        Slots it(R, q, words);
+        for (bool more = true; more;) {
+            int id[kChunk];
+            bool member[kChunk];
+            double4 v[kChunk];
+#pragma unroll
+            for (int u = 0; u < kChunk; ++u) {
+                member[u] = false;
+                const int r = more ? it.next(seed, member[u]) : -1;
+                more = r >= 0;
+                id[u] = more ? R.ids[base + r] : -1;
+            }
+#pragma unroll
+            for (int u = 0; u < kChunk; ++u) v[u] = R.rec[id[u] >= 0 ? id[u] : a];
+#pragma unroll
+            for (int u = 0; u < kChunk; ++u) {
+                if (id[u] < 0) continue;
+                const double DX = ax - v[u].x, DY = ay - v[u].y;
+                if (member[u]) {
+                    const double d2 = (x1 - v[u].x) * (x1 - v[u].x) + (y1 - v[u].y) * (y1 - v[u].y);  // :231-240
+                    length += sqrt(d2);
+                    x1 = v[u].x;
+                    y1 = v[u].y;
+                    ++len;
+                    row[len] = static_cast<unsigned>(id[u] - id0) + 1;
+                }
+                if (DX * DX + DY * DY < E.close_thr) continue;  // the default bundle
+                const bool branch_a = (DX * ca + DY * sa) < 0;
+                const double sn = v[u].z, cn = v[u].w;
+                const double sd = branch_a ? -R.sin_dt : R.sin_dt;  // the lower constraint's theta_n -+ dt
+                const double s0n = __builtin_fma(sn, R.cos_dt, cn * sd), c0n = __builtin_fma(cn, R.cos_dt, -(sn * sd));
+                const double s1n = __builtin_fma(sn, R.cos_dt, -(cn * sd)), c1n = __builtin_fma(cn, R.cos_dt, sn * sd);
+                const double tt = __builtin_fma(s2, DX, -(c2 * DY));
+                const double den =
+                    __builtin_fma(-2.0 * ox, tt, __builtin_fma(DX, DX, __builtin_fma(DY, DY, -E.dx2)) + ox * ox);
+                const double s0 = __builtin_fma(s2, c0n, -(c2 * s0n)), s1 = __builtin_fma(s2, c1n, -(c2 * s1n));
+                const double d0 = __builtin_fma(-s0, ox, __builtin_fma(DX, c0n, DY * s0n));
+                const double d1 = __builtin_fma(-s1, ox, __builtin_fma(DX, c1n, DY * s1n));
+                vague = vague || !(fabs(den) >= R.min_den && fabs(d0) >= R.min_den && fabs(d1) >= R.min_den);
+                const double pp = den * d0, ppp = pp * d1;
+                double y = __builtin_amdgcn_rcp(ppp);
+                y = __builtin_fma(y, __builtin_fma(-ppp, y, 1.0), y);
+                const double w = y * d1, yx = 2.0 * (w * d0);
+                const double lo = fmax((tt - ox - E.dx) * yx, s0 * (w * den));
+                const double hi = fmin((tt - ox + E.dx) * yx, s1 * (y * pp));
+                if (lo > lo1) {
+                    lo2 = lo1;
+                    lo1 = lo;
+                    lo_id = id[u];
+                } else {
+                    lo2 = fmax(lo2, lo);
+                }
+                if (hi < hi1) {
+                    hi2 = hi1;
+                    hi1 = hi;
+                    hi_id = id[u];
+                } else {
+                    hi2 = fmin(hi2, hi);
+                }
+            }
+        }
+    }
+    for (int l = len; l < R.G; ++l) row[l + 1] = 0u;
+
+    // each approximate bound is within max_k 2^-27 of the exact one
+    double k_min = -E.max_k, k_max = E.max_k;
+    const double tol = E.max_k * 0x1p-25;
+    const bool lo_at = lo1 >= -E.max_k - tol, hi_at = hi1 <= E.max_k + tol;  // not at the clamp
+    const bool all_lo = vague || (lo_at && !(lo1 - lo2 > tol && lo1 > -E.max_k + tol));
+    const bool all_hi = vague || (hi_at && !(hi2 - hi1 > tol && hi1 < E.max_k - tol));
+#pragma unroll 1
+    for (int side = 0; side < 2; ++side) {
+        const bool upper = side != 0, all = upper ? all_hi : all_lo;
+        double v = upper ? k_max : k_min;
+        int id = all || !(upper ? hi_at : lo_at) ? -1 : (upper ? hi_id : lo_id);
+        int seed_id = -1;
+        Slots it(R, q, words);
+        bool member;
+        if (all) {
+            // the running bundle in the order it was formed: the seed's first
+            // (bundle_intersection, :838-841)
+            int r;
+            for (int s = -1; s != seed;) {
+                r = it.next(seed, member);
+                s = it.s - 1;
+            }
+            id = seed_id = R.ids[base + r];
+            it.restart();
+        }
+        while (id >= 0) {
+            const double e = exact_bound(E, upper, ax, ay, sa, ca, T2t, s2, c2, ox, id);
+            if (upper ? v > e : v < e) v = e;
+            if (!all) break;
+            do {
+                const int r = it.next(seed, member);
+                id = r >= 0 ? R.ids[base + r] : -1;
+            } while (id == seed_id);
+        }
+        k_max = upper ? v : k_max;
+        k_min = upper ? k_min : v;
+    }
+    write_info(R, o, ax, ay, at, (meta >> 8) & 1u, c, k_max, k_min, length, len);
 }
 
 // compact_curvelet_output (cpu_curvelet.hpp:282-303) in two passes.  First,
-// one thread per staging slot: an accepted slot (its rank among the anchor's
-// accepted rows, or -1) names its output row in slot_of_row.  Then one thread
-// per output row records it; the row count (the last row offset) stays on
-// the device, and the rows beyond the caller's buffers are left out (the host
-// reports them).
-__global__ __launch_bounds__(kBlock) void k_row_slots(RecordArgs R, int *__restrict__ slot_of_row,
-                                                      const unsigned *__restrict__ num_rows, unsigned *__restrict__ scal)
+// one thread per anchor: its rows (contiguous, from its row offset) learn
+// their anchor.  Then one thread per output row records it; the row count
+// (the last row offset) stays on the device, and rows beyond the caller's
+// buffers are left out (the host reports them).  Block 0 also puts the
+// counts the host reads into the scalars: the rows, and with `partial` the
+// fused kernel's per-wave sums (adding those up with atomics on one address
+// would cost ~11 ns each, 45 us for 4,096 waves at the kernel's end).
+__global__ __launch_bounds__(kBlock) void k_row_anchors(int n, const unsigned *__restrict__ row_off, unsigned max_rows,
+                                                        int *__restrict__ row_anchor,
+                                                        const unsigned *__restrict__ partial, int waves,
+                                                        unsigned *__restrict__ scal)
 {
-    const int q = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-    if (q == 0) scal[S_ROWS] = *num_rows;  // read back with the other scalars
-    if (q >= R.pairs) return;
-    const int rk = R.st_rank[q];
-    if (rk < 0) return;
-    const unsigned o = R.row_off[R.pair_anchor[q]] + static_cast<unsigned>(rk);
-    if (o < R.max_rows) slot_of_row[o] = q;
+    const int a = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+    if (a < n) {
+        const unsigned o1 = min(row_off[a + 1], max_rows);
+        for (unsigned o = row_off[a]; o < o1; ++o) row_anchor[o] = a;
+    }
+    if (blockIdx.x != 0) return;
+    if (threadIdx.x == 0) scal[S_ROWS] = row_off[n];
+    if (!partial) return;
+    unsigned long long vp = 0, is = 0;
+    for (int w = static_cast<int>(threadIdx.x); w < waves; w += kBlock) {
+        vp += partial[3 * w];
+        is += static_cast<unsigned long long>(partial[3 * w + 1]) |
+              static_cast<unsigned long long>(partial[3 * w + 2]) << 32;
+    }
+    __shared__ unsigned long long s_vp[kBlock / 64], s_is[kBlock / 64];
+    vp = wave_sum_u64(vp);
+    is = wave_sum_u64(is);
+    if ((threadIdx.x & 63) == 0) {
+        s_vp[threadIdx.x >> 6] = vp;
+        s_is[threadIdx.x >> 6] = is;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kBlock / 64; ++w) {
+            vp += s_vp[w];
+            is += s_is[w];
+        }
+        scal[S_VALID] = static_cast<unsigned>(vp);
+        scal[S_COUNT] = static_cast<unsigned>(is);
+        scal[S_COUNT + 1] = static_cast<unsigned>(is >> 32);
+    }
 }
 
-template <bool F32>
-__global__ __launch_bounds__(kBlock) void k_record(RecordArgs R, const int *__restrict__ slot_of_row,
-                                                   const unsigned *__restrict__ num_rows)
+enum { ROWS_FUSED = 0, ROWS_GENERAL = 1, ROWS_FLOAT = 2 };
+
+template <int KIND>
+__global__ __launch_bounds__(kBlock) void k_record(RecordArgs R, const int *__restrict__ row_anchor)
 {
-    const unsigned rows = min(*num_rows, R.max_rows);
+    const unsigned rows = min(R.row_off[R.n], R.max_rows);
     const unsigned stride = gridDim.x * blockDim.x;
-    for (unsigned o = blockIdx.x * blockDim.x + threadIdx.x; o < rows; o += stride)
-        record_row<F32>(R, o, slot_of_row[o]);
+    for (unsigned o = blockIdx.x * blockDim.x + threadIdx.x; o < rows; o += stride) {
+        if constexpr (KIND == ROWS_FUSED)
+            record_row_fused(R, o, row_anchor[o]);
+        else
+            record_row<KIND == ROWS_FLOAT>(R, o, row_anchor[o]);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -2846,7 +2191,6 @@ struct GenArgs {
     int *st_ids;
     unsigned *st_meta;
     double *st_k;
-    int *st_rank;
     unsigned *acc_count;
     unsigned *valid_pairs;
     unsigned long long *intersections;
@@ -3027,7 +2371,6 @@ __global__ __launch_bounds__(64 * kGenWaves) void k_curvelets_generic(GenArgs<T>
                 wave_sync();  // the dedup row is read by every lane
             }
         }
-        for (int k = lane; k < deg; k += 64) A.st_rank[base + k] = k < static_cast<int>(nacc) ? k : -1;
         if (lane == 0) A.acc_count[a] = nacc;
         wave_sync();  // the scratch is rewritten by the next anchor
     }
@@ -3169,14 +2512,7 @@ int read_scalars(cvg_context *ctx)
 
 constexpr int kSpecMiss = 1000;  // internal: a guessed size did not hold (never returned to callers)
 
-int queue_edge_trig(cvg_context *ctx, const cvg_params &p);
-int queue_pair_setup(cvg_context *ctx, const cvg_params &p, unsigned long long pair_cap);
-// Bytes of the pair-flag buffer for pairs pairs: whole 32-bit words, since
-// k_bucket reads each anchor's run of flags a word at a time.
-inline size_t cls_bytes(unsigned long long pairs)
-{
-    return static_cast<size_t>((pairs + 4) & ~3ULL);
-}
+int queue_setup(cvg_context *ctx);
 
 // Neighbour counts, CSR offsets, then the gathering pass, the distance sort
 // and the CSR fill (preprocess.hpp:186-274) over either cell layout.  The
@@ -3222,6 +2558,7 @@ int graph_scans(cvg_context *ctx, const Cells &cells, int n, unsigned R, unsigne
         if (ctx->max_deg >= (1u << 23))
             return fail(ctx, CVG_ERR_UNSUPPORTED, "an anchor has 2^23 or more neighbours");
         ctx->truncated = ctx->mailbox[S_TRUNC];
+        ctx->wide_theta = ctx->mailbox[S_WIDE] != 0;
         return CVG_OK;
     };
     int fill_cap;
@@ -3229,7 +2566,7 @@ int graph_scans(cvg_context *ctx, const Cells &cells, int n, unsigned R, unsigne
     if (spec) {
         fill_cap = ctx->spec_fill_cap;
         pair_cap = std::min({ctx->d_cand.bytes / sizeof(Cand), ctx->d_ids.bytes / sizeof(int),
-                             ctx->d_d2.bytes / sizeof(double), ctx->d_pair_anchor.bytes / sizeof(int)});
+                             ctx->d_d2.bytes / sizeof(double)});
         // below the fill's saturated offset, so that any saturated sum misses
         pair_cap = std::min<unsigned long long>(pair_cap, kFillSumMax - 1);
     } else {
@@ -3239,7 +2576,6 @@ int graph_scans(cvg_context *ctx, const Cells &cells, int n, unsigned R, unsigne
         CVG_TRY(ensure(ctx, ctx->d_cand, np * sizeof(Cand)));
         CVG_TRY(ensure(ctx, ctx->d_ids, np * sizeof(int)));
         CVG_TRY(ensure(ctx, ctx->d_d2, np * sizeof(double)));
-        CVG_TRY(ensure(ctx, ctx->d_pair_anchor, np * sizeof(int)));
         fill_cap = static_cast<int>(std::max(ctx->max_deg, 1u));
         pair_cap = np;
     }
@@ -3248,7 +2584,7 @@ int graph_scans(cvg_context *ctx, const Cells &cells, int n, unsigned R, unsigne
     // its candidates in LDS
     using FillFn = void (*)(int, const double *, const double *, const int *, const int *, Cells, int, double,
                             const int *, const int *, const double2 *, unsigned *, Cand *, int *, double *,
-                            int *, int *, unsigned, int, const int *, const long long *, unsigned *, bool,
+                            int *, unsigned, int, const int *, const long long *, unsigned *, bool,
                             unsigned long long, unsigned long long *, unsigned, unsigned);
     const size_t per_seg = static_cast<size_t>(fill_seg_doubles(fill_cap, count_in_fill)) * sizeof(double);
     int G = ctx->fill_lanes;
@@ -3289,7 +2625,7 @@ int graph_scans(cvg_context *ctx, const Cells &cells, int n, unsigned R, unsigne
                        st, n, as<double>(ctx->d_x), as<double>(ctx->d_y), as<int>(ctx->d_cx), as<int>(ctx->d_cy),
                        cells, static_cast<int>(R), rad2, as<int>(ctx->d_sorted), as<int>(ctx->d_scell),
                        as<double2>(ctx->d_sxy), as<unsigned>(ctx->d_off), as<Cand>(ctx->d_cand),
-                       as<int>(ctx->d_ids), as<double>(ctx->d_d2), as<int>(ctx->d_pair_anchor),
+                       as<int>(ctx->d_ids), as<double>(ctx->d_d2),
                        as<int>(ctx->d_tmp_ids), max_cand, fill_cap, num_maps > 1 ? as<int>(ctx->d_map) : nullptr,
                        as<long long>(ctx->d_eoff), scal, ctx->f32, pair_cap, lb, epoch, ctx->lookback_spins);
     hipLaunchKernelGGL(k_tie_sort, dim3(std::min(blocks_for(n), 64)), dim3(kBlock), 0, st, as<int>(ctx->d_tmp_ids),
@@ -3298,24 +2634,21 @@ int graph_scans(cvg_context *ctx, const Cells &cells, int n, unsigned R, unsigne
     CVG_HIP(ctx, hipGetLastError());
     if (spec) {
         // the sizes come back while the device already runs the curvelet
-        // stage's per-edge trig
+        // stage's first kernels
         CVG_HIP(ctx, hipMemcpyAsync(ctx->mailbox, ctx->d_scal.ptr, kScalarWords * sizeof(unsigned),
                                     hipMemcpyDeviceToHost, st));
         CVG_HIP(ctx, hipEventRecord(ctx->ev_read, st));
-        if (ctx->early_params && !ctx->edge_trig_queued) {
-            CVG_TRY(queue_edge_trig(ctx, *ctx->early_params));
-            CVG_TRY(queue_pair_setup(ctx, *ctx->early_params, pair_cap));
-        }
+        if (ctx->early_setup) CVG_TRY(queue_setup(ctx));
         CVG_HIP(ctx, hipEventSynchronize(ctx->ev_read));
         if (ctx->mailbox[S_BAD] || ctx->mailbox[S_MISS]) {
-            // the queued per-pair launch found the miss and did nothing: the
-            // graph built again queues it again (k_edge_trig's rows still hold)
-            ctx->pair_setup_queued = false;
+            // k_order found the miss and did nothing: the graph built again
+            // needs both kernels again
+            ctx->setup_queued = false;
             return kSpecMiss;  // the exact path reports bad input
         }
         const int rc = take_counts();
         if (rc != CVG_OK) {
-            ctx->pair_setup_queued = false;
+            ctx->setup_queued = false;
             return rc;
         }
     }
@@ -3379,8 +2712,7 @@ int build_graph(cvg_context *ctx, int n, int sz, const double *d_edges, double r
     ctx->graph_ready = false;
     ctx->curvelets_ready = false;
     ctx->counts_pending = false;
-    ctx->edge_trig_queued = false;  // a new graph: its per-edge trig is queued again
-    ctx->pair_setup_queued = false;
+    ctx->setup_queued = false;  // a new graph: its edge records and lists are queued again
     if (n <= 0 || sz < 4 || d_edges == nullptr)  // preprocess.hpp:197
         return fail(ctx, CVG_ERR_INVALID_ARGUMENT, "build_neighbor_csr_graph: need num_edges > 0, sz_edge_data >= 4");
     if (R > 4096) return fail(ctx, CVG_ERR_UNSUPPORTED, "neighbor_radius above 4096 cells");
@@ -3600,8 +2932,8 @@ struct Derived {
     double dt, dx, dx2, close_thr, max_k, nrad;
     unsigned kx, kt, K, G;
     int cpl;
-    std::vector<double> off_x, off_t, rank_ox;
-    std::vector<int> rank_j, rank_cell, rank_elig;
+    std::vector<double> off_x, off_t, rank_ox, rank_ot, rank_so, rank_co;
+    std::vector<int> rank_cell, rank_elig;
     int rank_of_cell0;
 };
 
@@ -3637,73 +2969,81 @@ int derive(cvg_context *ctx, const cvg_params &p, Derived &d)
     }
     std::stable_sort(order.begin(), order.end(), [&](int u, int v) { return dist[u] < dist[v]; });
     d.rank_ox.resize(d.K);
-    d.rank_j.resize(d.K);
+    d.rank_ot.resize(d.K);
+    d.rank_so.resize(d.K);
+    d.rank_co.resize(d.K);
     d.rank_cell.resize(d.K);
     d.rank_elig.resize(d.K);
     for (unsigned r = 0; r < d.K; ++r) {
         const int c = order[r];
         d.rank_cell[r] = c;
         d.rank_ox[r] = d.off_x[c / d.kt];
-        d.rank_j[r] = c % d.kt;
+        d.rank_ot[r] = d.off_t[c % d.kt];
+        d.rank_so[r] = std::sin(d.off_t[c % d.kt]);
+        d.rank_co[r] = std::cos(d.off_t[c % d.kt]);
         d.rank_elig[r] = dist[c] < 100.0 ? 1 : 0;
         if (c == 0) d.rank_of_cell0 = static_cast<int>(r);
     }
     return CVG_OK;
 }
 
-// Per-edge trig of the fused stage (k_edge_trig), which needs only the
-// edges' orientations and the parameters: queued by build_curvelets, or
-// earlier, while the graph stage's last host read is in flight.
-int queue_edge_trig(cvg_context *ctx, const cvg_params &p)
+// The fused stage's edge records and anchor lists, which need only the graph:
+// queued by build_curvelets, or earlier, while the graph stage's last host
+// read is in flight.
+int queue_setup(cvg_context *ctx)
 {
-    Derived d;
-    CVG_TRY(derive(ctx, p, d));
     const int n = ctx->n;
-    if (static_cast<unsigned long long>(n) * (d.kt + 3) > 0xffffffffull)
-        return fail(ctx, CVG_ERR_UNSUPPORTED, "more than 2^32 (edge, angle) items in one run");
-    const int ntrig = cvg::TRIG_GRID + 2 * static_cast<int>(d.kt);
-    CVG_TRY(ensure(ctx, ctx->d_trig, static_cast<size_t>(ntrig) * n * sizeof(double)));
-    CVG_TRY(ensure(ctx, ctx->d_tdd, static_cast<size_t>(8 + 4 * d.kt) * n * sizeof(double)));
-    hipLaunchKernelGGL(k_edge_trig, dim3(blocks_for(static_cast<long long>(n) * (d.kt + 3))), dim3(kBlock), 0,
-                       ctx->stream, n, as<double>(ctx->d_th), d.dt, static_cast<int>(d.kt), p.st,
-                       as<double>(ctx->d_trig), as<double>(ctx->d_tdd), as<unsigned>(ctx->d_scal));
+    CVG_TRY(ensure(ctx, ctx->d_rec, static_cast<size_t>(n) * sizeof(double4)));
+    CVG_TRY(ensure(ctx, ctx->d_lists, static_cast<size_t>(kLists) * n * sizeof(int4)));
+    CVG_TRY(ensure(ctx, ctx->d_acc, static_cast<size_t>(n) * sizeof(unsigned)));
+    hipLaunchKernelGGL(k_edge_rec, dim3(blocks_for(n)), dim3(kBlock), 0, ctx->stream, n, as<double>(ctx->d_x),
+                       as<double>(ctx->d_y), as<double>(ctx->d_th), as<double4>(ctx->d_rec),
+                       as<unsigned>(ctx->d_scal));
+    hipLaunchKernelGGL(k_order, dim3(blocks_for(n, kOrderBlock)), dim3(kOrderBlock), 0, ctx->stream, n,
+                       as<int>(ctx->d_sorted), as<unsigned>(ctx->d_off), as<int4>(ctx->d_lists),
+                       as<unsigned>(ctx->d_acc), as<unsigned>(ctx->d_scal));
     CVG_HIP(ctx, hipGetLastError());
-    ctx->edge_trig_queued = true;
+    ctx->setup_queued = true;
     return CVG_OK;
 }
 
-// The per-pair records and sines (k_pair_trig with the record, Kt = 7),
-// queued behind k_edge_trig while the graph stage's count read is in flight:
-// the launch covers the CSR buffers' capacity pair_cap and takes the pair
-// count from the device.  Only where the pair buffers already hold that
-// capacity: nothing is allocated before the counts are known.
-int queue_pair_setup(cvg_context *ctx, const cvg_params &p, unsigned long long pair_cap)
+// Whether the fused kernel's fixed-point bounds can be trusted for this graph
+// and these parameters, and the smallest denominator at which they can (a
+// smaller one is settled by its certain sign, with quotients far beyond
+// max_k, or leaves the cell open); min_prod bounds the product of the three
+// where one is that small.
+//
+// u = 2^-53; S >= |DX| + |DY| over the window, X = dx + max |delta_x2|,
+// B = S + X.  Angles are below 72 (|theta| <= 64), so theta + delta is rounded
+// by up to 64 u and a difference of two by 128 u.  Against the reference's own
+// rounded evaluation:
+//   rotated sin/cos              68 u     (64 u the angle, the rest rounding)
+//   s0, s1                      352 u     (two rotated pairs, the difference)
+//   numerators                  max(152 B, 352) u
+//   denominators                max(64 B^2, 360 B) u
+// A quotient up to 2 max_k is then off by at most
+// (num error + 2 max_k den error) / |den|.  min_den keeps four times that
+// within 8 fixed-point units (max_k 2^-27).  num_err and den_err are four times the errors.
+struct FusedLimits {
+    double min_den, num_err, den_err, min_prod;
+};
+
+bool fused_limits(const cvg_context *ctx, const Derived &d, FusedLimits *lim)
 {
-    Derived d;
-    CVG_TRY(derive(ctx, p, d));
-    constexpr int kt = 7;
-    if (d.kt != kt || ctx->arena || pair_cap == 0 || pair_cap > static_cast<unsigned long long>(INT_MAX))
-        return CVG_OK;
-    // after a much larger map the capacity would launch mostly idle
-    // workgroups: then the launch waits for the count (ctx->pairs still holds
-    // the last graph's)
-    if (pair_cap > 2ULL * static_cast<unsigned long long>(std::max(ctx->pairs, 0)) + 65536ULL) return CVG_OK;
-    if (ctx->d_cls.bytes < cls_bytes(pair_cap) || ctx->d_prec.bytes < pair_cap * 8 * sizeof(double) ||
-        ctx->d_psin.bytes < pair_cap * kt * 2 * sizeof(double))
-        return CVG_OK;
-    const int cap = static_cast<int>(pair_cap);
-    const int n = ctx->n;
-    const PrepArgs P{as<double>(ctx->d_x), as<double>(ctx->d_y), as<double>(ctx->d_trig), d.close_thr,
-                     as<unsigned char>(ctx->d_cls), as<double>(ctx->d_prec)};
-    const auto fn = k_pair_trig<kt, true>;
-    hipLaunchKernelGGL(fn, dim3(blocks_for(cap)), dim3(kBlock), kBlock * kt * sizeof(double2),
-                       ctx->stream, cap, n, kt, as<int>(ctx->d_pair_anchor), as<int>(ctx->d_ids),
-                       static_cast<const unsigned char *>(as<unsigned char>(ctx->d_cls)), as<double>(ctx->d_th), p.st,
-                       d.dt, as<double>(ctx->d_tdd), as<double>(ctx->d_psin), P,
-                       static_cast<const unsigned *>(as<unsigned>(ctx->d_scal)));
-    CVG_HIP(ctx, hipGetLastError());
-    ctx->pair_setup_queued = true;
-    return CVG_OK;
+    double xmax = 0.0, tmax = std::fabs(d.dt);
+    for (double v : d.off_x) xmax = std::max(xmax, std::fabs(v));
+    for (double v : d.off_t) tmax = std::max(tmax, std::fabs(v));
+    double S = 2.0 * (static_cast<double>(ctx->nbr_radius) + 1.0);
+    if (ctx->rad >= 0.0) S = std::min(S, 1.5 * ctx->rad);
+    const double B = S + d.dx + xmax;
+    if (!(d.dx >= 0.0) || !(d.max_k > 0.0) || !(tmax <= 8.0) || !(B <= 1e5) || ctx->wide_theta) return false;
+    const double u = std::ldexp(1.0, -53);
+    const double num = std::max(152.0 * B, 352.0) * u, den = std::max(64.0 * B * B, 360.0 * B) * u;
+    lim->num_err = 4.0 * num;
+    lim->den_err = 4.0 * den;
+    lim->min_den = 4.0 * (num + 2.0 * d.max_k * den) / (d.max_k * std::ldexp(1.0, -27));
+    lim->min_prod = 1.01 * lim->min_den * B * std::max(B, B * B + d.dx2);
+    return lim->min_den <= 0.05;
 }
 
 // The parameter tables to d_tables, unless the same bytes are already there
@@ -3841,11 +3181,12 @@ int finish_curvelets(cvg_context *ctx)
 
 // compact_curvelet_output + record_curvelet_chain (cpu_curvelet.hpp:258-303):
 // row offsets from the per-anchor accepted counts, then every accepted
-// staging row to its row (R carries the grid and info parameters), and the
-// counts back with the stream.  Outputs are sized by their bound (one row per
+// staging row to its row (R carries the grid and info parameters; fused_waves:
+// the fused kernel's per-wave sums to add up), and the counts back with the
+// stream.  Outputs are sized by their bound (one row per
 // CSR pair at most), so the record runs without a host round trip; the
 // counts are read at the first query (finish_curvelets).
-int record_rows(cvg_context *ctx, const cvg_params &p, RecordArgs R, int st_stride)
+int record_rows(cvg_context *ctx, const cvg_params &p, RecordArgs R, int st_stride, int fused_waves)
 {
     hipStream_t st = ctx->stream;
     const int n = ctx->n;
@@ -3861,35 +3202,35 @@ int record_rows(cvg_context *ctx, const cvg_params &p, RecordArgs R, int st_stri
         out_chains = as<unsigned>(ctx->d_chains);
         out_info = as<double>(ctx->d_info);
     }
-    R.pairs = pairs;
-    R.pair_anchor = as<int>(ctx->d_pair_anchor);
+    R.n = n;
     R.map_of = ctx->num_maps > 1 ? as<int>(ctx->d_map) : nullptr;
     R.map_eoff = as<long long>(ctx->d_eoff);
     R.x = as<double>(ctx->d_x);
     R.y = as<double>(ctx->d_y);
     R.th = as<double>(ctx->d_th);
-    R.st_rank = as<int>(ctx->d_st_rank);
     R.row_off = as<unsigned>(ctx->d_rowoff);
-    R.st_ids = as<int>(ctx->d_st_ids);
+    R.off = as<unsigned>(ctx->d_off);
+    R.ids = as<int>(ctx->d_ids);
     R.st_meta = as<unsigned>(ctx->d_st_meta);
+    R.st_ids = as<int>(ctx->d_st_ids);
     R.st_k = as<double>(ctx->d_st_k);
     R.st_stride = st_stride;
     R.chains = out_chains;
     R.info = out_info;
     R.max_rows = ctx->caller_chains ? ctx->caller_rows : UINT_MAX;
     if (pairs > 0) {
-        CVG_TRY(ensure(ctx, ctx->d_rowslot, np * sizeof(int)));
-        int *slots = as<int>(ctx->d_rowslot);
-        hipLaunchKernelGGL(k_row_slots, dim3(blocks_for(pairs)), dim3(kBlock), 0, st, R, slots,
-                           static_cast<const unsigned *>(as<unsigned>(ctx->d_rowoff) + n), as<unsigned>(ctx->d_scal));
+        CVG_TRY(ensure(ctx, ctx->d_rowanchor, np * sizeof(int)));
+        int *row_anchor = as<int>(ctx->d_rowanchor);
+        hipLaunchKernelGGL(k_row_anchors, dim3(blocks_for(n)), dim3(kBlock), 0, st, n, R.row_off, R.max_rows,
+                           row_anchor, static_cast<const unsigned *>(fused_waves > 0 ? as<unsigned>(ctx->d_partial) : nullptr),
+                           fused_waves, as<unsigned>(ctx->d_scal));
         // a resident grid strides over the rows (their count is on the device)
-        const auto rec = R.f32 ? k_record<true> : k_record<false>;
+        const auto rec = R.f32 ? k_record<ROWS_FLOAT> : (fused_waves > 0 ? k_record<ROWS_FUSED> : k_record<ROWS_GENERAL>);
         int occ = 0;
         CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(rec), kBlock, 0, &occ));
         const long long resident = static_cast<long long>(std::max(occ, 1)) * ctx->num_cu;
         const int grid = static_cast<int>(std::min(resident, static_cast<long long>(blocks_for(pairs))));
-        hipLaunchKernelGGL(rec, dim3(grid), dim3(kBlock), 0, st, R, static_cast<const int *>(slots),
-                           static_cast<const unsigned *>(as<unsigned>(ctx->d_rowoff) + n));
+        hipLaunchKernelGGL(rec, dim3(grid), dim3(kBlock), 0, st, R, static_cast<const int *>(row_anchor));
     }
     CVG_HIP(ctx, hipGetLastError());
     // the counts (the row count in S_ROWS when there are pairs; none otherwise)
@@ -3979,7 +3320,6 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
     CVG_TRY(ensure(ctx, ctx->d_st_ids, np * cap * sizeof(int)));
     CVG_TRY(ensure(ctx, ctx->d_st_meta, np * sizeof(unsigned)));
     CVG_TRY(ensure(ctx, ctx->d_st_k, np * 2 * sizeof(double)));
-    CVG_TRY(ensure(ctx, ctx->d_st_rank, np * sizeof(int)));
     CVG_TRY(ensure(ctx, ctx->d_acc, static_cast<size_t>(n) * sizeof(unsigned)));
     CVG_TRY(ensure(ctx, ctx->d_rowoff, static_cast<size_t>(n + 1) * sizeof(unsigned)));
     unsigned *scal = as<unsigned>(ctx->d_scal);
@@ -4027,7 +3367,6 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
     A.st_ids = as<int>(ctx->d_st_ids);
     A.st_meta = as<unsigned>(ctx->d_st_meta);
     A.st_k = as<double>(ctx->d_st_k);
-    A.st_rank = as<int>(ctx->d_st_rank);
     A.acc_count = as<unsigned>(ctx->d_acc);
     A.valid_pairs = scal + S_VALID;
     A.intersections = reinterpret_cast<unsigned long long *>(scal + S_COUNT);
@@ -4053,7 +3392,7 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
         R.off_x = reinterpret_cast<const double *>(tb + o_off_x);
         R.off_t = reinterpret_cast<const double *>(tb + o_off_t);
     }
-    return record_rows(ctx, p, R, cap);
+    return record_rows(ctx, p, R, cap, 0);
 }
 
 int build_curvelets(cvg_context *ctx, const cvg_params &p)
@@ -4063,239 +3402,157 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     ctx->curvelets_ready = false;
     Derived d;
     CVG_TRY(derive(ctx, p, d));
-    // the fused kernel holds a chain in the lanes of a wave and up to four
-    // 64-neighbour chunks per anchor; other maps take the general kernel
-    if (d.G > 64 || ctx->max_deg > 256 || ctx->force_generic) {
-        ctx->edge_trig_queued = false;  // the general kernel computes its own trig
-        ctx->pair_setup_queued = false;
+    // the fused kernel's masks hold up to 256 neighbours, and its error bound
+    // has a range; other maps take the general kernel
+    FusedLimits lim;
+    if (d.G > 64 || ctx->max_deg > 256 || ctx->force_generic || !fused_limits(ctx, d, &lim)) {
+        ctx->setup_queued = false;
         return build_curvelets_generic<double>(ctx, p);
     }
     hipStream_t st = ctx->stream;
     const int n = ctx->n;
     const int pairs = ctx->pairs;
 
-    // bucket capacities (neighbour slots per workgroup)
-    std::vector<int> caps = {4, 6, 8, 11, 16, 24, 32, 48, 64};
-    const int maxcap = static_cast<int>(std::max<unsigned>(ctx->max_deg, 1u));
-    while (!caps.empty() && caps.back() >= maxcap) caps.pop_back();
-    caps.push_back(maxcap);
-    const int nb = static_cast<int>(caps.size());
-    if (nb > kMaxBuckets) return fail(ctx, CVG_ERR_STATE, "internal: too many buckets");
-
     // parameter tables
     std::vector<char> blob;
     const size_t o_rank_ox = put(blob, d.rank_ox);
-    const size_t o_rank_j = put(blob, d.rank_j);
+    const size_t o_rank_ot = put(blob, d.rank_ot);
+    const size_t o_rank_so = put(blob, d.rank_so);
+    const size_t o_rank_co = put(blob, d.rank_co);
     const size_t o_rank_cell = put(blob, d.rank_cell);
     const size_t o_rank_elig = put(blob, d.rank_elig);
     const size_t o_off_x = put(blob, d.off_x);
     const size_t o_off_t = put(blob, d.off_t);
-    const size_t o_caps = put(blob, caps);
     CVG_TRY(upload_tables(ctx, blob));
-    char *tb = static_cast<char *>(ctx->d_tables.ptr);
-    Tables T;
-    T.rank_ox = reinterpret_cast<double *>(tb + o_rank_ox);
-    T.rank_j = reinterpret_cast<int *>(tb + o_rank_j);
-    T.rank_cell = reinterpret_cast<int *>(tb + o_rank_cell);
-    T.rank_elig = reinterpret_cast<int *>(tb + o_rank_elig);
-    T.off_x = reinterpret_cast<double *>(tb + o_off_x);
-    T.off_t = reinterpret_cast<double *>(tb + o_off_t);
-    T.caps = reinterpret_cast<int *>(tb + o_caps);
+    const char *tb = static_cast<const char *>(ctx->d_tables.ptr);
+    const double *off_x = reinterpret_cast<const double *>(tb + o_off_x);
+    const double *off_t = reinterpret_cast<const double *>(tb + o_off_t);
 
-    // per-edge trig, per-pair classes and sines, buckets
-    if (!ctx->edge_trig_queued) CVG_TRY(queue_edge_trig(ctx, p));
-    ctx->edge_trig_queued = false;
-    const bool pair_setup_queued = ctx->pair_setup_queued;
-    ctx->pair_setup_queued = false;
-    CVG_TRY(ensure(ctx, ctx->d_cls, cls_bytes(pairs)));
-    CVG_TRY(ensure(ctx, ctx->d_prec, static_cast<size_t>(std::max(pairs, 1)) * 8 * sizeof(double)));
-    CVG_TRY(ensure(ctx, ctx->d_psin, static_cast<size_t>(std::max(pairs, 1)) * d.kt * 2 * sizeof(double)));
-    CVG_TRY(ensure(ctx, ctx->d_lists, static_cast<size_t>(nb) * n * sizeof(int4)));
+    // edge records and anchor lists
+    if (!ctx->setup_queued) CVG_TRY(queue_setup(ctx));
+    ctx->setup_queued = false;
     unsigned *scal = as<unsigned>(ctx->d_scal);
-    if (static_cast<unsigned long long>(pairs) * d.kt > 0xffffffffull)
-        return fail(ctx, CVG_ERR_UNSUPPORTED, "more than 2^32 (pair, angle) items in one run");
-    if (pairs > 0 && !pair_setup_queued) {
-        const PrepArgs P{as<double>(ctx->d_x), as<double>(ctx->d_y), as<double>(ctx->d_trig), d.close_thr,
-                         as<unsigned char>(ctx->d_cls), as<double>(ctx->d_prec)};
-        // Kt = 7 (the default grid): one kernel forms the pairs' records and
-        // sines; other grids run the record first
-        const bool fused_prep = d.kt == 7;
-        if (!fused_prep)
-            hipLaunchKernelGGL(k_pair_prep, dim3(blocks_for(pairs)), dim3(kBlock), 0, st, pairs, n,
-                               as<int>(ctx->d_pair_anchor), as<int>(ctx->d_ids), P);
-        const size_t trig_lds = d.kt <= static_cast<unsigned>(kPairTrigMaxKt) ? kBlock * d.kt * sizeof(double2) : 0;
-        const auto trig_fn = fused_prep ? k_pair_trig<7, true> : k_pair_trig<0, false>;
-        hipLaunchKernelGGL(trig_fn, dim3(blocks_for(pairs)), dim3(kBlock), trig_lds, st,
-                           pairs, n, static_cast<int>(d.kt), as<int>(ctx->d_pair_anchor), as<int>(ctx->d_ids),
-                           static_cast<const unsigned char *>(as<unsigned char>(ctx->d_cls)), as<double>(ctx->d_th),
-                           p.st, d.dt, as<double>(ctx->d_tdd), as<double>(ctx->d_psin), P,
-                           static_cast<const unsigned *>(nullptr));
-    }
-    hipLaunchKernelGGL(k_bucket, dim3(blocks_for(n, kBucketBlock)), dim3(kBucketBlock), 0, st, n, as<int>(ctx->d_sorted),
-                       as<unsigned char>(ctx->d_cls), as<unsigned>(ctx->d_off), nb, T.caps, as<int4>(ctx->d_lists),
-                       scal);
-    CVG_HIP(ctx, hipGetLastError());
 
-    // staging
-    const int st_stride = static_cast<int>(std::max(d.G, 1u));
-    const int chain_stride = static_cast<int>(std::max(d.G, 1u));
+    // staging: an anchor's rows start at its first CSR slot
     const size_t np = static_cast<size_t>(std::max(pairs, 1));
-    CVG_TRY(ensure(ctx, ctx->d_st_ids, np * st_stride * sizeof(int)));
+    const bool wide = ctx->max_deg > 64;
+    CVG_TRY(ensure(ctx, ctx->d_st_mask, np * (wide ? 4 : 1) * sizeof(ulonglong2)));
     CVG_TRY(ensure(ctx, ctx->d_st_meta, np * sizeof(unsigned)));
-    CVG_TRY(ensure(ctx, ctx->d_st_k, np * 2 * sizeof(double)));
-    CVG_TRY(ensure(ctx, ctx->d_st_rank, np * sizeof(int)));
-    CVG_TRY(ensure(ctx, ctx->d_acc, static_cast<size_t>(n) * sizeof(unsigned)));
     CVG_TRY(ensure(ctx, ctx->d_rowoff, static_cast<size_t>(n + 1) * sizeof(unsigned)));
 
     FusedArgs A{};
-    A.n = n;
-    A.prec = as<double>(ctx->d_prec);
-    A.trig = as<double>(ctx->d_trig);
-    A.psin = as<double>(ctx->d_psin);
+    A.rec = as<double4>(ctx->d_rec);
     A.ids = as<int>(ctx->d_ids);
-    A.pflag = as<unsigned char>(ctx->d_cls);
-    A.chain_stride = chain_stride;
-    A.st_stride = st_stride;
-    A.dx = d.dx;
-    A.dx2 = d.dx2;
-    A.max_k = d.max_k;
-    A.kt = static_cast<int>(d.kt);
+    A.th = as<double>(ctx->d_th);
     A.K = static_cast<int>(d.K);
     A.G = static_cast<int>(d.G);
-    A.rank_ox = T.rank_ox;
-    A.rank_j = T.rank_j;
-    A.rank_cell = T.rank_cell;
-    A.rank_elig = T.rank_elig;
+    A.rank_ox = reinterpret_cast<const double *>(tb + o_rank_ox);
+    A.rank_ot = reinterpret_cast<const double *>(tb + o_rank_ot);
+    A.rank_so = reinterpret_cast<const double *>(tb + o_rank_so);
+    A.rank_co = reinterpret_cast<const double *>(tb + o_rank_co);
+    A.rank_elig = reinterpret_cast<const int *>(tb + o_rank_elig);
     A.rank_of_cell0 = d.rank_of_cell0;
-    A.st_ids = as<int>(ctx->d_st_ids);
+    A.two_dx = 2.0 * d.dx;
+    A.max_k = d.max_k;
+    A.sin_dt = std::sin(d.dt);
+    A.cos_dt = std::cos(d.dt);
+    A.dx = d.dx;
+    A.dx2 = d.dx2;
+    A.close_thr = d.close_thr;
+    A.scale = static_cast<double>(kFixOne) / d.max_k;
+    A.exact = ExactGrid{as<double>(ctx->d_x), as<double>(ctx->d_y), as<double>(ctx->d_th), off_x, off_t, d.dt, d.dx, d.dx2,
+                        d.close_thr, d.max_k, static_cast<int>(d.kt)};
+    A.min_den = lim.min_den;
+    A.num_err = lim.num_err;
+    A.den_err = lim.den_err;
+    A.min_prod = lim.min_prod;
+    A.st_mask = as<ulonglong2>(ctx->d_st_mask);
+    A.mask_plane = np;
     A.st_meta = as<unsigned>(ctx->d_st_meta);
-    A.st_k = as<double>(ctx->d_st_k);
-    A.st_rank = as<int>(ctx->d_st_rank);
     A.acc_count = as<unsigned>(ctx->d_acc);
-    A.valid_pairs = scal + S_VALID;
-    A.intersections = reinterpret_cast<unsigned long long *>(scal + S_COUNT);
 
-    // per bucket: 64-neighbour chunks of the lane-indexed lists (degree <= 2 x
-    // the bucket's key and <= the map's largest); heavy buckets share one anchor
-    // among the waves of a workgroup, light ones pack one anchor per wave;
-    // bundles go to global memory only when one anchor's slice alone exceeds
-    // LDS.  Each launch is persistent: as many anchor streams as stay resident
-    // (the occupancy query accounts for registers and LDS), each looping over
-    // its share of the bucket's list.
-    struct Launch {
-        int nch, wpb, apb, dcap, grid;
-        bool gb, coop;
-        size_t slice;
-        unsigned shmem;
-        FusedKernel fn;
-    };
-    std::vector<Launch> plan(nb);
-    std::vector<size_t> gb_off(nb, 0);
-    size_t gb_total = 0;
-    for (int b = 0; b < nb; ++b) {
-        Launch &l = plan[b];
-        l.dcap = std::min(2 * caps[b], static_cast<int>(std::max(ctx->max_deg, 1u)));
-        const int need = (l.dcap + 63) / 64;
-        if (need > 4) return build_curvelets_generic<double>(ctx, p);
-        l.nch = need <= 1 ? 1 : (need <= 2 ? 2 : 4);
-        l.gb = false;
-        l.coop = caps[b] >= ctx->coop_min_cap;
-        l.slice = anchor_carve(caps[b], l.dcap, A.K, A.kt, chain_stride, true, l.nch).bytes;
-        if (l.coop) {
-            l.wpb = ctx->coop_waves;
-        } else {
-            l.wpb = 4;
-            while (l.wpb > 1 && l.slice * l.wpb > ctx->lds_limit) l.wpb >>= 1;
-        }
-        if (l.slice > ctx->lds_limit) {
-            l.gb = true;
-            l.coop = false;
-            l.wpb = 1;
-            l.slice = anchor_carve(caps[b], l.dcap, A.K, A.kt, chain_stride, false, l.nch).bytes;
-            if (l.slice > ctx->lds_limit) return build_curvelets_generic<double>(ctx, p);
-        }
-        l.apb = l.coop ? 1 : l.wpb;
-        l.shmem = static_cast<unsigned>(l.slice * l.apb);
-        l.fn = fused_kernel(d.cpl, l.nch, l.gb, l.coop);
-        if (!l.fn) return fail(ctx, CVG_ERR_STATE, "internal: no fused kernel for this grid");
-        int occ = 0;
-        CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(l.fn), 64 * l.wpb, l.shmem, &occ));
-        // the bucket sizes stay on the device: every launch gets the resident
-        // grid (streams beyond the bucket's length exit at once), at most one
-        // stream per anchor of the map
-        long long resident = static_cast<long long>(std::max(occ, 1)) * ctx->num_cu;
-        // Launches run four at a time: a light bucket's persistent grid sized
-        // for the whole GPU has workgroups that are dispatched late and still
-        // own a full share of the list, which stretches the stage's tail.  A
-        // grid in proportion to the run's edges fits its lists better; large
-        // maps and batches, whose launches run longer, keep the full one.
-        if (caps[b] < kHeavyCap) {
-            const int pct = ctx->grid_pct > 0 ? ctx->grid_pct : auto_grid_pct(n);
-            resident = std::max(1LL, resident * pct / 100);
-        }
-        const long long max_blocks = (static_cast<long long>(n) + l.apb - 1) / l.apb;
-        l.grid = static_cast<int>(std::min(resident, max_blocks));
-        if (l.gb) {
-            gb_off[b] = gb_total;
-            gb_total += static_cast<size_t>(l.grid) * l.apb * caps[b] * A.K * 2;
-        }
+    // A persistent launch (as many waves as stay resident, each looping over
+    // its share of the lists), then the anchors it leaves open; anchors of more
+    // than 64 neighbours, where the map has any, beside it on an auxiliary
+    // stream.  The slots keep kFusedWavesPerSimd waves per SIMD resident; a
+    // run's bundles beyond them (under 1% of the runs) go to device memory.
+    const FusedKernel fn = fused_kernel(d.cpl);
+    const ExactKernel fn_open = exact_kernel<1>(d.cpl), fn_wide = exact_kernel<4>(d.cpl);
+    A.slots = std::max(kSmallRun, kFusedSlots / d.cpl);
+    const unsigned slice = static_cast<unsigned>(slice_carve(A.slots, d.cpl).bytes);
+    const unsigned shmem = slice * kFusedWaves;
+    int occ = 0, occ_wide = 0, occ_open = 0;
+    CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(fn), 64 * kFusedWaves, shmem, &occ));
+    CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(fn_open), 64, slice, &occ_open));
+    CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(fn_wide), 64, slice, &occ_wide));
+    // bundle words in device memory per wave
+    const size_t word = static_cast<size_t>(d.cpl) * 64;
+    const size_t spill_main = std::max(0, static_cast<int>(std::min(ctx->max_deg, 64u)) - A.slots) * word;
+    const size_t spill_exact = std::max(0, static_cast<int>(ctx->max_deg) - A.slots) * word;
+    long long blocks = static_cast<long long>(std::max(occ, 1)) * ctx->num_cu;
+    if (ctx->grid_pct > 0) blocks = std::max(1LL, blocks * ctx->grid_pct / 100);
+    blocks = std::min(blocks, (static_cast<long long>(n) + kFusedWaves - 1) / kFusedWaves);
+    long long blocks_wide = wide ? std::min<long long>(n, static_cast<long long>(std::max(occ_wide, 1)) * ctx->num_cu) : 0;
+    long long blocks_open = std::min<long long>(n, ctx->num_cu);
+    // (the no-alloc scratch leaves a smaller grid's worth)
+    if (ctx->arena && spill_exact > 0) {
+        const long long fit = static_cast<long long>((size_t(6) << 20) / (spill_exact * sizeof(int2)));
+        blocks = std::max(1LL, std::min(blocks, fit / kFusedWaves));
+        blocks_wide = std::min(blocks_wide, std::max(1LL, fit));
+        blocks_open = std::max(1LL, std::min(blocks_open, fit));
     }
-    if (gb_total > 0) CVG_TRY(ensure(ctx, ctx->d_gbundle, gb_total * sizeof(double)));
+    const int waves_main = static_cast<int>(blocks) * kFusedWaves;
+    const int waves = waves_main + static_cast<int>(blocks_wide + blocks_open);
+    CVG_TRY(ensure(ctx, ctx->d_gbundle, (std::max<size_t>(spill_main * waves_main, spill_exact * blocks_open) +
+                                         spill_exact * blocks_wide) * sizeof(int2)));
+    CVG_TRY(ensure(ctx, ctx->d_partial, static_cast<size_t>(waves) * 3 * sizeof(unsigned)));
+    A.lists = as<int4>(ctx->d_lists);
+    A.list_len = scal + kBucketBase;
+    A.n = n;
+    FusedArgs X = A;  // the exact kernel's
 
-    // bucket launches: the short-list bucket 0 (most anchors) alone on the main
-    // stream, the long-list buckets round-robin over the auxiliary streams,
-    // longest lists first, so their long-latency work starts at once and
-    // overlaps the bulk
     const int ring = static_cast<int>(ctx->fused_runs % cvg_context::kFusedRing);
     CVG_TRY(record_timing(ctx, ctx->ev[3], st));
     CVG_TRY(record_timing(ctx, ctx->fused_ev[ring][0], st));
-    const hipEvent_t fork = ctx->timed_run ? ctx->ev[3] : ctx->ev_fork;
-    if (!ctx->timed_run) CVG_HIP(ctx, hipEventRecord(fork, st));
-    for (int i = 0; i < 3; ++i) CVG_HIP(ctx, hipStreamWaitEvent(ctx->aux[i], fork, 0));
-    bool aux_used[3] = {false, false, false};
-    int rr = 0;
-    GateArgs gate{};
-    for (int b = nb - 1; b >= 0; --b) {
-        const int slot = b == 0 ? 0 : 1 + (rr++ % 3);
-        hipStream_t ls = slot == 0 ? st : ctx->aux[slot - 1];
-        if (slot > 0) aux_used[slot - 1] = true;
-        const Launch &l = plan[b];
-        A.list = as<int4>(ctx->d_lists) + static_cast<size_t>(b) * n;
-        A.list_len = scal + kBucketBase + b * kBucketStride;
-        A.nb_cap = caps[b];
-        const bool heavy = b > 0 && caps[b] >= kHeavyCap;  // on an auxiliary stream
-        A.started = heavy ? scal + kStartedWord : nullptr;
-        if (heavy) {
-            gate.bucket[gate.nheavy] = b;
-            gate.streams[gate.nheavy] = l.grid * l.apb;
-            ++gate.nheavy;
-        }
-        if (b == 0 && gate.nheavy > 0) {
-            hipLaunchKernelGGL(k_gate, dim3(1), dim3(64), 0, st, gate, static_cast<const unsigned *>(scal),
-                               ctx->gate_naps);
-            CVG_HIP(ctx, hipGetLastError());
-        }
-        A.deg_cap = l.dcap;
-        A.g_bundle = l.gb ? as<double>(ctx->d_gbundle) + gb_off[b] : nullptr;
-        hipLaunchKernelGGL(l.fn, dim3(l.grid), dim3(64 * l.wpb), l.shmem, ls, A);
-        CVG_HIP(ctx, hipGetLastError());
+    X.spill_stride = spill_exact;
+    if (wide) {
+        const hipEvent_t fork = ctx->timed_run ? ctx->ev[3] : ctx->ev_fork;
+        if (!ctx->timed_run) CVG_HIP(ctx, hipEventRecord(fork, st));
+        CVG_HIP(ctx, hipStreamWaitEvent(ctx->aux, fork, 0));
+        X.spill = as<int2>(ctx->d_gbundle);
+        X.partial = as<unsigned>(ctx->d_partial);
+        hipLaunchKernelGGL(fn_wide, dim3(static_cast<unsigned>(blocks_wide)), dim3(64), slice, ctx->aux, X,
+                           static_cast<int>(L_WIDE));
+        CVG_HIP(ctx, hipEventRecord(ctx->ev_join, ctx->aux));
     }
-    for (int i = 0; i < 3; ++i) {
-        if (!aux_used[i]) continue;
-        CVG_HIP(ctx, hipEventRecord(ctx->ev_join[i], ctx->aux[i]));
-        CVG_HIP(ctx, hipStreamWaitEvent(st, ctx->ev_join[i], 0));
-    }
+    A.spill = as<int2>(ctx->d_gbundle) + spill_exact * blocks_wide;
+    A.spill_stride = spill_main;
+    A.partial = as<unsigned>(ctx->d_partial) + 3 * blocks_wide;
+    hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(blocks)), dim3(64 * kFusedWaves), shmem, st, A);
+    X.spill = A.spill;
+    X.partial = A.partial + 3 * waves_main;
+    hipLaunchKernelGGL(fn_open, dim3(static_cast<unsigned>(blocks_open)), dim3(64), slice, st, X,
+                       static_cast<int>(L_OPEN));
+    CVG_HIP(ctx, hipGetLastError());
+    if (wide) CVG_HIP(ctx, hipStreamWaitEvent(st, ctx->ev_join, 0));
     CVG_TRY(record_timing(ctx, ctx->ev[4], st));
     CVG_TRY(record_timing(ctx, ctx->fused_ev[ring][1], st));
     if (ctx->timed_run) ++ctx->fused_runs;
-    // every anchor is in exactly one bucket, so every acc_count entry is written
     RecordArgs R{};
     R.G = static_cast<int>(d.G);
     R.kt = static_cast<int>(d.kt);
     R.nrad = d.nrad;
-    R.off_x = T.off_x;
-    R.off_t = T.off_t;
-    return record_rows(ctx, p, R, st_stride);
+    R.off_x = off_x;
+    R.off_t = off_t;
+    R.exact = A.exact;
+    R.st_mask = A.st_mask;
+    R.rec = A.rec;
+    R.rank_cell = reinterpret_cast<const int *>(tb + o_rank_cell);
+    R.sin_dt = A.sin_dt;
+    R.cos_dt = A.cos_dt;
+    R.min_den = A.min_den;
+    R.mask_plane = A.mask_plane;
+    return record_rows(ctx, p, R, 0, waves);
 }
 
 bool same_params(const cvg_params &a, const cvg_params &b)
@@ -4322,10 +3579,10 @@ int run_common(cvg_context *ctx, int n, int sz, const double *d_edges, const cvg
     ctx->timed_run = timed || stats || ctx->event_timing;
     CVG_TRY(record_timing(ctx, ctx->ev[0], ctx->stream));
     ctx->use_cellrank = false;
-    ctx->edge_trig_queued = false;
-    ctx->early_params = (!f32 && p->group_max_sz <= 64 && !ctx->force_generic) ? p : nullptr;
+    ctx->setup_queued = false;
+    ctx->early_setup = !f32 && p->group_max_sz <= 64 && !ctx->force_generic;
     const int rc = build_graph(ctx, n, sz, d_edges, p->nrad, 3u, p->max_candidates, num_maps, eoff);  // main.cpp:48: 3
-    ctx->early_params = nullptr;
+    ctx->early_setup = false;
     if (rc != CVG_OK) return rc;
     CVG_TRY(record_timing(ctx, ctx->ev[1], ctx->stream));
     CVG_TRY(build_curvelets(ctx, *p));
@@ -4569,11 +3826,9 @@ int cvg_create(int device, cvg_context **out_ctx)
     do {
         if (hipSetDevice(device) != hipSuccess) { rc = CVG_ERR_DEVICE; break; }
         if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) { rc = CVG_ERR_DEVICE; break; }
-        for (int i = 0; i < 3 && rc == CVG_OK; ++i) {
-            if (hipStreamCreateWithFlags(&ctx->aux[i], hipStreamNonBlocking) != hipSuccess ||
-                hipEventCreateWithFlags(&ctx->ev_join[i], hipEventDisableTiming) != hipSuccess)
-                rc = CVG_ERR_DEVICE;
-        }
+        if (hipStreamCreateWithFlags(&ctx->aux, hipStreamNonBlocking) != hipSuccess ||
+            hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess)
+            rc = CVG_ERR_DEVICE;
         if (rc != CVG_OK) break;
         for (auto &e : ctx->ev)
             if (hipEventCreate(&e) != hipSuccess) rc = CVG_ERR_DEVICE;
@@ -4614,7 +3869,6 @@ int cvg_create(int device, cvg_context **out_ctx)
         if (const char *v = std::getenv("CVG_SPARSE_CELLS")) ctx->force_sparse = std::atoi(v) != 0;
         if (const char *v = std::getenv("CVG_GENERIC_KERNEL")) ctx->force_generic = std::atoi(v) != 0;
         if (const char *v = std::getenv("CVG_SPECULATE")) ctx->spec_off = std::atoi(v) == 0;
-        if (const char *v = std::getenv("CVG_GATE_NAPS")) ctx->gate_naps = std::min(std::max(0, std::atoi(v)), 400);
         if (const char *v = std::getenv("CVG_LOOKBACK_SPINS"))
             ctx->lookback_spins = static_cast<unsigned>(std::min<long long>(std::max(0LL, std::atoll(v)), kLookbackSpins));
     } while (false);
@@ -4645,11 +3899,9 @@ void cvg_destroy(cvg_context *ctx)
         if (ctx->h_stage[b]) (void)hipHostFree(ctx->h_stage[b]);
         if (ctx->ev_stage[b]) (void)hipEventDestroy(ctx->ev_stage[b]);
     }
-    for (int i = 0; i < 3; ++i) {
-        if (ctx->aux[i]) (void)hipStreamSynchronize(ctx->aux[i]);
-        if (ctx->ev_join[i]) (void)hipEventDestroy(ctx->ev_join[i]);
-        if (ctx->aux[i]) (void)hipStreamDestroy(ctx->aux[i]);
-    }
+    if (ctx->aux) (void)hipStreamSynchronize(ctx->aux);
+    if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
+    if (ctx->aux) (void)hipStreamDestroy(ctx->aux);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -5016,22 +4268,16 @@ int cvg_autotune_batch(cvg_context *ctx, int num_maps, const int *num_edges, int
     CVG_TRY(cvg_get_tuning(ctx, &cur));
     double cur_ms = 0.0;
     CVG_TRY(time_of(cur, &cur_ms));
-    // coordinate descent: the cooperative threshold, its waves, the scan
-    // lanes, the light buckets' grid
-    const int keys[] = {4, 6, 8, 11, 16, 1 << 30};
-    const int waves[] = {2, 4};
-    const int lanes[] = {8, 16, 32};
+    // coordinate descent: the scan lanes, then the curvelet launch's grid
+    const int lanes[] = {8, 16, 32, 64};
     const int grids[] = {25, 50, 75, 100};
-    for (int field = 0; field < 4; ++field) {
-        const int *vals = field == 0 ? keys : (field == 1 ? waves : (field == 2 ? lanes : grids));
-        const int nv = field == 0 ? 6 : (field == 1 ? 2 : (field == 2 ? 3 : 4));
+    for (int field = 0; field < 2; ++field) {
+        const int *vals = field == 0 ? lanes : grids;
         cvg_tuning base = cur;
-        for (int k = 0; k < nv; ++k) {
+        for (int k = 0; k < 4; ++k) {
             cvg_tuning t = base;
-            int &slot = field == 0 ? t.coop_min_key
-                                   : (field == 1 ? t.coop_waves : (field == 2 ? t.window_lanes : t.grid_pct));
-            const int old = field == 0 ? base.coop_min_key
-                                       : (field == 1 ? base.coop_waves : (field == 2 ? base.window_lanes : base.grid_pct));
+            int &slot = field == 0 ? t.window_lanes : t.grid_pct;
+            const int old = field == 0 ? base.window_lanes : base.grid_pct;
             if (vals[k] == old) continue;
             slot = vals[k];
             double ms = 0.0;

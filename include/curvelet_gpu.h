@@ -266,14 +266,11 @@ int cvg_get_batch_map_curvelets(cvg_context *ctx, int map, unsigned *chains, dou
  * defaults' 1920x1080 tuning.  The environment variables CVG_COOP_MIN_CAP,
  * CVG_COOP_WAVES and CVG_FILL_LANES set the initial values of a new context. */
 typedef struct cvg_tuning {
-    int coop_min_key;  /* anchor buckets whose key (max(forward, backward) + neither
-                          neighbours) is at least this run one anchor per workgroup of
-                          coop_waves waves; lighter ones one anchor per wave (>= 1) */
-    int coop_waves;    /* 1, 2 or 4 */
+    int coop_min_key;  /* at least 1; kept for callers that set it, no launch depends on it */
+    int coop_waves;    /* 1, 2 or 4; likewise */
     int window_lanes;  /* lanes per anchor in the neighbour-window scans: 8, 16, 32 or 64 */
-    int grid_pct;      /* grid of the light buckets' curvelet launches as a percentage of
-                          their resident capacity, 5..100; 0 = automatic (10 plus one
-                          percent per 4,000 edges in the run, at most 100) */
+    int grid_pct;      /* grid of the curvelet launch as a percentage of its resident
+                          capacity, 5..100; 0 = automatic (all of it) */
 } cvg_tuning;
 typedef struct cvg_tuning_trial {
     cvg_tuning tuning;

@@ -249,6 +249,13 @@ struct FusedArgs {
     ulonglong2 *st_mask;             // (hypotheses, chain) per row
     size_t mask_plane;               // entries between the 64-bit planes of st_mask
     unsigned *st_meta;
+    // float maps: the reference's float operands, and rows as the general
+    // kernel stages them
+    float dt_f, dx_f, max_k_f, close_f;
+    const int *rank_cell;
+    int *st_ids;
+    int st_stride;
+    double *st_k;
     unsigned *acc_count;
     unsigned *partial;               // per wave: valid pairs, then two words of the intersection count
 };
@@ -279,6 +286,7 @@ __host__ __device__ inline SliceCarve slice_carve(int slots, int cpl)
 template <int CPL>
 struct WaveCells {
     double ox[CPL], m2ox[CPL], ox2[CPL], oxp[CPL], so[CPL], co[CPL];
+    double ot[CPL];  // (float maps)
     unsigned long long emask[CPL];  // cells that can be a best one
 };
 
@@ -300,9 +308,40 @@ struct alignas(8) Bounds {
     int lo, hi;
 };
 
-// One anchor on one wave.  EXACT = false returns true, with nothing counted,
-// when some comparison is closer than the approximate bounds can decide;
-// EXACT = true makes such comparisons on the exact bounds.
+// Float maps (the reference's float instantiation).  Its bounds are formed by
+// its own float operations, which take a lane no division longer than the
+// approximations above; only the correctly rounded float sines come from
+// doubles: rotations, as above, corrected for the angle's rounding to float,
+// and certain unless within kSineErr of where the float changes.  Bounds are
+// compared as integers of the same order.  720p float map (92,070 edges): 4,860
+// us on the general kernel, whose two correctly rounded sines a cell are some
+// 600 instructions; 327 us so, and 347 us for the anchors left to the general one.
+enum { M_FAST = 0, M_EXACT = 1, M_FLOAT = 2 };
+
+// Beyond what the rotations are off by: sums of an orientation (up to 64) and
+// an offset 2^-47, their sines and cosines 2^-51 each, the products 2^-50.
+constexpr double kSineErr = 0x1p-44;
+
+// v as float; `bad` gets a bit where v + kSineErr or v - kSineErr rounds
+// differently.
+__device__ __forceinline__ float sure_float(double v, unsigned &bad)
+{
+    const float f = static_cast<float>(v + kSineErr);
+    bad |= __float_as_uint(f) ^ __float_as_uint(static_cast<float>(v - kSineErr));
+    return f;
+}
+
+// Floats as integers of the same order, and back (no -0.0f).
+__device__ __forceinline__ int float_key(float v)
+{
+    const int b = __float_as_int(v);
+    return b ^ ((b >> 31) & INT_MAX);
+}
+__device__ __forceinline__ float key_float(int k) { return __int_as_float(k ^ ((k >> 31) & INT_MAX)); }
+
+// One anchor on one wave.  M_FAST and M_FLOAT return true, with nothing
+// counted, when something is closer than they can decide; M_EXACT makes such
+// comparisons on the exact bounds.
 //
 // Lane = neighbour forms the pairs' direction class, flags and
 // cell-independent terms (16 records in LDS at a time, in run order).  Then,
@@ -329,12 +368,17 @@ struct alignas(8) Bounds {
 // k_max are left to the record, where a lane has a row of its own.
 //
 // NW: 64-bit words of a slot or neighbour mask (64 NW neighbours at most).
-template <int CPL, int NW, bool EXACT>
+//
+// nid, nb, nth: lane's neighbour (of the first 64), its record and orientation.
+template <int CPL, int NW, int MODE>
 __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CPL> &W, char *sl, int2 *spill, int a,
-                                          unsigned base, int deg, const double4 nb, unsigned &vp_sum,
-                                          unsigned long long &isect_sum)
+                                          unsigned base, int deg, int nid, const double4 nb, double nth,
+                                          unsigned &vp_sum, unsigned long long &isect_sum)
 {
     typedef unsigned long long u64;
+    constexpr bool EXACT = MODE == M_EXACT, FLT = MODE == M_FLOAT;
+    static_assert(!FLT || NW == 1, "float maps: up to 64 neighbours");
+    constexpr int kTol = FLT ? 0 : kFixTol;
     constexpr int NC = NW;  // 64-seed (64-neighbour) chunks
     const int lane = threadIdx.x & 63;
     const int G = A.G;
@@ -364,7 +408,11 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
     // and in between open.  Not EXACT: a lane's smallest t + kFixTol, as
     // unsigned, says at the end whether any of its comparisons was open.
     unsigned closest = ~0u;
-    auto note = [&](int t) { closest = min(closest, static_cast<unsigned>(t + kFixTol)); };
+    auto note = [&](int t) {
+        if (MODE == M_FAST) closest = min(closest, static_cast<unsigned>(t + kFixTol));
+    };
+    unsigned bad = 0u;        // M_FLOAT: nonzero where a float sine is uncertain
+    float least = A.max_k_f;  // M_FLOAT: the smallest magnitude of a bound (a zero's sign would be lost)
     auto is_open = [&](int t) -> u64 {
         return __builtin_amdgcn_ballot_w64(static_cast<unsigned>(t + kFixTol) <= 2u * kFixTol);
     };
@@ -374,11 +422,24 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
     const double ax = uload(ar), ay = uload(ar + 1), sa = uload(ar + 2), ca = uload(ar + 3);
     // sin/cos of theta_a + delta_t2 by rotation
     double sT[CPL], cT[CPL];
+    float T2[CPL], sf[CPL], cf[CPL];  // M_FLOAT: the angle, its sine and cosine
 #pragma unroll
     for (int m = 0; m < CPL; ++m) {
         sT[m] = __builtin_fma(sa, W.co[m], ca * W.so[m]);
         cT[m] = __builtin_fma(ca, W.co[m], -(sa * W.so[m]));
+        if constexpr (FLT) {
+            const double th = uload(A.th + a);
+            T2[m] = static_cast<float>(th) + static_cast<float>(W.ot[m]);  // :702
+            const double e = static_cast<double>(T2[m]) - (th + W.ot[m]);
+            const double s = sT[m], c = cT[m];
+            sT[m] = __builtin_fma(e, __builtin_fma(-0.5 * e, s, c), s);
+            cT[m] = __builtin_fma(-e, __builtin_fma(0.5 * e, c, s), c);
+            sf[m] = sure_float(sT[m], bad);
+            cf[m] = sure_float(cT[m], bad);
+        }
     }
+
+    [[maybe_unused]] const float fsa = sure_float(sa, bad), fca = sure_float(ca, bad);
 
     // EXACT: the exact bounds of neighbour b at this lane's cell of group m
     auto exact_cell = [&](int m, int b, double &lo, double &hi) {
@@ -405,13 +466,18 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             const bool in = 64 * c + lane < deg;
             const double vx = q.x - ax, vy = q.y - ay;
             cl[c] = in && vx * vx + vy * vy < A.close_thr;  // :682 (DX^2 + DY^2, the same squares)
+            if constexpr (FLT) {
+                const float fx = static_cast<float>(ax) - static_cast<float>(q.x);
+                const float fy = static_cast<float>(ay) - static_cast<float>(q.y);
+                cl[c] = in && fx * fx + fy * fy < A.close_f;
+            }
             int k;
             if constexpr (EXACT) {
                 k = in ? cvg::direction_class(ax, ay, ca, sa, q.x, q.y, c_sincos_tab, c_atan_tab) : 3;
             } else {
                 // (direction_class's projection and a bound at least as strict)
                 const double p = vx * ca + vy * sa;
-                open |= __ballot(in && !(fabs(p) > 1e-12 * (fabs(vx) + fabs(vy))));
+                open |= __ballot(in && !(fabs(p) > (FLT ? 1e-5 : 1e-12) * (fabs(vx) + fabs(vy))));
                 k = p > 0 ? 1 : 2;
             }
             cls[c] = in ? k : 3;
@@ -462,6 +528,49 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
         for (int c = 0; c < NC; ++c) {
             if (NC > 1 && 64 * c >= deg) continue;
             const double4 q = c > 0 ? load_rec(c) : nb;
+            if constexpr (FLT) {
+                // M_FLOAT: the sines and cosines, DX^2 and DY^2, DX, DY and
+                // the angles, DX cos and DY sin
+                const float fx = static_cast<float>(ax) - static_cast<float>(q.x);
+                const float fy = static_cast<float>(ay) - static_cast<float>(q.y);
+                const bool branch_a = (fx * fca + fy * fsa) < 0;  // :690
+                double s[2], co[2];
+                float T0[2], cx[2], sy[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const bool minus = (k == 0) == branch_a;
+                    const float fth = static_cast<float>(nth);
+                    const double d = minus ? -static_cast<double>(A.dt_f) : static_cast<double>(A.dt_f);
+                    const double sd = minus ? -A.sin_dt : A.sin_dt;
+                    T0[k] = minus ? fth - A.dt_f : fth + A.dt_f;
+                    const double e = static_cast<double>(T0[k]) - (nth + d);
+                    const double s0 = __builtin_fma(q.z, A.cos_dt, q.w * sd);
+                    const double c0 = __builtin_fma(q.w, A.cos_dt, -(q.z * sd));
+                    s[k] = __builtin_fma(e, __builtin_fma(-0.5 * e, s0, c0), s0);
+                    co[k] = __builtin_fma(-e, __builtin_fma(0.5 * e, c0, s0), c0);
+                    cx[k] = fx * sure_float(co[k], bad);  // :730-733
+                    sy[k] = fy * sure_float(s[k], bad);
+                }
+                if (pos[c] >= 0 && (pos[c] >> 4) == b) {
+                    const lds_ptr<double2> o = rec + (pos[c] & 15) * 5;
+                    o[0].x = s[0];
+                    o[0].y = co[0];
+                    o[1].x = s[1];
+                    o[1].y = co[1];
+                    o[2].x = static_cast<double>(fx * fx);
+                    o[2].y = static_cast<double>(fy * fy);
+                    const lds_ptr<float4> f = (lds_ptr<float4>)(o + 3);
+                    f[0].x = fx;
+                    f[0].y = fy;
+                    f[0].z = T0[0];
+                    f[0].w = T0[1];
+                    f[1].x = cx[0];
+                    f[1].y = sy[0];
+                    f[1].z = cx[1];
+                    f[1].w = sy[1];
+                }
+                continue;
+            }
             const double DX = ax - q.x, DY = ay - q.y;
             const bool branch_a = (DX * ca + DY * sa) < 0;  // :690
             const double sd = branch_a ? -A.sin_dt : A.sin_dt;
@@ -524,9 +633,49 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                     // the default bundle [-max_k, max_k]
 #pragma unroll
                     for (int m = 0; m < CPL; ++m) {
-                        v[m].lo = -kFixOne;
-                        v[m].hi = kFixOne;
+                        v[m].lo = FLT ? float_key(-A.max_k_f) : -kFixOne;
+                        v[m].hi = FLT ? float_key(A.max_k_f) : kFixOne;
                     }
+                } else if constexpr (FLT) {
+                    // compute_curve_bundle<float>; its branches differ (a
+                    // power of two on both sides of a quotient apart) in the
+                    // angles' order only
+                    const lds_ptr<float4> f = (lds_ptr<float4>)(q + 3);
+                    const float DX = f[0].x, DY = f[0].y;
+                    const double DX2 = q[2].x, DY2 = q[2].y;
+                    u64 any = 0ULL;
+#pragma unroll
+                    for (int m = 0; m < CPL; ++m) {
+                        const float o = static_cast<float>(W.ox[m]);
+                        const float tt = sf[m] * DX - cf[m] * DY;  // :705
+                        const float ttm = tt - o;
+                        // :711 (the first product is exact)
+                        const float den = static_cast<float>(
+                            __builtin_fma(W.m2ox[m], static_cast<double>(tt), DX2) + DY2 - A.dx2 + W.ox2[m]);
+                        const float kx0 = 2.0f * (ttm - A.dx_f) / den, kx1 = 2.0f * (ttm + A.dx_f) / den;
+                        float kt[2];
+#pragma unroll
+                        for (int k = 0; k < 2; ++k) {
+                            const double s0 = q[k].x, c0 = q[k].y;
+                            const float T0 = k == 0 ? f[0].z : f[0].w;
+                            const float cx = k == 0 ? f[1].x : f[1].z, sy = k == 0 ? f[1].y : f[1].w;
+                            const double e = static_cast<double>(T2[m] - T0) -
+                                             (static_cast<double>(T2[m]) - static_cast<double>(T0));
+                            const double s = __builtin_fma(sT[m], c0, -(cT[m] * s0));
+                            const double c = __builtin_fma(cT[m], c0, sT[m] * s0);
+                            const float sn = sure_float(__builtin_fma(e, __builtin_fma(-0.5 * e, s, c), s), bad);
+                            kt[k] = sn / (-sn * o + cx + sy);
+                        }
+                        // the reference's compare-and-assign, which ignores NaN
+                        const float lo = __builtin_fmaxf(__builtin_fmaxf(-A.max_k_f, kx0), kt[0]);
+                        const float hi = __builtin_fminf(__builtin_fminf(A.max_k_f, kx1), kt[1]);
+                        least = __builtin_fminf(least, __builtin_fminf(__builtin_fabsf(lo), __builtin_fabsf(hi)));
+                        const bool ok = hi > lo;
+                        v[m].lo = ok ? float_key(lo) : INT_MAX;
+                        v[m].hi = ok ? float_key(hi) : INT_MIN;
+                        any |= __builtin_amdgcn_ballot_w64(ok);
+                    }
+                    if (any == 0ULL) continue;  // bundle_valid_check, :821-830
                 } else {
                     const double DX = q[0].x, DY = q[0].y, r2 = q[1].x, C0 = q[1].y, C1 = q[2].x;
                     const double s0n = q[2].y, c0n = q[3].x, s1n = q[3].y, c1n = q[4].x;
@@ -551,7 +700,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                         int lo = max(fix(k0), fix(s0 * yd0));
                         int hi = min(fix(k1), fix(s1 * yd1));
                         const int t = min(sub_sat(hi, lo), min(sub_sat(hi, -kFixOne), sub_sat(kFixOne, lo)));
-                        if (!EXACT) note(t);
+                        note(t);
                         bool ok = t > kFixTol;
                         u64 T = __builtin_amdgcn_ballot_w64(ok);
                         u64 U = EXACT ? is_open(t) : 0ULL;
@@ -656,6 +805,35 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
         };
         auto put_row = [&](unsigned rank, const u64 (&chain)[NW], int best, int seed) {
             const size_t q = static_cast<size_t>(base) + rank;
+            if constexpr (FLT) {
+                // the slots' edges are in `pm`; k_max and k_min over the
+                // members' and the seed's bundles at the best cell
+                const lds_ptr<int> slot_id = (lds_ptr<int>)pm;
+                const lds_ptr<Bounds> at = (lds_ptr<Bounds>)(sl + cv.bun) + best;
+                const mem_ptr<Bounds> far = (mem_ptr<Bounds>)spill + best;
+                const mem_ptr<int> ids = (mem_ptr<int>)A.st_ids + q * A.st_stride;
+                int len = 0, lo = INT_MIN, hi = INT_MAX;
+                ids[len++] = a;
+                for (u64 set = chain[0] | 1ULL << seed; set != 0ULL; set &= set - 1ULL) {
+                    const int s = __builtin_ctzll(set);
+                    if ((chain[0] >> s) & 1ULL) ids[len++] = slot_id[s];
+                    int l, h;
+                    if (s < slots) {
+                        l = at[s * CPL * 64].lo;
+                        h = at[s * CPL * 64].hi;
+                    } else {
+                        l = far[(s - slots) * CPL * 64].lo;
+                        h = far[(s - slots) * CPL * 64].hi;
+                    }
+                    lo = max(lo, l);
+                    hi = min(hi, h);
+                }
+                ((mem_ptr<unsigned>)A.st_meta)[q] = static_cast<unsigned>(len) | (run == 0 ? 0x8000u : 0u) |
+                                                    static_cast<unsigned>(A.rank_cell[best]) << 16;
+                ((mem_ptr<double>)A.st_k)[2 * q] = static_cast<double>(key_float(hi));
+                ((mem_ptr<double>)A.st_k)[2 * q + 1] = static_cast<double>(key_float(lo));
+                return;
+            }
 #pragma unroll
             for (int w = 0; w < NW; ++w)
                 if (w == 0 || deg > 64) {
@@ -673,6 +851,16 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 if (best < 0 && e != 0ULL) best = 64 * m + __builtin_ctzll(e);
             }
             return best < 0 ? A.rank_of_cell0 : best;
+        };
+        auto slot_ids = [&]() {  // M_FLOAT: the slots' edges into `pm`
+            if constexpr (FLT) {
+                wave_sync();  // the last reads there are done, and every bundle is written
+                if (__builtin_amdgcn_inverse_ballot_w64(hyp[0]))
+                    ((lds_ptr<int>)pm)[__builtin_amdgcn_mbcnt_hi(
+                        static_cast<unsigned>(hyp[0] >> 32),
+                        __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(hyp[0]), 0u))] = nid;
+                wave_sync();
+            }
         };
         auto rank_of = [&](u64 acc) -> unsigned {
             return nacc + static_cast<unsigned>(__builtin_amdgcn_mbcnt_hi(
@@ -710,7 +898,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                             redo |= is_open(t) != 0ULL ? 1ULL << (8 * i + k) : 0ULL;
                         else
                             note(t);
-                        P[m] = set_lane64(P[m], __builtin_amdgcn_ballot_w64(t > kFixTol), 8 * i + k);
+                        P[m] = set_lane64(P[m], __builtin_amdgcn_ballot_w64(t > kTol), 8 * i + k);
                     }
                 }
             }
@@ -726,7 +914,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                         const int t = min(sub_sat(bk.hi, bi.lo), sub_sat(bi.hi, bk.lo));
                         const u64 U = is_open(t);
                         if (U != 0ULL)
-                            P[m] = set_lane64(P[m], (__builtin_amdgcn_ballot_w64(t > kFixTol) & ~U) | exact_run(m, U, set),
+                            P[m] = set_lane64(P[m], (__builtin_amdgcn_ballot_w64(t > kTol) & ~U) | exact_run(m, U, set),
                                               ik);
                     }
                 }
@@ -795,6 +983,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             }
             const bool keep = j == k && j < R && members >= 2 && ((dup >> (lane & 56)) & 0xffULL) == 0ULL;
             const u64 acc = __builtin_amdgcn_ballot_w64(keep);
+            if (FLT && acc != 0ULL) slot_ids();
             if (keep) {
                 u64 row[NW];
 #pragma unroll
@@ -822,8 +1011,10 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             for (int m = 0; m < CPL; ++m) {
                 // (clamped at -+max_k)
                 cur[m] = get_bundle(j, m);
-                cur[m].lo = max(cur[m].lo, -kFixOne);
-                cur[m].hi = min(cur[m].hi, kFixOne);
+                if (!FLT) {
+                    cur[m].lo = max(cur[m].lo, -kFixOne);
+                    cur[m].hi = min(cur[m].hi, kFixOne);
+                }
                 nx[m] = get_bundle(0, m);
             }
             u64 S[NW];
@@ -837,7 +1028,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 for (int m = 0; m < CPL; ++m) {
                     n[m].lo = max(cur[m].lo, nx[m].lo);
                     n[m].hi = min(cur[m].hi, nx[m].hi);
-                    T |= __builtin_amdgcn_ballot_w64(sub_sat(n[m].hi, n[m].lo) > kFixTol);
+                    T |= __builtin_amdgcn_ballot_w64(sub_sat(n[m].hi, n[m].lo) > kTol);
                 }
                 const int hn = h + 1 < R ? h + 1 : h;
 #pragma unroll
@@ -872,7 +1063,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
 #pragma unroll
             for (int m = 0; m < CPL; ++m) {
                 const int t = sub_sat(cur[m].hi, cur[m].lo);
-                u64 T = __builtin_amdgcn_ballot_w64(t > kFixTol);
+                u64 T = __builtin_amdgcn_ballot_w64(t > kTol);
                 if constexpr (EXACT) {
                     const u64 U = is_open(t);
                     if (U != 0ULL) {
@@ -922,11 +1113,13 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                     acc &= ~same;
                 }
             }
+            if (FLT && acc != 0ULL) slot_ids();
             if (__builtin_amdgcn_inverse_ballot_w64(acc)) put_row(rank_of(acc), sm[c], best_cell(sM[c]), j);
             nacc += static_cast<unsigned>(__popcll(acc));
         }
     }
-    if (!EXACT && (open | __builtin_amdgcn_ballot_w64(closest <= 2u * kFixTol)) != 0ULL) return true;
+    if (MODE == M_FAST && (open | __builtin_amdgcn_ballot_w64(closest <= 2u * kFixTol)) != 0ULL) return true;
+    if (FLT && (open | __builtin_amdgcn_ballot_w64(bad != 0u || least == 0.0f)) != 0ULL) return true;
     if (lane == 0) ((mem_ptr<unsigned>)A.acc_count)[a] = nacc;
     vp_sum += vp;
     isect_sum += isect + (lane == 0 ? isect_u : 0u);
@@ -946,7 +1139,7 @@ __device__ __forceinline__ void put_sums(unsigned *partial, int g, unsigned vp, 
     }
 }
 
-template <int CPL>
+template <int CPL, bool FLT = false>
 __device__ __forceinline__ WaveCells<CPL> wave_cells(const FusedArgs &A)
 {
     WaveCells<CPL> W;
@@ -957,8 +1150,9 @@ __device__ __forceinline__ WaveCells<CPL> wave_cells(const FusedArgs &A)
         const int r = live ? rho : 0;
         W.ox[m] = A.rank_ox[r];
         W.m2ox[m] = -2.0 * W.ox[m];
-        W.ox2[m] = W.ox[m] * W.ox[m];
+        W.ox2[m] = FLT ? static_cast<double>(static_cast<float>(W.ox[m]) * static_cast<float>(W.ox[m])) : W.ox[m] * W.ox[m];
         W.oxp[m] = W.ox[m] + A.dx;
+        W.ot[m] = A.rank_ot[r];
         W.so[m] = A.rank_so[r];
         W.co[m] = A.rank_co[r];
         W.emask[m] = __ballot(live && A.rank_elig[r] != 0);
@@ -989,8 +1183,8 @@ __device__ __forceinline__ void load_entry(const int4 *p, int &a, unsigned &base
 // for the approximate bounds go to the open list.  (Done again here, their
 // code costs the main loop its registers: 1,272 us against 720 on the 1080p
 // map.)
-template <int CPL>
-__global__ __launch_bounds__(64 * kFusedWaves, CPL == 1 ? kFusedWavesPerSimd + 1 : kFusedWavesPerSimd)
+template <int CPL, bool FLT>
+__global__ __launch_bounds__(64 * kFusedWaves, CPL == 1 && !FLT ? kFusedWavesPerSimd + 1 : kFusedWavesPerSimd)
 void k_curvelets(FusedArgs A)
 {
     extern __shared__ double lds[];
@@ -1002,7 +1196,7 @@ void k_curvelets(FusedArgs A)
     unsigned long long isect = 0;  // bundle intersections the reference tests (per lane)
     char *sl = reinterpret_cast<char *>(lds) + static_cast<size_t>(wave) * slice_carve(A.slots, CPL).bytes;
     int2 *spill = A.spill + static_cast<size_t>(g) * A.spill_stride;
-    const WaveCells<CPL> W = wave_cells<CPL>(A);
+    const WaveCells<CPL> W = wave_cells<CPL, FLT>(A);
 
     // the wave's entries: a cursor into the current list
     int list = L_FIRST - 1, left = 0, at = g;
@@ -1023,20 +1217,24 @@ void k_curvelets(FusedArgs A)
         if (id >= 0) v = A.rec[id];
         return v;
     };
+    auto load_th = [&](int id) -> double { return FLT && id >= 0 ? A.th[id] : 0.0; };
     int a = 0, deg, na = 0, ndeg = -1;
     unsigned base = 0, nbase = 0;
     next(a, base, deg);
-    double4 nb = load_rec(load_id(base, deg));
+    int id = load_id(base, deg);
+    double4 nb = load_rec(id);
+    double nth = load_th(id);
     if (deg >= 0) next(na, nbase, ndeg);
     int nid = load_id(nbase, ndeg);
     while (deg >= 0) {
         // start the next anchor's loads
         const double4 nnb = load_rec(nid);
+        const double nnth = load_th(nid);
         int nna = 0, nndeg = -1;
         unsigned nnbase = 0;
         if (ndeg >= 0) next(nna, nnbase, nndeg);
         const int nnid = load_id(nnbase, nndeg);
-        if (do_anchor<CPL, 1, false>(A, W, sl, spill, a, base, deg, nb, vp, isect)) {
+        if (do_anchor<CPL, 1, FLT ? M_FLOAT : M_FAST>(A, W, sl, spill, a, base, deg, id, nb, nth, vp, isect)) {
             if (lane == 0)
                 A.lists[static_cast<size_t>(L_OPEN) * A.n + atomicAdd(A.list_len + L_OPEN * kBucketStride, 1u)] =
                     make_int4(a, static_cast<int>(base), deg, 0);
@@ -1045,6 +1243,8 @@ void k_curvelets(FusedArgs A)
         base = nbase;
         deg = ndeg;
         nb = nnb;
+        nth = nnth;
+        id = nid;
         na = nna;
         nbase = nnbase;
         ndeg = nndeg;
@@ -1075,7 +1275,7 @@ __global__ __launch_bounds__(64, 4) void k_curvelets_exact(FusedArgs A, int list
             load_entry(A.lists + static_cast<size_t>(list) * A.n + L, a, base, deg);
             double4 nb = make_double4(0.0, 0.0, 0.0, 1.0);
             if (lane < deg) nb = A.rec[A.ids[base + lane]];
-            (void)do_anchor<CPL, NW, true>(A, W, reinterpret_cast<char *>(lds), spill, a, base, deg, nb, vp, isect);
+            (void)do_anchor<CPL, NW, M_EXACT>(A, W, reinterpret_cast<char *>(lds), spill, a, base, deg, 0, nb, 0.0, vp, isect);
         }
     }
     put_sums(A.partial, g, vp, isect);
@@ -1085,9 +1285,10 @@ using FusedKernel = void (*)(FusedArgs);
 using ExactKernel = void (*)(FusedArgs, int);
 
 // by cells per lane
+template <bool FLT>
 inline FusedKernel fused_kernel(int cpl)
 {
-    return cpl == 1 ? k_curvelets<1> : (cpl == 2 ? k_curvelets<2> : k_curvelets<4>);
+    return cpl == 1 ? k_curvelets<1, FLT> : (cpl == 2 ? k_curvelets<2, FLT> : k_curvelets<4, FLT>);
 }
 template <int NW>
 inline ExactKernel exact_kernel(int cpl)

@@ -2024,7 +2024,9 @@ __global__ __launch_bounds__(kBlock) void k_row_anchors(int n, const unsigned *_
             vp += s_vp[w];
             is += s_is[w];
         }
-        scal[S_VALID] = static_cast<unsigned>(vp);
+        // (beside what k_curvelets_generic counted of the same map)
+        is += static_cast<unsigned long long>(scal[S_COUNT]) | static_cast<unsigned long long>(scal[S_COUNT + 1]) << 32;
+        scal[S_VALID] += static_cast<unsigned>(vp);
         scal[S_COUNT] = static_cast<unsigned>(is);
         scal[S_COUNT + 1] = static_cast<unsigned>(is >> 32);
     }
@@ -2203,6 +2205,10 @@ struct GenArgs {
     unsigned *acc_count;
     unsigned *valid_pairs;
     unsigned long long *intersections;
+    // the anchors of these two lists (lengths first, kBucketStride apart) in
+    // place of 0 .. n - 1
+    const int4 *list[2];
+    const unsigned *list_len;
 };
 
 constexpr int kGenWaves = 4;  // waves per workgroup of k_curvelets_generic
@@ -2246,7 +2252,10 @@ __global__ __launch_bounds__(64 * kGenWaves) void k_curvelets_generic(GenArgs<T>
     }
     unsigned vpw = 0;
     unsigned long long isect = 0;
-    for (int a = w; a < A.n; a += nwaves) {
+    const int n0 = A.list_len ? static_cast<int>(A.list_len[0]) : 0;
+    const int total = A.list_len ? n0 + static_cast<int>(A.list_len[kBucketStride]) : A.n;
+    for (int i = w; i < total; i += nwaves) {
+        const int a = !A.list_len ? i : (i < n0 ? A.list[0][i].x : A.list[1][i - n0].x);
         const unsigned base = A.off[a];
         const int deg = static_cast<int>(A.off[a + 1] - base);
         const T ax = static_cast<T>(A.x[a]), ay = static_cast<T>(A.y[a]);
@@ -3261,6 +3270,53 @@ int record_rows(cvg_context *ctx, const cvg_params &p, RecordArgs R, int st_stri
     return CVG_OK;
 }
 
+// The launch of k_curvelets: as many waves as stay resident, each looping over
+// its share of the lists.  The slots keep kFusedWavesPerSimd waves per SIMD
+// resident; a run's bundles beyond them (under 1% of the runs) go to device
+// memory, `spill` words per wave.
+struct FusedShape {
+    FusedKernel fn;
+    int slots;
+    unsigned shmem;
+    size_t spill;
+    long long waves;
+};
+
+template <bool FLT>
+int fused_shape(cvg_context *ctx, int K, FusedShape *f)
+{
+    const int cpl = K <= 64 ? 1 : (K <= 128 ? 2 : 4);
+    f->fn = fused_kernel<FLT>(cpl);
+    f->slots = std::max(kSmallRun, kFusedSlots / cpl);
+    f->shmem = static_cast<unsigned>(slice_carve(f->slots, cpl).bytes) * kFusedWaves;
+    int occ = 0;
+    CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(f->fn), 64 * kFusedWaves, f->shmem, &occ));
+    f->spill = static_cast<size_t>(std::max(0, static_cast<int>(std::min(ctx->max_deg, 64u)) - f->slots)) * cpl * 64;
+    long long blocks = static_cast<long long>(std::max(occ, 1)) * ctx->num_cu;
+    if (ctx->grid_pct > 0) blocks = std::max(1LL, blocks * ctx->grid_pct / 100);
+    blocks = std::min(blocks, (static_cast<long long>(ctx->n) + kFusedWaves - 1) / kFusedWaves);
+    // (the no-alloc scratch leaves a smaller grid's worth)
+    if (ctx->arena && f->spill > 0)
+        blocks = std::max(1LL, std::min(blocks, static_cast<long long>((size_t(6) << 20) / (f->spill * sizeof(int2))) /
+                                                    kFusedWaves));
+    f->waves = blocks * kFusedWaves;
+    return CVG_OK;
+}
+
+// Whether the fused kernel's float sines can be trusted for this graph and
+// these parameters (kSineErr): orientations up to kWideTheta, offsets up to 8,
+// and bounds and coordinates differences that stay finite and normal.
+template <typename T>
+bool float_limits(const cvg_context *ctx, double dx, double max_k, const std::vector<T> &off_x,
+                  const std::vector<T> &off_t, double dt)
+{
+    double xmax = 0.0, tmax = std::fabs(dt);
+    for (T v : off_x) xmax = std::max(xmax, std::fabs(static_cast<double>(v)));
+    for (T v : off_t) tmax = std::max(tmax, std::fabs(static_cast<double>(v)));
+    const double S = 2.0 * (static_cast<double>(ctx->nbr_radius) + 1.0);
+    return dx >= 1e-9 && max_k >= 1e-9 && max_k <= 1e9 && tmax <= 8.0 && S + dx + xmax <= 1e5 && !ctx->wide_theta;
+}
+
 // The curvelet stage on k_curvelets_generic: the float instantiation
 // (run_curvelet<float>: the parameters cast to float as main.cpp:22-30 casts
 // them, the bundle grid of init_curvelet_storage (:73-74) from float dx / sx
@@ -3323,6 +3379,16 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
     std::vector<char> blob;
     const size_t o_off_x = put(blob, off_x), o_off_t = put(blob, off_t), o_inf_x = put(blob, inf_x),
                  o_inf_t = put(blob, inf_t), o_crank = put(blob, cell_rank), o_rcell = put(blob, rank_cell);
+    // in rank order: delta_x2, delta_t2, its sine and cosine
+    std::vector<double> rank(4 * static_cast<size_t>(K));
+    for (int r = 0; r < K; ++r) {
+        const double ot = static_cast<double>(off_t[rank_cell[r] % kt]);
+        rank[r] = static_cast<double>(off_x[rank_cell[r] / kt]);
+        rank[K + r] = ot;
+        rank[2 * K + r] = std::sin(ot);
+        rank[3 * K + r] = std::cos(ot);
+    }
+    const size_t o_rank = put(blob, rank), o_elig = put(blob, std::vector<int>(K, 1));
     CVG_TRY(upload_tables(ctx, blob));
     char *tb = static_cast<char *>(ctx->d_tables.ptr);
 
@@ -3333,7 +3399,20 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
     CVG_TRY(ensure(ctx, ctx->d_acc, static_cast<size_t>(n) * sizeof(unsigned)));
     CVG_TRY(ensure(ctx, ctx->d_rowoff, static_cast<size_t>(n + 1) * sizeof(unsigned)));
     unsigned *scal = as<unsigned>(ctx->d_scal);
-    CVG_HIP(ctx, hipMemsetAsync(scal + S_VALID, 0, (kScalarBufWords - S_VALID) * sizeof(unsigned), st));
+    // float maps: the fused kernel, then this one on the anchors it leaves (a
+    // sine, a direction or a zero it cannot settle, or more than 64
+    // neighbours).  The lists hold up to 256 neighbours' anchors; below three
+    // edges no chain is long enough, and this kernel counts the intersections.
+    const bool fused = kFloat && G >= 3 && G <= 64 && ctx->max_deg <= 256 && !ctx->force_generic &&
+                       float_limits(ctx, p.dx, p.max_k, off_x, off_t, dt) &&
+                       *std::max_element(cell_rank.begin(), cell_rank.end()) < K;
+    if (!fused) {
+        ctx->setup_queued = false;
+        CVG_HIP(ctx, hipMemsetAsync(scal + S_VALID, 0, (kScalarBufWords - S_VALID) * sizeof(unsigned), st));
+    } else {
+        if (!ctx->setup_queued) CVG_TRY(queue_setup(ctx));
+        ctx->setup_queued = false;
+    }
 
     // one wave per anchor, as many waves as the per-wave scratch allows
     const size_t per_wave = static_cast<size_t>(max_deg) * K * 2 * sizeof(T) +
@@ -3348,7 +3427,10 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
     const size_t sf_ints = nwaves * max_deg;
     const size_t sa_ints = nwaves * max_deg * (cap + 1);
     const size_t sc_ints = nwaves * cap;
-    CVG_TRY(ensure(ctx, ctx->d_gbundle, sb_elems * sizeof(T) + (sf_ints + sa_ints + sc_ints) * sizeof(int) + 512));
+    const size_t general_bytes = sb_elems * sizeof(T) + (sf_ints + sa_ints + sc_ints) * sizeof(int) + 512;
+    FusedShape f{};
+    if (fused) CVG_TRY(fused_shape<true>(ctx, K, &f));
+    CVG_TRY(ensure(ctx, ctx->d_gbundle, std::max(general_bytes, f.spill * static_cast<size_t>(f.waves) * sizeof(int2))));
     GenArgs<T> A{};
     A.n = n;
     A.x = as<double>(ctx->d_x);
@@ -3383,6 +3465,46 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
     const int ring = static_cast<int>(ctx->fused_runs % cvg_context::kFusedRing);
     CVG_TRY(record_timing(ctx, ctx->ev[3], st));
     CVG_TRY(record_timing(ctx, ctx->fused_ev[ring][0], st));
+    if (fused) {
+        FusedArgs M{};
+        M.rec = as<double4>(ctx->d_rec);
+        M.ids = A.ids;
+        M.th = A.th;
+        M.K = K;
+        M.G = G;
+        M.rank_ox = reinterpret_cast<const double *>(tb + o_rank);
+        M.rank_ot = M.rank_ox + K;
+        M.rank_so = M.rank_ot + K;
+        M.rank_co = M.rank_so + K;
+        M.rank_elig = reinterpret_cast<const int *>(tb + o_elig);
+        M.rank_cell = A.rank_cell;
+        M.sin_dt = std::sin(static_cast<double>(dt));
+        M.cos_dt = std::cos(static_cast<double>(dt));
+        M.dx2 = A.dx2;
+        M.dt_f = dt;
+        M.dx_f = dx;
+        M.max_k_f = max_k;
+        M.close_f = A.close_thr;
+        M.st_ids = A.st_ids;
+        M.st_stride = cap;
+        M.st_k = A.st_k;
+        M.st_meta = A.st_meta;
+        M.acc_count = A.acc_count;
+        M.lists = as<int4>(ctx->d_lists);
+        M.list_len = scal + kBucketBase;
+        M.n = n;
+        M.slots = f.slots;
+        M.spill = as<int2>(ctx->d_gbundle);
+        M.spill_stride = f.spill;
+        CVG_TRY(ensure(ctx, ctx->d_partial, static_cast<size_t>(f.waves) * 3 * sizeof(unsigned)));
+        M.partial = as<unsigned>(ctx->d_partial);
+        hipLaunchKernelGGL(f.fn, dim3(static_cast<unsigned>(f.waves / kFusedWaves)), dim3(64 * kFusedWaves), f.shmem, st,
+                           M);
+        A.list[0] = M.lists + static_cast<size_t>(L_OPEN) * n;
+        A.list[1] = M.lists + static_cast<size_t>(L_WIDE) * n;
+        A.list_len = M.list_len;
+        static_assert(L_WIDE == L_OPEN + 1, "the lists' lengths follow each other");
+    }
     hipLaunchKernelGGL(k_curvelets_generic<T>, dim3(blocks), dim3(64 * kGenWaves), 0, st, A);
     CVG_HIP(ctx, hipGetLastError());
     CVG_TRY(record_timing(ctx, ctx->ev[4], st));
@@ -3402,7 +3524,7 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
         R.off_x = reinterpret_cast<const double *>(tb + o_off_x);
         R.off_t = reinterpret_cast<const double *>(tb + o_off_t);
     }
-    return record_rows(ctx, p, R, cap, 0);
+    return record_rows(ctx, p, R, cap, static_cast<int>(f.waves));
 }
 
 int build_curvelets(cvg_context *ctx, const cvg_params &p)
@@ -3481,39 +3603,27 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     A.st_meta = as<unsigned>(ctx->d_st_meta);
     A.acc_count = as<unsigned>(ctx->d_acc);
 
-    // A persistent launch (as many waves as stay resident, each looping over
-    // its share of the lists), then the anchors it leaves open; anchors of more
-    // than 64 neighbours, where the map has any, beside it on an auxiliary
-    // stream.  The slots keep kFusedWavesPerSimd waves per SIMD resident; a
-    // run's bundles beyond them (under 1% of the runs) go to device memory.
-    const FusedKernel fn = fused_kernel(d.cpl);
+    // k_curvelets, then the anchors it leaves open; anchors of more than 64
+    // neighbours, where the map has any, beside it on an auxiliary stream
+    FusedShape f{};
+    CVG_TRY(fused_shape<false>(ctx, A.K, &f));
     const ExactKernel fn_open = exact_kernel<1>(d.cpl), fn_wide = exact_kernel<4>(d.cpl);
-    A.slots = std::max(kSmallRun, kFusedSlots / d.cpl);
-    const unsigned slice = static_cast<unsigned>(slice_carve(A.slots, d.cpl).bytes);
-    const unsigned shmem = slice * kFusedWaves;
-    int occ = 0, occ_wide = 0, occ_open = 0;
-    CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(fn), 64 * kFusedWaves, shmem, &occ));
-    CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(fn_open), 64, slice, &occ_open));
+    A.slots = f.slots;
+    const unsigned slice = f.shmem / kFusedWaves;
+    int occ_wide = 0;
+    CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(fn_open), 64, slice, nullptr));
     CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(fn_wide), 64, slice, &occ_wide));
-    // bundle words in device memory per wave
-    const size_t word = static_cast<size_t>(d.cpl) * 64;
-    const size_t spill_main = std::max(0, static_cast<int>(std::min(ctx->max_deg, 64u)) - A.slots) * word;
-    const size_t spill_exact = std::max(0, static_cast<int>(ctx->max_deg) - A.slots) * word;
-    long long blocks = static_cast<long long>(std::max(occ, 1)) * ctx->num_cu;
-    if (ctx->grid_pct > 0) blocks = std::max(1LL, blocks * ctx->grid_pct / 100);
-    blocks = std::min(blocks, (static_cast<long long>(n) + kFusedWaves - 1) / kFusedWaves);
+    const size_t spill_exact = static_cast<size_t>(std::max(0, static_cast<int>(ctx->max_deg) - A.slots)) * d.cpl * 64;
     long long blocks_wide = wide ? std::min<long long>(n, static_cast<long long>(std::max(occ_wide, 1)) * ctx->num_cu) : 0;
     long long blocks_open = std::min<long long>(n, ctx->num_cu);
-    // (the no-alloc scratch leaves a smaller grid's worth)
     if (ctx->arena && spill_exact > 0) {
         const long long fit = static_cast<long long>((size_t(6) << 20) / (spill_exact * sizeof(int2)));
-        blocks = std::max(1LL, std::min(blocks, fit / kFusedWaves));
         blocks_wide = std::min(blocks_wide, std::max(1LL, fit));
         blocks_open = std::max(1LL, std::min(blocks_open, fit));
     }
-    const int waves_main = static_cast<int>(blocks) * kFusedWaves;
+    const int waves_main = static_cast<int>(f.waves);
     const int waves = waves_main + static_cast<int>(blocks_wide + blocks_open);
-    CVG_TRY(ensure(ctx, ctx->d_gbundle, (std::max<size_t>(spill_main * waves_main, spill_exact * blocks_open) +
+    CVG_TRY(ensure(ctx, ctx->d_gbundle, (std::max<size_t>(f.spill * waves_main, spill_exact * blocks_open) +
                                          spill_exact * blocks_wide) * sizeof(int2)));
     CVG_TRY(ensure(ctx, ctx->d_partial, static_cast<size_t>(waves) * 3 * sizeof(unsigned)));
     A.lists = as<int4>(ctx->d_lists);
@@ -3536,9 +3646,9 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
         CVG_HIP(ctx, hipEventRecord(ctx->ev_join, ctx->aux));
     }
     A.spill = as<int2>(ctx->d_gbundle) + spill_exact * blocks_wide;
-    A.spill_stride = spill_main;
+    A.spill_stride = f.spill;
     A.partial = as<unsigned>(ctx->d_partial) + 3 * blocks_wide;
-    hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(blocks)), dim3(64 * kFusedWaves), shmem, st, A);
+    hipLaunchKernelGGL(f.fn, dim3(static_cast<unsigned>(f.waves / kFusedWaves)), dim3(64 * kFusedWaves), f.shmem, st, A);
     X.spill = A.spill;
     X.partial = A.partial + 3 * waves_main;
     hipLaunchKernelGGL(fn_open, dim3(static_cast<unsigned>(blocks_open)), dim3(64), slice, st, X,
@@ -3590,7 +3700,7 @@ int run_common(cvg_context *ctx, int n, int sz, const double *d_edges, const cvg
     CVG_TRY(record_timing(ctx, ctx->ev[0], ctx->stream));
     ctx->use_cellrank = false;
     ctx->setup_queued = false;
-    ctx->early_setup = !f32 && p->group_max_sz <= 64 && !ctx->force_generic;
+    ctx->early_setup = p->group_max_sz <= 64 && !ctx->force_generic;
     const int rc = build_graph(ctx, n, sz, d_edges, p->nrad, 3u, p->max_candidates, num_maps, eoff);  // main.cpp:48: 3
     ctx->early_setup = false;
     if (rc != CVG_OK) return rc;

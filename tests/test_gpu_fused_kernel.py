@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 from curvelet_construction_on_gpu_amd import Context, CurveletParams
+from oracle import OracleF32
 
 pytestmark = pytest.mark.gpu
 
@@ -93,3 +94,59 @@ def test_parameter_range(both, oracle_cr, dx, dt, max_k, nrad):
     rng = np.random.default_rng(7)
     e = np.stack([rng.uniform(0, 30, 500), rng.uniform(0, 30, 500), rng.uniform(-3, 3, 500), np.ones(500)], axis=1)
     same_bits(both, oracle_cr, e, CurveletParams(dx=dx, dt_deg=dt, max_k=max_k, nrad=nrad, sx=dx / 4))
+
+
+@pytest.fixture(scope="module")
+def oracle_f32_cr():
+    return OracleF32(cr=True)
+
+
+def same_bits_float(both, oracle_f32_cr, edges, p):
+    e = np.ascontiguousarray(edges, dtype=np.float32)
+    want = oracle_f32_cr.run(e, p)
+    counts = []
+    for ctx in both:
+        stats = ctx.run_f32(e, p)
+        chains, info = ctx.curvelets()
+        assert stats["valid_pairs"] == want["valid_pairs"]
+        assert np.array_equal(chains, want["chains"])
+        assert np.array_equal(info.view(np.uint64), want["info"].view(np.uint64))
+        counts.append(stats["intersections"])
+    assert counts[0] == counts[1]
+
+
+@pytest.mark.parametrize("group", [2, 3, 7, 12])
+@pytest.mark.parametrize("run", [1, 2, 8, 9, 14, 15, 32, 33, 65])
+def test_float_run_lengths(both, oracle_f32_cr, run, group):
+    same_bits_float(both, oracle_f32_cr, lines(run, seed=run), CurveletParams(group_max_sz=group, max_candidates=256))
+
+
+@pytest.mark.parametrize("sx,st", [(0.1, 0.08), (0.05, 0.08), (0.05, 0.04)])
+@pytest.mark.parametrize("cand", [64, 65])
+def test_float_list_lengths_and_cells(both, oracle_f32_cr, sx, st, cand):
+    rng = np.random.default_rng(cand)
+    e = np.stack([rng.uniform(0, 10, 420), rng.uniform(0, 10, 420), rng.uniform(0, 0.8, 420), np.ones(420)], axis=1)
+    same_bits_float(both, oracle_f32_cr, e, CurveletParams(sx=sx, st=st, group_max_sz=6, max_candidates=cand))
+
+
+@pytest.mark.parametrize("angle", [0.0, np.pi / 2, np.pi / 4])
+def test_float_equal_bounds(both, oracle_f32_cr, angle):
+    xs, ys = np.meshgrid(np.arange(12) * 1.0, np.arange(9) * 1.0)
+    e = np.stack([xs.ravel(), ys.ravel(), np.full(xs.size, angle), np.ones(xs.size)], axis=1)
+    same_bits_float(both, oracle_f32_cr, e, CurveletParams(group_max_sz=5))
+
+
+@pytest.mark.parametrize("top", [63.9, 64.0, 64.1, 1e5])
+def test_float_orientation_range(both, oracle_f32_cr, top):
+    e = lines(6, seed=3)
+    e[:, 2] += 2 * np.pi * np.floor((top - e[:, 2].max()) / (2 * np.pi))
+    e[0, 2] = top
+    same_bits_float(both, oracle_f32_cr, e, CurveletParams(group_max_sz=7))
+
+
+@pytest.mark.parametrize("dx,dt,max_k,nrad", [(0.2, 2.0, 2.0, 3.0), (1.5, 40.0, 0.05, 5.0), (0.4, 15.0, 1e-6, 3.5),
+                                              (0.4, 15.0, 1e4, 3.5), (12.0, 15.0, 0.3, 3.5)])
+def test_float_parameter_range(both, oracle_f32_cr, dx, dt, max_k, nrad):
+    rng = np.random.default_rng(7)
+    e = np.stack([rng.uniform(0, 30, 500), rng.uniform(0, 30, 500), rng.uniform(-3, 3, 500), np.ones(500)], axis=1)
+    same_bits_float(both, oracle_f32_cr, e, CurveletParams(dx=dx, dt_deg=dt, max_k=max_k, nrad=nrad, sx=dx / 4))

@@ -45,6 +45,8 @@
 #include <atomic>
 #include <chrono>
 #include <climits>
+#include <condition_variable>
+#include <functional>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -112,6 +114,75 @@ struct GridDesc {
 
 }  // namespace
 
+// Up to 11 helper threads for the copies out of page-locked blocks (the
+// calling thread is another): started at a context's first such download,
+// parked between downloads, joined with the context.
+struct CopyCrew {
+    std::mutex mu;
+    std::condition_variable wake, idle;
+    std::vector<std::thread> threads;
+    const std::function<void()> *job = nullptr;
+    unsigned long long serial = 0;
+    int active = 0;
+    bool started = false, stop = false;
+
+    // The helpers run *fn once each, those that wake before end().
+    void begin(const std::function<void()> *fn)
+    {
+        if (!started) {
+            started = true;
+            const unsigned hw = std::thread::hardware_concurrency();
+            const int count = static_cast<int>(std::min<unsigned>(hw > 1 ? hw - 1 : 0, 11));
+            for (int w = 0; w < count; ++w) {
+                try {
+                    threads.emplace_back([this] { loop(); });
+                } catch (...) {
+                    break;  // fewer helpers
+                }
+            }
+        }
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            job = fn;
+            ++serial;
+        }
+        wake.notify_all();
+    }
+    void end()
+    {
+        std::unique_lock<std::mutex> lk(mu);
+        job = nullptr;
+        idle.wait(lk, [this] { return active == 0; });
+    }
+    ~CopyCrew()
+    {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            stop = true;
+        }
+        wake.notify_all();
+        for (auto &th : threads) th.join();
+    }
+
+private:
+    void loop()
+    {
+        unsigned long long seen = 0;
+        std::unique_lock<std::mutex> lk(mu);
+        while (true) {
+            wake.wait(lk, [&] { return stop || (job && serial != seen); });
+            if (stop) return;
+            seen = serial;
+            const std::function<void()> *fn = job;
+            ++active;
+            lk.unlock();
+            (*fn)();
+            lk.lock();
+            if (--active == 0) idle.notify_all();
+        }
+    }
+};
+
 struct cvg_context {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -158,6 +229,7 @@ struct cvg_context {
     unsigned *mailbox = nullptr;  // pinned host scalars read back after syncs
     // page-locked staging blocks for downloads into pageable caller memory
     void *h_stage[2] = {nullptr, nullptr};
+    CopyCrew crew;
     hipEvent_t ev_stage[2] = {nullptr, nullptr};
 
     // graph
@@ -3751,6 +3823,30 @@ int upload(cvg_context *ctx, int n, int sz, const double *host, const double **d
     return CVG_OK;
 }
 
+__global__ __launch_bounds__(kBlock) void k_widen(long long count, const float *__restrict__ in,
+                                                  double *__restrict__ out)
+{
+    const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < count) out[i] = static_cast<double>(in[i]);
+}
+
+// Float edges, held exactly as doubles on the device (widened there: half the
+// bytes over the link, and no host copy).  The caller's array is free on return.
+int upload_f32(cvg_context *ctx, int n, int sz, const float *host, const double **dptr)
+{
+    const size_t count = static_cast<size_t>(n) * sz;
+    CVG_TRY(ensure(ctx, ctx->d_edges_up, count * (sizeof(double) + sizeof(float))));
+    double *wide = as<double>(ctx->d_edges_up);
+    float *in = reinterpret_cast<float *>(wide + count);
+    CVG_HIP(ctx, hipMemcpyAsync(in, host, count * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+    CVG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    hipLaunchKernelGGL(k_widen, dim3(blocks_for(static_cast<long long>(count))), dim3(kBlock), 0, ctx->stream,
+                       static_cast<long long>(count), in, wide);
+    CVG_HIP(ctx, hipGetLastError());
+    *dptr = wide;
+    return CVG_OK;
+}
+
 // This device's copy of `scratch`, resolved once per device with that device
 // current (each GPU holds its own copy at its own address).
 constexpr int kMaxDevices = 64;
@@ -3779,6 +3875,7 @@ int scratch_address(cvg_context *ctx)
 // k + 1's DMA runs.
 constexpr size_t kStageBytes = static_cast<size_t>(4) << 20;
 constexpr size_t kStageMinBytes = static_cast<size_t>(1) << 20;
+constexpr size_t kSliceBytes = static_cast<size_t>(128) << 10;
 
 struct Segment {
     void *dst;
@@ -3834,58 +3931,50 @@ int download(cvg_context *ctx, std::initializer_list<Segment> segs)
         CVG_HIP(ctx, hipEventRecord(ctx->ev_stage[b], st));
         return CVG_OK;
     };
-    // host copy-out: nw helper threads and this one split each chunk; the
-    // chunk a helper may copy is published in `ready`, and `done` counts
-    // finished slices (every helper does one slice per chunk)
-    const unsigned hw = std::thread::hardware_concurrency();
-    const int nw = static_cast<int>(std::min<unsigned>(hw > 1 ? hw - 1 : 0, 11));
-    const int parts = nw + 1;
-    std::atomic<long long> ready{-1};
-    std::atomic<long long> done{0};
-    std::atomic<bool> quit{false};
-    auto slice = [&](size_t k, int part) {
-        const size_t len = chunks[k].len;
-        const size_t per = ((len + parts - 1) / parts + 63) & ~static_cast<size_t>(63);
-        const size_t o = std::min(len, per * part), e = std::min(len, o + per);
-        if (e > o) std::memcpy(chunks[k].dst + o, static_cast<const char *>(ctx->h_stage[k & 1]) + o, e - o);
-    };
-    std::vector<std::thread> pool;
-    for (int w = 0; w < nw; ++w) {
-        try {
-            pool.emplace_back([&, w] {
-                for (size_t k = 0; k < nchunk; ++k) {
-                    while (ready.load(std::memory_order_acquire) < static_cast<long long>(k)) {
-                        if (quit.load(std::memory_order_relaxed)) return;
-                        std::this_thread::yield();
-                    }
-                    slice(k, w + 1);
-                    done.fetch_add(1, std::memory_order_release);
-                }
-            });
-        } catch (...) {
-            break;  // fewer helpers: the slices of missing ones are copied below
-        }
-    }
-    const int started = static_cast<int>(pool.size());
     int rc = issue(0);
+    if (rc == CVG_OK && nchunk > 1) rc = issue(1);
+    // host copy-out: this thread and the context's helpers take kSliceBytes
+    // slices in order; chunks below `ready` are in their blocks, and copied[b]
+    // counts block b's slices out again.  The helpers outlive the call:
+    // starting them took longer than copying a chunk.
+    constexpr size_t kSlices = kStageBytes / kSliceBytes;
+    std::atomic<size_t> next{0}, ready{0};
+    std::atomic<size_t> copied[2] = {{0}, {0}};
+    std::atomic<bool> quit{false};
+    auto take = [&](size_t limit) -> bool {  // one slice of a chunk below limit
+        size_t s = next.load(std::memory_order_relaxed);
+        do {
+            if (s >= limit * kSlices) return false;
+        } while (!next.compare_exchange_weak(s, s + 1, std::memory_order_relaxed));
+        const size_t k = s / kSlices, o = (s % kSlices) * kSliceBytes;
+        while (ready.load(std::memory_order_acquire) <= k) {
+            if (quit.load(std::memory_order_relaxed)) return false;
+            std::this_thread::yield();
+        }
+        if (o < chunks[k].len)
+            std::memcpy(chunks[k].dst + o, static_cast<const char *>(ctx->h_stage[k & 1]) + o,
+                        std::min(kSliceBytes, chunks[k].len - o));
+        copied[k & 1].fetch_add(1, std::memory_order_release);
+        return true;
+    };
+    const std::function<void()> help = [&] {
+        while (take(nchunk)) {
+        }
+    };
+    if (rc == CVG_OK) ctx->crew.begin(&help);
     for (size_t k = 0; rc == CVG_OK && k < nchunk; ++k) {
-        // block (k + 1) & 1 last held chunk k - 1: every slice of it is copied
-        while (done.load(std::memory_order_acquire) < static_cast<long long>(k) * started) std::this_thread::yield();
-        if (k + 1 < nchunk) rc = issue(k + 1);
-        if (rc != CVG_OK) break;
         if (hipEventSynchronize(ctx->ev_stage[k & 1]) != hipSuccess) {
             rc = fail(ctx, CVG_ERR_DEVICE, "download: staging copy failed");
             break;
         }
-        ready.store(static_cast<long long>(k), std::memory_order_release);
-        slice(k, 0);
-        for (int w = started + 1; w < parts; ++w) slice(k, w);
+        ready.store(k + 1, std::memory_order_release);
+        while (take(k + 1)) {
+        }
+        while (copied[k & 1].load(std::memory_order_acquire) < (k / 2 + 1) * kSlices) std::this_thread::yield();
+        if (k + 2 < nchunk) rc = issue(k + 2);
     }
-    if (rc == CVG_OK)
-        while (done.load(std::memory_order_acquire) < static_cast<long long>(nchunk) * started)
-            std::this_thread::yield();
     quit.store(true, std::memory_order_relaxed);
-    for (auto &t : pool) t.join();
+    ctx->crew.end();
     // the direct copies, and after a failure any DMA still aimed at a block
     if (hipStreamSynchronize(st) != hipSuccess && rc == CVG_OK)
         rc = fail(ctx, CVG_ERR_DEVICE, "download: device-to-host copy failed");
@@ -4053,14 +4142,8 @@ int cvg_build_neighbor_csr_graph_f32(cvg_context *ctx, int num_edges, int sz_edg
     CVG_TRY(check_ctx(ctx));
     if (!edges || num_edges <= 0 || sz_edge_data < 4)
         return fail(ctx, CVG_ERR_INVALID_ARGUMENT, "build_neighbor_csr_graph: need num_edges > 0, sz_edge_data >= 4");
-    std::vector<double> wide;
-    try {
-        wide.assign(edges, edges + static_cast<size_t>(num_edges) * sz_edge_data);
-    } catch (...) {
-        return fail(ctx, CVG_ERR_OUT_OF_MEMORY, "host allocation failed");
-    }
     const double *d = nullptr;
-    CVG_TRY(upload(ctx, num_edges, sz_edge_data, wide.data(), &d));
+    CVG_TRY(upload_f32(ctx, num_edges, sz_edge_data, edges, &d));
     ctx->use_cellrank = false;
     ctx->f32 = true;
     CVG_TRY(build_graph(ctx, num_edges, sz_edge_data, d, rad, neighbor_radius, max_candidates));
@@ -4161,17 +4244,8 @@ int cvg_run_f32(cvg_context *ctx, int num_edges, int sz_edge_data, const float *
     CVG_TRY(check_ctx(ctx));
     if (!params || !edges || num_edges <= 0 || sz_edge_data < 4)
         return fail(ctx, CVG_ERR_INVALID_ARGUMENT, "cvg_run_f32: bad arguments");
-    // the float values held exactly as doubles on the device
-    std::vector<double> wide;
-    try {
-        wide.assign(edges, edges + static_cast<size_t>(num_edges) * sz_edge_data);
-    } catch (...) {
-        return fail(ctx, CVG_ERR_OUT_OF_MEMORY, "cvg_run_f32: host allocation failed");
-    }
     const double *d = nullptr;
-    CVG_TRY(upload(ctx, num_edges, sz_edge_data, wide.data(), &d));
-    // the upload must have left the host vector before it goes away
-    CVG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    CVG_TRY(upload_f32(ctx, num_edges, sz_edge_data, edges, &d));
     return run_common(ctx, num_edges, sz_edge_data, d, params, stats, 1, nullptr, true);
 }
 

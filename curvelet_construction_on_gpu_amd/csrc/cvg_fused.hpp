@@ -17,7 +17,7 @@
 //
 // Measured on the 1080p map (207,326 edges, 2.04M pairs, G = 7): 1,000 us for
 // the kernel on exact bounds and 141 us for its sines pass (345 MB) before; now
-// 530 us, and 83 us for the few anchors left open.
+// 473 us, and 81 us for the few anchors left open.
 #ifndef CVG_FUSED_HPP
 #define CVG_FUSED_HPP
 
@@ -239,7 +239,7 @@ struct FusedArgs {
     const double *rank_ox, *rank_ot, *rank_so, *rank_co;
     const int *rank_elig;
     int rank_of_cell0;
-    double sin_dt, cos_dt, dx, two_dx, dx2, close_thr, max_k;
+    double sin_dt, cos_dt, dx, four_dx, dx2, close_thr, max_k;
     double scale;                    // kFixOne / max_k
     double min_den, num_err, den_err;  // fused_limits
     double min_prod;                 // below it a product of the three denominators may have a small one
@@ -261,9 +261,11 @@ struct FusedArgs {
 };
 
 constexpr int kFusedWaves = 4;  // anchor streams (waves) per workgroup
-constexpr int kFusedWavesPerSimd = 4;
-constexpr int kFusedSlots = 14;  // bundle slots at one cell per lane
-constexpr int kPairBatch = 16;  // pair records in LDS at a time
+constexpr int kFusedWavesPerSimd = 5;  // at one cell per lane (double maps)
+constexpr int kFusedSlots = 12;  // bundle slots at one cell per lane
+// pair records in LDS at a time, as a power of two (with two cells per lane 16
+// of them would cost a resident wave per SIMD)
+__host__ __device__ constexpr int batch_log(int cpl) { return cpl == 1 ? 4 : 3; }
 constexpr int kSmallRun = 8;    // runs up to here grow on cell masks
 
 struct SliceCarve {
@@ -277,7 +279,7 @@ __host__ __device__ inline SliceCarve slice_carve(int slots, int cpl)
     SliceCarve c{};
     c.bun = 0;
     c.rec = c.bun + slots * cpl * 64 * 8;
-    c.pm = c.rec + kPairBatch * 80;
+    c.pm = c.rec + (80 << batch_log(cpl));
     c.bytes = c.pm + 64 * cpl * 8;
     return c;
 }
@@ -285,8 +287,8 @@ __host__ __device__ inline SliceCarve slice_carve(int slots, int cpl)
 // A lane's cells: lanes without one repeat the first.
 template <int CPL>
 struct WaveCells {
-    double ox[CPL], m2ox[CPL], ox2[CPL], oxp[CPL], so[CPL], co[CPL];
-    double ot[CPL];  // (float maps)
+    double ox[CPL], oxp2[CPL], so[CPL], co[CPL];
+    double m2ox[CPL], ox2[CPL], ot[CPL];  // (float maps)
     unsigned long long emask[CPL];  // cells that can be a best one
 };
 
@@ -379,6 +381,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
     constexpr bool EXACT = MODE == M_EXACT, FLT = MODE == M_FLOAT;
     static_assert(!FLT || NW == 1, "float maps: up to 64 neighbours");
     constexpr int kTol = FLT ? 0 : kFixTol;
+    constexpr int kLog = batch_log(CPL), kLast = (1 << kLog) - 1;
     constexpr int NC = NW;  // 64-seed (64-neighbour) chunks
     const int lane = threadIdx.x & 63;
     const int G = A.G;
@@ -518,7 +521,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             }
     }
 
-    // the pair records of batch b (places 16 b .. 16 b + 15) into LDS: DX, DY,
+    // the pair records of batch b (that many places from its number times as many) into LDS: DX, DY,
     // DX^2 + DY^2 - dx^2, and for the lower and the upper orientation
     // constraint (theta_n -+ dt, by branch, :736, :799) the sine and cosine of
     // the angle and DX cos + DY sin
@@ -551,8 +554,8 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                     cx[k] = fx * sure_float(co[k], bad);  // :730-733
                     sy[k] = fy * sure_float(s[k], bad);
                 }
-                if (pos[c] >= 0 && (pos[c] >> 4) == b) {
-                    const lds_ptr<double2> o = rec + (pos[c] & 15) * 5;
+                if (pos[c] >= 0 && (pos[c] >> kLog) == b) {
+                    const lds_ptr<double2> o = rec + (pos[c] & kLast) * 5;
                     o[0].x = s[0];
                     o[0].y = co[0];
                     o[1].x = s[1];
@@ -576,8 +579,8 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             const double sd = branch_a ? -A.sin_dt : A.sin_dt;
             const double s0 = __builtin_fma(q.z, A.cos_dt, q.w * sd), c0 = __builtin_fma(q.w, A.cos_dt, -(q.z * sd));
             const double s1 = __builtin_fma(q.z, A.cos_dt, -(q.w * sd)), c1 = __builtin_fma(q.w, A.cos_dt, q.z * sd);
-            if (pos[c] >= 0 && (pos[c] >> 4) == b) {
-                const lds_ptr<double2> o = rec + (pos[c] & 15) * 5;
+            if (pos[c] >= 0 && (pos[c] >> kLog) == b) {
+                const lds_ptr<double2> o = rec + (pos[c] & kLast) * 5;
                 o[0].x = DX;
                 o[0].y = DY;
                 o[1].x = __builtin_fma(DX, DX, __builtin_fma(DY, DY, -A.dx2));
@@ -614,15 +617,142 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
 #pragma unroll
         for (int w = 0; w < NW; ++w) place[w] = 0ULL;
 
-        // the run's bundles (compute_curve_bundle, :636-819)
+        // the bundle of the pair at place p (record q, not close): the lane's
+        // cells and, as bits, those with hi > lo (compute_curve_bundle, :636-819)
+        auto bundle = [&](int p, lds_ptr<double2> q, Bounds (&v)[CPL]) __attribute__((always_inline)) -> u64 {
+            if constexpr (FLT) {
+                // compute_curve_bundle<float>; its branches differ (a
+                // power of two on both sides of a quotient apart) in the
+                // angles' order only
+                const lds_ptr<float4> f = (lds_ptr<float4>)(q + 3);
+                const float DX = f[0].x, DY = f[0].y;
+                const double DX2 = q[2].x, DY2 = q[2].y;
+                u64 any = 0ULL;
+#pragma unroll
+                for (int m = 0; m < CPL; ++m) {
+                    const float o = static_cast<float>(W.ox[m]);
+                    const float tt = sf[m] * DX - cf[m] * DY;  // :705
+                    const float ttm = tt - o;
+                    // :711 (the first product is exact)
+                    const float den = static_cast<float>(
+                        __builtin_fma(W.m2ox[m], static_cast<double>(tt), DX2) + DY2 - A.dx2 + W.ox2[m]);
+                    const float kx0 = 2.0f * (ttm - A.dx_f) / den, kx1 = 2.0f * (ttm + A.dx_f) / den;
+                    float kt[2];
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+                        const double s0 = q[k].x, c0 = q[k].y;
+                        const float T0 = k == 0 ? f[0].z : f[0].w;
+                        const float cx = k == 0 ? f[1].x : f[1].z, sy = k == 0 ? f[1].y : f[1].w;
+                        const double e = static_cast<double>(T2[m] - T0) -
+                                         (static_cast<double>(T2[m]) - static_cast<double>(T0));
+                        const double s = __builtin_fma(sT[m], c0, -(cT[m] * s0));
+                        const double c = __builtin_fma(cT[m], c0, sT[m] * s0);
+                        const float sn = sure_float(__builtin_fma(e, __builtin_fma(-0.5 * e, s, c), s), bad);
+                        kt[k] = sn / (-sn * o + cx + sy);
+                    }
+                    // the reference's compare-and-assign, which ignores NaN
+                    const float lo = __builtin_fmaxf(__builtin_fmaxf(-A.max_k_f, kx0), kt[0]);
+                    const float hi = __builtin_fminf(__builtin_fminf(A.max_k_f, kx1), kt[1]);
+                    least = __builtin_fminf(least, __builtin_fminf(__builtin_fabsf(lo), __builtin_fabsf(hi)));
+                    const bool ok = hi > lo;
+                    v[m].lo = ok ? float_key(lo) : INT_MAX;
+                    v[m].hi = ok ? float_key(hi) : INT_MIN;
+                    any |= __builtin_amdgcn_ballot_w64(ok);
+                }
+                return any;
+            } else {
+                const double DX = q[0].x, DY = q[0].y, r2 = q[1].x, C0 = q[1].y, C1 = q[2].x;
+                const double s0n = q[2].y, c0n = q[3].x, s1n = q[3].y, c1n = q[4].x;
+                u64 any = 0ULL;  // cells with hi > lo
+#pragma unroll
+                for (int m = 0; m < CPL; ++m) {
+                    const double tt = __builtin_fma(sT[m], DX, -(cT[m] * DY));
+                    const double den = __builtin_fma(W.ox[m], __builtin_fma(-2.0, tt, W.ox[m]), r2);
+                    const double x0 = __builtin_fma(2.0, tt, -W.oxp2[m]);  // :712's numerator
+                    const double s0 = __builtin_fma(sT[m], c0n, -(cT[m] * s0n));
+                    const double s1 = __builtin_fma(sT[m], c1n, -(cT[m] * s1n));
+                    const double d0 = __builtin_fma(-s0, W.ox[m], C0);
+                    const double d1 = __builtin_fma(-s1, W.ox[m], C1);
+                    // 1 / den, 1 / d0 and 1 / d1 (times scale) from one reciprocal
+                    const double pp = den * d0, ppp = pp * d1;
+                    double y = __builtin_amdgcn_rcp(ppp);
+                    y = __builtin_fma(y, __builtin_fma(-ppp, y, 1.0), y);
+                    y *= A.scale;
+                    const double yd1 = y * pp, w = y * d1;
+                    const double yd0 = w * den, yx = w * d0;
+                    const double k0 = x0 * yx, k1 = __builtin_fma(A.four_dx, yx, k0);
+                    int lo = max(fix(k0), fix(s0 * yd0));
+                    int hi = min(fix(k1), fix(s1 * yd1));
+                    const int t = min(sub_sat(hi, lo), min(sub_sat(hi, -kFixOne), sub_sat(kFixOne, lo)));
+                    note(t);
+                    bool ok = t > kFixTol;
+                    u64 T = __builtin_amdgcn_ballot_w64(ok);
+                    u64 U = EXACT ? is_open(t) : 0ULL;
+                    // a small denominator (then the product is small as well)
+                    // settles nothing unless its sign is certain and its
+                    // quotients lie well beyond max_k, where they stay either way
+                    if (__builtin_amdgcn_ballot_w64(!(fabs(ppp) >= A.min_prod)) != 0ULL) {
+                        auto weak = [&](double n, double d) {
+                            return !(fabs(d) >= A.min_den) &&
+                                   !(fabs(d) > A.den_err && fabs(n) > 4.0 * A.max_k * fabs(d) + A.num_err);
+                        };
+                        const bool bad = weak(x0, den) || weak(x0 + A.four_dx, den) ||
+                                         weak(s0, d0) || weak(s1, d1);
+                        if (EXACT)
+                            U |= __builtin_amdgcn_ballot_w64(bad);
+                        else
+                            closest = bad ? 0u : closest;
+                    }
+                    if constexpr (EXACT) {
+                        if (U != 0ULL) {
+                            const int b = neighbour(p);
+                            bool valid = false;
+                            if (__builtin_amdgcn_inverse_ballot_w64(U)) {
+                                double elo = 0.0, ehi = 0.0;
+                                exact_cell(m, b, elo, ehi);
+                                valid = ehi > elo;
+                                lo = fix(elo * A.scale);
+                                hi = max(fix(ehi * A.scale), lo + 1);
+                            }
+                            T = (T & ~U) | __ballot(valid);
+                            ok = __builtin_amdgcn_inverse_ballot_w64(T);
+                        }
+                    }
+                    v[m].lo = ok ? lo : INT_MAX;
+                    v[m].hi = ok ? hi : INT_MIN;
+                    any |= T;
+                }
+                return any;
+            }
+        };
+        // (FAST's bounds are clamped by the comparisons)
+        const int def_lo = FLT ? float_key(-A.max_k_f) : -kFixOne, def_hi = FLT ? float_key(A.max_k_f) : kFixOne;
+
+        // the run's bundles, a batch of records at a time
         lds_ptr<Bounds> bp = bun;  // the next slot
         for (int p = p0; p < p1;) {
-            if ((p >> 4) != batch) {
-                batch = p >> 4;
+            if ((p >> kLog) != batch) {
+                batch = p >> kLog;
                 fill_batch(batch);
             }
-            const int pe = min(p1, (p | 15) + 1);
-            lds_ptr<double2> q = rec + (p & 15) * 5;
+            const int pe = min(p1, (p | kLast) + 1);
+            lds_ptr<double2> q = rec + (p & kLast) * 5;
+            if (!EXACT && R + pe - p <= slots && ((closep[0] >> (p & 63)) & ((1ULL << (pe - p)) - 1ULL)) == 0ULL) {
+                // (most batches: no close pair, and slots for all)
+                for (; p < pe; ++p, q += 5) {
+                    Bounds v[CPL];
+                    if (bundle(p, q, v) == 0ULL) continue;  // bundle_valid_check, :821-830
+#pragma unroll
+                    for (int m = 0; m < CPL; ++m) {
+                        bp[m * 64].lo = v[m].lo;
+                        bp[m * 64].hi = v[m].hi;
+                    }
+                    bp += CPL * 64;
+                    place[0] |= 1ULL << (p & 63);
+                }
+                R = __popcll(place[0]);
+                continue;
+            }
             for (; p < pe; ++p, q += 5) {
                 bool close = false;
 #pragma unroll
@@ -633,114 +763,13 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                     // the default bundle [-max_k, max_k]
 #pragma unroll
                     for (int m = 0; m < CPL; ++m) {
-                        v[m].lo = FLT ? float_key(-A.max_k_f) : -kFixOne;
-                        v[m].hi = FLT ? float_key(A.max_k_f) : kFixOne;
+                        v[m].lo = def_lo;
+                        v[m].hi = def_hi;
                     }
-                } else if constexpr (FLT) {
-                    // compute_curve_bundle<float>; its branches differ (a
-                    // power of two on both sides of a quotient apart) in the
-                    // angles' order only
-                    const lds_ptr<float4> f = (lds_ptr<float4>)(q + 3);
-                    const float DX = f[0].x, DY = f[0].y;
-                    const double DX2 = q[2].x, DY2 = q[2].y;
-                    u64 any = 0ULL;
-#pragma unroll
-                    for (int m = 0; m < CPL; ++m) {
-                        const float o = static_cast<float>(W.ox[m]);
-                        const float tt = sf[m] * DX - cf[m] * DY;  // :705
-                        const float ttm = tt - o;
-                        // :711 (the first product is exact)
-                        const float den = static_cast<float>(
-                            __builtin_fma(W.m2ox[m], static_cast<double>(tt), DX2) + DY2 - A.dx2 + W.ox2[m]);
-                        const float kx0 = 2.0f * (ttm - A.dx_f) / den, kx1 = 2.0f * (ttm + A.dx_f) / den;
-                        float kt[2];
-#pragma unroll
-                        for (int k = 0; k < 2; ++k) {
-                            const double s0 = q[k].x, c0 = q[k].y;
-                            const float T0 = k == 0 ? f[0].z : f[0].w;
-                            const float cx = k == 0 ? f[1].x : f[1].z, sy = k == 0 ? f[1].y : f[1].w;
-                            const double e = static_cast<double>(T2[m] - T0) -
-                                             (static_cast<double>(T2[m]) - static_cast<double>(T0));
-                            const double s = __builtin_fma(sT[m], c0, -(cT[m] * s0));
-                            const double c = __builtin_fma(cT[m], c0, sT[m] * s0);
-                            const float sn = sure_float(__builtin_fma(e, __builtin_fma(-0.5 * e, s, c), s), bad);
-                            kt[k] = sn / (-sn * o + cx + sy);
-                        }
-                        // the reference's compare-and-assign, which ignores NaN
-                        const float lo = __builtin_fmaxf(__builtin_fmaxf(-A.max_k_f, kx0), kt[0]);
-                        const float hi = __builtin_fminf(__builtin_fminf(A.max_k_f, kx1), kt[1]);
-                        least = __builtin_fminf(least, __builtin_fminf(__builtin_fabsf(lo), __builtin_fabsf(hi)));
-                        const bool ok = hi > lo;
-                        v[m].lo = ok ? float_key(lo) : INT_MAX;
-                        v[m].hi = ok ? float_key(hi) : INT_MIN;
-                        any |= __builtin_amdgcn_ballot_w64(ok);
-                    }
-                    if (any == 0ULL) continue;  // bundle_valid_check, :821-830
-                } else {
-                    const double DX = q[0].x, DY = q[0].y, r2 = q[1].x, C0 = q[1].y, C1 = q[2].x;
-                    const double s0n = q[2].y, c0n = q[3].x, s1n = q[3].y, c1n = q[4].x;
-                    u64 any = 0ULL;  // cells with hi > lo
-#pragma unroll
-                    for (int m = 0; m < CPL; ++m) {
-                        const double tt = __builtin_fma(sT[m], DX, -(cT[m] * DY));
-                        const double den = __builtin_fma(W.m2ox[m], tt, r2 + W.ox2[m]);
-                        const double x0 = tt - W.oxp[m];  // half of :712's numerator
-                        const double s0 = __builtin_fma(sT[m], c0n, -(cT[m] * s0n));
-                        const double s1 = __builtin_fma(sT[m], c1n, -(cT[m] * s1n));
-                        const double d0 = __builtin_fma(-s0, W.ox[m], C0);
-                        const double d1 = __builtin_fma(-s1, W.ox[m], C1);
-                        // 1 / den, 1 / d0 and 1 / d1 (times scale) from one reciprocal
-                        const double pp = den * d0, ppp = pp * d1;
-                        double y = __builtin_amdgcn_rcp(ppp);
-                        y = __builtin_fma(y, __builtin_fma(-ppp, y, 1.0), y);
-                        y *= A.scale;
-                        const double yd1 = y * pp, w = y * d1;
-                        const double yd0 = w * den, yx = w * (d0 + d0);
-                        const double k0 = x0 * yx, k1 = __builtin_fma(A.two_dx, yx, k0);
-                        int lo = max(fix(k0), fix(s0 * yd0));
-                        int hi = min(fix(k1), fix(s1 * yd1));
-                        const int t = min(sub_sat(hi, lo), min(sub_sat(hi, -kFixOne), sub_sat(kFixOne, lo)));
-                        note(t);
-                        bool ok = t > kFixTol;
-                        u64 T = __builtin_amdgcn_ballot_w64(ok);
-                        u64 U = EXACT ? is_open(t) : 0ULL;
-                        // a small denominator (then the product is small as well)
-                        // settles nothing unless its sign is certain and its
-                        // quotients lie well beyond max_k, where they stay either way
-                        if (__builtin_amdgcn_ballot_w64(!(fabs(ppp) >= A.min_prod)) != 0ULL) {
-                            auto weak = [&](double n, double d) {
-                                return !(fabs(d) >= A.min_den) &&
-                                       !(fabs(d) > A.den_err && fabs(n) > 4.0 * A.max_k * fabs(d) + A.num_err);
-                            };
-                            const bool bad = weak(2.0 * x0, den) || weak(2.0 * x0 + 2.0 * A.two_dx, den) ||
-                                             weak(s0, d0) || weak(s1, d1);
-                            if (EXACT)
-                                U |= __builtin_amdgcn_ballot_w64(bad);
-                            else
-                                closest = bad ? 0u : closest;
-                        }
-                        if constexpr (EXACT) {
-                            if (U != 0ULL) {
-                                const int b = neighbour(p);
-                                bool valid = false;
-                                if (__builtin_amdgcn_inverse_ballot_w64(U)) {
-                                    double elo = 0.0, ehi = 0.0;
-                                    exact_cell(m, b, elo, ehi);
-                                    valid = ehi > elo;
-                                    lo = fix(elo * A.scale);
-                                    hi = max(fix(ehi * A.scale), lo + 1);
-                                }
-                                T = (T & ~U) | __ballot(valid);
-                                ok = __builtin_amdgcn_inverse_ballot_w64(T);
-                            }
-                        }
-                        v[m].lo = ok ? lo : INT_MAX;
-                        v[m].hi = ok ? hi : INT_MIN;
-                        any |= T;
-                    }
-                    if (any == 0ULL) continue;  // bundle_valid_check, :821-830
+                } else if (bundle(p, q, v) == 0ULL) {
+                    continue;
                 }
-                ++vp;
+                if (EXACT) ++vp;
                 if (EXACT && run == 2) continue;
                 if (R < slots) {
 #pragma unroll
@@ -762,6 +791,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 ++R;
             }
         }
+        if (!EXACT) vp += static_cast<unsigned>(R);
         // a chain longer than 2 takes two hypotheses and G >= 3
         if ((EXACT && run == 2) || R < 2 || G < 3) continue;
 
@@ -875,20 +905,17 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             u64 P[CPL];
             u64 redo = 0ULL;  // EXACT: bit 8 i + k: the pair has an open cell
 #pragma unroll
-            for (int i = 0; i < kSmallRun; ++i)
+            for (int m = 0; m < CPL; ++m) P[m] = 0ULL;
+            auto meet = [&](auto slot) -> bool {
+                constexpr int i = decltype(slot)::value;
+                if (i >= R) return false;
+                asm volatile("");  // (a branch: runs of 2 to 4 slots would do the work of 8)
 #pragma unroll
-                for (int m = 0; m < CPL; ++m) {  // (slots >= kSmallRun)
+                for (int m = 0; m < CPL; ++m) {
                     b[i][m].lo = bun[(i * CPL + m) * 64].lo;
                     b[i][m].hi = bun[(i * CPL + m) * 64].hi;
-                }
-#pragma unroll
-            for (int m = 0; m < CPL; ++m) P[m] = 0ULL;
-#pragma unroll
-            for (int i = 0; i < kSmallRun; ++i) {
-                if (i >= R) break;
-#pragma unroll
-                for (int m = 0; m < CPL; ++m)
                     P[m] = set_lane64(P[m], __builtin_amdgcn_ballot_w64(b[i][m].hi > b[i][m].lo), 9 * i);
+                }
 #pragma unroll
                 for (int k = 0; k < i; ++k) {
 #pragma unroll
@@ -901,7 +928,9 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                         P[m] = set_lane64(P[m], __builtin_amdgcn_ballot_w64(t > kTol), 8 * i + k);
                     }
                 }
-            }
+                return true;
+            };
+            each(meet, std::make_integer_sequence<int, kSmallRun>{});
             if constexpr (EXACT) {
                 for (; redo != 0ULL; redo &= redo - 1ULL) {
                     const int ik = __builtin_ctzll(redo), i = ik >> 3, k = ik & 7;
@@ -936,8 +965,9 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             const u64 ones = 0x0101010101010101ULL;
             u64 count = 0ULL, stop = 0ULL;  // per seed, one byte each
             u64 chain = 0ULL;               // byte j: seed j's chain, as slots
-            auto step = [&](auto slot) -> bool {
+            auto grow = [&](auto slot, auto full) -> bool {
                 constexpr int h = decltype(slot)::value;
+                constexpr bool limited = decltype(full)::value;
                 if (h >= R) return false;
                 u64 nz = 0ULL;
 #pragma unroll
@@ -965,7 +995,13 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 }
                 return true;
             };
-            each(step, std::make_integer_sequence<int, kSmallRun>{});
+            if (limited) {
+                auto step = [&](auto slot) -> bool { return grow(slot, std::true_type{}); };
+                each(step, std::make_integer_sequence<int, kSmallRun>{});
+            } else {
+                auto step = [&](auto slot) -> bool { return grow(slot, std::false_type{}); };
+                each(step, std::make_integer_sequence<int, kSmallRun>{});
+            }
             // rows, lane 9 j = seed j: kept with more than 2 edges (:549) and
             // no earlier seed with the same chain (lane 8 j + k compares j's
             // with k's)
@@ -1139,7 +1175,7 @@ __device__ __forceinline__ void put_sums(unsigned *partial, int g, unsigned vp, 
     }
 }
 
-template <int CPL, bool FLT = false>
+template <int CPL>
 __device__ __forceinline__ WaveCells<CPL> wave_cells(const FusedArgs &A)
 {
     WaveCells<CPL> W;
@@ -1150,8 +1186,8 @@ __device__ __forceinline__ WaveCells<CPL> wave_cells(const FusedArgs &A)
         const int r = live ? rho : 0;
         W.ox[m] = A.rank_ox[r];
         W.m2ox[m] = -2.0 * W.ox[m];
-        W.ox2[m] = FLT ? static_cast<double>(static_cast<float>(W.ox[m]) * static_cast<float>(W.ox[m])) : W.ox[m] * W.ox[m];
-        W.oxp[m] = W.ox[m] + A.dx;
+        W.ox2[m] = static_cast<double>(static_cast<float>(W.ox[m]) * static_cast<float>(W.ox[m]));
+        W.oxp2[m] = 2.0 * (W.ox[m] + A.dx);
         W.ot[m] = A.rank_ot[r];
         W.so[m] = A.rank_so[r];
         W.co[m] = A.rank_co[r];
@@ -1175,16 +1211,15 @@ __device__ __forceinline__ void load_entry(const int4 *p, int &a, unsigned &base
 // Persistent: one wave per anchor (do_anchor), wave g takes entries g,
 // g + waves, ... of the concatenated lists.  The neighbours' records of the
 // next anchor, the ids of the one after it and the list entry of the third are
-// in flight while an anchor is worked on.  Bound by instruction issue: the
-// SIMDs issue about one instruction of any kind per four cycles from start to
-// end (counters; 820 vector, 490 scalar and 90 LDS instructions an anchor), and
-// waves that take entries from a shared counter instead of a fixed share end
-// together but no sooner (741 us against 724 at the time).  Anchors with a comparison too close
+// in flight while an anchor is worked on.  Bound by instruction issue and
+// latency together: on the 1080p map one to four waves per SIMD take 1,145,
+// 723, 574 and 516 us, five 473 (770 vector, 440 scalar and 90 LDS instructions
+// an anchor).  Anchors with a comparison too close
 // for the approximate bounds go to the open list.  (Done again here, their
 // code costs the main loop its registers: 1,272 us against 720 on the 1080p
 // map.)
 template <int CPL, bool FLT>
-__global__ __launch_bounds__(64 * kFusedWaves, CPL == 1 && !FLT ? kFusedWavesPerSimd + 1 : kFusedWavesPerSimd)
+__global__ __launch_bounds__(64 * kFusedWaves, CPL == 1 && !FLT ? kFusedWavesPerSimd : 4)
 void k_curvelets(FusedArgs A)
 {
     extern __shared__ double lds[];
@@ -1196,7 +1231,7 @@ void k_curvelets(FusedArgs A)
     unsigned long long isect = 0;  // bundle intersections the reference tests (per lane)
     char *sl = reinterpret_cast<char *>(lds) + static_cast<size_t>(wave) * slice_carve(A.slots, CPL).bytes;
     int2 *spill = A.spill + static_cast<size_t>(g) * A.spill_stride;
-    const WaveCells<CPL> W = wave_cells<CPL, FLT>(A);
+    const WaveCells<CPL> W = wave_cells<CPL>(A);
 
     // the wave's entries: a cursor into the current list
     int list = L_FIRST - 1, left = 0, at = g;

@@ -3344,7 +3344,7 @@ int record_rows(cvg_context *ctx, const cvg_params &p, RecordArgs R, int st_stri
 
 // The launch of k_curvelets: as many waves as stay resident, each looping over
 // its share of the lists.  The slots keep kFusedWavesPerSimd waves per SIMD
-// resident; a run's bundles beyond them (under 1% of the runs) go to device
+// resident (720p map: 263 us at five, 288 at four, 339 at three); a run's bundles beyond them (under 1% of the runs) go to device
 // memory, `spill` words per wave.
 struct FusedShape {
     FusedKernel fn;
@@ -3656,7 +3656,7 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     A.rank_co = reinterpret_cast<const double *>(tb + o_rank_co);
     A.rank_elig = reinterpret_cast<const int *>(tb + o_rank_elig);
     A.rank_of_cell0 = d.rank_of_cell0;
-    A.two_dx = 2.0 * d.dx;
+    A.four_dx = 4.0 * d.dx;
     A.max_k = d.max_k;
     A.sin_dt = std::sin(d.dt);
     A.cos_dt = std::cos(d.dt);
@@ -3676,7 +3676,11 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     A.acc_count = as<unsigned>(ctx->d_acc);
 
     // k_curvelets, then the anchors it leaves open; anchors of more than 64
-    // neighbours, where the map has any, beside it on an auxiliary stream
+    // neighbours, where the map has any, beside it on an auxiliary stream.
+    // Those are launched second: k_curvelets' waves then all start at once
+    // (a late one ends late, each has its share), and theirs take the place of
+    // the first that end.  (Launched first they cost the 3840x2160 map's
+    // k_curvelets 1,806 us against 1,566.)
     FusedShape f{};
     CVG_TRY(fused_shape<false>(ctx, A.K, &f));
     const ExactKernel fn_open = exact_kernel<1>(d.cpl), fn_wide = exact_kernel<4>(d.cpl);
@@ -3707,9 +3711,13 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     CVG_TRY(record_timing(ctx, ctx->ev[3], st));
     CVG_TRY(record_timing(ctx, ctx->fused_ev[ring][0], st));
     X.spill_stride = spill_exact;
+    const hipEvent_t fork = ctx->timed_run ? ctx->ev[3] : ctx->ev_fork;
+    if (wide && !ctx->timed_run) CVG_HIP(ctx, hipEventRecord(fork, st));
+    A.spill = as<int2>(ctx->d_gbundle) + spill_exact * blocks_wide;
+    A.spill_stride = f.spill;
+    A.partial = as<unsigned>(ctx->d_partial) + 3 * blocks_wide;
+    hipLaunchKernelGGL(f.fn, dim3(static_cast<unsigned>(f.waves / kFusedWaves)), dim3(64 * kFusedWaves), f.shmem, st, A);
     if (wide) {
-        const hipEvent_t fork = ctx->timed_run ? ctx->ev[3] : ctx->ev_fork;
-        if (!ctx->timed_run) CVG_HIP(ctx, hipEventRecord(fork, st));
         CVG_HIP(ctx, hipStreamWaitEvent(ctx->aux, fork, 0));
         X.spill = as<int2>(ctx->d_gbundle);
         X.partial = as<unsigned>(ctx->d_partial);
@@ -3717,10 +3725,6 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
                            static_cast<int>(L_WIDE));
         CVG_HIP(ctx, hipEventRecord(ctx->ev_join, ctx->aux));
     }
-    A.spill = as<int2>(ctx->d_gbundle) + spill_exact * blocks_wide;
-    A.spill_stride = f.spill;
-    A.partial = as<unsigned>(ctx->d_partial) + 3 * blocks_wide;
-    hipLaunchKernelGGL(f.fn, dim3(static_cast<unsigned>(f.waves / kFusedWaves)), dim3(64 * kFusedWaves), f.shmem, st, A);
     X.spill = A.spill;
     X.partial = A.partial + 3 * waves_main;
     hipLaunchKernelGGL(fn_open, dim3(static_cast<unsigned>(blocks_open)), dim3(64), slice, st, X,

@@ -299,13 +299,6 @@ using lds_ptr = __attribute__((address_space(3))) T *;
 template <typename T>
 using mem_ptr = __attribute__((address_space(1))) T *;
 
-// f(0), f(1), ... as constants, until one returns false.
-template <class F, int... I>
-__device__ __forceinline__ void each(F &f, std::integer_sequence<int, I...>)
-{
-    (void)(f(std::integral_constant<int, I>{}) && ...);
-}
-
 struct alignas(8) Bounds {
     int lo, hi;
 };

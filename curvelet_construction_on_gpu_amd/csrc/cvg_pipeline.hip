@@ -1213,6 +1213,26 @@ __device__ inline double bcast(double v, int lane)
 
 __device__ inline int bcast(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 
+// f(0), f(1), ... as constants, until one returns false.
+template <class F, int... I>
+__device__ __forceinline__ void each(F &f, std::integer_sequence<int, I...>)
+{
+    (void)(f(std::integral_constant<int, I>{}) && ...);
+}
+
+// v of lane J of the lane's row of 16, and of the lane N before it in the row
+// (0 before the first): a register move each, where a shuffle is an LDS trip.
+template <int J>
+__device__ __forceinline__ int row_lane(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, 0x150 + J, 0xf, 0xf, true);
+}
+template <int N>
+__device__ __forceinline__ int row_before(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, 0x110 + N, 0xf, 0xf, true);
+}
+
 // The neighbour-window scans give each anchor a segment of G lanes (64 / G
 // anchors per wave).  The window is rows py = cy-R..cy+R; in each row the cells
 // cx-R..cx+R are one contiguous range of the cell-sorted arrays
@@ -1229,13 +1249,21 @@ __device__ inline void window_rows(const Cells &cells, int cx, int cy, int R, in
     rs = 0;
     if (valid && r <= 2 * R) cells.row(cx, cy - R + r, R, rs, len);
     int inc = len;
+    if constexpr (G == 16) {
+        inc += row_before<1>(inc);
+        inc += row_before<2>(inc);
+        inc += row_before<4>(inc);
+        inc += row_before<8>(inc);
+        tot = row_lane<15>(inc);
+    } else {
 #pragma unroll
-    for (int o = 1; o < G; o <<= 1) {
-        const int v = __shfl_up(inc, o, G);
-        if (sl >= o) inc += v;
+        for (int o = 1; o < G; o <<= 1) {
+            const int v = __shfl_up(inc, o, G);
+            if (sl >= o) inc += v;
+        }
+        tot = __shfl(inc, G - 1, G);
     }
     pre = inc - len;
-    tot = __shfl(inc, G - 1, G);
 }
 
 // Sorted position of the t-th candidate (0 <= t < tot) of rows rb..rb+nrows-1,
@@ -1244,11 +1272,23 @@ template <int G>
 __device__ inline int window_pos(int rs, int pre, int tot, int nrows, int t)
 {
     int k = -1;
+    if constexpr (G == 16) {
+        const int shift = rs - pre;
+        auto row = [&](auto slot) -> bool {
+            constexpr int j = decltype(slot)::value;
+            if (j >= nrows) return false;
+            const int pj = row_lane<j>(pre), sj = row_lane<j>(shift);  // (both by every lane)
+            k = t >= pj ? t + sj : k;
+            return true;
+        };
+        each(row, std::make_integer_sequence<int, G>{});
+    } else {
 #pragma unroll 8
-    for (int j = 0; j < nrows; ++j) {
-        const int pj = __shfl(pre, j, G);
-        const int sj = __shfl(rs, j, G);
-        if (t >= pj) k = sj + (t - pj);
+        for (int j = 0; j < nrows; ++j) {
+            const int pj = __shfl(pre, j, G);
+            const int sj = __shfl(rs, j, G);
+            if (t >= pj) k = sj + (t - pj);
+        }
     }
     return t < tot ? k : -1;
 }
@@ -1422,6 +1462,23 @@ __device__ inline int list_rank(const double *ld, const int *lcell, int dg, int 
     return rank;
 }
 
+// The ranks of lists without exact ties: entry i (distance di) comes after the
+// entries below it.  Four vector instructions an entry, against some 15 of
+// all kinds in list_rank; the entries from dg to dmax must hold infinity.  `upto` counts
+// the entries up to di: rank + 1 unless some other entry ties.
+__device__ __forceinline__ int plain_rank(const double *ld, int dmax, double di, int &upto)
+{
+    int rank = 0;
+    upto = 0;
+#pragma unroll 4
+    for (int j = 0; j < dmax; ++j) {
+        const double dj = ld[j];
+        rank += dj < di ? 1 : 0;
+        upto += dj <= di ? 1 : 0;
+    }
+    return rank;
+}
+
 // LDS doubles per k_fill_csr segment of list capacity cap: d2 (8 B), id and
 // cell (4 B each), and with the counting variant the sorted order (4 B).
 __host__ __device__ inline int fill_seg_doubles(int cap, bool count)
@@ -1438,6 +1495,9 @@ __host__ __device__ inline int fill_seg_doubles(int cap, bool count)
 // position, which is the insertion-sort order std::sort yields up to 16
 // entries); lists with ties and more than 16 entries get their scan-order
 // copy in `cand` and are queued for the std::sort replay (k_tie_sort).
+// Bound by instruction issue, and with COUNT by the look-back.  (10 maps of
+// 519,391 edges: 164 us when every entry pair was also compared for ties and
+// cells and the window's rows went through LDS shuffles, 99 us now.)
 // COUNT: no counting pass ran.  Each segment counts its in-radius candidates
 // over the whole window (the degree is the count capped at max_candidates,
 // preprocess.hpp:165), the workgroup finds its anchors' offsets with the
@@ -1520,7 +1580,6 @@ __global__ __launch_bounds__(64 * kFillWaves) void k_fill_csr(int n, const doubl
     const int lim = COUNT ? static_cast<int>(min(max_cand, static_cast<unsigned>(INT_MAX))) : dg;
     const int keep = COUNT ? min(lim, cap) : dg;  // candidates stored in LDS
     int kept = 0;
-    int last_cell = -1;  // cell of the last kept candidate
     bool ambiguous = false;
     bool done = !valid;
     for (int rb = 0; rb <= 2 * R && __ballot(!done) != 0ULL; rb += G) {
@@ -1549,18 +1608,17 @@ __global__ __launch_bounds__(64 * kFillWaves) void k_fill_csr(int n, const doubl
             }
             // a max_candidates cut inside one cell makes the kept set depend on
             // the within-cell order: compare the first dropped candidate's cell
-            // with the last kept one's
-            const unsigned long long bm = __ballot(pass && pos == lim) & segmask;
-            const unsigned long long pm = __ballot(pass && pos == lim - 1) & segmask;
-            const int bcell = __shfl(cell, bm != 0ULL ? __ffsll(static_cast<long long>(bm)) - 1 : lane);
-            const int pcell = __shfl(cell, pm != 0ULL ? __ffsll(static_cast<long long>(pm)) - 1 : lane);
-            const int hcell = __shfl(cell, m != 0ULL ? 63 - __clzll(static_cast<long long>(m)) : lane);
-            if (bm != 0ULL) {
-                const int prev = pm != 0ULL ? pcell : last_cell;
-                if (lim > 0 && prev == bcell) ambiguous = true;
-                done = true;
-            } else if (m != 0ULL) {
-                if (kept + __popcll(m) <= lim) last_cell = hcell;
+            // with the last kept one's (not in LDS only if the list outgrew it,
+            // and then the build is repeated)
+            const unsigned long long cut = __ballot(pass && pos == lim);
+            if (cut != 0ULL) {
+                wave_sync();
+                const unsigned long long bm = cut & segmask;
+                const int bcell = __shfl(cell, bm != 0ULL ? __ffsll(static_cast<long long>(bm)) - 1 : lane);
+                if (bm != 0ULL) {
+                    if (lim > 0 && lim <= keep && lcell[lim - 1] == bcell) ambiguous = true;
+                    done = true;
+                }
             }
             kept += __popcll(m);
             // without a cut (dg < max_candidates) nothing passes after the dg-th
@@ -1602,17 +1660,29 @@ __global__ __launch_bounds__(64 * kFillWaves) void k_fill_csr(int n, const doubl
         wave_sync();
         bool tie = false, shared = false;
         const int dmax = wave_max_over_segments<G>(dr);
+        for (int j = dr + sl; j < dmax; j += G) ld[j] = INFINITY;
+        wave_sync();
         for (int i0 = 0; i0 < dmax; i0 += G) {
             const int i = i0 + sl;
-            const bool active = i < dr;
-            double di = 0.0;
-            int celli = -1;
-            if (active) {
-                di = ld[i];
-                celli = lcell[i];
+            int upto;
+            const int rank = plain_rank(ld, dmax, i < dr ? ld[i] : 0.0, upto);
+            tie = tie || (i < dr && upto != rank + 1);
+            if (i < dr) lord[rank] = i;
+        }
+        if (__ballot(tie) != 0ULL) {
+            tie = false;
+            for (int i0 = 0; i0 < dmax; i0 += G) {
+                const int i = i0 + sl;
+                const bool active = i < dr;
+                double di = 0.0;
+                int celli = -1;
+                if (active) {
+                    di = ld[i];
+                    celli = lcell[i];
+                }
+                const int rank = list_rank(ld, lcell, dr, dmax, i, active, di, celli, tie, shared, ambiguous);
+                if (active) lord[rank] = i;
             }
-            const int rank = list_rank(ld, lcell, dr, dmax, i, active, di, celli, tie, shared, ambiguous);
-            if (active) lord[rank] = i;
         }
         __syncthreads();
         if (threadIdx.x < 64) {
@@ -1665,7 +1735,23 @@ __global__ __launch_bounds__(64 * kFillWaves) void k_fill_csr(int n, const doubl
     bool tie = false;
     bool shared = false;
     const int dmax = wave_max_over_segments<G>(dg);
+    for (int j = dg + sl; j < dmax; j += G) ld[j] = INFINITY;
+    wave_sync();
     for (int i0 = 0; i0 < dmax; i0 += G) {
+        const int i = i0 + sl;
+        const double di = i < dg ? ld[i] : 0.0;
+        int upto;
+        const int rank = plain_rank(ld, dmax, di, upto);
+        tie = tie || (i < dg && upto != rank + 1);
+        if (i < dg) {
+            ids[o + rank] = lid[i];
+            d2[o + rank] = di;
+        }
+    }
+    const bool again = __ballot(tie) != 0ULL;
+    if (again) __threadfence();  // the places are written again
+    tie = false;
+    for (int i0 = 0; again && i0 < dmax; i0 += G) {
         const int i = i0 + sl;
         const bool active = i < dg;
         double di = 0.0;
@@ -2604,6 +2690,10 @@ constexpr int kSpecMiss = 1000;  // internal: a guessed size did not hold (never
 
 int queue_setup(cvg_context *ctx);
 
+// Maps of up to this many edges count in the fill: at 24,809 edges that saves
+// 10 us of 300, at 107,415 it costs 9 of 505, at 851,141 it costs 120 of 2,340.
+constexpr int kCountInFillMax = 65536;
+
 // Neighbour counts, CSR offsets, then the gathering pass, the distance sort
 // and the CSR fill (preprocess.hpp:186-274) over either cell layout.  The
 // pair count and largest degree size the fill; with spec they are not read
@@ -2619,9 +2709,11 @@ int graph_scans(cvg_context *ctx, const Cells &cells, int n, unsigned R, unsigne
     const size_t ni = static_cast<size_t>(n) * sizeof(int);
     CVG_TRY(ensure(ctx, ctx->d_off, static_cast<size_t>(n + 1) * sizeof(unsigned)));
     // on guessed buffers the fill counts the lists itself and finds the
-    // offsets in the same pass; otherwise a counting pass and the offsets
-    // scan size the buffers first
-    const bool count_in_fill = spec;
+    // offsets in the same pass (its workgroups' look-back makes a chain of n / 16
+    // links, which a large map waits for); otherwise a counting pass and the
+    // offsets scan come first
+    const bool count_in_fill = spec && (n <= kCountInFillMax ||
+                                        static_cast<unsigned long long>(n) * max_cand > static_cast<unsigned>(INT_MAX));
     if (!count_in_fill) {
         CVG_TRY(ensure(ctx, ctx->d_deg, ni));
         using CountFn = void (*)(int, const double *, const double *, const int *, const int *, Cells, int, double,

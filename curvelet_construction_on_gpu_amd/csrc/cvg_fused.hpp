@@ -17,7 +17,8 @@
 //
 // Measured on the 1080p map (207,326 edges, 2.04M pairs, G = 7): 1,000 us for
 // the kernel on exact bounds and 141 us for its sines pass (345 MB) before; now
-// 473 us, and 81 us for the few anchors left open.
+// 473 us, and 65 us for the few anchors left open (81 us before they shared a
+// bound's sides and members out over the lanes).
 #ifndef CVG_FUSED_HPP
 #define CVG_FUSED_HPP
 
@@ -65,22 +66,15 @@ __device__ inline double exact_bound(const ExactGrid &E, bool upper, double ax, 
     return v;
 }
 
-// Both bounds at the cell (ox, ot) of anchor a.  Out of line: the exact
-// kernel's few anchors spend their time on instruction fetch, and its callers
-// share this copy.
-__device__ __noinline__ double2 exact_bounds(ExactGrid E, double ax, double ay, double sa, double ca, double T2t,
-                                             double ox, int b)
+// A lane's bound (lo, or hi with `upper`) at the cell (ox, ot) of anchor a.
+// Out of line: the exact kernel's few anchors spend much of their time on
+// instruction fetch, and its callers share this copy.
+__device__ __noinline__ double exact_value(ExactGrid E, bool upper, double ax, double ay, double sa, double ca,
+                                           double T2t, double ox, int b)
 {
     double s2, c2;
     cvg::cr_sincos<false>(T2t, c_sincos_tab, &s2, &c2);
-    double2 r = make_double2(0.0, 0.0);
-#pragma unroll 1
-    for (int side = 0; side < 2; ++side) {
-        const double v = exact_bound(E, side != 0, ax, ay, sa, ca, T2t, s2, c2, ox, b);
-        r.x = side == 0 ? v : r.x;
-        r.y = side == 0 ? r.y : v;
-    }
-    return r;
+    return exact_bound(E, upper, ax, ay, sa, ca, T2t, s2, c2, ox, b);
 }
 
 // Per edge: (x, y, sin theta, cos theta), the correctly rounded pair.  Block 0
@@ -437,12 +431,39 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
 
     [[maybe_unused]] const float fsa = sure_float(sa, bad), fca = sure_float(ca, bad);
 
-    // EXACT: the exact bounds of neighbour b at this lane's cell of group m
-    auto exact_cell = [&](int m, int b, double &lo, double &hi) {
-        const int rho = lane + 64 * m < A.K ? lane + 64 * m : 0;
-        const double2 v = exact_bounds(A.exact, ax, ay, sa, ca, A.th[a] + A.rank_ot[rho], A.rank_ox[rho], b);
-        lo = v.x;
-        hi = v.y;
+    // EXACT: for the lanes U, the largest lo and smallest hi at their cell of
+    // group m over `members` neighbours (edge b, or those listed in LDS where
+    // the pair records are): a (cell, member, side) per lane, as a bound is a
+    // long chain of double operations and few cells are open at a time
+    const lds_ptr<int> listed = (lds_ptr<int>)(sl + cv.rec);
+    const lds_ptr<double> value = (lds_ptr<double>)(sl + cv.bytes - 512);
+    auto exact_set = [&](int m, u64 U, int members, int b, double &lo, double &hi) {
+        lo = -INFINITY;
+        hi = INFINITY;
+        const int mine = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                             static_cast<unsigned>(U >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(U), 0u))) *
+                         members;
+        const int items = 2 * __popcll(U) * members;
+#pragma unroll 1
+        for (int t0 = 0; t0 < items; t0 += 64) {
+            const int q = (t0 + lane) >> 1, at = q / members;
+            int rho = 0, k = 0;
+#pragma unroll 1
+            for (u64 u = U; u != 0ULL; u &= u - 1ULL, ++k) rho = at == k ? __builtin_ctzll(u) + 64 * m : rho;
+            rho = rho < A.K ? rho : 0;
+            double v = 0.0;
+            if (t0 + lane < items)
+                v = exact_value(A.exact, (lane & 1) != 0, ax, ay, sa, ca, A.th[a] + A.rank_ot[rho], A.rank_ox[rho],
+                                b >= 0 ? b : listed[q - at * members]);
+            wave_sync();  // the last values are read
+            value[lane] = v;
+            wave_sync();
+            if (__builtin_amdgcn_inverse_ballot_w64(U))
+                for (int i = max(mine, t0 >> 1); i < min(mine + members, (t0 >> 1) + 32); ++i) {
+                    lo = fmax(lo, value[2 * i - t0]);
+                    hi = fmin(hi, value[2 * i - t0 + 1]);
+                }
+        }
     };
 
     // direction classes (:459-461), lane = neighbour; a neighbour's place in
@@ -698,16 +719,13 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                     }
                     if constexpr (EXACT) {
                         if (U != 0ULL) {
-                            const int b = neighbour(p);
-                            bool valid = false;
+                            double elo, ehi;
+                            exact_set(m, U, 1, neighbour(p), elo, ehi);
                             if (__builtin_amdgcn_inverse_ballot_w64(U)) {
-                                double elo = 0.0, ehi = 0.0;
-                                exact_cell(m, b, elo, ehi);
-                                valid = ehi > elo;
                                 lo = fix(elo * A.scale);
                                 hi = max(fix(ehi * A.scale), lo + 1);
                             }
-                            T = (T & ~U) | __ballot(valid);
+                            T = (T & ~U) | (__builtin_amdgcn_ballot_w64(ehi > elo) & U);
                             ok = __builtin_amdgcn_inverse_ballot_w64(T);
                         }
                     }
@@ -800,31 +818,33 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
         // EXACT: whether the running bundle of the slots in `set` is valid, in
         // the lanes U of cell group m
         auto exact_run = [&](int m, u64 U, const u64 (&set)[NW]) -> u64 {
-            double lo = 0.0, hi = 0.0;
-            bool begun = false;
-            int s = 0;
-#pragma unroll 1
-            for (int p = p0; p < p1; ++p) {
-                u64 word = place[0], in = set[0];
+            int members = 0;
 #pragma unroll
-                for (int w = 1; w < NW; ++w) {
-                    word = (p >> 6) == w ? place[w] : word;
+            for (int w = 0; w < NW; ++w) members += __popcll(set[w]);
+            wave_sync();
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                if (!__builtin_amdgcn_inverse_ballot_w64(hyp[c])) continue;
+                int s = 0, rank = 0;  // the neighbour's slot, and its place among the members
+                u64 in = 0ULL;
+#pragma unroll
+                for (int w = 0; w < NW; ++w) {
+                    const int at = pos[c] - 64 * w;
+                    s += __popcll(at >= 64 ? place[w] : (at > 0 ? place[w] & ((1ULL << at) - 1ULL) : 0ULL));
+                }
+#pragma unroll
+                for (int w = 0; w < NW; ++w) {
+                    const int at = s - 64 * w;
+                    rank += __popcll(at >= 64 ? set[w] : (at > 0 ? set[w] & ((1ULL << at) - 1ULL) : 0ULL));
                     in = (s >> 6) == w ? set[w] : in;
                 }
-                if (!((word >> (p & 63)) & 1ULL)) continue;
-                const bool member = (in >> (s & 63)) & 1ULL;
-                ++s;
-                if (!member) continue;
-                const int b = neighbour(p);
-                if (__builtin_amdgcn_inverse_ballot_w64(U)) {
-                    double elo = 0.0, ehi = 0.0;
-                    exact_cell(m, b, elo, ehi);
-                    lo = !begun || lo < elo ? elo : lo;
-                    hi = !begun || hi > ehi ? ehi : hi;
-                }
-                begun = true;
+                if ((in >> (s & 63)) & 1ULL) listed[rank] = A.ids[base + 64 * c + lane];
             }
-            return __ballot(hi > lo) & U;
+            batch = -1;  // (the pair records are gone)
+            wave_sync();
+            double lo, hi;
+            exact_set(m, U, members, -1, lo, hi);
+            return __builtin_amdgcn_ballot_w64(hi > lo) & U;
         };
         auto put_row = [&](unsigned rank, const u64 (&chain)[NW], int best, int seed) {
             const size_t q = static_cast<size_t>(base) + rank;

@@ -304,8 +304,25 @@ struct alignas(8) Bounds {
 // and certain unless within kSineErr of where the float changes.  Bounds are
 // compared as integers of the same order.  720p float map (92,070 edges): 4,860
 // us on the general kernel, whose two correctly rounded sines a cell are some
-// 600 instructions; 327 us so, and 347 us for the anchors left to the general one.
-enum { M_FAST = 0, M_EXACT = 1, M_FLOAT = 2 };
+// 600 instructions; 322 us so, and 56 us for the anchors left open (346 us when
+// those went to the general kernel).
+// M_FLOAT leaves an anchor with an uncertain sine or direction open;
+// M_FLOAT_EXACT takes the correctly rounded ones there.
+enum { M_FAST = 0, M_EXACT = 1, M_FLOAT = 2, M_FLOAT_EXACT = 3 };
+
+__device__ inline int direction_class_f(float ax, float ay, float at, float nx, float ny, float cos_at, float sin_at);
+
+// (out of line, as exact_value)
+__device__ __noinline__ float exact_sine(float x, bool cosine)
+{
+    float s, c;
+    cvg::cr_sincosf(x, c_sincos_tab, &s, &c);
+    return cosine ? c : s;
+}
+__device__ __noinline__ int exact_direction(float ax, float ay, float at, float nx, float ny, float ca, float sa)
+{
+    return direction_class_f(ax, ay, at, nx, ny, ca, sa);
+}
 
 // Beyond what the rotations are off by: sums of an orientation (up to 64) and
 // an offset 2^-47, their sines and cosines 2^-51 each, the products 2^-50.
@@ -330,7 +347,8 @@ __device__ __forceinline__ float key_float(int k) { return __int_as_float(k ^ ((
 
 // One anchor on one wave.  M_FAST and M_FLOAT return true, with nothing
 // counted, when something is closer than they can decide; M_EXACT makes such
-// comparisons on the exact bounds.
+// comparisons on the exact bounds, and M_FLOAT_EXACT returns true only for a
+// bound of zero, whose sign the integers lose.
 //
 // Lane = neighbour forms the pairs' direction class, flags and
 // cell-independent terms (16 records in LDS at a time, in run order).  Then,
@@ -365,7 +383,8 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                                           unsigned &vp_sum, unsigned long long &isect_sum)
 {
     typedef unsigned long long u64;
-    constexpr bool EXACT = MODE == M_EXACT, FLT = MODE == M_FLOAT;
+    constexpr bool EXACT = MODE == M_EXACT, FLT = MODE >= M_FLOAT, SINES = MODE == M_FLOAT_EXACT;
+    constexpr bool CLASSES = EXACT || SINES;  // exact directions, with the third class
     static_assert(!FLT || NW == 1, "float maps: up to 64 neighbours");
     constexpr int kTol = FLT ? 0 : kFixTol;
     constexpr int kLog = batch_log(CPL), kLast = (1 << kLog) - 1;
@@ -402,7 +421,21 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
         if (MODE == M_FAST) closest = min(closest, static_cast<unsigned>(t + kFixTol));
     };
     unsigned bad = 0u;        // M_FLOAT: nonzero where a float sine is uncertain
-    float least = A.max_k_f;  // M_FLOAT: the smallest magnitude of a bound (a zero's sign would be lost)
+    // the float of v, an approximation of x's sine or cosine, in the lanes `in`
+    auto sure = [&](double v, float x, bool cosine, bool in) -> float {
+        unsigned u = 0u;
+        float f = sure_float(v, u);
+        u = in ? u : 0u;
+        if constexpr (SINES) {
+            if (__builtin_amdgcn_ballot_w64(u != 0u) != 0ULL) {
+                if (u != 0u) f = exact_sine(x, cosine);
+            }
+        } else {
+            bad |= u;
+        }
+        return f;
+    };
+    float least = A.max_k_f;  // float maps: the smallest magnitude of a bound (a zero's sign would be lost)
     auto is_open = [&](int t) -> u64 {
         return __builtin_amdgcn_ballot_w64(static_cast<unsigned>(t + kFixTol) <= 2u * kFixTol);
     };
@@ -412,7 +445,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
     const double ax = uload(ar), ay = uload(ar + 1), sa = uload(ar + 2), ca = uload(ar + 3);
     // sin/cos of theta_a + delta_t2 by rotation
     double sT[CPL], cT[CPL];
-    float T2[CPL], sf[CPL], cf[CPL];  // M_FLOAT: the angle, its sine and cosine
+    float T2[CPL], sf[CPL], cf[CPL];  // float maps: the angle, its sine and cosine
 #pragma unroll
     for (int m = 0; m < CPL; ++m) {
         sT[m] = __builtin_fma(sa, W.co[m], ca * W.so[m]);
@@ -424,12 +457,17 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             const double s = sT[m], c = cT[m];
             sT[m] = __builtin_fma(e, __builtin_fma(-0.5 * e, s, c), s);
             cT[m] = __builtin_fma(-e, __builtin_fma(0.5 * e, c, s), c);
-            sf[m] = sure_float(sT[m], bad);
-            cf[m] = sure_float(cT[m], bad);
+            sf[m] = sure(sT[m], T2[m], false, true);
+            cf[m] = sure(cT[m], T2[m], true, true);
         }
     }
 
-    [[maybe_unused]] const float fsa = sure_float(sa, bad), fca = sure_float(ca, bad);
+    [[maybe_unused]] float fth = 0.0f, fsa = 0.0f, fca = 0.0f;
+    if constexpr (FLT) {
+        fth = static_cast<float>(uload(A.th + a));
+        fsa = sure(sa, fth, false, true);
+        fca = sure(ca, fth, true, true);
+    }
 
     // EXACT: for the lanes U, the largest lo and smallest hi at their cell of
     // group m over `members` neighbours (edge b, or those listed in LDS where
@@ -491,6 +529,11 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             int k;
             if constexpr (EXACT) {
                 k = in ? cvg::direction_class(ax, ay, ca, sa, q.x, q.y, c_sincos_tab, c_atan_tab) : 3;
+            } else if constexpr (SINES) {
+                k = 3;
+                if (in)
+                    k = exact_direction(static_cast<float>(ax), static_cast<float>(ay), fth, static_cast<float>(q.x),
+                                        static_cast<float>(q.y), fca, fsa);
             } else {
                 // (direction_class's projection and a bound at least as strict)
                 const double p = vx * ca + vy * sa;
@@ -499,9 +542,9 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             }
             cls[c] = in ? k : 3;
             n1 += __popcll(__ballot(cls[c] == 1));
-            if (EXACT) n2 += __popcll(__ballot(cls[c] == 2));
+            if (CLASSES) n2 += __popcll(__ballot(cls[c] == 2));
         }
-        if (!EXACT) n2 = deg - n1;
+        if (!CLASSES) n2 = deg - n1;
         int b1 = 0, b2 = n1, b0 = n1 + n2;
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
@@ -510,7 +553,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                     static_cast<unsigned>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m), 0u)));
             };
             const u64 m1 = __ballot(cls[c] == 1);
-            if constexpr (EXACT) {
+            if constexpr (CLASSES) {
                 const u64 m2 = __ballot(cls[c] == 2), m0 = __ballot(cls[c] == 0);
                 pos[c] = cls[c] == 1 ? b1 + below(m1) : cls[c] == 2 ? b2 + below(m2) : b0 + below(m0);
                 b2 += __popcll(m2);
@@ -556,17 +599,17 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
                     const bool minus = (k == 0) == branch_a;
-                    const float fth = static_cast<float>(nth);
+                    const float fn = static_cast<float>(nth);
                     const double d = minus ? -static_cast<double>(A.dt_f) : static_cast<double>(A.dt_f);
                     const double sd = minus ? -A.sin_dt : A.sin_dt;
-                    T0[k] = minus ? fth - A.dt_f : fth + A.dt_f;
+                    T0[k] = minus ? fn - A.dt_f : fn + A.dt_f;
                     const double e = static_cast<double>(T0[k]) - (nth + d);
                     const double s0 = __builtin_fma(q.z, A.cos_dt, q.w * sd);
                     const double c0 = __builtin_fma(q.w, A.cos_dt, -(q.z * sd));
                     s[k] = __builtin_fma(e, __builtin_fma(-0.5 * e, s0, c0), s0);
                     co[k] = __builtin_fma(-e, __builtin_fma(0.5 * e, c0, s0), c0);
-                    cx[k] = fx * sure_float(co[k], bad);  // :730-733
-                    sy[k] = fy * sure_float(s[k], bad);
+                    cx[k] = fx * sure(co[k], T0[k], true, pos[c] >= 0);  // :730-733
+                    sy[k] = fy * sure(s[k], T0[k], false, pos[c] >= 0);
                 }
                 if (pos[c] >= 0 && (pos[c] >> kLog) == b) {
                     const lds_ptr<double2> o = rec + (pos[c] & kLast) * 5;
@@ -623,7 +666,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
     int batch = -1;
     unsigned nacc = 0, vp = 0, isect_u = 0;  // isect_u: the wave's, isect: the lane's
     unsigned isect = 0;
-    for (int run = 0; run < (EXACT ? 3 : 2); ++run) {
+    for (int run = 0; run < (CLASSES ? 3 : 2); ++run) {
         const int p0 = run == 0 ? 0 : (run == 1 ? n1 : n1 + n2);
         const int p1 = run == 0 ? n1 : (run == 1 ? n1 + n2 : deg);
         int R = 0;      // hypotheses of the run
@@ -661,7 +704,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                                          (static_cast<double>(T2[m]) - static_cast<double>(T0));
                         const double s = __builtin_fma(sT[m], c0, -(cT[m] * s0));
                         const double c = __builtin_fma(cT[m], c0, sT[m] * s0);
-                        const float sn = sure_float(__builtin_fma(e, __builtin_fma(-0.5 * e, s, c), s), bad);
+                        const float sn = sure(__builtin_fma(e, __builtin_fma(-0.5 * e, s, c), s), T2[m] - T0, false, true);
                         kt[k] = sn / (-sn * o + cx + sy);
                     }
                     // the reference's compare-and-assign, which ignores NaN
@@ -748,7 +791,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             }
             const int pe = min(p1, (p | kLast) + 1);
             lds_ptr<double2> q = rec + (p & kLast) * 5;
-            if (!EXACT && R + pe - p <= slots && ((closep[0] >> (p & 63)) & ((1ULL << (pe - p)) - 1ULL)) == 0ULL) {
+            if (!CLASSES && R + pe - p <= slots && ((closep[0] >> (p & 63)) & ((1ULL << (pe - p)) - 1ULL)) == 0ULL) {
                 // (most batches: no close pair, and slots for all)
                 for (; p < pe; ++p, q += 5) {
                     Bounds v[CPL];
@@ -780,8 +823,8 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 } else if (bundle(p, q, v) == 0ULL) {
                     continue;
                 }
-                if (EXACT) ++vp;
-                if (EXACT && run == 2) continue;
+                if (CLASSES) ++vp;
+                if (CLASSES && run == 2) continue;
                 if (R < slots) {
 #pragma unroll
                     for (int m = 0; m < CPL; ++m) {
@@ -802,9 +845,9 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 ++R;
             }
         }
-        if (!EXACT) vp += static_cast<unsigned>(R);
+        if (!CLASSES) vp += static_cast<unsigned>(R);
         // a chain longer than 2 takes two hypotheses and G >= 3
-        if ((EXACT && run == 2) || R < 2 || G < 3) continue;
+        if ((CLASSES && run == 2) || R < 2 || G < 3) continue;
 
         u64 hyp[NW];  // the run's hypotheses as bits over the neighbour list
 #pragma unroll
@@ -1329,6 +1372,38 @@ __global__ __launch_bounds__(64, 4) void k_curvelets_exact(FusedArgs A, int list
     put_sums(A.partial, g, vp, isect);
 }
 
+// Float maps: the anchors k_curvelets left open.  Those with a zero bound join
+// the wide ones, for the general kernel.
+template <int CPL>
+__global__ __launch_bounds__(64, 4) void k_curvelets_float_open(FusedArgs A)
+{
+    extern __shared__ double lds[];
+    const int lane = threadIdx.x & 63;
+    const int g = static_cast<int>(blockIdx.x);
+    const int total = static_cast<int>(uload(A.list_len + L_OPEN * kBucketStride));
+    unsigned vp = 0;
+    unsigned long long isect = 0;
+    if (g < total) {
+        const WaveCells<CPL> W = wave_cells<CPL>(A);
+        int2 *spill = A.spill + static_cast<size_t>(g) * A.spill_stride;
+        for (int L = g; L < total; L += static_cast<int>(gridDim.x)) {
+            int a, deg;
+            unsigned base;
+            load_entry(A.lists + static_cast<size_t>(L_OPEN) * A.n + L, a, base, deg);
+            const int id = lane < deg ? A.ids[base + lane] : -1;
+            const double4 nb = id >= 0 ? A.rec[id] : make_double4(0.0, 0.0, 0.0, 1.0);
+            const double nth = id >= 0 ? A.th[id] : 0.0;
+            if (do_anchor<CPL, 1, M_FLOAT_EXACT>(A, W, reinterpret_cast<char *>(lds), spill, a, base, deg, id, nb, nth, vp,
+                                                 isect)) {
+                if (lane == 0)
+                    A.lists[static_cast<size_t>(L_WIDE) * A.n + atomicAdd(A.list_len + L_WIDE * kBucketStride, 1u)] =
+                        make_int4(a, static_cast<int>(base), deg, 0);
+            }
+        }
+    }
+    put_sums(A.partial, g, vp, isect);
+}
+
 using FusedKernel = void (*)(FusedArgs);
 using ExactKernel = void (*)(FusedArgs, int);
 
@@ -1337,6 +1412,10 @@ template <bool FLT>
 inline FusedKernel fused_kernel(int cpl)
 {
     return cpl == 1 ? k_curvelets<1, FLT> : (cpl == 2 ? k_curvelets<2, FLT> : k_curvelets<4, FLT>);
+}
+inline FusedKernel float_open_kernel(int cpl)
+{
+    return cpl == 1 ? k_curvelets_float_open<1> : (cpl == 2 ? k_curvelets_float_open<2> : k_curvelets_float_open<4>);
 }
 template <int NW>
 inline ExactKernel exact_kernel(int cpl)

@@ -2363,9 +2363,7 @@ struct GenArgs {
     unsigned *acc_count;
     unsigned *valid_pairs;
     unsigned long long *intersections;
-    // the anchors of these two lists (lengths first, kBucketStride apart) in
-    // place of 0 .. n - 1
-    const int4 *list[2];
+    const int4 *list;  // the anchors of this list in place of 0 .. n - 1
     const unsigned *list_len;
 };
 
@@ -2410,10 +2408,9 @@ __global__ __launch_bounds__(64 * kGenWaves) void k_curvelets_generic(GenArgs<T>
     }
     unsigned vpw = 0;
     unsigned long long isect = 0;
-    const int n0 = A.list_len ? static_cast<int>(A.list_len[0]) : 0;
-    const int total = A.list_len ? n0 + static_cast<int>(A.list_len[kBucketStride]) : A.n;
+    const int total = A.list ? static_cast<int>(*A.list_len) : A.n;
     for (int i = w; i < total; i += nwaves) {
-        const int a = !A.list_len ? i : (i < n0 ? A.list[0][i].x : A.list[1][i - n0].x);
+        const int a = A.list ? A.list[i].x : i;
         const unsigned base = A.off[a];
         const int deg = static_cast<int>(A.off[a + 1] - base);
         const T ax = static_cast<T>(A.x[a]), ay = static_cast<T>(A.y[a]);
@@ -3563,9 +3560,9 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
     CVG_TRY(ensure(ctx, ctx->d_acc, static_cast<size_t>(n) * sizeof(unsigned)));
     CVG_TRY(ensure(ctx, ctx->d_rowoff, static_cast<size_t>(n + 1) * sizeof(unsigned)));
     unsigned *scal = as<unsigned>(ctx->d_scal);
-    // float maps: the fused kernel, then this one on the anchors it leaves (a
-    // sine, a direction or a zero it cannot settle, or more than 64
-    // neighbours).  The lists hold up to 256 neighbours' anchors; below three
+    // float maps: the fused kernel, then its exact form on the anchors it
+    // leaves, then this one on those of a zero bound or more than 64
+    // neighbours.  The lists hold up to 256 neighbours' anchors; below three
     // edges no chain is long enough, and this kernel counts the intersections.
     const bool fused = kFloat && G >= 3 && G <= 64 && ctx->max_deg <= 256 && !ctx->force_generic &&
                        float_limits(ctx, p.dx, p.max_k, off_x, off_t, dt) &&
@@ -3594,6 +3591,7 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
     const size_t general_bytes = sb_elems * sizeof(T) + (sf_ints + sa_ints + sc_ints) * sizeof(int) + 512;
     FusedShape f{};
     if (fused) CVG_TRY(fused_shape<true>(ctx, K, &f));
+    const long long open_waves = fused ? std::min(f.waves, static_cast<long long>(ctx->num_cu)) : 0;
     CVG_TRY(ensure(ctx, ctx->d_gbundle, std::max(general_bytes, f.spill * static_cast<size_t>(f.waves) * sizeof(int2))));
     GenArgs<T> A{};
     A.n = n;
@@ -3660,14 +3658,17 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
         M.slots = f.slots;
         M.spill = as<int2>(ctx->d_gbundle);
         M.spill_stride = f.spill;
-        CVG_TRY(ensure(ctx, ctx->d_partial, static_cast<size_t>(f.waves) * 3 * sizeof(unsigned)));
+        CVG_TRY(ensure(ctx, ctx->d_partial, static_cast<size_t>(f.waves + open_waves) * 3 * sizeof(unsigned)));
         M.partial = as<unsigned>(ctx->d_partial);
         hipLaunchKernelGGL(f.fn, dim3(static_cast<unsigned>(f.waves / kFusedWaves)), dim3(64 * kFusedWaves), f.shmem, st,
                            M);
-        A.list[0] = M.lists + static_cast<size_t>(L_OPEN) * n;
-        A.list[1] = M.lists + static_cast<size_t>(L_WIDE) * n;
-        A.list_len = M.list_len;
-        static_assert(L_WIDE == L_OPEN + 1, "the lists' lengths follow each other");
+        const FusedKernel open = float_open_kernel(K <= 64 ? 1 : (K <= 128 ? 2 : 4));
+        const unsigned slice = f.shmem / kFusedWaves;
+        CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(open), 64, slice, nullptr));
+        M.partial += 3 * f.waves;
+        hipLaunchKernelGGL(open, dim3(static_cast<unsigned>(open_waves)), dim3(64), slice, st, M);
+        A.list = M.lists + static_cast<size_t>(L_WIDE) * n;
+        A.list_len = M.list_len + L_WIDE * kBucketStride;
     }
     hipLaunchKernelGGL(k_curvelets_generic<T>, dim3(blocks), dim3(64 * kGenWaves), 0, st, A);
     CVG_HIP(ctx, hipGetLastError());
@@ -3688,7 +3689,7 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
         R.off_x = reinterpret_cast<const double *>(tb + o_off_x);
         R.off_t = reinterpret_cast<const double *>(tb + o_off_t);
     }
-    return record_rows(ctx, p, R, cap, static_cast<int>(f.waves));
+    return record_rows(ctx, p, R, cap, static_cast<int>(f.waves + open_waves));
 }
 
 int build_curvelets(cvg_context *ctx, const cvg_params &p)

@@ -1218,7 +1218,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
     return false;
 }
 
-// One wave's sums into its place (k_row_anchors adds the places up).
+// One wave's sums into its place (k_record adds the places up).
 __device__ __forceinline__ void put_sums(unsigned *partial, int g, unsigned vp, unsigned long long isect)
 {
 #pragma unroll

@@ -29,9 +29,8 @@
 //           k_curvelets_exact the same on exact bounds, for anchors whose
 //                             comparisons the approximations leave open and
 //                             those of more than 64 neighbours
-//           scan              per-anchor accepted counts -> output row offsets
-//           k_row_anchors     row -> anchor, and the counts into the scalars
-//                             read back with the stream
+//           scan              per-anchor accepted counts -> output row offsets,
+//                             and each row's anchor
 //           k_record          chain rows (1-based) and the 10 info columns
 //
 // The reference path this replaces is cpu_curvelet (preprocess.hpp,
@@ -565,8 +564,18 @@ __global__ __launch_bounds__(1024) void k_scan_tile_sums(unsigned *tile_sums, in
     }
 }
 
+// (item base + k's places out[base + k] up to `limit` in `owner` get its number)
+__device__ inline void set_owners(const unsigned (&o)[kScanItems], const unsigned (&v)[kScanItems], long long base,
+                                  int *owner, unsigned limit)
+{
+    for (int k = 0; k < kScanItems; ++k) {
+        const unsigned end = min(o[k] + v[k], limit);
+        for (unsigned q = o[k]; q < end; ++q) owner[q] = static_cast<int>(base) + k;
+    }
+}
+
 __global__ __launch_bounds__(kBlock) void k_scan_apply(const unsigned *in, long long n, const unsigned *tile_prefix,
-                                                       int ntiles, unsigned *out)
+                                                       int ntiles, unsigned *out, int *owner, unsigned limit)
 {
     __shared__ unsigned lw[kBlock / 64];
     const long long base = static_cast<long long>(blockIdx.x) * kScanTile + threadIdx.x * kScanItems;
@@ -589,6 +598,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_apply(const unsigned *in, long 
         for (int k = 0; k < kScanItems; ++k)
             if (base + k < n) out[base + k] = o[k];
     }
+    if (owner) set_owners(o, v, base, owner, limit);
     if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = tile_prefix[ntiles];
 }
 
@@ -661,7 +671,7 @@ __device__ inline unsigned scan_lookback(unsigned long long *st, unsigned epoch,
 __global__ __launch_bounds__(kBlock) void k_scan_1pass(const unsigned *__restrict__ in, long long n,
                                                        unsigned *__restrict__ out, unsigned *__restrict__ total,
                                                        unsigned long long *__restrict__ lb, unsigned epoch,
-                                                       unsigned max_spins)
+                                                       unsigned max_spins, int *__restrict__ owner, unsigned limit)
 {
     __shared__ unsigned lw[kBlock / 64];
     __shared__ unsigned s_base;
@@ -692,6 +702,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_1pass(const unsigned *__restric
         for (int k = 0; k < kScanItems; ++k)
             if (base + k < n) out[base + k] = o[k];
     }
+    if (owner) set_owners(o, v, base, owner, limit);
     if (tile == static_cast<int>(gridDim.x) - 1 && threadIdx.x == 0) {
         out[n] = s_base + agg;
         if (total) *total = s_base + agg;
@@ -700,10 +711,11 @@ __global__ __launch_bounds__(kBlock) void k_scan_1pass(const unsigned *__restric
 
 // out has n + 1 entries (the tile buffer is sized here).  With stat_max set,
 // the maximum of the inputs goes to *stat_max and the number of inputs >= thr
-// to *stat_cnt.
+// to *stat_cnt.  With owner, places out[i] .. out[i + 1] - 1 of it below limit
+// get i (the rows' anchors: a kernel for them took 11 us on the 1080p map).
 int exclusive_scan(cvg_context *ctx, const unsigned *in, long long n, unsigned *out, DevBuf &tiles,
                    unsigned *stat_max = nullptr, unsigned *stat_cnt = nullptr, unsigned thr = 0,
-                   unsigned *stat_total = nullptr)
+                   unsigned *stat_total = nullptr, int *owner = nullptr, unsigned limit = 0)
 {
     const int ntiles = static_cast<int>((n + kScanTile - 1) / kScanTile);
     CVG_TRY(ensure(ctx, tiles, static_cast<size_t>(3) * (ntiles + 1) * sizeof(unsigned)));
@@ -723,7 +735,8 @@ int exclusive_scan(cvg_context *ctx, const unsigned *in, long long n, unsigned *
                            stat_max, stat_cnt, static_cast<unsigned *>(nullptr));
     }
     if (ntiles > 0)
-        hipLaunchKernelGGL(k_scan_apply, dim3(ntiles), dim3(kBlock), 0, ctx->stream, in, n, t, ntiles, out);
+        hipLaunchKernelGGL(k_scan_apply, dim3(ntiles), dim3(kBlock), 0, ctx->stream, in, n, t, ntiles, out,
+                           owner, limit);
     else
         CVG_HIP(ctx, hipMemcpyAsync(out, t, sizeof(unsigned), hipMemcpyDeviceToDevice, ctx->stream));
     CVG_HIP(ctx, hipGetLastError());
@@ -739,10 +752,12 @@ int exclusive_scan(cvg_context *ctx, const unsigned *in, long long n, unsigned *
 // (17.8 against ~14 us).
 constexpr long long kScan1PassMaxTiles = 256;
 
-int exclusive_scan_1pass(cvg_context *ctx, const unsigned *in, long long n, unsigned *out, DevBuf &tiles)
+int exclusive_scan_1pass(cvg_context *ctx, const unsigned *in, long long n, unsigned *out, DevBuf &tiles,
+                         int *owner = nullptr, unsigned limit = 0)
 {
     const long long ntiles = (n + kScanTile - 1) / kScanTile;
-    if (ntiles > kScan1PassMaxTiles || ntiles == 0) return exclusive_scan(ctx, in, n, out, tiles);
+    if (ntiles > kScan1PassMaxTiles || ntiles == 0)
+        return exclusive_scan(ctx, in, n, out, tiles, nullptr, nullptr, 0, nullptr, owner, limit);
     CVG_TRY(ensure(ctx, ctx->d_scanstat, static_cast<size_t>(ntiles) * sizeof(unsigned long long)));
     if (++ctx->scan_epoch >= (1u << 30)) ctx->scan_epoch = 1;  // words hold epoch << 32 below the 2-bit flag
     if (ctx->d_scanstat.ptr != ctx->scanstat_zero_ptr || ctx->d_scanstat.bytes != ctx->scanstat_zero_bytes ||
@@ -753,7 +768,7 @@ int exclusive_scan_1pass(cvg_context *ctx, const unsigned *in, long long n, unsi
     }
     hipLaunchKernelGGL(k_scan_1pass, dim3(static_cast<unsigned>(ntiles)), dim3(kBlock), 0, ctx->stream, in, n, out,
                        static_cast<unsigned *>(nullptr), as<unsigned long long>(ctx->d_scanstat), ctx->scan_epoch,
-                       ctx->lookback_spins);
+                       ctx->lookback_spins, owner, limit);
     CVG_HIP(ctx, hipGetLastError());
     return CVG_OK;
 }
@@ -1786,14 +1801,26 @@ __global__ __launch_bounds__(64 * kFillWaves) void k_fill_csr(int n, const doubl
     }
 }
 
+// The scalars to the host's page-locked copy, by one workgroup (read there once
+// the kernel has ended): a copy of its own is a launch and some 4 us.
+__device__ inline void send_scalars(const unsigned *scal, unsigned *mail)
+{
+    const int i = static_cast<int>(threadIdx.x);
+    if (i < static_cast<int>(kScalarWords))
+        __hip_atomic_store(&mail[i], scal[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Anchors whose (more than 16) candidates contain exact distance ties: replay
 // libstdc++'s introsort on the scan-order list k_fill_csr left in cand.
 // Grid-stride over the device-side count, so no host round trip is needed.
+// With mail, the scalars (final by now) go to the host as well.
 __global__ __launch_bounds__(kBlock) void k_tie_sort(const int *__restrict__ tie_list,
                                                      const unsigned *__restrict__ scal,
                                                      const unsigned *__restrict__ off, Cand *__restrict__ cand,
-                                                     int *__restrict__ ids, double *__restrict__ d2)
+                                                     int *__restrict__ ids, double *__restrict__ d2,
+                                                     unsigned *__restrict__ mail)
 {
+    if (mail && blockIdx.x == 0) send_scalars(scal, mail);
     const unsigned count = scal[S_TIES];
     for (unsigned t = blockIdx.x * blockDim.x + threadIdx.x; t < count; t += gridDim.x * blockDim.x) {
         const int a = tie_list[t];
@@ -2142,33 +2169,20 @@ __device__ inline void record_row_fused(const RecordArgs &R, unsigned o, int a)
     write_info(R, o, ax, ay, at, (meta >> 8) & 1u, c, k_max, k_min, length, len);
 }
 
-// compact_curvelet_output (cpu_curvelet.hpp:282-303) in two passes.  First,
-// one thread per anchor: its rows (contiguous, from its row offset) learn
-// their anchor.  Then one thread per output row records it; the row count
-// (the last row offset) stays on the device, and rows beyond the caller's
-// buffers are left out (the host reports them).  Block 0 also puts the
-// counts the host reads into the scalars: the rows, and with `partial` the
-// fused kernel's per-wave sums (adding those up with atomics on one address
-// would cost ~11 ns each, 45 us for 4,096 waves at the kernel's end).
-__global__ __launch_bounds__(kBlock) void k_row_anchors(int n, const unsigned *__restrict__ row_off, unsigned max_rows,
-                                                        int *__restrict__ row_anchor,
-                                                        const unsigned *__restrict__ partial, int waves,
-                                                        unsigned *__restrict__ scal)
+// The run's counts into the scalars and to the host, by one workgroup: the row
+// count and, with partial, the fused kernels' per-wave sums (beside what
+// k_curvelets_generic counted of the same map).  (Adding those up with atomics
+// on one address would cost ~11 ns each, 45 us for 4,096 waves.)
+__device__ inline void finish_counts(unsigned rows, const unsigned *__restrict__ partial, int waves, unsigned *scal,
+                                     unsigned *mail)
 {
-    const int a = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-    if (a < n) {
-        const unsigned o1 = min(row_off[a + 1], max_rows);
-        for (unsigned o = row_off[a]; o < o1; ++o) row_anchor[o] = a;
-    }
-    if (blockIdx.x != 0) return;
-    if (threadIdx.x == 0) scal[S_ROWS] = row_off[n];
-    if (!partial) return;
     unsigned long long vp = 0, is = 0;
-    for (int w = static_cast<int>(threadIdx.x); w < waves; w += kBlock) {
-        vp += partial[3 * w];
-        is += static_cast<unsigned long long>(partial[3 * w + 1]) |
-              static_cast<unsigned long long>(partial[3 * w + 2]) << 32;
-    }
+    if (partial)
+        for (int w = static_cast<int>(threadIdx.x); w < waves; w += kBlock) {
+            vp += partial[3 * w];
+            is += static_cast<unsigned long long>(partial[3 * w + 1]) |
+                  static_cast<unsigned long long>(partial[3 * w + 2]) << 32;
+        }
     __shared__ unsigned long long s_vp[kBlock / 64], s_is[kBlock / 64];
     vp = wave_sum_u64(vp);
     is = wave_sum_u64(is);
@@ -2182,19 +2196,28 @@ __global__ __launch_bounds__(kBlock) void k_row_anchors(int n, const unsigned *_
             vp += s_vp[w];
             is += s_is[w];
         }
-        // (beside what k_curvelets_generic counted of the same map)
         is += static_cast<unsigned long long>(scal[S_COUNT]) | static_cast<unsigned long long>(scal[S_COUNT + 1]) << 32;
         scal[S_VALID] += static_cast<unsigned>(vp);
         scal[S_COUNT] = static_cast<unsigned>(is);
         scal[S_COUNT + 1] = static_cast<unsigned>(is >> 32);
+        scal[S_ROWS] = rows;
     }
+    __syncthreads();
+    send_scalars(scal, mail);
 }
 
+// compact_curvelet_output (cpu_curvelet.hpp:282-303): one thread per output row
+// (the offsets scan left each row's anchor).  The row count (the last row
+// offset) stays on the device, and rows beyond the caller's buffers are left
+// out (the host reports them).
 enum { ROWS_FUSED = 0, ROWS_GENERAL = 1, ROWS_FLOAT = 2 };
 
 template <int KIND>
-__global__ __launch_bounds__(kBlock) void k_record(RecordArgs R, const int *__restrict__ row_anchor)
+__global__ __launch_bounds__(kBlock) void k_record(RecordArgs R, const int *__restrict__ row_anchor,
+                                                   const unsigned *__restrict__ partial, int waves, unsigned *scal,
+                                                   unsigned *mail)
 {
+    if (blockIdx.x == 0) finish_counts(R.row_off[R.n], partial, waves, scal, mail);
     const unsigned rows = min(R.row_off[R.n], R.max_rows);
     const unsigned stride = gridDim.x * blockDim.x;
     for (unsigned o = blockIdx.x * blockDim.x + threadIdx.x; o < rows; o += stride) {
@@ -2809,13 +2832,12 @@ int graph_scans(cvg_context *ctx, const Cells &cells, int n, unsigned R, unsigne
                        as<long long>(ctx->d_eoff), scal, ctx->f32, pair_cap, lb, epoch, ctx->lookback_spins);
     hipLaunchKernelGGL(k_tie_sort, dim3(std::min(blocks_for(n), 64)), dim3(kBlock), 0, st, as<int>(ctx->d_tmp_ids),
                        scal, as<unsigned>(ctx->d_off), as<Cand>(ctx->d_cand), as<int>(ctx->d_ids),
-                       as<double>(ctx->d_d2));
+                       as<double>(ctx->d_d2),
+                       spec ? ctx->mailbox : static_cast<unsigned *>(nullptr));
     CVG_HIP(ctx, hipGetLastError());
     if (spec) {
         // the sizes come back while the device already runs the curvelet
         // stage's first kernels
-        CVG_HIP(ctx, hipMemcpyAsync(ctx->mailbox, ctx->d_scal.ptr, kScalarWords * sizeof(unsigned),
-                                    hipMemcpyDeviceToHost, st));
         CVG_HIP(ctx, hipEventRecord(ctx->ev_read, st));
         if (ctx->early_setup) CVG_TRY(queue_setup(ctx));
         CVG_HIP(ctx, hipEventSynchronize(ctx->ev_read));
@@ -3372,7 +3394,10 @@ int record_rows(cvg_context *ctx, const cvg_params &p, RecordArgs R, int st_stri
     const int n = ctx->n;
     const int pairs = ctx->pairs;
     const size_t np = static_cast<size_t>(std::max(pairs, 1));
-    CVG_TRY(exclusive_scan_1pass(ctx, as<unsigned>(ctx->d_acc), n, as<unsigned>(ctx->d_rowoff), ctx->d_tiles));
+    CVG_TRY(ensure(ctx, ctx->d_rowanchor, np * sizeof(int)));
+    R.max_rows = ctx->caller_chains ? ctx->caller_rows : UINT_MAX;
+    CVG_TRY(exclusive_scan_1pass(ctx, as<unsigned>(ctx->d_acc), n, as<unsigned>(ctx->d_rowoff), ctx->d_tiles,
+                                 as<int>(ctx->d_rowanchor), R.max_rows));
     ctx->width = static_cast<unsigned>(R.G) + 1;
     unsigned *out_chains = ctx->caller_chains;
     double *out_info = ctx->caller_info;
@@ -3397,25 +3422,22 @@ int record_rows(cvg_context *ctx, const cvg_params &p, RecordArgs R, int st_stri
     R.st_stride = st_stride;
     R.chains = out_chains;
     R.info = out_info;
-    R.max_rows = ctx->caller_chains ? ctx->caller_rows : UINT_MAX;
     if (pairs > 0) {
-        CVG_TRY(ensure(ctx, ctx->d_rowanchor, np * sizeof(int)));
-        int *row_anchor = as<int>(ctx->d_rowanchor);
-        hipLaunchKernelGGL(k_row_anchors, dim3(blocks_for(n)), dim3(kBlock), 0, st, n, R.row_off, R.max_rows,
-                           row_anchor, static_cast<const unsigned *>(fused_waves > 0 ? as<unsigned>(ctx->d_partial) : nullptr),
-                           fused_waves, as<unsigned>(ctx->d_scal));
         // a resident grid strides over the rows (their count is on the device)
         const auto rec = R.f32 ? k_record<ROWS_FLOAT> : (fused_waves > 0 ? k_record<ROWS_FUSED> : k_record<ROWS_GENERAL>);
         int occ = 0;
         CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(rec), kBlock, 0, &occ));
         const long long resident = static_cast<long long>(std::max(occ, 1)) * ctx->num_cu;
         const int grid = static_cast<int>(std::min(resident, static_cast<long long>(blocks_for(pairs))));
-        hipLaunchKernelGGL(rec, dim3(grid), dim3(kBlock), 0, st, R, static_cast<const int *>(row_anchor));
+        hipLaunchKernelGGL(rec, dim3(grid), dim3(kBlock), 0, st, R, as<int>(ctx->d_rowanchor),
+                           static_cast<const unsigned *>(fused_waves > 0 ? as<unsigned>(ctx->d_partial) : nullptr),
+                           fused_waves, as<unsigned>(ctx->d_scal), ctx->mailbox);
     }
     CVG_HIP(ctx, hipGetLastError());
-    // the counts (the row count in S_ROWS when there are pairs; none otherwise)
-    CVG_HIP(ctx, hipMemcpyAsync(ctx->mailbox, ctx->d_scal.ptr, kScalarWords * sizeof(unsigned),
-                                hipMemcpyDeviceToHost, st));
+    // (without pairs nothing was recorded: the scalars as they are)
+    if (pairs <= 0)
+        CVG_HIP(ctx, hipMemcpyAsync(ctx->mailbox, ctx->d_scal.ptr, kScalarWords * sizeof(unsigned),
+                                    hipMemcpyDeviceToHost, st));
     if (ctx->num_maps > 1) {
         const int M = ctx->num_maps;
         CVG_TRY(ensure(ctx, ctx->d_maprow, (static_cast<size_t>(M) + 1) * sizeof(unsigned)));

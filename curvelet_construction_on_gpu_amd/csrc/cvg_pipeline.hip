@@ -847,7 +847,7 @@ enum {
     S_WIDE = 15
 };
 constexpr int kScalarWords = S_WIDE + 1;  // the words read back to the host
-constexpr int kMaxLists = 6;
+constexpr int kMaxLists = 16;
 constexpr int kBucketStride = 32;  // words
 constexpr int kBucketBase = 32;    // list b's length at [kBucketBase + b * kBucketStride]
 constexpr int kScalarBufWords = kBucketBase + kMaxLists * kBucketStride;

@@ -3603,7 +3603,14 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
                             static_cast<size_t>(max_deg) * (cap + 1) * sizeof(int) + static_cast<size_t>(cap) * sizeof(int) +
                             256;
     long long waves = std::min<long long>(n, static_cast<long long>(ctx->num_cu) * 16);
-    waves = std::max(1LL, std::min<long long>(waves, static_cast<long long>((size_t(512) << 20) / per_wave)));
+    size_t budget = size_t(512) << 20;
+    if (ctx->arena) {
+        // (what the no-alloc scratch has left after the record's buffers)
+        const size_t later = np * sizeof(int) + static_cast<size_t>(n) * 2 * sizeof(unsigned) + (size_t(256) << 10);
+        const size_t left = kScratchBytes - std::min(kScratchBytes, ctx->arena_used);
+        budget = left > later ? left - later : 0;
+    }
+    waves = std::max(1LL, std::min<long long>(waves, static_cast<long long>(budget / per_wave) / kGenWaves * kGenWaves));
     const int blocks = static_cast<int>((waves + kGenWaves - 1) / kGenWaves);
     const size_t nwaves = static_cast<size_t>(blocks) * kGenWaves;
     const size_t sb_elems = nwaves * max_deg * K * 2;

@@ -17,7 +17,7 @@
 //
 // Measured on the 1080p map (207,326 edges, 2.04M pairs, G = 7): 1,000 us for
 // the kernel on exact bounds and 141 us for its sines pass (345 MB) before; now
-// 473 us, and 65 us for the few anchors left open (81 us before they shared a
+// 455 us, and 65 us for the few anchors left open (81 us before they shared a
 // bound's sides and members out over the lanes).
 #ifndef CVG_FUSED_HPP
 #define CVG_FUSED_HPP

@@ -242,7 +242,7 @@ struct cvg_context {
     unsigned max_deg = 0;
     unsigned truncated = 0;
     unsigned ambiguous = 0;
-    bool wide_theta = false;  // some |theta| above kWideTheta
+    unsigned wide_theta = 0;  // 1: some |theta| above kWideTheta, 3: above kMaxTheta
     int gx0 = 0, gy0 = 0, gw = 0, gh = 0;
     // d_grid's leading cell counts known to be zero (while d_grid is grid_zero_ptr)
     const void *grid_zero_ptr = nullptr;
@@ -852,9 +852,10 @@ constexpr int kBucketStride = 32;  // words
 constexpr int kBucketBase = 32;    // list b's length at [kBucketBase + b * kBucketStride]
 constexpr int kScalarBufWords = kBucketBase + kMaxLists * kBucketStride;
 
-// Orientations the fused kernel's error bound covers (fused_limits); maps
-// with larger ones take the general kernel.
-constexpr double kWideTheta = 64.0;
+// Orientations the fused kernel's error bounds cover (fused_limits): up to the
+// second it allows for 64 times the rounding of the angles; maps with larger
+// ones take the general kernel.
+constexpr double kWideTheta = 64.0, kMaxTheta = 4096.0;
 
 // Cells are (lrint(x), lrint(y)) (preprocess.hpp:85-86).  Coordinates must be
 // finite with |x|, |y| < 2^31 - 2^13 (so that every window cell cx +- R of the
@@ -888,7 +889,7 @@ __global__ __launch_bounds__(kBlock) void k_prep_edges(int n, int sz, const doub
         const double tv = e[static_cast<long long>(i) * sz + 2];
         const bool ok = fabs(xv) < kMaxCoord && fabs(yv) < kMaxCoord && fabs(tv) <= DBL_MAX;
         if (!ok) atomicOr(&sbad, 1);
-        if (!(fabs(tv) <= kWideTheta)) atomicOr(&sbad, 2);
+        if (!(fabs(tv) <= kWideTheta)) atomicOr(&sbad, fabs(tv) <= kMaxTheta ? 2 : 6);
         const int ix = ok ? static_cast<int>(rint(xv)) : 0;
         const int iy = ok ? static_cast<int>(rint(yv)) : 0;
         x[i] = xv;
@@ -969,7 +970,7 @@ __global__ __launch_bounds__(1024) void k_bbox_finish(int nparts, const int *__r
         scal[S_MINY] = static_cast<unsigned>(v[2]);
         scal[S_MAXY] = static_cast<unsigned>(v[3]);
         scal[S_BAD] = v[4] & 1 ? 1u : 0u;
-        scal[S_WIDE] = v[4] & 2 ? 1u : 0u;
+        scal[S_WIDE] = static_cast<unsigned>(v[4]) >> 1;
         if (spec_on) {
             const bool fits = static_cast<long long>(v[0]) - R >= spec.x0 &&
                               static_cast<long long>(v[1]) + R <= static_cast<long long>(spec.x0) + spec.w - 1 &&
@@ -2760,7 +2761,7 @@ int graph_scans(cvg_context *ctx, const Cells &cells, int n, unsigned R, unsigne
         if (ctx->max_deg >= (1u << 23))
             return fail(ctx, CVG_ERR_UNSUPPORTED, "an anchor has 2^23 or more neighbours");
         ctx->truncated = ctx->mailbox[S_TRUNC];
-        ctx->wide_theta = ctx->mailbox[S_WIDE] != 0;
+        ctx->wide_theta = ctx->mailbox[S_WIDE];
         return CVG_OK;
     };
     int fill_cap;
@@ -3217,7 +3218,8 @@ int queue_setup(cvg_context *ctx)
 //
 // u = 2^-53; S >= |DX| + |DY| over the window, X = dx + max |delta_x2|,
 // B = S + X.  Angles are below 72 (|theta| <= 64), so theta + delta is rounded
-// by up to 64 u and a difference of two by 128 u.  Against the reference's own
+// by up to 64 u and a difference of two by 128 u (64 times that up to |theta| =
+// 4096: all of the below is then scaled).  Against the reference's own
 // rounded evaluation:
 //   rotated sin/cos              68 u     (64 u the angle, the rest rounding)
 //   s0, s1                      352 u     (two rotated pairs, the difference)
@@ -3238,14 +3240,15 @@ bool fused_limits(const cvg_context *ctx, const Derived &d, FusedLimits *lim)
     double S = 2.0 * (static_cast<double>(ctx->nbr_radius) + 1.0);
     if (ctx->rad >= 0.0) S = std::min(S, 1.5 * ctx->rad);
     const double B = S + d.dx + xmax;
-    if (!(d.dx >= 0.0) || !(d.max_k > 0.0) || !(tmax <= 8.0) || !(B <= 1e5) || ctx->wide_theta) return false;
-    const double u = std::ldexp(1.0, -53);
+    if (!(d.dx >= 0.0) || !(d.max_k > 0.0) || !(tmax <= 8.0) || !(B <= 1e5) || ctx->wide_theta > 1) return false;
+    const double u = std::ldexp(ctx->wide_theta ? 64.0 : 1.0, -53);
     const double num = std::max(152.0 * B, 352.0) * u, den = std::max(64.0 * B * B, 360.0 * B) * u;
     lim->num_err = 4.0 * num;
     lim->den_err = 4.0 * den;
     lim->min_den = 4.0 * (num + 2.0 * d.max_k * den) / (d.max_k * std::ldexp(1.0, -27));
     lim->min_prod = 1.01 * lim->min_den * B * std::max(B, B * B + d.dx2);
-    return lim->min_den <= 0.05;
+    // (denominators are of the order of 1; beyond, too many would be open)
+    return lim->min_den <= 0.25;
 }
 
 // The parameter tables to d_tables, unless the same bytes are already there
@@ -3498,7 +3501,7 @@ bool float_limits(const cvg_context *ctx, double dx, double max_k, const std::ve
     for (T v : off_x) xmax = std::max(xmax, std::fabs(static_cast<double>(v)));
     for (T v : off_t) tmax = std::max(tmax, std::fabs(static_cast<double>(v)));
     const double S = 2.0 * (static_cast<double>(ctx->nbr_radius) + 1.0);
-    return dx >= 1e-9 && max_k >= 1e-9 && max_k <= 1e9 && tmax <= 8.0 && S + dx + xmax <= 1e5 && !ctx->wide_theta;
+    return dx >= 1e-9 && max_k >= 1e-9 && max_k <= 1e9 && tmax <= 8.0 && S + dx + xmax <= 1e5 && ctx->wide_theta == 0;
 }
 
 // The curvelet stage on k_curvelets_generic: the float instantiation

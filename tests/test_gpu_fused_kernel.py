@@ -80,7 +80,7 @@ def test_equal_bounds(both, oracle_cr, angle, sx, st):
     same_bits(both, oracle_cr, e, CurveletParams(sx=sx, st=st, group_max_sz=5))
 
 
-@pytest.mark.parametrize("top", [63.9, 64.0, 64.1, 1e5])
+@pytest.mark.parametrize("top", [63.9, 64.0, 64.1, 500.0, 4095.9, 4096.0, 4096.1, 1e5])
 def test_orientation_range(both, oracle_cr, top):
     e = lines(6, seed=3)
     e[:, 2] += 2 * np.pi * np.floor((top - e[:, 2].max()) / (2 * np.pi))
@@ -89,7 +89,8 @@ def test_orientation_range(both, oracle_cr, top):
 
 
 @pytest.mark.parametrize("dx,dt,max_k,nrad", [(0.4, 15.0, 0.3, 3.5), (0.2, 2.0, 2.0, 3.0), (1.5, 40.0, 0.05, 5.0),
-                                              (0.4, 15.0, 1e-6, 3.5), (0.4, 15.0, 1e4, 3.5)])
+                                              (0.4, 15.0, 1e-6, 3.5), (0.4, 15.0, 1e-3, 3.5),
+                                              (0.4, 15.0, 1e4, 3.5)])
 def test_parameter_range(both, oracle_cr, dx, dt, max_k, nrad):
     rng = np.random.default_rng(7)
     e = np.stack([rng.uniform(0, 30, 500), rng.uniform(0, 30, 500), rng.uniform(-3, 3, 500), np.ones(500)], axis=1)

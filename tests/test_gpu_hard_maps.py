@@ -1,0 +1,42 @@
+"""Maps whose distances, bounds, orientations or parameters put the kernels on
+their slower branches: the time stays of the order of an ordinary map's of the
+same size (the shortest of several runs, against a factor far above what is
+measured and far below what the fault behind each test cost)."""
+import numpy as np
+import pytest
+
+from curvelet_construction_on_gpu_amd import Context, CurveletParams, synth_edges
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    return Context()
+
+
+@pytest.fixture(scope="module")
+def frame():
+    return synth_edges("C3", 1003)
+
+
+def on_pixels(e):
+    """The map at whole pixels, one edge each."""
+    e = e.copy()
+    e[:, :2] = np.rint(e[:, :2])
+    _, first = np.unique(e[:, :2], axis=0, return_index=True)
+    return np.ascontiguousarray(e[np.sort(first)])
+
+
+def shortest(ctx, e, p, key, runs=7):
+    return min(ctx.run(e, p)[key] for _ in range(runs))
+
+
+def test_graph_of_tied_distances(ctx, frame):
+    """Nearly every list has exact ties; the fill took 1,100 us of it (about
+    100 without ties) while tied places were written twice."""
+    p = CurveletParams()
+    e = on_pixels(frame)
+    apart = e.copy()
+    apart[:, :2] += np.random.default_rng(1).uniform(-0.3, 0.3, (len(e), 2))
+    assert shortest(ctx, e, p, "ms_graph") < 3.0 * shortest(ctx, apart, p, "ms_graph")

@@ -161,12 +161,8 @@ __device__ __forceinline__ T uload(const T *p)
     return *(const __attribute__((address_space(4))) T *)p;
 }
 
-// Fixed point: max_k is 2^30; conversions and differences saturate.  Two
-// approximate bounds whose difference is beyond kFixTol compare as the exact
-// ones do: each is off by at most 8 units from the formulas (fused_limits
-// keeps the denominators where that holds) and 1 from the conversion.
-constexpr int kFixOne = 1 << 30;
-constexpr int kFixTol = 18;
+using cvg::kFixOne;
+using cvg::kFixTol;
 
 // v_cvt_i32_f64: truncates and saturates (NaN gives 0), where the C++ cast is
 // undefined out of range.
@@ -409,11 +405,11 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
         return v;
     };
     // Each comparison's t = hi - lo: true above kFixTol, false below -kFixTol,
-    // and in between open.  Not EXACT: a lane's smallest t + kFixTol, as
-    // unsigned, says at the end whether any of its comparisons was open.
+    // and in between open.  Not EXACT: a lane's smallest open_key says at the
+    // end whether any of its comparisons was open.
     unsigned closest = ~0u;
     auto note = [&](int t) {
-        if (MODE == M_FAST) closest = min(closest, static_cast<unsigned>(t + kFixTol));
+        if (MODE == M_FAST) closest = min(closest, cvg::open_key(t));
     };
     unsigned bad = 0u;        // M_FLOAT: nonzero where a float sine is uncertain
     // the float of v, an approximation of x's sine or cosine, in the lanes `in`
@@ -432,7 +428,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
     };
     float least = A.max_k_f;  // float maps: the smallest magnitude of a bound (a zero's sign would be lost)
     auto is_open = [&](int t) -> u64 {
-        return __builtin_amdgcn_ballot_w64(static_cast<unsigned>(t + kFixTol) <= 2u * kFixTol);
+        return __builtin_amdgcn_ballot_w64(cvg::open_key(t) <= 2u * kFixTol);
     };
     u64 open = 0ULL;
 

@@ -64,6 +64,7 @@
 
 #include "../../include/curvelet_gpu.h"
 #include "cvg_device.hpp"
+#include "cvg_fixed.hpp"
 #include "cvg_math.hpp"
 #include "cvg_stlsort.hpp"
 

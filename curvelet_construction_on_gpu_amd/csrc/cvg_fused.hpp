@@ -47,9 +47,10 @@ __device__ inline double exact_bound(const ExactGrid &E, bool upper, double ax, 
     const bool branch_a = (DX * ca + DY * sa) < 0;  // :690
     const double tt = s2 * DX - c2 * DY;
     const double ttm = tt - ox;
-    const double den = -2.0 * ox * tt + DX2 + DY2 - E.dx2 + ox * ox;
+    // (:711; :774 negates the sum, so that an exact zero is -0 there)
+    const double u = 2.0 * ox * tt - DX2 - DY2 + E.dx2 - ox * ox;
     const double x = upper ? ttm + E.dx : ttm - E.dx;
-    const double kx = (branch_a ? 2.0 * x : x) / (branch_a ? den : den / 2.0);
+    const double kx = (branch_a ? 2.0 * x : x) / (branch_a ? 0.0 - u : -u / 2.0);
     const double T0 = branch_a == upper ? nt + E.dt : nt - E.dt;
     double s0, c0;
     cvg::cr_sincos<false>(T0, c_sincos_tab, &s0, &c0);
@@ -339,7 +340,7 @@ __device__ __forceinline__ float key_float(int k) { return __int_as_float(k ^ ((
 // One anchor on one wave.  M_FAST and M_FLOAT return true, with nothing
 // counted, when something is closer than they can decide; M_EXACT makes such
 // comparisons on the exact bounds, and M_FLOAT_EXACT returns true only for a
-// bound of zero, whose sign the integers lose.
+// bound or denominator of zero, whose sign is lost.
 //
 // Lane = neighbour forms the pairs' direction class, flags and
 // cell-independent terms (16 records in LDS at a time, in run order).  Then,
@@ -426,7 +427,9 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
         }
         return f;
     };
-    float least = A.max_k_f;  // float maps: the smallest magnitude of a bound (a zero's sign would be lost)
+    // float maps: the smallest magnitude of a bound or of its first denominator
+    // (a zero's sign would be lost: :774 makes it -0)
+    float least = A.max_k_f;
     auto is_open = [&](int t) -> u64 {
         return __builtin_amdgcn_ballot_w64(cvg::open_key(t) <= 2u * kFixTol);
     };
@@ -701,7 +704,8 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                     // the reference's compare-and-assign, which ignores NaN
                     const float lo = __builtin_fmaxf(__builtin_fmaxf(-A.max_k_f, kx0), kt[0]);
                     const float hi = __builtin_fminf(__builtin_fminf(A.max_k_f, kx1), kt[1]);
-                    least = __builtin_fminf(least, __builtin_fminf(__builtin_fabsf(lo), __builtin_fabsf(hi)));
+                    least = __builtin_fminf(__builtin_fminf(least, __builtin_fabsf(den)),
+                                            __builtin_fminf(__builtin_fabsf(lo), __builtin_fabsf(hi)));
                     const bool ok = hi > lo;
                     v[m].lo = ok ? float_key(lo) : INT_MAX;
                     v[m].hi = ok ? float_key(hi) : INT_MIN;

@@ -10,19 +10,21 @@
 // formed approximately, with a proven error bound: sines by rotating the edges'
 // correctly rounded sin/cos, one reciprocal for the three denominators, the
 // result in 32-bit fixed point.  A comparison whose margin exceeds the error
-// bound is decided by it.  An anchor with any closer comparison is done again,
-// and then those comparisons are made on the exact bounds (the reference's
-// operands and rounding points, correctly rounded math, IEEE divisions).  The
-// results are the reference's bit for bit.
+// bound is decided by it.  An anchor with any closer comparison is done again
+// on the reference's own bounds (its operands and rounding points, correctly
+// rounded math, IEEE divisions, doubles).  The results are the reference's bit
+// for bit.
 //
 // Measured on the 1080p map (207,326 edges, 2.04M pairs, G = 7): 1,000 us for
 // the kernel on exact bounds and 141 us for its sines pass (345 MB) before; now
-// 455 us, and 65 us for the few anchors left open (81 us before they shared a
-// bound's sides and members out over the lanes).
+// 460 us, and 68 us for the few anchors left open, which is one wave's time for
+// one of them.  The same map at whole pixels and 16 orientations leaves about
+// half of its anchors open: 0.70 ms.  (Their open comparisons alone made on
+// exact bounds, on 256 waves: 1.51 ms, and 4.2 ms with all orientations zero.)
 #ifndef CVG_FUSED_HPP
 #define CVG_FUSED_HPP
 
-// The grid and edges of exact_bounds.
+// The grid and edges of exact_bound.
 struct ExactGrid {
     const double *x, *y, *th;
     const double *off_x, *off_t;  // delta_x2, delta_t2 (cpu_curvelet.hpp:697-698)
@@ -67,15 +69,18 @@ __device__ inline double exact_bound(const ExactGrid &E, bool upper, double ax, 
     return v;
 }
 
-// A lane's bound (lo, or hi with `upper`) at the cell (ox, ot) of anchor a.
-// Out of line: the exact kernel's few anchors spend much of their time on
-// instruction fetch, and its callers share this copy.
-__device__ __noinline__ double exact_value(ExactGrid E, bool upper, double ax, double ay, double sa, double ca,
-                                           double T2t, double ox, int b)
+// Correctly rounded, of any finite angle; out of line: the direct kernel's
+// anchors are often few, and then spend much of their time on instruction fetch.
+__device__ __noinline__ double2 direct_sincos(double x)
 {
-    double s2, c2;
-    cvg::cr_sincos<false>(T2t, c_sincos_tab, &s2, &c2);
-    return exact_bound(E, upper, ax, ay, sa, ca, T2t, s2, c2, ox, b);
+    double s, c;
+    cvg::cr_sincos(x, c_sincos_tab, &s, &c);
+    return make_double2(s, c);
+}
+__device__ __noinline__ double direct_sin(double x) { return cvg::cr_sin(x, c_sincos_tab); }
+__device__ __noinline__ int direct_class(double ax, double ay, double ca, double sa, double nx, double ny)
+{
+    return cvg::direction_class(ax, ay, ca, sa, nx, ny, c_sincos_tab, c_atan_tab);
 }
 
 // Per edge: (x, y, sin theta, cos theta), the correctly rounded pair.  Block 0
@@ -100,7 +105,7 @@ __global__ __launch_bounds__(kBlock) void k_edge_rec(int n, const double *__rest
 }
 
 // Anchors in spatial (cell) order in lists by falling degree: first those of
-// more than 64 neighbours (for k_curvelets_exact), then k_curvelets': its waves
+// more than 64 neighbours (for k_curvelets_direct), then k_curvelets': its waves
 // take entries round robin over those concatenated lists, so each gets its
 // share of long and short anchors, and the kernel's tail consists of the
 // shortest.  Narrow lists keep the shares alike: with 14 of them in place of
@@ -216,6 +221,7 @@ struct FusedArgs {
     const double *th;
     ExactGrid exact;
     const int *ids;
+    const unsigned *off;  // CSR offsets
     int4 *lists;         // kLists x n entries (anchor, CSR base, degree, -)
     unsigned *list_len;  // entry counts, kBucketStride words apart (device; k_order's, and the open list's)
     int n;
@@ -224,21 +230,22 @@ struct FusedArgs {
     // whether it can be a best cell
     const double *rank_ox, *rank_ot, *rank_so, *rank_co;
     const int *rank_elig;
+    const int *rank_cell;
+    float inv_kt;  // 1 / exact.kt
     int rank_of_cell0;
     double sin_dt, cos_dt, dx, four_dx, dx2, close_thr, max_k;
     double scale;                    // kFixOne / max_k
     double min_den, num_err, den_err;  // fused_limits
     double min_prod;                 // below it a product of the three denominators may have a small one
     int slots;                       // bundle slots in LDS; a run's other bundles go to `spill`
-    int2 *spill;
-    size_t spill_stride;             // per wave
+    char *spill;
+    size_t spill_stride;             // bytes per wave
     ulonglong2 *st_mask;             // (hypotheses, chain) per row
     size_t mask_plane;               // entries between the 64-bit planes of st_mask
     unsigned *st_meta;
     // float maps: the reference's float operands, and rows as the general
     // kernel stages them
     float dt_f, dx_f, max_k_f, close_f;
-    const int *rank_cell;
     int *st_ids;
     int st_stride;
     double *st_k;
@@ -254,19 +261,44 @@ constexpr int kFusedSlots = 12;  // bundle slots at one cell per lane
 __host__ __device__ constexpr int batch_log(int cpl) { return cpl == 1 ? 4 : 3; }
 constexpr int kSmallRun = 8;    // runs up to here grow on cell masks
 
+constexpr int kLeftOpen = 16;   // a wave's anchors waiting to be appended to another list
+
 struct SliceCarve {
-    int bun, rec, pm, bytes;
+    int bun, rec, pm, sines, left, bytes;
 };
 
 // One wave's LDS slice: bundle slots (lo, hi per lane), the pair records of
-// one batch (80 B each), and the mask matrix of a small run.
+// one batch (80 B each), the mask matrix of a small run, and the anchors left
+// open.  With 12 slots that is 8,000 B, four of them the 25 blocks of 1,280 B that
+// let a fifth workgroup onto a CU.
 __host__ __device__ inline SliceCarve slice_carve(int slots, int cpl)
 {
     SliceCarve c{};
     c.bun = 0;
     c.rec = c.bun + slots * cpl * 64 * 8;
     c.pm = c.rec + (80 << batch_log(cpl));
-    c.bytes = c.pm + 64 * cpl * 8;
+    c.left = c.pm + 64 * cpl * 8;
+    c.bytes = c.left + kLeftOpen * 4;
+    return c;
+}
+
+// The same with bounds in doubles, 16 pair records at a time, and the
+// transport sines of direct_pairs(kt) pairs.
+constexpr int kDirectSlots = 8;
+__host__ __device__ inline int direct_pairs_log(int kt)
+{
+    int log = 4;
+    while (log > 0 && (2 * kt << log) > 128) --log;
+    return log;
+}
+__host__ __device__ inline SliceCarve direct_carve(int slots, int cpl, int kt)
+{
+    SliceCarve c{};
+    c.bun = 0;
+    c.rec = c.bun + slots * cpl * 64 * 16;
+    c.pm = c.rec + 16 * 80;
+    c.sines = c.pm + 64 * cpl * 8;
+    c.bytes = c.sines + (2 * kt << direct_pairs_log(kt)) * 8;
     return c;
 }
 
@@ -274,7 +306,9 @@ __host__ __device__ inline SliceCarve slice_carve(int slots, int cpl)
 template <int CPL>
 struct WaveCells {
     double ox[CPL], oxp2[CPL], so[CPL], co[CPL];
-    double m2ox[CPL], ox2[CPL], ot[CPL];  // (float maps)
+    double m2ox[CPL], ox2[CPL];  // (float maps)
+    double ot[CPL];
+    int j[CPL];  // (direct) the cell's orientation offset
     unsigned long long emask[CPL];  // cells that can be a best one
 };
 
@@ -285,8 +319,9 @@ using lds_ptr = __attribute__((address_space(3))) T *;
 template <typename T>
 using mem_ptr = __attribute__((address_space(1))) T *;
 
-struct alignas(8) Bounds {
-    int lo, hi;
+template <typename V>
+struct alignas(2 * sizeof(V)) BoundsOf {
+    V lo, hi;
 };
 
 // Float maps (the reference's float instantiation).  Its bounds are formed by
@@ -300,11 +335,11 @@ struct alignas(8) Bounds {
 // those went to the general kernel).
 // M_FLOAT leaves an anchor with an uncertain sine or direction open;
 // M_FLOAT_EXACT takes the correctly rounded ones there.
-enum { M_FAST = 0, M_EXACT = 1, M_FLOAT = 2, M_FLOAT_EXACT = 3 };
+enum { M_FAST = 0, M_DIRECT = 1, M_FLOAT = 2, M_FLOAT_EXACT = 3 };
 
 __device__ inline int direction_class_f(float ax, float ay, float at, float nx, float ny, float cos_at, float sin_at);
 
-// (out of line, as exact_value)
+// (out of line, as direct_sin)
 __device__ __noinline__ float exact_sine(float x, bool cosine)
 {
     float s, c;
@@ -338,9 +373,14 @@ __device__ __forceinline__ int float_key(float v)
 __device__ __forceinline__ float key_float(int k) { return __int_as_float(k ^ ((k >> 31) & INT_MAX)); }
 
 // One anchor on one wave.  M_FAST and M_FLOAT return true, with nothing
-// counted, when something is closer than they can decide; M_EXACT makes such
-// comparisons on the exact bounds, and M_FLOAT_EXACT returns true only for a
-// bound or denominator of zero, whose sign is lost.
+// counted, when something is closer than they can decide; M_DIRECT forms the
+// reference's own bounds, and M_FLOAT_EXACT returns true only for a bound or
+// denominator of zero, whose sign is lost.
+//
+// M_DIRECT: correctly rounded sines and four IEEE divisions a cell, bounds in
+// doubles.  A pair's transport sines depend on the cell's orientation offset
+// alone (sin(T2t - T0), :728-729): the lanes take (pair, side, offset) items,
+// 7 to a side in place of 63 cells, and the cells read them in LDS.
 //
 // Lane = neighbour forms the pairs' direction class, flags and
 // cell-independent terms (16 records in LDS at a time, in run order).  Then,
@@ -349,7 +389,8 @@ __device__ __forceinline__ float key_float(int k) { return __int_as_float(k ^ ((
 // valid one; CPL cells per lane), each run's bundles: forward neighbours,
 // backward, neither (validity only, for the count).  A valid (or close) pair
 // is a hypothesis and takes the next slot; its cells with hi <= lo are stored
-// as (largest, smallest), so that they compare as invalid from then on.
+// as (largest, smallest), so that they compare as invalid from then on (M_DIRECT:
+// as they are).
 //
 // Growth.  A chain's running bundle is max lo, min hi over its members, so it
 // is valid at a cell exactly where every member's lo lies below every member's
@@ -370,21 +411,23 @@ __device__ __forceinline__ float key_float(int k) { return __int_as_float(k ^ ((
 //
 // nid, nb, nth: lane's neighbour (of the first 64), its record and orientation.
 template <int CPL, int NW, int MODE>
-__device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CPL> &W, char *sl, int2 *spill, int a,
+__device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CPL> &W, char *sl, char *spill, int a,
                                           unsigned base, int deg, int nid, const double4 nb, double nth,
                                           unsigned &vp_sum, unsigned long long &isect_sum)
 {
     typedef unsigned long long u64;
-    constexpr bool EXACT = MODE == M_EXACT, FLT = MODE >= M_FLOAT, SINES = MODE == M_FLOAT_EXACT;
-    constexpr bool CLASSES = EXACT || SINES;  // exact directions, with the third class
+    constexpr bool DIRECT = MODE == M_DIRECT, FLT = MODE >= M_FLOAT, SINES = MODE == M_FLOAT_EXACT;
+    constexpr bool CLASSES = DIRECT || SINES;  // exact directions, with the third class
     static_assert(!FLT || NW == 1, "float maps: up to 64 neighbours");
+    using V = typename std::conditional<DIRECT, double, int>::type;
+    using Bounds = BoundsOf<V>;
     constexpr int kTol = FLT ? 0 : kFixTol;
-    constexpr int kLog = batch_log(CPL), kLast = (1 << kLog) - 1;
+    constexpr int kLog = DIRECT ? 4 : batch_log(CPL), kLast = (1 << kLog) - 1;
     constexpr int NC = NW;  // 64-seed (64-neighbour) chunks
     const int lane = threadIdx.x & 63;
     const int G = A.G;
     const int slots = A.slots;
-    const SliceCarve cv = slice_carve(A.slots, CPL);
+    const SliceCarve cv = DIRECT ? direct_carve(A.slots, CPL, A.exact.kt) : slice_carve(A.slots, CPL);
     const lds_ptr<Bounds> bun = (lds_ptr<Bounds>)(sl + cv.bun) + lane;
     const lds_ptr<double2> rec = (lds_ptr<double2>)(sl + cv.rec);
     const lds_ptr<u64> pm = (lds_ptr<u64>)(sl + cv.pm);
@@ -405,8 +448,8 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
         if (64 * c + lane < deg) v = A.rec[A.ids[base + 64 * c + lane]];
         return v;
     };
-    // Each comparison's t = hi - lo: true above kFixTol, false below -kFixTol,
-    // and in between open.  Not EXACT: a lane's smallest open_key says at the
+    // M_FAST, each comparison's t = hi - lo: true above kFixTol, false below
+    // -kFixTol, and in between open.  A lane's smallest open_key says at the
     // end whether any of its comparisons was open.
     unsigned closest = ~0u;
     auto note = [&](int t) {
@@ -430,18 +473,21 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
     // float maps: the smallest magnitude of a bound or of its first denominator
     // (a zero's sign would be lost: :774 makes it -0)
     float least = A.max_k_f;
-    auto is_open = [&](int t) -> u64 {
-        return __builtin_amdgcn_ballot_w64(cvg::open_key(t) <= 2u * kFixTol);
-    };
     u64 open = 0ULL;
 
     const double *ar = reinterpret_cast<const double *>(A.rec + a);
     const double ax = uload(ar), ay = uload(ar + 1), sa = uload(ar + 2), ca = uload(ar + 3);
-    // sin/cos of theta_a + delta_t2 by rotation
+    // sin/cos of theta_a + delta_t2 (by rotation)
     double sT[CPL], cT[CPL];
     float T2[CPL], sf[CPL], cf[CPL];  // float maps: the angle, its sine and cosine
 #pragma unroll
     for (int m = 0; m < CPL; ++m) {
+        if constexpr (DIRECT) {
+            const double2 t = direct_sincos(uload(A.th + a) + W.ot[m]);  // :702
+            sT[m] = t.x;
+            cT[m] = t.y;
+            continue;
+        }
         sT[m] = __builtin_fma(sa, W.co[m], ca * W.so[m]);
         cT[m] = __builtin_fma(ca, W.co[m], -(sa * W.so[m]));
         if constexpr (FLT) {
@@ -462,41 +508,6 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
         fsa = sure(sa, fth, false, true);
         fca = sure(ca, fth, true, true);
     }
-
-    // EXACT: for the lanes U, the largest lo and smallest hi at their cell of
-    // group m over `members` neighbours (edge b, or those listed in LDS where
-    // the pair records are): a (cell, member, side) per lane, as a bound is a
-    // long chain of double operations and few cells are open at a time
-    const lds_ptr<int> listed = (lds_ptr<int>)(sl + cv.rec);
-    const lds_ptr<double> value = (lds_ptr<double>)(sl + cv.bytes - 512);
-    auto exact_set = [&](int m, u64 U, int members, int b, double &lo, double &hi) {
-        lo = -INFINITY;
-        hi = INFINITY;
-        const int mine = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
-                             static_cast<unsigned>(U >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(U), 0u))) *
-                         members;
-        const int items = 2 * __popcll(U) * members;
-#pragma unroll 1
-        for (int t0 = 0; t0 < items; t0 += 64) {
-            const int q = (t0 + lane) >> 1, at = q / members;
-            int rho = 0, k = 0;
-#pragma unroll 1
-            for (u64 u = U; u != 0ULL; u &= u - 1ULL, ++k) rho = at == k ? __builtin_ctzll(u) + 64 * m : rho;
-            rho = rho < A.K ? rho : 0;
-            double v = 0.0;
-            if (t0 + lane < items)
-                v = exact_value(A.exact, (lane & 1) != 0, ax, ay, sa, ca, A.th[a] + A.rank_ot[rho], A.rank_ox[rho],
-                                b >= 0 ? b : listed[q - at * members]);
-            wave_sync();  // the last values are read
-            value[lane] = v;
-            wave_sync();
-            if (__builtin_amdgcn_inverse_ballot_w64(U))
-                for (int i = max(mine, t0 >> 1); i < min(mine + members, (t0 >> 1) + 32); ++i) {
-                    lo = fmax(lo, value[2 * i - t0]);
-                    hi = fmin(hi, value[2 * i - t0 + 1]);
-                }
-        }
-    };
 
     // direction classes (:459-461), lane = neighbour; a neighbour's place in
     // run order (forward, backward, neither; CSR order within)
@@ -521,8 +532,9 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 cl[c] = in && fx * fx + fy * fy < A.close_f;
             }
             int k;
-            if constexpr (EXACT) {
-                k = in ? cvg::direction_class(ax, ay, ca, sa, q.x, q.y, c_sincos_tab, c_atan_tab) : 3;
+            if constexpr (DIRECT) {
+                k = 3;
+                if (in) k = direct_class(ax, ay, ca, sa, q.x, q.y);
             } else if constexpr (SINES) {
                 k = 3;
                 if (in)
@@ -627,6 +639,20 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             }
             const double DX = ax - q.x, DY = ay - q.y;
             const bool branch_a = (DX * ca + DY * sa) < 0;  // :690
+            if constexpr (DIRECT) {
+                // DX, DY, their squares, the angles; below: DX cos and DY sin
+                if (pos[c] >= 0 && (pos[c] >> kLog) == b) {
+                    const double th = c > 0 ? A.th[A.ids[base + 64 * c + lane]] : nth;
+                    const lds_ptr<double2> o = rec + (pos[c] & kLast) * 5;
+                    o[0].x = DX;
+                    o[0].y = DY;
+                    o[1].x = DX * DX;
+                    o[1].y = DY * DY;
+                    o[4].x = branch_a ? th - A.exact.dt : th + A.exact.dt;
+                    o[4].y = branch_a ? th + A.exact.dt : th - A.exact.dt;
+                }
+                continue;
+            }
             const double sd = branch_a ? -A.sin_dt : A.sin_dt;
             const double s0 = __builtin_fma(q.z, A.cos_dt, q.w * sd), c0 = __builtin_fma(q.w, A.cos_dt, -(q.z * sd));
             const double s1 = __builtin_fma(q.z, A.cos_dt, -(q.w * sd)), c1 = __builtin_fma(q.w, A.cos_dt, q.z * sd);
@@ -644,20 +670,36 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             }
         }
         wave_sync();
-    };
-
-    // EXACT: the edge at place p
-    auto neighbour = [&](int p) -> int {
-        int r = 0;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const u64 m = __ballot(pos[c] == p);
-            if (m != 0ULL) r = 64 * c + __builtin_ctzll(m);
+        if constexpr (DIRECT) {
+            const int pair = lane >> 1;
+            if (lane < 32 && (b << kLog) + pair < deg) {
+                const lds_ptr<double2> o = rec + pair * 5;
+                const double2 t = direct_sincos((lane & 1) != 0 ? o[4].y : o[4].x);
+                o[2 + (lane & 1)].x = o[0].x * t.y;  // :730-733
+                o[2 + (lane & 1)].y = o[0].y * t.x;
+            }
+            wave_sync();
         }
-        return A.ids[base + r];
     };
 
-    int batch = -1;
+    // M_DIRECT: the transport sines of one group of pairs of the batch in LDS
+    const int slog = DIRECT ? direct_pairs_log(A.exact.kt) : 0;
+    const lds_ptr<double> sines = (lds_ptr<double>)(sl + cv.sines);
+    auto fill_sines = [&](int group) {
+        const int kt = A.exact.kt;
+        const int items = 2 * kt * min(1 << slog, deg - (group << slog));
+        const double th = uload(A.th + a);
+        wave_sync();  // the last group's reads are done
+#pragma unroll 1
+        for (int t = lane; t < items; t += 64) {
+            const int side = static_cast<int>((static_cast<float>(t) + 0.5f) * A.inv_kt);  // 2 pair + side
+            const lds_ptr<double2> o = rec + (((group << slog) + (side >> 1)) & kLast) * 5;
+            sines[t] = direct_sin(th + A.exact.off_t[t - side * kt] - ((side & 1) != 0 ? o[4].y : o[4].x));
+        }
+        wave_sync();
+    };
+
+    int batch = -1, group = -1;
     unsigned nacc = 0, vp = 0, isect_u = 0;  // isect_u: the wave's, isect: the lane's
     unsigned isect = 0;
     for (int run = 0; run < (CLASSES ? 3 : 2); ++run) {
@@ -712,6 +754,37 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                     any |= __builtin_amdgcn_ballot_w64(ok);
                 }
                 return any;
+            } else if constexpr (DIRECT) {
+                const double DX = q[0].x, DY = q[0].y, DX2 = q[1].x, DY2 = q[1].y;
+                const double cx0 = q[2].x, sy0 = q[2].y, cx1 = q[3].x, sy1 = q[3].y;
+                // the branches (:711-751, :774-806) differ in powers of two and
+                // in the angles' order
+                const bool branch_a = (DX * ca + DY * sa) < 0;
+                const double fn = branch_a ? 2.0 : 1.0;
+                const lds_ptr<double> sn = sines + 2 * A.exact.kt * (p & ((1 << slog) - 1));
+                u64 any = 0ULL;
+#pragma unroll
+                for (int m = 0; m < CPL; ++m) {
+                    const double ox = W.ox[m];
+                    const double tt = sT[m] * DX - cT[m] * DY;  // :705
+                    const double ttm = tt - ox;
+                    // (as exact_bound's)
+                    const double u = 2.0 * ox * tt - DX2 - DY2 + A.exact.dx2 - ox * ox;
+                    const double den = branch_a ? 0.0 - u : -u / 2.0;
+                    const double s0 = sn[W.j[m]], s1 = sn[W.j[m] + A.exact.kt];
+                    const double kx0 = fn * (ttm - A.exact.dx) / den, kx1 = fn * (ttm + A.exact.dx) / den;
+                    const double kt0 = s0 / (-s0 * ox + cx0 + sy0), kt1 = s1 / (-s1 * ox + cx1 + sy1);
+                    // the reference's compare-and-assign, which ignores NaN
+                    double lo = -A.exact.max_k, hi = A.exact.max_k;
+                    lo = lo < kx0 ? kx0 : lo;
+                    lo = lo < kt0 ? kt0 : lo;
+                    hi = hi > kx1 ? kx1 : hi;
+                    hi = hi > kt1 ? kt1 : hi;
+                    v[m].lo = lo;
+                    v[m].hi = hi;
+                    any |= __builtin_amdgcn_ballot_w64(hi > lo);
+                }
+                return any;
             } else {
                 const double DX = q[0].x, DY = q[0].y, r2 = q[1].x, C0 = q[1].y, C1 = q[2].x;
                 const double s0n = q[2].y, c0n = q[3].x, s1n = q[3].y, c1n = q[4].x;
@@ -737,9 +810,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                     int hi = min(fix(k1), fix(s1 * yd1));
                     const int t = min(sub_sat(hi, lo), min(sub_sat(hi, -kFixOne), sub_sat(kFixOne, lo)));
                     note(t);
-                    bool ok = t > kFixTol;
-                    u64 T = __builtin_amdgcn_ballot_w64(ok);
-                    u64 U = EXACT ? is_open(t) : 0ULL;
+                    const bool ok = t > kFixTol;
                     // a small denominator (then the product is small as well)
                     // settles nothing unless its sign is certain and its
                     // quotients lie well beyond max_k, where they stay either way
@@ -750,32 +821,24 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                         };
                         const bool bad = weak(x0, den) || weak(x0 + A.four_dx, den) ||
                                          weak(s0, d0) || weak(s1, d1);
-                        if (EXACT)
-                            U |= __builtin_amdgcn_ballot_w64(bad);
-                        else
-                            closest = bad ? 0u : closest;
-                    }
-                    if constexpr (EXACT) {
-                        if (U != 0ULL) {
-                            double elo, ehi;
-                            exact_set(m, U, 1, neighbour(p), elo, ehi);
-                            if (__builtin_amdgcn_inverse_ballot_w64(U)) {
-                                lo = fix(elo * A.scale);
-                                hi = max(fix(ehi * A.scale), lo + 1);
-                            }
-                            T = (T & ~U) | (__builtin_amdgcn_ballot_w64(ehi > elo) & U);
-                            ok = __builtin_amdgcn_inverse_ballot_w64(T);
-                        }
+                        closest = bad ? 0u : closest;
                     }
                     v[m].lo = ok ? lo : INT_MAX;
                     v[m].hi = ok ? hi : INT_MIN;
-                    any |= T;
+                    any |= __builtin_amdgcn_ballot_w64(ok);
                 }
                 return any;
             }
         };
         // (FAST's bounds are clamped by the comparisons)
-        const int def_lo = FLT ? float_key(-A.max_k_f) : -kFixOne, def_hi = FLT ? float_key(A.max_k_f) : kFixOne;
+        V def_lo, def_hi;
+        if constexpr (DIRECT) {
+            def_lo = -A.exact.max_k;
+            def_hi = A.exact.max_k;
+        } else {
+            def_lo = FLT ? float_key(-A.max_k_f) : -kFixOne;
+            def_hi = FLT ? float_key(A.max_k_f) : kFixOne;
+        }
 
         // the run's bundles, a batch of records at a time
         lds_ptr<Bounds> bp = bun;  // the next slot
@@ -784,7 +847,11 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 batch = p >> kLog;
                 fill_batch(batch);
             }
-            const int pe = min(p1, (p | kLast) + 1);
+            if (DIRECT && (p >> slog) != group) {
+                group = p >> slog;
+                fill_sines(group);
+            }
+            const int pe = min(p1, (DIRECT ? p | ((1 << slog) - 1) : p | kLast) + 1);
             lds_ptr<double2> q = rec + (p & kLast) * 5;
             if (!CLASSES && R + pe - p <= slots && ((closep[0] >> (p & 63)) & ((1ULL << (pe - p)) - 1ULL)) == 0ULL) {
                 // (most batches: no close pair, and slots for all)
@@ -853,37 +920,6 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 if ((pos[c] >> 6) == w) word = place[w];
             hyp[c] = __builtin_amdgcn_ballot_w64(pos[c] >= 0 && ((word >> (pos[c] & 63)) & 1ULL) != 0ULL);
         }
-        // EXACT: whether the running bundle of the slots in `set` is valid, in
-        // the lanes U of cell group m
-        auto exact_run = [&](int m, u64 U, const u64 (&set)[NW]) -> u64 {
-            int members = 0;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) members += __popcll(set[w]);
-            wave_sync();
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                if (!__builtin_amdgcn_inverse_ballot_w64(hyp[c])) continue;
-                int s = 0, rank = 0;  // the neighbour's slot, and its place among the members
-                u64 in = 0ULL;
-#pragma unroll
-                for (int w = 0; w < NW; ++w) {
-                    const int at = pos[c] - 64 * w;
-                    s += __popcll(at >= 64 ? place[w] : (at > 0 ? place[w] & ((1ULL << at) - 1ULL) : 0ULL));
-                }
-#pragma unroll
-                for (int w = 0; w < NW; ++w) {
-                    const int at = s - 64 * w;
-                    rank += __popcll(at >= 64 ? set[w] : (at > 0 ? set[w] & ((1ULL << at) - 1ULL) : 0ULL));
-                    in = (s >> 6) == w ? set[w] : in;
-                }
-                if ((in >> (s & 63)) & 1ULL) listed[rank] = A.ids[base + 64 * c + lane];
-            }
-            batch = -1;  // (the pair records are gone)
-            wave_sync();
-            double lo, hi;
-            exact_set(m, U, members, -1, lo, hi);
-            return __builtin_amdgcn_ballot_w64(hi > lo) & U;
-        };
         auto put_row = [&](unsigned rank, const u64 (&chain)[NW], int best, int seed) {
             const size_t q = static_cast<size_t>(base) + rank;
             if constexpr (FLT) {
@@ -953,8 +989,8 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             // the compatibility masks of every two slots: lane 8 i + k, the
             // cells where slots i and k are valid together
             Bounds b[kSmallRun][CPL];
+            u64 own[kSmallRun][CPL];  // M_DIRECT: the slots' own valid cells
             u64 P[CPL];
-            u64 redo = 0ULL;  // EXACT: bit 8 i + k: the pair has an open cell
 #pragma unroll
             for (int m = 0; m < CPL; ++m) P[m] = 0ULL;
             auto meet = [&](auto slot) -> bool {
@@ -965,40 +1001,27 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 for (int m = 0; m < CPL; ++m) {
                     b[i][m].lo = bun[(i * CPL + m) * 64].lo;
                     b[i][m].hi = bun[(i * CPL + m) * 64].hi;
-                    P[m] = set_lane64(P[m], __builtin_amdgcn_ballot_w64(b[i][m].hi > b[i][m].lo), 9 * i);
+                    own[i][m] = __builtin_amdgcn_ballot_w64(b[i][m].hi > b[i][m].lo);
+                    P[m] = set_lane64(P[m], own[i][m], 9 * i);
                 }
 #pragma unroll
                 for (int k = 0; k < i; ++k) {
 #pragma unroll
                     for (int m = 0; m < CPL; ++m) {
-                        const int t = min(sub_sat(b[k][m].hi, b[i][m].lo), sub_sat(b[i][m].hi, b[k][m].lo));
-                        if (EXACT)
-                            redo |= is_open(t) != 0ULL ? 1ULL << (8 * i + k) : 0ULL;
-                        else
+                        if constexpr (DIRECT) {
+                            const u64 both = __builtin_amdgcn_ballot_w64(b[k][m].hi > b[i][m].lo) &
+                                             __builtin_amdgcn_ballot_w64(b[i][m].hi > b[k][m].lo);
+                            P[m] = set_lane64(P[m], both & own[i][m] & own[k][m], 8 * i + k);
+                        } else {
+                            const int t = min(sub_sat(b[k][m].hi, b[i][m].lo), sub_sat(b[i][m].hi, b[k][m].lo));
                             note(t);
-                        P[m] = set_lane64(P[m], __builtin_amdgcn_ballot_w64(t > kTol), 8 * i + k);
+                            P[m] = set_lane64(P[m], __builtin_amdgcn_ballot_w64(t > kTol), 8 * i + k);
+                        }
                     }
                 }
                 return true;
             };
             each(meet, std::make_integer_sequence<int, kSmallRun>{});
-            if constexpr (EXACT) {
-                for (; redo != 0ULL; redo &= redo - 1ULL) {
-                    const int ik = __builtin_ctzll(redo), i = ik >> 3, k = ik & 7;
-                    u64 set[NW];
-#pragma unroll
-                    for (int w = 0; w < NW; ++w) set[w] = w == 0 ? 1ULL << i | 1ULL << k : 0ULL;
-#pragma unroll
-                    for (int m = 0; m < CPL; ++m) {
-                        const Bounds bi = get_bundle(i, m), bk = get_bundle(k, m);
-                        const int t = min(sub_sat(bk.hi, bi.lo), sub_sat(bi.hi, bk.lo));
-                        const u64 U = is_open(t);
-                        if (U != 0ULL)
-                            P[m] = set_lane64(P[m], (__builtin_amdgcn_ballot_w64(t > kTol) & ~U) | exact_run(m, U, set),
-                                              ik);
-                    }
-                }
-            }
             // the upper triangle, and the rows in LDS
             u64 C[CPL];
             wave_sync();  // (the last matrix's reads are done)
@@ -1081,6 +1104,12 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             continue;
         }
 
+        auto valid_lanes = [&](const Bounds &b) -> u64 {
+            if constexpr (DIRECT)
+                return __builtin_amdgcn_ballot_w64(b.hi > b.lo);
+            else
+                return __builtin_amdgcn_ballot_w64(sub_sat(b.hi, b.lo) > kTol);
+        };
         // longer runs: seed by seed, lane = cell: the running bundle over the
         // hypotheses in CSR order
         u64 sm[NC][NW];   // lane = seed (of chunk c): the chain's slots
@@ -1098,7 +1127,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             for (int m = 0; m < CPL; ++m) {
                 // (clamped at -+max_k)
                 cur[m] = get_bundle(j, m);
-                if (!FLT) {
+                if constexpr (MODE == M_FAST) {
                     cur[m].lo = max(cur[m].lo, -kFixOne);
                     cur[m].hi = min(cur[m].hi, kFixOne);
                 }
@@ -1113,27 +1142,16 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 u64 T = 0ULL;
 #pragma unroll
                 for (int m = 0; m < CPL; ++m) {
-                    n[m].lo = max(cur[m].lo, nx[m].lo);
-                    n[m].hi = min(cur[m].hi, nx[m].hi);
-                    T |= __builtin_amdgcn_ballot_w64(sub_sat(n[m].hi, n[m].lo) > kTol);
+                    n[m].lo = cur[m].lo < nx[m].lo ? nx[m].lo : cur[m].lo;
+                    n[m].hi = cur[m].hi > nx[m].hi ? nx[m].hi : cur[m].hi;
+                    T |= valid_lanes(n[m]);
                 }
                 const int hn = h + 1 < R ? h + 1 : h;
 #pragma unroll
                 for (int m = 0; m < CPL; ++m) nx[m] = get_bundle(hn, m);
-                if (T == 0ULL && h != j) {
-                    // (a step with a certainly valid cell is settled by it)
-                    if constexpr (EXACT) {
-                        u64 set[NW];
-#pragma unroll
-                        for (int w = 0; w < NW; ++w)
-                            set[w] = S[w] | ((h >> 6) == w ? 1ULL << (h & 63) : 0ULL) |
-                                     ((j >> 6) == w ? 1ULL << (j & 63) : 0ULL);
-#pragma unroll
-                        for (int m = 0; m < CPL; ++m) {
-                            const u64 U = is_open(sub_sat(n[m].hi, n[m].lo));
-                            if (U != 0ULL) T |= exact_run(m, U, set);
-                        }
-                    } else {
+                if constexpr (MODE == M_FAST) {
+                    if (T == 0ULL && h != j) {
+                        // (a step with a certainly valid cell is settled by it)
 #pragma unroll
                         for (int m = 0; m < CPL; ++m) note(sub_sat(n[m].hi, n[m].lo));
                     }
@@ -1149,19 +1167,8 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             }
 #pragma unroll
             for (int m = 0; m < CPL; ++m) {
-                const int t = sub_sat(cur[m].hi, cur[m].lo);
-                u64 T = __builtin_amdgcn_ballot_w64(t > kTol);
-                if constexpr (EXACT) {
-                    const u64 U = is_open(t);
-                    if (U != 0ULL) {
-                        u64 set[NW];
-#pragma unroll
-                        for (int w = 0; w < NW; ++w) set[w] = S[w] | ((j >> 6) == w ? 1ULL << (j & 63) : 0ULL);
-                        T = (T & ~U) | exact_run(m, U, set);
-                    }
-                } else {
-                    note(t);
-                }
+                if constexpr (MODE == M_FAST) note(sub_sat(cur[m].hi, cur[m].lo));
+                const u64 T = valid_lanes(cur[m]);
 #pragma unroll
                 for (int c = 0; c < NC; ++c)
                     if (NC == 1 || (j >> 6) == c) sM[c][m] = set_lane64(sM[c][m], T, j & 63);
@@ -1213,6 +1220,37 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
     return false;
 }
 
+// A wave's anchors for another list, kept in LDS and appended several at a
+// time: an atomic each, ~11 ns on the one counter, took 2 ms where most anchors
+// of a 1080p map were left open.
+struct LeftOpen {
+    const FusedArgs &A;
+    lds_ptr<int> buf;
+    int list, count = 0;
+    __device__ void put(int a)
+    {
+        if ((threadIdx.x & 63) == 0) buf[count] = a;
+        if (++count == kLeftOpen) flush();
+    }
+    __device__ void flush()
+    {
+        if (count == 0) return;
+        wave_sync();
+        const int lane = threadIdx.x & 63;
+        unsigned at = 0;
+        if (lane == 0) at = atomicAdd(A.list_len + list * kBucketStride, static_cast<unsigned>(count));
+        at = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(at)));
+        if (lane < count) {
+            const int a = buf[lane];
+            const unsigned o0 = A.off[a], o1 = A.off[a + 1];
+            A.lists[static_cast<size_t>(list) * A.n + at + lane] =
+                make_int4(a, static_cast<int>(o0), static_cast<int>(o1 - o0), 0);
+        }
+        wave_sync();
+        count = 0;
+    }
+};
+
 // One wave's sums into its place (k_record adds the places up).
 __device__ __forceinline__ void put_sums(unsigned *partial, int g, unsigned vp, unsigned long long isect)
 {
@@ -1240,6 +1278,7 @@ __device__ __forceinline__ WaveCells<CPL> wave_cells(const FusedArgs &A)
         W.ox2[m] = static_cast<double>(static_cast<float>(W.ox[m]) * static_cast<float>(W.ox[m]));
         W.oxp2[m] = 2.0 * (W.ox[m] + A.dx);
         W.ot[m] = A.rank_ot[r];
+        W.j[m] = A.rank_cell[r] % A.exact.kt;
         W.so[m] = A.rank_so[r];
         W.co[m] = A.rank_co[r];
         W.emask[m] = __ballot(live && A.rank_elig[r] != 0);
@@ -1281,7 +1320,7 @@ void k_curvelets(FusedArgs A)
     unsigned vp = 0;               // valid or close pairs of this wave's anchors
     unsigned long long isect = 0;  // bundle intersections the reference tests (per lane)
     char *sl = reinterpret_cast<char *>(lds) + static_cast<size_t>(wave) * slice_carve(A.slots, CPL).bytes;
-    int2 *spill = A.spill + static_cast<size_t>(g) * A.spill_stride;
+    char *spill = A.spill + static_cast<size_t>(g) * A.spill_stride;
     const WaveCells<CPL> W = wave_cells<CPL>(A);
 
     // the wave's entries: a cursor into the current list
@@ -1312,6 +1351,8 @@ void k_curvelets(FusedArgs A)
     double nth = load_th(id);
     if (deg >= 0) next(na, nbase, ndeg);
     int nid = load_id(nbase, ndeg);
+    LeftOpen open{A, (lds_ptr<int>)(sl + slice_carve(A.slots, CPL).left), L_OPEN};
+    int lead = -6;  // open anchors' lead over the others
     while (deg >= 0) {
         // start the next anchor's loads
         const double4 nnb = load_rec(nid);
@@ -1320,10 +1361,13 @@ void k_curvelets(FusedArgs A)
         unsigned nnbase = 0;
         if (ndeg >= 0) next(nna, nnbase, nndeg);
         const int nnid = load_id(nnbase, nndeg);
-        if (do_anchor<CPL, 1, FLT ? M_FLOAT : M_FAST>(A, W, sl, spill, a, base, deg, id, nb, nth, vp, isect)) {
-            if (lane == 0)
-                A.lists[static_cast<size_t>(L_OPEN) * A.n + atomicAdd(A.list_len + L_OPEN * kBucketStride, 1u)] =
-                    make_int4(a, static_cast<int>(base), deg, 0);
+        // (where most anchors turn out open, the rest go there at once: their
+        // work here would be done twice)
+        --lead;
+        if (lead >= 0 ||
+            do_anchor<CPL, 1, FLT ? M_FLOAT : M_FAST>(A, W, sl, spill, a, base, deg, id, nb, nth, vp, isect)) {
+            lead += 2;
+            open.put(a);
         }
         a = na;
         base = nbase;
@@ -1336,39 +1380,41 @@ void k_curvelets(FusedArgs A)
         ndeg = nndeg;
         nid = nnid;
     }
+    open.flush();
     put_sums(A.partial, g, vp, isect);
 }
 
-// The anchors of one list, with close comparisons made on the exact bounds:
-// those k_curvelets left open, or those of 65 to 256 neighbours.  One wave per
-// workgroup, at the registers the main kernel leaves on a SIMD, so that the
-// latter run beside it.
+// The anchors of one list on their own bounds: those k_curvelets left open
+// or those of 65 to 256 neighbours.  One wave per workgroup; the grid is what
+// stays resident, since on whole-pixel maps most anchors can be open, and waves
+// without an anchor leave at once (k_record adds up the others' sums).
 template <int CPL, int NW>
-__global__ __launch_bounds__(64, 4) void k_curvelets_exact(FusedArgs A, int list)
+__global__ __launch_bounds__(64, CPL == 1 ? 4 : 2) void k_curvelets_direct(FusedArgs A, int list)
 {
     extern __shared__ double lds[];
     const int lane = threadIdx.x & 63;
     const int g = static_cast<int>(blockIdx.x);
     const int total = static_cast<int>(uload(A.list_len + list * kBucketStride));
+    if (g >= total) return;
     unsigned vp = 0;
     unsigned long long isect = 0;
-    if (g < total) {
-        const WaveCells<CPL> W = wave_cells<CPL>(A);
-        int2 *spill = A.spill + static_cast<size_t>(g) * A.spill_stride;
-        for (int L = g; L < total; L += static_cast<int>(gridDim.x)) {
-            int a, deg;
-            unsigned base;
-            load_entry(A.lists + static_cast<size_t>(list) * A.n + L, a, base, deg);
-            double4 nb = make_double4(0.0, 0.0, 0.0, 1.0);
-            if (lane < deg) nb = A.rec[A.ids[base + lane]];
-            (void)do_anchor<CPL, NW, M_EXACT>(A, W, reinterpret_cast<char *>(lds), spill, a, base, deg, 0, nb, 0.0, vp, isect);
-        }
+    const WaveCells<CPL> W = wave_cells<CPL>(A);
+    char *spill = A.spill + static_cast<size_t>(g) * A.spill_stride;
+    for (int L = g; L < total; L += static_cast<int>(gridDim.x)) {
+        int a, deg;
+        unsigned base;
+        load_entry(A.lists + static_cast<size_t>(list) * A.n + L, a, base, deg);
+        const int id = lane < deg ? A.ids[base + lane] : -1;
+        const double4 nb = id >= 0 ? A.rec[id] : make_double4(0.0, 0.0, 0.0, 1.0);
+        const double nth = id >= 0 ? A.th[id] : 0.0;
+        (void)do_anchor<CPL, NW, M_DIRECT>(A, W, reinterpret_cast<char *>(lds), spill, a, base, deg, 0, nb, nth, vp,
+                                           isect);
     }
     put_sums(A.partial, g, vp, isect);
 }
 
-// Float maps: the anchors k_curvelets left open.  Those with a zero bound join
-// the wide ones, for the general kernel.
+// Float maps: the anchors k_curvelets left open.  Those with a zero bound or
+// denominator join the wide ones, for the general kernel.
 template <int CPL>
 __global__ __launch_bounds__(64, 4) void k_curvelets_float_open(FusedArgs A)
 {
@@ -1376,31 +1422,28 @@ __global__ __launch_bounds__(64, 4) void k_curvelets_float_open(FusedArgs A)
     const int lane = threadIdx.x & 63;
     const int g = static_cast<int>(blockIdx.x);
     const int total = static_cast<int>(uload(A.list_len + L_OPEN * kBucketStride));
+    if (g >= total) return;
     unsigned vp = 0;
     unsigned long long isect = 0;
-    if (g < total) {
-        const WaveCells<CPL> W = wave_cells<CPL>(A);
-        int2 *spill = A.spill + static_cast<size_t>(g) * A.spill_stride;
-        for (int L = g; L < total; L += static_cast<int>(gridDim.x)) {
-            int a, deg;
-            unsigned base;
-            load_entry(A.lists + static_cast<size_t>(L_OPEN) * A.n + L, a, base, deg);
-            const int id = lane < deg ? A.ids[base + lane] : -1;
-            const double4 nb = id >= 0 ? A.rec[id] : make_double4(0.0, 0.0, 0.0, 1.0);
-            const double nth = id >= 0 ? A.th[id] : 0.0;
-            if (do_anchor<CPL, 1, M_FLOAT_EXACT>(A, W, reinterpret_cast<char *>(lds), spill, a, base, deg, id, nb, nth, vp,
-                                                 isect)) {
-                if (lane == 0)
-                    A.lists[static_cast<size_t>(L_WIDE) * A.n + atomicAdd(A.list_len + L_WIDE * kBucketStride, 1u)] =
-                        make_int4(a, static_cast<int>(base), deg, 0);
-            }
-        }
+    const WaveCells<CPL> W = wave_cells<CPL>(A);
+    char *spill = A.spill + static_cast<size_t>(g) * A.spill_stride;
+    char *sl = reinterpret_cast<char *>(lds);
+    LeftOpen zero{A, (lds_ptr<int>)(sl + slice_carve(A.slots, CPL).left), L_WIDE};
+    for (int L = g; L < total; L += static_cast<int>(gridDim.x)) {
+        int a, deg;
+        unsigned base;
+        load_entry(A.lists + static_cast<size_t>(L_OPEN) * A.n + L, a, base, deg);
+        const int id = lane < deg ? A.ids[base + lane] : -1;
+        const double4 nb = id >= 0 ? A.rec[id] : make_double4(0.0, 0.0, 0.0, 1.0);
+        const double nth = id >= 0 ? A.th[id] : 0.0;
+        if (do_anchor<CPL, 1, M_FLOAT_EXACT>(A, W, sl, spill, a, base, deg, id, nb, nth, vp, isect)) zero.put(a);
     }
+    zero.flush();
     put_sums(A.partial, g, vp, isect);
 }
 
 using FusedKernel = void (*)(FusedArgs);
-using ExactKernel = void (*)(FusedArgs, int);
+using DirectKernel = void (*)(FusedArgs, int);
 
 // by cells per lane
 template <bool FLT>
@@ -1413,9 +1456,9 @@ inline FusedKernel float_open_kernel(int cpl)
     return cpl == 1 ? k_curvelets_float_open<1> : (cpl == 2 ? k_curvelets_float_open<2> : k_curvelets_float_open<4>);
 }
 template <int NW>
-inline ExactKernel exact_kernel(int cpl)
+inline DirectKernel direct_kernel(int cpl)
 {
-    return cpl == 1 ? k_curvelets_exact<1, NW> : (cpl == 2 ? k_curvelets_exact<2, NW> : k_curvelets_exact<4, NW>);
+    return cpl == 1 ? k_curvelets_direct<1, NW> : (cpl == 2 ? k_curvelets_direct<2, NW> : k_curvelets_direct<4, NW>);
 }
 
 #endif

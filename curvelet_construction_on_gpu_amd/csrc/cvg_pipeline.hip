@@ -26,9 +26,9 @@
 //           k_curvelets       one wave per anchor: bundles (lane = cell) from
 //                             certified approximations, chain growth, dedup,
 //                             staging rows (cvg_fused.hpp)
-//           k_curvelets_exact the same on exact bounds, for anchors whose
-//                             comparisons the approximations leave open and
-//                             those of more than 64 neighbours
+//           k_curvelets_direct  the same on the reference's own bounds, for
+//                             anchors whose comparisons the approximations
+//                             leave open and those of more than 64 neighbours
 //           scan              per-anchor accepted counts -> output row offsets,
 //                             and each row's anchor
 //           k_record          chain rows (1-based) and the 10 info columns
@@ -2176,20 +2176,32 @@ __device__ inline void record_row_fused(const RecordArgs &R, unsigned o, int a)
     write_info(R, o, ax, ay, at, (meta >> 8) & 1u, c, k_max, k_min, length, len);
 }
 
+// The fused kernels' per-wave sums: `main` of them, then `open` places of which
+// as many hold one as the open list has anchors, then the wide list's.
+struct FusedSums {
+    int main, open, wide;
+};
+
 // The run's counts into the scalars and to the host, by one workgroup: the row
 // count and, with partial, the fused kernels' per-wave sums (beside what
 // k_curvelets_generic counted of the same map).  (Adding those up with atomics
 // on one address would cost ~11 ns each, 45 us for 4,096 waves.)
-__device__ inline void finish_counts(unsigned rows, const unsigned *__restrict__ partial, int waves, unsigned *scal,
-                                     unsigned *mail)
+__device__ inline void finish_counts(unsigned rows, const unsigned *__restrict__ partial, FusedSums sums,
+                                     unsigned *scal, unsigned *mail)
 {
     unsigned long long vp = 0, is = 0;
-    if (partial)
-        for (int w = static_cast<int>(threadIdx.x); w < waves; w += kBlock) {
+    if (partial) {
+        const auto held = [&](int places, int list) {
+            return static_cast<int>(min(static_cast<unsigned>(places), scal[kBucketBase + list * kBucketStride]));
+        };
+        const int head = sums.main + held(sums.open, L_OPEN), waves = head + held(sums.wide, L_WIDE);
+        for (int i = static_cast<int>(threadIdx.x); i < waves; i += kBlock) {
+            const int w = i < head ? i : i - head + sums.main + sums.open;
             vp += partial[3 * w];
             is += static_cast<unsigned long long>(partial[3 * w + 1]) |
                   static_cast<unsigned long long>(partial[3 * w + 2]) << 32;
         }
+    }
     __shared__ unsigned long long s_vp[kBlock / 64], s_is[kBlock / 64];
     vp = wave_sum_u64(vp);
     is = wave_sum_u64(is);
@@ -2221,10 +2233,10 @@ enum { ROWS_FUSED = 0, ROWS_GENERAL = 1, ROWS_FLOAT = 2 };
 
 template <int KIND>
 __global__ __launch_bounds__(kBlock) void k_record(RecordArgs R, const int *__restrict__ row_anchor,
-                                                   const unsigned *__restrict__ partial, int waves, unsigned *scal,
-                                                   unsigned *mail)
+                                                   const unsigned *__restrict__ partial, FusedSums sums,
+                                                   unsigned *scal, unsigned *mail)
 {
-    if (blockIdx.x == 0) finish_counts(R.row_off[R.n], partial, waves, scal, mail);
+    if (blockIdx.x == 0) finish_counts(R.row_off[R.n], partial, sums, scal, mail);
     const unsigned rows = min(R.row_off[R.n], R.max_rows);
     const unsigned stride = gridDim.x * blockDim.x;
     for (unsigned o = blockIdx.x * blockDim.x + threadIdx.x; o < rows; o += stride) {
@@ -3392,12 +3404,12 @@ int finish_curvelets(cvg_context *ctx)
 
 // compact_curvelet_output + record_curvelet_chain (cpu_curvelet.hpp:258-303):
 // row offsets from the per-anchor accepted counts, then every accepted
-// staging row to its row (R carries the grid and info parameters; fused_waves:
-// the fused kernel's per-wave sums to add up), and the counts back with the
+// staging row to its row (R carries the grid and info parameters; sums:
+// the fused kernels' per-wave sums to add up), and the counts back with the
 // stream.  Outputs are sized by their bound (one row per
 // CSR pair at most), so the record runs without a host round trip; the
 // counts are read at the first query (finish_curvelets).
-int record_rows(cvg_context *ctx, const cvg_params &p, RecordArgs R, int st_stride, int fused_waves)
+int record_rows(cvg_context *ctx, const cvg_params &p, RecordArgs R, int st_stride, FusedSums sums)
 {
     hipStream_t st = ctx->stream;
     const int n = ctx->n;
@@ -3433,14 +3445,14 @@ int record_rows(cvg_context *ctx, const cvg_params &p, RecordArgs R, int st_stri
     R.info = out_info;
     if (pairs > 0) {
         // a resident grid strides over the rows (their count is on the device)
-        const auto rec = R.f32 ? k_record<ROWS_FLOAT> : (fused_waves > 0 ? k_record<ROWS_FUSED> : k_record<ROWS_GENERAL>);
+        const auto rec = R.f32 ? k_record<ROWS_FLOAT> : (sums.main > 0 ? k_record<ROWS_FUSED> : k_record<ROWS_GENERAL>);
         int occ = 0;
         CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(rec), kBlock, 0, &occ));
         const long long resident = static_cast<long long>(std::max(occ, 1)) * ctx->num_cu;
         const int grid = static_cast<int>(std::min(resident, static_cast<long long>(blocks_for(pairs))));
         hipLaunchKernelGGL(rec, dim3(grid), dim3(kBlock), 0, st, R, as<int>(ctx->d_rowanchor),
-                           static_cast<const unsigned *>(fused_waves > 0 ? as<unsigned>(ctx->d_partial) : nullptr),
-                           fused_waves, as<unsigned>(ctx->d_scal), ctx->mailbox);
+                           static_cast<const unsigned *>(sums.main > 0 ? as<unsigned>(ctx->d_partial) : nullptr),
+                           sums, as<unsigned>(ctx->d_scal), ctx->mailbox);
     }
     CVG_HIP(ctx, hipGetLastError());
     // (without pairs nothing was recorded: the scalars as they are)
@@ -3471,9 +3483,16 @@ struct FusedShape {
     FusedKernel fn;
     int slots;
     unsigned shmem;
-    size_t spill;
+    size_t spill;  // bytes per wave
     long long waves;
 };
+
+// Waves whose spill regions fit: the no-alloc scratch leaves 6 MiB.
+long long spill_fit(const cvg_context *ctx, size_t spill)
+{
+    const size_t room = ctx->arena ? size_t(6) << 20 : size_t(1) << 30;
+    return spill == 0 ? LLONG_MAX : std::max(1LL, static_cast<long long>(room / spill));
+}
 
 template <bool FLT>
 int fused_shape(cvg_context *ctx, int K, FusedShape *f)
@@ -3484,15 +3503,35 @@ int fused_shape(cvg_context *ctx, int K, FusedShape *f)
     f->shmem = static_cast<unsigned>(slice_carve(f->slots, cpl).bytes) * kFusedWaves;
     int occ = 0;
     CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(f->fn), 64 * kFusedWaves, f->shmem, &occ));
-    f->spill = static_cast<size_t>(std::max(0, static_cast<int>(std::min(ctx->max_deg, 64u)) - f->slots)) * cpl * 64;
+    f->spill = static_cast<size_t>(std::max(0, static_cast<int>(std::min(ctx->max_deg, 64u)) - f->slots)) * cpl * 64 *
+               sizeof(int2);
     long long blocks = static_cast<long long>(std::max(occ, 1)) * ctx->num_cu;
     if (ctx->grid_pct > 0) blocks = std::max(1LL, blocks * ctx->grid_pct / 100);
     blocks = std::min(blocks, (static_cast<long long>(ctx->n) + kFusedWaves - 1) / kFusedWaves);
-    // (the no-alloc scratch leaves a smaller grid's worth)
-    if (ctx->arena && f->spill > 0)
-        blocks = std::max(1LL, std::min(blocks, static_cast<long long>((size_t(6) << 20) / (f->spill * sizeof(int2))) /
-                                                    kFusedWaves));
+    blocks = std::max(1LL, std::min(blocks, spill_fit(ctx, f->spill) / kFusedWaves));
     f->waves = blocks * kFusedWaves;
+    return CVG_OK;
+}
+
+// The launch of k_curvelets_direct on lists of up to 64 NW neighbours.
+struct DirectShape {
+    DirectKernel fn;
+    unsigned shmem;
+    size_t spill;  // bytes per wave
+    long long waves;
+};
+
+template <int NW>
+int direct_shape(cvg_context *ctx, int cpl, int kt, DirectShape *f)
+{
+    f->fn = direct_kernel<NW>(cpl);
+    f->shmem = static_cast<unsigned>(direct_carve(kDirectSlots, cpl, kt).bytes);
+    int occ = 0;
+    CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(f->fn), 64, f->shmem, &occ));
+    f->spill = static_cast<size_t>(std::max(0, static_cast<int>(std::min(ctx->max_deg, 64u * NW)) - kDirectSlots)) *
+               cpl * 64 * sizeof(double2);
+    f->waves = std::min({static_cast<long long>(ctx->n), static_cast<long long>(std::max(occ, 1)) * ctx->num_cu,
+                         spill_fit(ctx, f->spill)});
     return CVG_OK;
 }
 
@@ -3630,8 +3669,12 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
     const size_t general_bytes = sb_elems * sizeof(T) + (sf_ints + sa_ints + sc_ints) * sizeof(int) + 512;
     FusedShape f{};
     if (fused) CVG_TRY(fused_shape<true>(ctx, K, &f));
-    const long long open_waves = fused ? std::min(f.waves, static_cast<long long>(ctx->num_cu)) : 0;
-    CVG_TRY(ensure(ctx, ctx->d_gbundle, std::max(general_bytes, f.spill * static_cast<size_t>(f.waves) * sizeof(int2))));
+    const FusedKernel open = float_open_kernel(K <= 64 ? 1 : (K <= 128 ? 2 : 4));
+    const unsigned slice = f.shmem / kFusedWaves;
+    int occ_open = 0;
+    if (fused) CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(open), 64, slice, &occ_open));
+    const long long open_waves = std::min(f.waves, static_cast<long long>(std::max(occ_open, 1)) * ctx->num_cu);
+    CVG_TRY(ensure(ctx, ctx->d_gbundle, std::max(general_bytes, f.spill * static_cast<size_t>(f.waves))));
     GenArgs<T> A{};
     A.n = n;
     A.x = as<double>(ctx->d_x);
@@ -3679,6 +3722,8 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
         M.rank_co = M.rank_so + K;
         M.rank_elig = reinterpret_cast<const int *>(tb + o_elig);
         M.rank_cell = A.rank_cell;
+        M.exact.kt = kt;
+        M.off = A.off;
         M.sin_dt = std::sin(static_cast<double>(dt));
         M.cos_dt = std::cos(static_cast<double>(dt));
         M.dx2 = A.dx2;
@@ -3695,15 +3740,12 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
         M.list_len = scal + kBucketBase;
         M.n = n;
         M.slots = f.slots;
-        M.spill = as<int2>(ctx->d_gbundle);
+        M.spill = as<char>(ctx->d_gbundle);
         M.spill_stride = f.spill;
         CVG_TRY(ensure(ctx, ctx->d_partial, static_cast<size_t>(f.waves + open_waves) * 3 * sizeof(unsigned)));
         M.partial = as<unsigned>(ctx->d_partial);
         hipLaunchKernelGGL(f.fn, dim3(static_cast<unsigned>(f.waves / kFusedWaves)), dim3(64 * kFusedWaves), f.shmem, st,
                            M);
-        const FusedKernel open = float_open_kernel(K <= 64 ? 1 : (K <= 128 ? 2 : 4));
-        const unsigned slice = f.shmem / kFusedWaves;
-        CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(open), 64, slice, nullptr));
         M.partial += 3 * f.waves;
         hipLaunchKernelGGL(open, dim3(static_cast<unsigned>(open_waves)), dim3(64), slice, st, M);
         A.list = M.lists + static_cast<size_t>(L_WIDE) * n;
@@ -3728,7 +3770,7 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
         R.off_x = reinterpret_cast<const double *>(tb + o_off_x);
         R.off_t = reinterpret_cast<const double *>(tb + o_off_t);
     }
-    return record_rows(ctx, p, R, cap, static_cast<int>(f.waves + open_waves));
+    return record_rows(ctx, p, R, cap, FusedSums{static_cast<int>(f.waves), static_cast<int>(open_waves), 0});
 }
 
 int build_curvelets(cvg_context *ctx, const cvg_params &p)
@@ -3779,6 +3821,7 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     FusedArgs A{};
     A.rec = as<double4>(ctx->d_rec);
     A.ids = as<int>(ctx->d_ids);
+    A.off = as<unsigned>(ctx->d_off);
     A.th = as<double>(ctx->d_th);
     A.K = static_cast<int>(d.K);
     A.G = static_cast<int>(d.G);
@@ -3787,6 +3830,7 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     A.rank_so = reinterpret_cast<const double *>(tb + o_rank_so);
     A.rank_co = reinterpret_cast<const double *>(tb + o_rank_co);
     A.rank_elig = reinterpret_cast<const int *>(tb + o_rank_elig);
+    A.rank_cell = reinterpret_cast<const int *>(tb + o_rank_cell);
     A.rank_of_cell0 = d.rank_of_cell0;
     A.four_dx = 4.0 * d.dx;
     A.max_k = d.max_k;
@@ -3813,53 +3857,47 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     // (a late one ends late, each has its share), and theirs take the place of
     // the first that end.  (Launched first they cost the 3840x2160 map's
     // k_curvelets 1,806 us against 1,566.)
+    A.exact.kt = static_cast<int>(d.kt);
+    A.inv_kt = 1.0f / static_cast<float>(d.kt);
     FusedShape f{};
+    DirectShape fo{}, fw{};
     CVG_TRY(fused_shape<false>(ctx, A.K, &f));
-    const ExactKernel fn_open = exact_kernel<1>(d.cpl), fn_wide = exact_kernel<4>(d.cpl);
-    A.slots = f.slots;
-    const unsigned slice = f.shmem / kFusedWaves;
-    int occ_wide = 0;
-    CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(fn_open), 64, slice, nullptr));
-    CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(fn_wide), 64, slice, &occ_wide));
-    const size_t spill_exact = static_cast<size_t>(std::max(0, static_cast<int>(ctx->max_deg) - A.slots)) * d.cpl * 64;
-    long long blocks_wide = wide ? std::min<long long>(n, static_cast<long long>(std::max(occ_wide, 1)) * ctx->num_cu) : 0;
-    long long blocks_open = std::min<long long>(n, ctx->num_cu);
-    if (ctx->arena && spill_exact > 0) {
-        const long long fit = static_cast<long long>((size_t(6) << 20) / (spill_exact * sizeof(int2)));
-        blocks_wide = std::min(blocks_wide, std::max(1LL, fit));
-        blocks_open = std::max(1LL, std::min(blocks_open, fit));
-    }
-    const int waves_main = static_cast<int>(f.waves);
-    const int waves = waves_main + static_cast<int>(blocks_wide + blocks_open);
-    CVG_TRY(ensure(ctx, ctx->d_gbundle, (std::max<size_t>(f.spill * waves_main, spill_exact * blocks_open) +
-                                         spill_exact * blocks_wide) * sizeof(int2)));
-    CVG_TRY(ensure(ctx, ctx->d_partial, static_cast<size_t>(waves) * 3 * sizeof(unsigned)));
+    CVG_TRY(direct_shape<1>(ctx, d.cpl, A.exact.kt, &fo));
+    if (wide) CVG_TRY(direct_shape<4>(ctx, d.cpl, A.exact.kt, &fw));
+    const FusedSums sums{static_cast<int>(f.waves), static_cast<int>(fo.waves), static_cast<int>(fw.waves)};
+    const size_t spill_wide = fw.spill * static_cast<size_t>(fw.waves);
+    CVG_TRY(ensure(ctx, ctx->d_gbundle, spill_wide + std::max(f.spill * static_cast<size_t>(f.waves),
+                                                              fo.spill * static_cast<size_t>(fo.waves))));
+    CVG_TRY(ensure(ctx, ctx->d_partial, static_cast<size_t>(f.waves + fo.waves + fw.waves) * 3 * sizeof(unsigned)));
     A.lists = as<int4>(ctx->d_lists);
     A.list_len = scal + kBucketBase;
     A.n = n;
-    FusedArgs X = A;  // the exact kernel's
+    FusedArgs X = A;  // the direct kernel's
+    X.slots = kDirectSlots;
+    A.slots = f.slots;
 
     const int ring = static_cast<int>(ctx->fused_runs % cvg_context::kFusedRing);
     CVG_TRY(record_timing(ctx, ctx->ev[3], st));
     CVG_TRY(record_timing(ctx, ctx->fused_ev[ring][0], st));
-    X.spill_stride = spill_exact;
     const hipEvent_t fork = ctx->timed_run ? ctx->ev[3] : ctx->ev_fork;
     if (wide && !ctx->timed_run) CVG_HIP(ctx, hipEventRecord(fork, st));
-    A.spill = as<int2>(ctx->d_gbundle) + spill_exact * blocks_wide;
+    A.spill = as<char>(ctx->d_gbundle) + spill_wide;
     A.spill_stride = f.spill;
-    A.partial = as<unsigned>(ctx->d_partial) + 3 * blocks_wide;
+    A.partial = as<unsigned>(ctx->d_partial);
     hipLaunchKernelGGL(f.fn, dim3(static_cast<unsigned>(f.waves / kFusedWaves)), dim3(64 * kFusedWaves), f.shmem, st, A);
     if (wide) {
         CVG_HIP(ctx, hipStreamWaitEvent(ctx->aux, fork, 0));
-        X.spill = as<int2>(ctx->d_gbundle);
-        X.partial = as<unsigned>(ctx->d_partial);
-        hipLaunchKernelGGL(fn_wide, dim3(static_cast<unsigned>(blocks_wide)), dim3(64), slice, ctx->aux, X,
+        X.spill = as<char>(ctx->d_gbundle);
+        X.spill_stride = fw.spill;
+        X.partial = A.partial + 3 * (f.waves + fo.waves);
+        hipLaunchKernelGGL(fw.fn, dim3(static_cast<unsigned>(fw.waves)), dim3(64), fw.shmem, ctx->aux, X,
                            static_cast<int>(L_WIDE));
         CVG_HIP(ctx, hipEventRecord(ctx->ev_join, ctx->aux));
     }
     X.spill = A.spill;
-    X.partial = A.partial + 3 * waves_main;
-    hipLaunchKernelGGL(fn_open, dim3(static_cast<unsigned>(blocks_open)), dim3(64), slice, st, X,
+    X.spill_stride = fo.spill;
+    X.partial = A.partial + 3 * f.waves;
+    hipLaunchKernelGGL(fo.fn, dim3(static_cast<unsigned>(fo.waves)), dim3(64), fo.shmem, st, X,
                        static_cast<int>(L_OPEN));
     CVG_HIP(ctx, hipGetLastError());
     if (wide) CVG_HIP(ctx, hipStreamWaitEvent(st, ctx->ev_join, 0));
@@ -3880,7 +3918,7 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     R.cos_dt = A.cos_dt;
     R.min_den = A.min_den;
     R.mask_plane = A.mask_plane;
-    return record_rows(ctx, p, R, 0, waves);
+    return record_rows(ctx, p, R, 0, sums);
 }
 
 bool same_params(const cvg_params &a, const cvg_params &b)

@@ -40,3 +40,34 @@ def test_graph_of_tied_distances(ctx, frame):
     apart = e.copy()
     apart[:, :2] += np.random.default_rng(1).uniform(-0.3, 0.3, (len(e), 2))
     assert shortest(ctx, e, p, "ms_graph") < 3.0 * shortest(ctx, apart, p, "ms_graph")
+
+
+def theta_zero(e):
+    e = on_pixels(e)
+    e[:, 2] = 0.0
+    return e
+
+
+def sixteen_thetas(e):
+    e = on_pixels(e)
+    e[:, 2] = np.rint(e[:, 2] / (np.pi / 8)) * (np.pi / 8)
+    return e
+
+
+@pytest.mark.parametrize("make,changes", [(theta_zero, {}), (sixteen_thetas, {}), (np.copy, {"max_k": 1e-3}),
+                                          (np.copy, {"max_k": 1e6})])
+def test_curvelets_of_open_anchors(ctx, frame, make, changes):
+    """Comparisons that the approximate bounds leave open, at most anchors.  256
+    waves, one for each of them at a time, took 8 to 85 times an ordinary map's time."""
+    ordinary = shortest(ctx, frame, CurveletParams(group_max_sz=7), "ms_curvelets")
+    assert shortest(ctx, make(frame), CurveletParams(group_max_sz=7, **changes), "ms_curvelets") < 6.0 * ordinary
+
+
+def test_float_curvelets_of_open_anchors(ctx, frame):
+    """Sines of exactly zero: 13 times an ordinary map's time before."""
+    p = CurveletParams()
+    e = np.ascontiguousarray(frame[::2], dtype=np.float32)
+    flat = e.copy()
+    flat[:, 2] = 0.0
+    run = lambda m: min(ctx.run_f32(m, p)["ms_curvelets"] for _ in range(7))
+    assert run(flat) < 6.0 * run(e)

@@ -154,6 +154,7 @@ _SIGNATURES = {
     "cvg_synth_preset": (C.c_int, [C.c_char_p, _P(_SynthConfig)]),
     "cvg_synth_generate": (C.c_int, [_P(_SynthConfig), C.c_ulonglong, _dp, C.c_int, _ip]),
     "cvg_debug_anchor_bundles": (C.c_int, [C.c_void_p, _P(_Params), C.c_int, _ucp, _ucp, _dp, _dp, _ip, _ip]),
+    "cvg_debug_route": (C.c_int, [C.c_void_p, _ip]),
     "cvg_math_eval": (C.c_int, [C.c_void_p, C.c_int, C.c_int, _dp, _dp, _dp]),
     "cvg_debug_cell_order": (C.c_int, [C.c_int, _dp, _dp, _ip]),
 }
@@ -492,6 +493,12 @@ class Context:
         self.check(self._lib.cvg_get_batch_map_curvelets(self._h, m, _ptr(chains, C.c_uint), _ptr(info, C.c_double)),
                    "get_batch_map_curvelets")
         return chains, info
+
+    def debug_route(self) -> str:
+        """The curvelet kernels the last run took: "fused", "direct" or "general"."""
+        r = C.c_int()
+        self.check(self._lib.cvg_debug_route(self._h, C.byref(r)), "debug_route")
+        return ("fused", "direct", "general")[r.value]
 
     def anchor_bundles(self, params: CurveletParams, anchor: int, max_deg: int):
         """Per-neighbour dir class, hypothesis flag and bundle cells of one anchor (device)."""

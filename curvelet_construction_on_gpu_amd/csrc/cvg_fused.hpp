@@ -282,13 +282,14 @@ __host__ __device__ inline SliceCarve slice_carve(int slots, int cpl)
     return c;
 }
 
-// The same with bounds in doubles, 16 pair records at a time, and the
-// transport sines of direct_pairs(kt) pairs.
+// The same with bounds in doubles, 16 pair records of 64 B at a time, and the
+// transport sines of a group of pairs, one to a lane as far as they go: at the
+// default grid 10,176 B, a sixteenth of a CU's.
 constexpr int kDirectSlots = 8;
 __host__ __device__ inline int direct_pairs_log(int kt)
 {
     int log = 4;
-    while (log > 0 && (2 * kt << log) > 128) --log;
+    while (log > 0 && (2 * kt << log) > 64) --log;
     return log;
 }
 __host__ __device__ inline SliceCarve direct_carve(int slots, int cpl, int kt)
@@ -296,7 +297,7 @@ __host__ __device__ inline SliceCarve direct_carve(int slots, int cpl, int kt)
     SliceCarve c{};
     c.bun = 0;
     c.rec = c.bun + slots * cpl * 64 * 16;
-    c.pm = c.rec + 16 * 80;
+    c.pm = c.rec + 16 * 64;
     c.sines = c.pm + 64 * cpl * 8;
     c.bytes = c.sines + (2 * kt << direct_pairs_log(kt)) * 8;
     return c;
@@ -483,9 +484,12 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
 #pragma unroll
     for (int m = 0; m < CPL; ++m) {
         if constexpr (DIRECT) {
-            const double2 t = direct_sincos(uload(A.th + a) + W.ot[m]);  // :702
-            sT[m] = t.x;
-            cT[m] = t.y;
+            sT[m] = cT[m] = 0.0;
+            if (A.exact.kt > 32) {  // (fewer: with the first pairs' below)
+                const double2 t = direct_sincos(uload(A.th + a) + W.ot[m]);  // :702
+                sT[m] = t.x;
+                cT[m] = t.y;
+            }
             continue;
         }
         sT[m] = __builtin_fma(sa, W.co[m], ca * W.so[m]);
@@ -640,16 +644,14 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             const double DX = ax - q.x, DY = ay - q.y;
             const bool branch_a = (DX * ca + DY * sa) < 0;  // :690
             if constexpr (DIRECT) {
-                // DX, DY, their squares, the angles; below: DX cos and DY sin
+                // DX, DY, the angles; below: DX cos and DY sin
                 if (pos[c] >= 0 && (pos[c] >> kLog) == b) {
                     const double th = c > 0 ? A.th[A.ids[base + 64 * c + lane]] : nth;
-                    const lds_ptr<double2> o = rec + (pos[c] & kLast) * 5;
+                    const lds_ptr<double2> o = rec + (pos[c] & kLast) * 4;
                     o[0].x = DX;
                     o[0].y = DY;
-                    o[1].x = DX * DX;
-                    o[1].y = DY * DY;
-                    o[4].x = branch_a ? th - A.exact.dt : th + A.exact.dt;
-                    o[4].y = branch_a ? th + A.exact.dt : th - A.exact.dt;
+                    o[3].x = branch_a ? th - A.exact.dt : th + A.exact.dt;
+                    o[3].y = branch_a ? th + A.exact.dt : th - A.exact.dt;
                 }
                 continue;
             }
@@ -671,12 +673,26 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
         }
         wave_sync();
         if constexpr (DIRECT) {
-            const int pair = lane >> 1;
-            if (lane < 32 && (b << kLog) + pair < deg) {
-                const lds_ptr<double2> o = rec + pair * 5;
-                const double2 t = direct_sincos((lane & 1) != 0 ? o[4].y : o[4].x);
-                o[2 + (lane & 1)].x = o[0].x * t.y;  // :730-733
-                o[2 + (lane & 1)].y = o[0].y * t.x;
+            // lanes 0-31: the batch's angles; 32 on: with the first batch, the
+            // anchor's with each offset (:702)
+            const int kt = A.exact.kt;
+            const bool mine = lane < 32 && (b << kLog) + (lane >> 1) < deg;
+            const bool with_t2 = b == 0 && kt <= 32;
+            const lds_ptr<double2> o = rec + (lane >> 1) * 4;
+            double x = 0.0;
+            if (mine) x = (lane & 1) != 0 ? o[3].y : o[3].x;
+            if (with_t2 && lane >= 32) x = uload(A.th + a) + A.exact.off_t[min(lane - 32, kt - 1)];
+            const double2 t = direct_sincos(x);
+            if (mine) {
+                o[1 + (lane & 1)].x = o[0].x * t.y;  // :730-733
+                o[1 + (lane & 1)].y = o[0].y * t.x;
+            }
+            if (with_t2) {
+#pragma unroll
+                for (int m = 0; m < CPL; ++m) {
+                    sT[m] = __shfl(t.x, 32 + W.j[m], 64);
+                    cT[m] = __shfl(t.y, 32 + W.j[m], 64);
+                }
             }
             wave_sync();
         }
@@ -693,8 +709,8 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
 #pragma unroll 1
         for (int t = lane; t < items; t += 64) {
             const int side = static_cast<int>((static_cast<float>(t) + 0.5f) * A.inv_kt);  // 2 pair + side
-            const lds_ptr<double2> o = rec + (((group << slog) + (side >> 1)) & kLast) * 5;
-            sines[t] = direct_sin(th + A.exact.off_t[t - side * kt] - ((side & 1) != 0 ? o[4].y : o[4].x));
+            const lds_ptr<double2> o = rec + (((group << slog) + (side >> 1)) & kLast) * 4;
+            sines[t] = direct_sin(th + A.exact.off_t[t - side * kt] - ((side & 1) != 0 ? o[3].y : o[3].x));
         }
         wave_sync();
     };
@@ -755,8 +771,8 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 }
                 return any;
             } else if constexpr (DIRECT) {
-                const double DX = q[0].x, DY = q[0].y, DX2 = q[1].x, DY2 = q[1].y;
-                const double cx0 = q[2].x, sy0 = q[2].y, cx1 = q[3].x, sy1 = q[3].y;
+                const double DX = q[0].x, DY = q[0].y, DX2 = DX * DX, DY2 = DY * DY;
+                const double cx0 = q[1].x, sy0 = q[1].y, cx1 = q[2].x, sy1 = q[2].y;
                 // the branches (:711-751, :774-806) differ in powers of two and
                 // in the angles' order
                 const bool branch_a = (DX * ca + DY * sa) < 0;
@@ -852,10 +868,11 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 fill_sines(group);
             }
             const int pe = min(p1, (DIRECT ? p | ((1 << slog) - 1) : p | kLast) + 1);
-            lds_ptr<double2> q = rec + (p & kLast) * 5;
+            constexpr int kRec = DIRECT ? 4 : 5;
+            lds_ptr<double2> q = rec + (p & kLast) * kRec;
             if (!CLASSES && R + pe - p <= slots && ((closep[0] >> (p & 63)) & ((1ULL << (pe - p)) - 1ULL)) == 0ULL) {
                 // (most batches: no close pair, and slots for all)
-                for (; p < pe; ++p, q += 5) {
+                for (; p < pe; ++p, q += kRec) {
                     Bounds v[CPL];
                     if (bundle(p, q, v) == 0ULL) continue;  // bundle_valid_check, :821-830
 #pragma unroll
@@ -869,7 +886,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 R = __popcll(place[0]);
                 continue;
             }
-            for (; p < pe; ++p, q += 5) {
+            for (; p < pe; ++p, q += kRec) {
                 bool close = false;
 #pragma unroll
                 for (int c = 0; c < NC; ++c)
@@ -959,6 +976,39 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                     o->y = chain[w];
                 }
             ((mem_ptr<unsigned>)A.st_meta)[q] = row_meta(best, run == 0, deg > 64, seed);
+            if constexpr (DIRECT) {
+                if (A.st_k == nullptr) return;  // (the record forms them)
+                // the running bundle at the best cell, the seed's first (:838-841)
+                const lds_ptr<Bounds> at = (lds_ptr<Bounds>)(sl + cv.bun) + best;
+                const mem_ptr<Bounds> far = (mem_ptr<Bounds>)spill + best;
+                double lo = 0.0, hi = 0.0;
+                int s = seed;
+                u64 set[NW];
+#pragma unroll
+                for (int w = 0; w < NW; ++w) set[w] = chain[w];
+                for (bool first = true;; first = false) {
+                    double l, h;
+                    if (s < slots) {
+                        l = at[s * CPL * 64].lo;
+                        h = at[s * CPL * 64].hi;
+                    } else {
+                        l = far[(s - slots) * CPL * 64].lo;
+                        h = far[(s - slots) * CPL * 64].hi;
+                    }
+                    lo = first || lo < l ? l : lo;
+                    hi = first || hi > h ? h : hi;
+                    s = -1;
+#pragma unroll
+                    for (int w = 0; w < NW; ++w)
+                        if (s < 0 && set[w] != 0ULL) {
+                            s = 64 * w + __builtin_ctzll(set[w]);
+                            set[w] &= set[w] - 1ULL;
+                        }
+                    if (s < 0) break;
+                }
+                ((mem_ptr<double>)A.st_k)[2 * q] = hi;
+                ((mem_ptr<double>)A.st_k)[2 * q + 1] = lo;
+            }
         };
         auto best_cell = [&](const u64 (&valid)[CPL]) -> int {  // fill_curvelet_info, :202-226
             int best = -1;
@@ -1384,31 +1434,70 @@ void k_curvelets(FusedArgs A)
     put_sums(A.partial, g, vp, isect);
 }
 
-// The anchors of one list on their own bounds: those k_curvelets left open
-// or those of 65 to 256 neighbours.  One wave per workgroup; the grid is what
-// stays resident, since on whole-pixel maps most anchors can be open, and waves
-// without an anchor leave at once (k_record adds up the others' sums).
+// A wave's entries of lists first .. last: numbers at, at + step, ... of their
+// concatenation.
+struct ListCursor {
+    const FusedArgs &A;
+    int list, last, left, at, step;
+    __device__ ListCursor(const FusedArgs &a, int first, int last_, int g, int step_)
+        : A(a), list(first - 1), last(last_), left(0), at(g), step(step_)
+    {
+    }
+    // deg = -1 at the end
+    __device__ __forceinline__ void next(int &a, unsigned &base, int &deg)
+    {
+        deg = -1;
+        while (at >= left) {
+            at -= left;
+            if (list == last) {
+                left = 0;
+                return;
+            }
+            ++list;
+            left = static_cast<int>(uload(A.list_len + list * kBucketStride));
+        }
+        load_entry(A.lists + static_cast<size_t>(list) * A.n + at, a, base, deg);
+        at += step;
+    }
+};
+
+// The anchors of some lists on their own bounds: those k_curvelets left open,
+// those of 65 to 256 neighbours, or all of a map that k_curvelets' error bound
+// does not cover.  One wave per workgroup; the grid is what stays resident, since
+// on whole-pixel maps most anchors can be open, and waves without an anchor leave
+// at once (k_record adds up the others' sums).  Bound by instruction issue: all
+// 207,326 anchors of the 1080p map take 1,090 us, 2,100 vector and 912 scalar
+// instructions each.  (Fourteen waves a CU in place of sixteen, with 80 B records
+// and 112 sines at a time, and the anchor's and pairs' sines in two calls: 1,370.
+// Quotients of one denominator on one refined reciprocal: 1,070.)
 template <int CPL, int NW>
-__global__ __launch_bounds__(64, CPL == 1 ? 4 : 2) void k_curvelets_direct(FusedArgs A, int list)
+__global__ __launch_bounds__(64, CPL == 1 ? 4 : 2) void k_curvelets_direct(FusedArgs A, int first, int last)
 {
     extern __shared__ double lds[];
     const int lane = threadIdx.x & 63;
     const int g = static_cast<int>(blockIdx.x);
-    const int total = static_cast<int>(uload(A.list_len + list * kBucketStride));
-    if (g >= total) return;
+    ListCursor entries(A, first, last, g, static_cast<int>(gridDim.x));
+    int a = 0, deg;
+    unsigned base = 0;
+    entries.next(a, base, deg);
+    if (deg < 0 && first == last) return;
     unsigned vp = 0;
     unsigned long long isect = 0;
     const WaveCells<CPL> W = wave_cells<CPL>(A);
     char *spill = A.spill + static_cast<size_t>(g) * A.spill_stride;
-    for (int L = g; L < total; L += static_cast<int>(gridDim.x)) {
-        int a, deg;
-        unsigned base;
-        load_entry(A.lists + static_cast<size_t>(list) * A.n + L, a, base, deg);
-        const int id = lane < deg ? A.ids[base + lane] : -1;
+    int id = lane < deg ? A.ids[base + lane] : -1;
+    while (deg >= 0) {
         const double4 nb = id >= 0 ? A.rec[id] : make_double4(0.0, 0.0, 0.0, 1.0);
         const double nth = id >= 0 ? A.th[id] : 0.0;
+        int na = 0, ndeg;
+        unsigned nbase = 0;
+        entries.next(na, nbase, ndeg);
+        id = lane < ndeg ? A.ids[nbase + lane] : -1;
         (void)do_anchor<CPL, NW, M_DIRECT>(A, W, reinterpret_cast<char *>(lds), spill, a, base, deg, 0, nb, nth, vp,
                                            isect);
+        a = na;
+        base = nbase;
+        deg = ndeg;
     }
     put_sums(A.partial, g, vp, isect);
 }
@@ -1443,7 +1532,7 @@ __global__ __launch_bounds__(64, 4) void k_curvelets_float_open(FusedArgs A)
 }
 
 using FusedKernel = void (*)(FusedArgs);
-using DirectKernel = void (*)(FusedArgs, int);
+using DirectKernel = void (*)(FusedArgs, int, int);
 
 // by cells per lane
 template <bool FLT>

@@ -183,6 +183,9 @@ private:
     }
 };
 
+// cvg_debug_route
+enum { ROUTE_FUSED = 0, ROUTE_DIRECT = 1, ROUTE_GENERAL = 2 };
+
 struct cvg_context {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -243,6 +246,7 @@ struct cvg_context {
     unsigned max_deg = 0;
     unsigned truncated = 0;
     unsigned ambiguous = 0;
+    int route = -1;  // the curvelet kernels of the last run (cvg_debug_route)
     unsigned wide_theta = 0;  // 1: some |theta| above kWideTheta, 3: above kMaxTheta
     int gx0 = 0, gy0 = 0, gw = 0, gh = 0;
     // d_grid's leading cell counts known to be zero (while d_grid is grid_zero_ptr)
@@ -854,8 +858,9 @@ constexpr int kBucketBase = 32;    // list b's length at [kBucketBase + b * kBuc
 constexpr int kScalarBufWords = kBucketBase + kMaxLists * kBucketStride;
 
 // Orientations the fused kernel's error bounds cover (fused_limits): up to the
-// second it allows for 64 times the rounding of the angles; maps with larger
-// ones take the general kernel.
+// second it allows for 64 times the rounding of the angles.  On maps with larger
+// ones every anchor takes its own bounds at once: 1.33 ms on the 1080p map
+// against 0.88 within the range (9.87 on the general kernel).
 constexpr double kWideTheta = 64.0, kMaxTheta = 4096.0;
 
 // Cells are (lrint(x), lrint(y)) (preprocess.hpp:85-86).  Coordinates must be
@@ -2011,7 +2016,9 @@ __device__ inline void record_row(const RecordArgs &R, unsigned o, int a)
 // (and the seed's) bundles at the best cell.  Approximate bounds (do_anchor's
 // formulas in doubles) say which member sets each, and only that one's exact
 // bound is formed; where two are closer than the approximation can tell, or
-// one lies at the clamp, every member's.
+// one lies at the clamp, every member's.  DIRECT (maps outside the approximation's
+// range): the kernel staged them.
+template <bool DIRECT>
 __device__ inline void record_row_fused(const RecordArgs &R, unsigned o, int a)
 {
     const unsigned base = R.off[a];
@@ -2026,8 +2033,8 @@ __device__ inline void record_row_fused(const RecordArgs &R, unsigned o, int a)
     const ExactGrid &E = R.exact;
     const double ox = E.off_x[c / R.kt];
     const double T2t = at + E.off_t[c % R.kt];
-    double s2, c2;
-    cvg::cr_sincos<false>(T2t, c_sincos_tab, &s2, &c2);
+    double s2 = 0.0, c2 = 0.0;
+    if (!DIRECT) cvg::cr_sincos<false>(T2t, c_sincos_tab, &s2, &c2);
 
     // the hypotheses in order, four loads at a time
     struct Slots {
@@ -2098,7 +2105,7 @@ __device__ inline void record_row_fused(const RecordArgs &R, unsigned o, int a)
                     ++len;
                     row[len] = static_cast<unsigned>(id[u] - id0) + 1;
                 }
-                if (DX * DX + DY * DY < E.close_thr) continue;  // the default bundle
+                if (DIRECT || DX * DX + DY * DY < E.close_thr) continue;  // (close: the default bundle)
                 const bool branch_a = (DX * ca + DY * sa) < 0;
                 const double sn = v[u].z, cn = v[u].w;
                 const double sd = branch_a ? -R.sin_dt : R.sin_dt;  // the lower constraint's theta_n -+ dt
@@ -2136,6 +2143,10 @@ __device__ inline void record_row_fused(const RecordArgs &R, unsigned o, int a)
     }
     for (int l = len; l < R.G; ++l) row[l + 1] = 0u;
 
+    if constexpr (DIRECT) {
+        write_info(R, o, ax, ay, at, (meta >> 8) & 1u, c, R.st_k[2 * q], R.st_k[2 * q + 1], length, len);
+        return;
+    }
     // each approximate bound is within max_k 2^-27 of the exact one
     double k_min = -E.max_k, k_max = E.max_k;
     const double tol = E.max_k * 0x1p-25;
@@ -2229,7 +2240,7 @@ __device__ inline void finish_counts(unsigned rows, const unsigned *__restrict__
 // (the offsets scan left each row's anchor).  The row count (the last row
 // offset) stays on the device, and rows beyond the caller's buffers are left
 // out (the host reports them).
-enum { ROWS_FUSED = 0, ROWS_GENERAL = 1, ROWS_FLOAT = 2 };
+enum { ROWS_FUSED = 0, ROWS_GENERAL = 1, ROWS_FLOAT = 2, ROWS_DIRECT = 3 };
 
 template <int KIND>
 __global__ __launch_bounds__(kBlock) void k_record(RecordArgs R, const int *__restrict__ row_anchor,
@@ -2240,8 +2251,8 @@ __global__ __launch_bounds__(kBlock) void k_record(RecordArgs R, const int *__re
     const unsigned rows = min(R.row_off[R.n], R.max_rows);
     const unsigned stride = gridDim.x * blockDim.x;
     for (unsigned o = blockIdx.x * blockDim.x + threadIdx.x; o < rows; o += stride) {
-        if constexpr (KIND == ROWS_FUSED)
-            record_row_fused(R, o, row_anchor[o]);
+        if constexpr (KIND == ROWS_FUSED || KIND == ROWS_DIRECT)
+            record_row_fused<KIND == ROWS_DIRECT>(R, o, row_anchor[o]);
         else
             record_row<KIND == ROWS_FLOAT>(R, o, row_anchor[o]);
     }
@@ -3445,7 +3456,9 @@ int record_rows(cvg_context *ctx, const cvg_params &p, RecordArgs R, int st_stri
     R.info = out_info;
     if (pairs > 0) {
         // a resident grid strides over the rows (their count is on the device)
-        const auto rec = R.f32 ? k_record<ROWS_FLOAT> : (sums.main > 0 ? k_record<ROWS_FUSED> : k_record<ROWS_GENERAL>);
+        const auto rec = R.f32 ? k_record<ROWS_FLOAT>
+                               : (sums.main == 0 ? k_record<ROWS_GENERAL>
+                                                 : (ctx->route == ROUTE_DIRECT ? k_record<ROWS_DIRECT> : k_record<ROWS_FUSED>));
         int occ = 0;
         CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(rec), kBlock, 0, &occ));
         const long long resident = static_cast<long long>(std::max(occ, 1)) * ctx->num_cu;
@@ -3638,6 +3651,7 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
     const bool fused = kFloat && G >= 3 && G <= 64 && ctx->max_deg <= 256 && !ctx->force_generic &&
                        float_limits(ctx, p.dx, p.max_k, off_x, off_t, dt) &&
                        *std::max_element(cell_rank.begin(), cell_rank.end()) < K;
+    ctx->route = fused ? ROUTE_FUSED : ROUTE_GENERAL;
     if (!fused) {
         ctx->setup_queued = false;
         CVG_HIP(ctx, hipMemsetAsync(scal + S_VALID, 0, (kScalarBufWords - S_VALID) * sizeof(unsigned), st));
@@ -3780,13 +3794,16 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     ctx->curvelets_ready = false;
     Derived d;
     CVG_TRY(derive(ctx, p, d));
-    // the fused kernel's masks hold up to 256 neighbours, and its error bound
-    // has a range; other maps take the general kernel
-    FusedLimits lim;
-    if (d.G > 64 || ctx->max_deg > 256 || ctx->force_generic || !fused_limits(ctx, d, &lim)) {
+    // the fused kernels' masks hold up to 256 neighbours; other maps take the
+    // general kernel.  The approximate bounds have a range; outside it every
+    // anchor takes its own bounds at once.
+    if (d.G > 64 || ctx->max_deg > 256 || ctx->force_generic) {
         ctx->setup_queued = false;
         return build_curvelets_generic<double>(ctx, p);
     }
+    FusedLimits lim{};
+    const bool approximate = fused_limits(ctx, d, &lim);
+    ctx->route = approximate ? ROUTE_FUSED : ROUTE_DIRECT;
     hipStream_t st = ctx->stream;
     const int n = ctx->n;
     const int pairs = ctx->pairs;
@@ -3850,6 +3867,10 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     A.mask_plane = np;
     A.st_meta = as<unsigned>(ctx->d_st_meta);
     A.acc_count = as<unsigned>(ctx->d_acc);
+    if (!approximate) {
+        CVG_TRY(ensure(ctx, ctx->d_st_k, np * 2 * sizeof(double)));
+        A.st_k = as<double>(ctx->d_st_k);
+    }
 
     // k_curvelets, then the anchors it leaves open; anchors of more than 64
     // neighbours, where the map has any, beside it on an auxiliary stream.
@@ -3864,11 +3885,13 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     CVG_TRY(fused_shape<false>(ctx, A.K, &f));
     CVG_TRY(direct_shape<1>(ctx, d.cpl, A.exact.kt, &fo));
     if (wide) CVG_TRY(direct_shape<4>(ctx, d.cpl, A.exact.kt, &fw));
-    const FusedSums sums{static_cast<int>(f.waves), static_cast<int>(fo.waves), static_cast<int>(fw.waves)};
+    if (!approximate) f = FusedShape{nullptr, 0, 0, fo.spill, fo.waves};  // (the direct kernel in its place)
+    const long long open_waves = approximate ? fo.waves : 0;
+    const FusedSums sums{static_cast<int>(f.waves), static_cast<int>(open_waves), static_cast<int>(fw.waves)};
     const size_t spill_wide = fw.spill * static_cast<size_t>(fw.waves);
     CVG_TRY(ensure(ctx, ctx->d_gbundle, spill_wide + std::max(f.spill * static_cast<size_t>(f.waves),
-                                                              fo.spill * static_cast<size_t>(fo.waves))));
-    CVG_TRY(ensure(ctx, ctx->d_partial, static_cast<size_t>(f.waves + fo.waves + fw.waves) * 3 * sizeof(unsigned)));
+                                                              fo.spill * static_cast<size_t>(open_waves))));
+    CVG_TRY(ensure(ctx, ctx->d_partial, static_cast<size_t>(f.waves + open_waves + fw.waves) * 3 * sizeof(unsigned)));
     A.lists = as<int4>(ctx->d_lists);
     A.list_len = scal + kBucketBase;
     A.n = n;
@@ -3884,21 +3907,31 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     A.spill = as<char>(ctx->d_gbundle) + spill_wide;
     A.spill_stride = f.spill;
     A.partial = as<unsigned>(ctx->d_partial);
-    hipLaunchKernelGGL(f.fn, dim3(static_cast<unsigned>(f.waves / kFusedWaves)), dim3(64 * kFusedWaves), f.shmem, st, A);
+    X.spill = A.spill;
+    X.spill_stride = fo.spill;
+    X.partial = A.partial;
+    if (approximate)
+        hipLaunchKernelGGL(f.fn, dim3(static_cast<unsigned>(f.waves / kFusedWaves)), dim3(64 * kFusedWaves), f.shmem, st,
+                           A);
+    else
+        hipLaunchKernelGGL(fo.fn, dim3(static_cast<unsigned>(fo.waves)), dim3(64), fo.shmem, st, X,
+                           static_cast<int>(L_FIRST), kLists - 1);
     if (wide) {
         CVG_HIP(ctx, hipStreamWaitEvent(ctx->aux, fork, 0));
         X.spill = as<char>(ctx->d_gbundle);
         X.spill_stride = fw.spill;
-        X.partial = A.partial + 3 * (f.waves + fo.waves);
+        X.partial = A.partial + 3 * (f.waves + open_waves);
         hipLaunchKernelGGL(fw.fn, dim3(static_cast<unsigned>(fw.waves)), dim3(64), fw.shmem, ctx->aux, X,
-                           static_cast<int>(L_WIDE));
+                           static_cast<int>(L_WIDE), static_cast<int>(L_WIDE));
         CVG_HIP(ctx, hipEventRecord(ctx->ev_join, ctx->aux));
     }
-    X.spill = A.spill;
-    X.spill_stride = fo.spill;
-    X.partial = A.partial + 3 * f.waves;
-    hipLaunchKernelGGL(fo.fn, dim3(static_cast<unsigned>(fo.waves)), dim3(64), fo.shmem, st, X,
-                       static_cast<int>(L_OPEN));
+    if (approximate) {
+        X.spill = A.spill;
+        X.spill_stride = fo.spill;
+        X.partial = A.partial + 3 * f.waves;
+        hipLaunchKernelGGL(fo.fn, dim3(static_cast<unsigned>(fo.waves)), dim3(64), fo.shmem, st, X,
+                           static_cast<int>(L_OPEN), static_cast<int>(L_OPEN));
+    }
     CVG_HIP(ctx, hipGetLastError());
     if (wide) CVG_HIP(ctx, hipStreamWaitEvent(st, ctx->ev_join, 0));
     CVG_TRY(record_timing(ctx, ctx->ev[4], st));
@@ -4759,6 +4792,15 @@ int cvg_synchronize(cvg_context *ctx)
 {
     CVG_TRY(check_ctx(ctx));
     CVG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return CVG_OK;
+}
+
+int cvg_debug_route(cvg_context *ctx, int *route)
+{
+    CVG_TRY(check_ctx(ctx));
+    if (!route) return fail(ctx, CVG_ERR_INVALID_ARGUMENT, "null route");
+    if (ctx->route < 0) return fail(ctx, CVG_ERR_STATE, "no curvelets");
+    *route = ctx->route;
     return CVG_OK;
 }
 

@@ -376,6 +376,13 @@ int cvg_synth_generate(const cvg_synth_config *config, unsigned long long seed, 
  * the direction filter (:459-461). */
 int cvg_debug_anchor_bundles(cvg_context *ctx, const cvg_params *params, int anchor, unsigned char *dir,
                              unsigned char *hyp, double *bmin, double *bmax, int *deg, int *cells);
+/* Which curvelet kernels the context's last run took: 0 the fused kernel on
+ * certified approximate bounds (anchors it leaves open on their own bounds), 1
+ * every anchor on its own bounds (orientations or parameters outside the
+ * approximation's range), 2 the general kernel (group_max_sz above 64, more
+ * than 256 neighbours; float maps outside the fused kernel's range).  Results
+ * never depend on it. */
+int cvg_debug_route(cvg_context *ctx, int *route);
 /* The within-cell order the library replays for order-ambiguous maps: for
  * each edge, its position inside its pixel cell after the reference's
  * std::sort of the edge ids by packed cell key (build_spatial_index_cpu,

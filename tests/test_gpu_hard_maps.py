@@ -71,3 +71,17 @@ def test_float_curvelets_of_open_anchors(ctx, frame):
     flat[:, 2] = 0.0
     run = lambda m: min(ctx.run_f32(m, p)["ms_curvelets"] for _ in range(7))
     assert run(flat) < 6.0 * run(e)
+
+
+def turned(e):
+    e = e.copy()
+    e[:, 2] += 2 * np.pi * 1000
+    return e
+
+
+@pytest.mark.parametrize("make,changes", [(turned, {}), (np.copy, {"max_k": 1e-6}), (np.copy, {"max_k": 0.0})])
+def test_curvelets_outside_the_approximations(ctx, frame, make, changes):
+    """Orientations and parameters that the approximate bounds do not cover: 11
+    to 18 times an ordinary map's time on the general kernel."""
+    ordinary = shortest(ctx, frame, CurveletParams(group_max_sz=7), "ms_curvelets")
+    assert shortest(ctx, make(frame), CurveletParams(group_max_sz=7, **changes), "ms_curvelets") < 6.0 * ordinary

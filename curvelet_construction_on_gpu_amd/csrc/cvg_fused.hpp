@@ -822,9 +822,12 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                     const double yd1 = y * pp, w = y * d1;
                     const double yd0 = w * den, yx = w * d0;
                     const double k0 = x0 * yx, k1 = __builtin_fma(A.four_dx, yx, k0);
-                    int lo = max(fix(k0), fix(s0 * yd0));
-                    int hi = min(fix(k1), fix(s1 * yd1));
-                    const int t = min(sub_sat(hi, lo), min(sub_sat(hi, -kFixOne), sub_sat(kFixOne, lo)));
+                    // (clamped to +-max_k as the reference's: a bundle beyond the
+                    // fixed-point range on both sides is not within the tolerance
+                    // of an invalid cell's values)
+                    const int lo = max(max(fix(k0), fix(s0 * yd0)), -kFixOne);
+                    const int hi = min(min(fix(k1), fix(s1 * yd1)), kFixOne);
+                    const int t = sub_sat(hi, lo);
                     note(t);
                     const bool ok = t > kFixTol;
                     // a small denominator (then the product is small as well)
@@ -846,7 +849,6 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 return any;
             }
         };
-        // (FAST's bounds are clamped by the comparisons)
         V def_lo, def_hi;
         if constexpr (DIRECT) {
             def_lo = -A.exact.max_k;
@@ -1175,12 +1177,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             Bounds cur[CPL], nx[CPL];
 #pragma unroll
             for (int m = 0; m < CPL; ++m) {
-                // (clamped at -+max_k)
                 cur[m] = get_bundle(j, m);
-                if constexpr (MODE == M_FAST) {
-                    cur[m].lo = max(cur[m].lo, -kFixOne);
-                    cur[m].hi = min(cur[m].hi, kFixOne);
-                }
                 nx[m] = get_bundle(0, m);
             }
             u64 S[NW];

@@ -85,3 +85,11 @@ def test_curvelets_outside_the_approximations(ctx, frame, make, changes):
     to 18 times an ordinary map's time on the general kernel."""
     ordinary = shortest(ctx, frame, CurveletParams(group_max_sz=7), "ms_curvelets")
     assert shortest(ctx, make(frame), CurveletParams(group_max_sz=7, **changes), "ms_curvelets") < 6.0 * ordinary
+
+
+@pytest.mark.parametrize("max_k", [0.02, 0.05, 0.1])
+def test_bounds_beyond_a_small_max_k(ctx, frame, max_k):
+    """Most bundles reach beyond max_k on both sides; none of those is close to
+    anything.  Their anchors were all left open: 2.5 times the ordinary time."""
+    ordinary = shortest(ctx, frame, CurveletParams(group_max_sz=7), "ms_curvelets")
+    assert shortest(ctx, frame, CurveletParams(group_max_sz=7, max_k=max_k), "ms_curvelets") < 1.5 * ordinary

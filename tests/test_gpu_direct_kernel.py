@@ -72,13 +72,13 @@ def test_mixed_orientations(both, oracle_cr, top):
     same_bits(both, oracle_cr, e, CurveletParams(group_max_sz=7))
 
 
-@pytest.mark.parametrize("dx,dt,max_k", [(0.4, 15.0, 1e-6), (0.4, 15.0, 0.0), (0.4, 15.0, -0.3), (0.0, 15.0, 0.3),
+@pytest.mark.parametrize("dx,dt,max_k", [(0.4, 15.0, 1e5), (0.4, 15.0, 0.0), (0.4, 15.0, -0.3), (0.0, 15.0, 0.3),
                                          (-0.02, 15.0, 0.3), (1e-70, 15.0, 0.3), (0.4, 600.0, 0.3)])
 def test_parameters(both, oracle_cr, dx, dt, max_k):
     rng = np.random.default_rng(7)
     e = np.stack([rng.uniform(0, 30, 500), rng.uniform(0, 30, 500), rng.uniform(-3, 3, 500), np.ones(500)], axis=1)
     e[1::25, :2] = e[::25, :2]  # some at the same place
-    e[:, 2] += FAR if dx >= 0.0 and dt < 100.0 and max_k > 1e-3 else 0.0
+    e[:, 2] += FAR if dx >= 0.0 and dt < 100.0 and 0.0 < max_k < 1.0 else 0.0
     same_bits(both, oracle_cr, e, CurveletParams(dx=dx, dt_deg=dt, max_k=max_k, st=0.08 if dt < 100.0 else 1.5))
 
 
@@ -86,8 +86,23 @@ def test_parameters(both, oracle_cr, dx, dt, max_k):
 def test_lattice(both, oracle_cr, angle):
     xs, ys = np.meshgrid(np.arange(12) * 1.0, np.arange(9) * 1.0)
     e = np.stack([xs.ravel(), ys.ravel(), np.full(xs.size, angle), np.ones(xs.size)], axis=1)
-    for max_k in (1e-6, 0.0):
+    for max_k in (1e5, 0.0):
         same_bits(both, oracle_cr, e, CurveletParams(max_k=max_k, group_max_sz=5))
+
+
+@pytest.mark.parametrize("max_k,turns,route", [(1e-9, 0, "fused"), (1e-6, 0, "fused"), (1e-3, 100, "fused"),
+                                               (0.05, 0, "fused"), (3000.0, 0, "fused"), (8000.0, 0, "direct"),
+                                               (0.3, 650, "fused"), (0.3, 653, "direct")])
+def test_where_the_route_changes(both, oracle_cr, max_k, turns, route):
+    """On either side of the approximate bounds' range, on a map and on a
+    lattice of it, whose bounds are often equal."""
+    rng = np.random.default_rng(11)
+    e = np.stack([rng.uniform(0, 30, 600), rng.uniform(0, 30, 600), rng.uniform(-3, 3, 600), np.ones(600)], axis=1)
+    q = np.unique(np.rint(e[:, :2]), axis=0)
+    lattice = np.concatenate([q, np.rint(e[:len(q), 2:3] * 4) / 4, np.ones((len(q), 1))], axis=1)
+    for m in (e, lattice):
+        m[:, 2] += 2 * np.pi * turns
+        same_bits(both, oracle_cr, m, CurveletParams(max_k=max_k, group_max_sz=5), route)
 
 
 @pytest.mark.parametrize("group", [4, 7])

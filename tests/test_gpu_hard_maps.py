@@ -93,3 +93,12 @@ def test_bounds_beyond_a_small_max_k(ctx, frame, max_k):
     anything.  Their anchors were all left open: 2.5 times the ordinary time."""
     ordinary = shortest(ctx, frame, CurveletParams(group_max_sz=7), "ms_curvelets")
     assert shortest(ctx, frame, CurveletParams(group_max_sz=7, max_k=max_k), "ms_curvelets") < 1.5 * ordinary
+
+
+@pytest.mark.parametrize("max_k", [1e-4, 1e5])
+def test_extreme_max_k(ctx, frame, max_k):
+    """Small: the approximate bounds still settle most anchors.  Large: their
+    units are too coarse, and the direct kernel takes all anchors at once."""
+    ordinary = shortest(ctx, frame, CurveletParams(group_max_sz=7), "ms_curvelets")
+    assert shortest(ctx, frame, CurveletParams(group_max_sz=7, max_k=max_k), "ms_curvelets") < 3.5 * ordinary
+    assert ctx.debug_route() == ("fused" if max_k < 1.0 else "direct")

@@ -1399,8 +1399,10 @@ void k_curvelets(FusedArgs A)
     if (deg >= 0) next(na, nbase, ndeg);
     int nid = load_id(nbase, ndeg);
     LeftOpen open{A, (lds_ptr<int>)(sl + slice_carve(A.slots, CPL).left), L_OPEN};
-    int lead = -6;  // open anchors' lead over the others
-    while (deg >= 0) {
+    // (where most anchors turn out open, the rest go there at once: their work
+    // here would be done twice)
+    int lead = -6;  // the open anchors' over the others
+    while (deg >= 0 && lead < 0) {
         // start the next anchor's loads
         const double4 nnb = load_rec(nid);
         const double nnth = load_th(nid);
@@ -1408,11 +1410,8 @@ void k_curvelets(FusedArgs A)
         unsigned nnbase = 0;
         if (ndeg >= 0) next(nna, nnbase, nndeg);
         const int nnid = load_id(nnbase, nndeg);
-        // (where most anchors turn out open, the rest go there at once: their
-        // work here would be done twice)
         --lead;
-        if (lead >= 0 ||
-            do_anchor<CPL, 1, FLT ? M_FLOAT : M_FAST>(A, W, sl, spill, a, base, deg, id, nb, nth, vp, isect)) {
+        if (do_anchor<CPL, 1, FLT ? M_FLOAT : M_FAST>(A, W, sl, spill, a, base, deg, id, nb, nth, vp, isect)) {
             lead += 2;
             open.put(a);
         }
@@ -1427,7 +1426,32 @@ void k_curvelets(FusedArgs A)
         ndeg = nndeg;
         nid = nnid;
     }
+    if (deg >= 0) open.put(a);
+    if (ndeg >= 0) open.put(na);
     open.flush();
+    while (ndeg >= 0) {
+        // the wave's next 64 entries, one to a lane
+        int l = list, rest = left;
+        long long i = at + static_cast<long long>(lane) * streams;
+        while (l < kLists && i >= rest) {
+            i -= rest;
+            ++l;
+            rest = l < kLists ? static_cast<int>(A.list_len[l * kBucketStride]) : 0;
+        }
+        const bool some = l < kLists;
+        const unsigned long long m = __ballot(some);
+        if (m == 0ULL) break;
+        unsigned to = 0;
+        if (lane == 0)
+            to = atomicAdd(A.list_len + L_OPEN * kBucketStride, static_cast<unsigned>(__popcll(m)));
+        to = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(to)));
+        if (some) A.lists[static_cast<size_t>(L_OPEN) * A.n + to + lane] = A.lists[static_cast<size_t>(l) * A.n + i];
+        if (m != ~0ULL) break;
+        // (on from the last lane's place)
+        list = __builtin_amdgcn_readlane(l, 63);
+        left = __builtin_amdgcn_readlane(rest, 63);
+        at = __builtin_amdgcn_readlane(static_cast<int>(i), 63) + streams;
+    }
     put_sums(A.partial, g, vp, isect);
 }
 

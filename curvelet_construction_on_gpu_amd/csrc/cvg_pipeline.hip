@@ -3269,7 +3269,8 @@ bool fused_limits(const cvg_context *ctx, const Derived &d, FusedLimits *lim)
     double S = 2.0 * (static_cast<double>(ctx->nbr_radius) + 1.0);
     if (ctx->rad >= 0.0) S = std::min(S, 1.5 * ctx->rad);
     const double B = S + d.dx + xmax;
-    if (!(d.dx >= 0.0) || !(d.max_k > 0.0) || !(tmax <= 8.0) || !(B <= 1e5) || ctx->wide_theta > 1) return false;
+    // (2^-100: kFixOne / max_k and its products with the quotients stay finite)
+    if (!(d.dx >= 0.0) || !(d.max_k >= 0x1p-100) || !(tmax <= 8.0) || !(B <= 1e5) || ctx->wide_theta > 1) return false;
     const double u = std::ldexp(ctx->wide_theta ? 64.0 : 1.0, -53);
     const double num = std::max(152.0 * B, 352.0) * u, den = std::max(64.0 * B * B, 360.0 * B) * u;
     lim->num_err = 4.0 * num;

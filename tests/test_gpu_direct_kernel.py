@@ -72,7 +72,8 @@ def test_mixed_orientations(both, oracle_cr, top):
     same_bits(both, oracle_cr, e, CurveletParams(group_max_sz=7))
 
 
-@pytest.mark.parametrize("dx,dt,max_k", [(0.4, 15.0, 1e5), (0.4, 15.0, 0.0), (0.4, 15.0, -0.3), (0.0, 15.0, 0.3),
+@pytest.mark.parametrize("dx,dt,max_k", [(0.4, 15.0, 1e5), (0.4, 15.0, np.inf), (0.4, 15.0, np.nan), (0.4, 15.0, 0.0),
+                                         (0.4, 15.0, -0.3), (0.0, 15.0, 0.3),
                                          (-0.02, 15.0, 0.3), (1e-70, 15.0, 0.3), (0.4, 600.0, 0.3)])
 def test_parameters(both, oracle_cr, dx, dt, max_k):
     rng = np.random.default_rng(7)
@@ -90,7 +91,8 @@ def test_lattice(both, oracle_cr, angle):
         same_bits(both, oracle_cr, e, CurveletParams(max_k=max_k, group_max_sz=5))
 
 
-@pytest.mark.parametrize("max_k,turns,route", [(1e-9, 0, "fused"), (1e-6, 0, "fused"), (1e-3, 100, "fused"),
+@pytest.mark.parametrize("max_k,turns,route", [(1e-305, 0, "direct"), (5e-31, 0, "direct"),
+                                               (1e-30, 0, "fused"), (1e-9, 0, "fused"), (1e-6, 0, "fused"), (1e-3, 100, "fused"),
                                                (0.05, 0, "fused"), (3000.0, 0, "fused"), (8000.0, 0, "direct"),
                                                (0.3, 650, "fused"), (0.3, 653, "direct")])
 def test_where_the_route_changes(both, oracle_cr, max_k, turns, route):

@@ -1,0 +1,103 @@
+"""Where the fused kernels' error bounds and buffers are nearest to their
+limits, bit for bit against the oracle with correctly rounded sin/cos:
+neighbours at opposite ends of the orientations' range (the differences of the
+angles round the most there), runs that just fill the twelve bundle slots in
+LDS, the general kernel on a nearly full no-alloc scratch array, and launch
+shapes.  There is no tolerance."""
+import numpy as np
+import pytest
+
+from curvelet_construction_on_gpu_amd import Context, CurveletParams
+from oracle import OracleF32
+from tests._inputs import edges_for
+from tests.test_gpu_fused_kernel import lines
+from tests.test_zz_no_alloc import bits, noalloc, pooled
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    return Context()
+
+
+def check(ctx, want, stats, route):
+    chains, info = ctx.curvelets()
+    assert ctx.debug_route() == route
+    assert stats["valid_pairs"] == want["valid_pairs"]
+    assert np.array_equal(chains, want["chains"])
+    assert np.array_equal(info.view(np.uint64), want["info"].view(np.uint64))
+
+
+def alternating(e, top):
+    """Whole turns up to +top and down to -top, from edge to edge."""
+    e = e.copy()
+    e[::2, 2] += 2 * np.pi * np.floor((top - np.abs(e[:, 2]).max()) / (2 * np.pi))
+    e[1::2, 2] -= 2 * np.pi * np.floor((top - np.abs(e[:, 2]).max()) / (2 * np.pi))
+    return e
+
+
+def scene(kind):
+    if kind == "lines":
+        return lines(9, seed=5)
+    if kind == "map":
+        return np.array(edges_for("synth:C1:1001"))
+    xs, ys = np.meshgrid(np.arange(14) * 1.0, np.arange(11) * 1.0)
+    th = np.random.default_rng(2).integers(0, 16, xs.size) * (np.pi / 8)
+    return np.stack([xs.ravel(), ys.ravel(), th, np.ones(xs.size)], axis=1)
+
+
+@pytest.mark.parametrize("kind", ["lines", "map", "lattice"])
+@pytest.mark.parametrize("top", [64.0, 4096.0])
+def test_opposite_orientations(ctx, oracle_cr, kind, top):
+    e = alternating(scene(kind), top)
+    assert 0.8 * top < np.abs(e[:, 2]).max() <= top
+    p = CurveletParams(group_max_sz=7)
+    check(ctx, oracle_cr.run(e, p), ctx.run(e, p), "fused")
+
+
+@pytest.mark.parametrize("kind", ["lines", "map", "lattice"])
+def test_float_opposite_orientations(ctx, kind):
+    e = alternating(scene(kind), 63.9).astype(np.float32)
+    p = CurveletParams(group_max_sz=7)
+    check(ctx, OracleF32(cr=True).run(e, p), ctx.run_f32(e, p), "fused")
+
+
+@pytest.mark.parametrize("group", [3, 7, 12, 13, 14])
+@pytest.mark.parametrize("run", [11, 12, 13])
+def test_runs_that_fill_the_slots(ctx, oracle_cr, run, group):
+    e = lines(run, seed=run)
+    p = CurveletParams(group_max_sz=group, max_candidates=256)
+    check(ctx, oracle_cr.run(e, p), ctx.run(e, p), "fused")
+    f = e.astype(np.float32)
+    check(ctx, OracleF32(cr=True).run(f, p), ctx.run_f32(f, p), "fused")
+
+
+@pytest.mark.parametrize("group", [4, 7])
+def test_noalloc_on_the_general_kernel(group, monkeypatch):
+    """Its per-wave buffers are made for device memory; on this map they do not
+    fit the scratch array, and the grid is what the array has left."""
+    monkeypatch.setenv("CVG_GENERIC_KERNEL", "1")
+    e = np.array(edges_for("synth:C1:1001"))
+    p = CurveletParams(group_max_sz=group)
+    with Context(0) as general:
+        want_c, want_i, want_v = pooled(general, e, p)
+        got_c, got_i, got_v = noalloc(general, e, p, len(want_c) + 3)
+        assert general.debug_route() == "general"
+    assert got_v == want_v
+    assert np.array_equal(got_c, want_c)
+    assert np.array_equal(bits(got_i), bits(want_i))
+
+
+@pytest.mark.parametrize("lanes", [8, 16, 32, 64])
+@pytest.mark.parametrize("pct", [5, 40, 0])
+def test_launch_shapes(oracle_cr, lanes, pct, monkeypatch):
+    """Lanes per anchor in the window scans, and the curvelet grid down to one
+    wave to many anchors (0: automatic)."""
+    monkeypatch.setenv("CVG_FILL_LANES", str(lanes))
+    monkeypatch.setenv("CVG_GRID_PCT", str(pct))
+    e = np.array(edges_for("synth:C1:1001"))
+    p = CurveletParams(group_max_sz=5)
+    with Context(0) as shaped:
+        for _ in range(2):  # the second run is on guessed sizes
+            check(shaped, oracle_cr.run(e, p), shaped.run(e, p), "fused")

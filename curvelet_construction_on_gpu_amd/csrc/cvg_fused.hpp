@@ -115,6 +115,17 @@ __global__ __launch_bounds__(kBlock) void k_edge_rec(int n, const double *__rest
 constexpr int kOrderBlock = 1024;  // few workgroups: one list-length atomic each per list
 enum { L_OPEN = 0, L_WIDE = 1, L_FIRST = 2, kLists = 16 };
 
+// The open list has n places, and so has the wide one, last (a double map
+// without lists of more than 64 does not use it).  An anchor is in one degree
+// list, so two of those share n, one from the front and one from the back.
+constexpr int kListRegions = L_FIRST + (kLists - L_FIRST) / 2;
+__host__ __device__ __forceinline__ long long entry_place(int list, long long i, int n)
+{
+    const int region = list == L_OPEN ? 0 : (list == L_WIDE ? kListRegions - 1 : 1 + (list - L_FIRST) / 2);
+    const bool back = list > L_FIRST && ((list - L_FIRST) & 1) != 0;
+    return static_cast<long long>(region) * n + (back ? n - 1 - i : i);
+}
+
 __device__ __forceinline__ int degree_list(unsigned deg)
 {
     constexpr unsigned kAbove[kLists - 1 - L_FIRST] = {48, 40, 32, 28, 24, 20, 17, 14, 12, 10, 8, 6, 4};
@@ -156,7 +167,7 @@ __global__ __launch_bounds__(kOrderBlock) void k_order(int n, const int *__restr
         s_base[threadIdx.x] = atomicAdd(&scal[kBucketBase + threadIdx.x * kBucketStride], s_count[threadIdx.x]);
     __syncthreads();
     if (b >= 0)
-        lists[static_cast<long long>(b) * n + s_base[b] + my_off] =
+        lists[entry_place(b, static_cast<long long>(s_base[b]) + my_off, n)] =
             make_int4(a, static_cast<int>(o0), static_cast<int>(o1 - o0), 0);
 }
 
@@ -222,7 +233,7 @@ struct FusedArgs {
     ExactGrid exact;
     const int *ids;
     const unsigned *off;  // CSR offsets
-    int4 *lists;         // kLists x n entries (anchor, CSR base, degree, -)
+    int4 *lists;         // (anchor, CSR base, degree, -), at entry_place
     unsigned *list_len;  // entry counts, kBucketStride words apart (device; k_order's, and the open list's)
     int n;
     int K, G;
@@ -1290,7 +1301,7 @@ struct LeftOpen {
         if (lane < count) {
             const int a = buf[lane];
             const unsigned o0 = A.off[a], o1 = A.off[a + 1];
-            A.lists[static_cast<size_t>(list) * A.n + at + lane] =
+            A.lists[entry_place(list, static_cast<long long>(at) + lane, A.n)] =
                 make_int4(a, static_cast<int>(o0), static_cast<int>(o1 - o0), 0);
         }
         wave_sync();
@@ -1380,7 +1391,7 @@ void k_curvelets(FusedArgs A)
             ++list;
             left = static_cast<int>(uload(A.list_len + list * kBucketStride));
         }
-        load_entry(A.lists + static_cast<size_t>(list) * A.n + at, ea, eb, ed);
+        load_entry(A.lists + entry_place(list, at, A.n), ea, eb, ed);
         at += streams;
     };
     auto load_id = [&](unsigned b0, int d0) -> int { return lane < d0 ? A.ids[b0 + lane] : -1; };
@@ -1445,7 +1456,7 @@ void k_curvelets(FusedArgs A)
         if (lane == 0)
             to = atomicAdd(A.list_len + L_OPEN * kBucketStride, static_cast<unsigned>(__popcll(m)));
         to = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(to)));
-        if (some) A.lists[static_cast<size_t>(L_OPEN) * A.n + to + lane] = A.lists[static_cast<size_t>(l) * A.n + i];
+        if (some) A.lists[entry_place(L_OPEN, static_cast<long long>(to) + lane, A.n)] = A.lists[entry_place(l, i, A.n)];
         if (m != ~0ULL) break;
         // (on from the last lane's place)
         list = __builtin_amdgcn_readlane(l, 63);
@@ -1477,7 +1488,7 @@ struct ListCursor {
             ++list;
             left = static_cast<int>(uload(A.list_len + list * kBucketStride));
         }
-        load_entry(A.lists + static_cast<size_t>(list) * A.n + at, a, base, deg);
+        load_entry(A.lists + entry_place(list, at, A.n), a, base, deg);
         at += step;
     }
 };
@@ -1542,7 +1553,7 @@ __global__ __launch_bounds__(64, 4) void k_curvelets_float_open(FusedArgs A)
     for (int L = g; L < total; L += static_cast<int>(gridDim.x)) {
         int a, deg;
         unsigned base;
-        load_entry(A.lists + static_cast<size_t>(L_OPEN) * A.n + L, a, base, deg);
+        load_entry(A.lists + entry_place(L_OPEN, L, A.n), a, base, deg);
         const int id = lane < deg ? A.ids[base + lane] : -1;
         const double4 nb = id >= 0 ? A.rec[id] : make_double4(0.0, 0.0, 0.0, 1.0);
         const double nth = id >= 0 ? A.th[id] : 0.0;

@@ -3226,7 +3226,9 @@ int queue_setup(cvg_context *ctx)
 {
     const int n = ctx->n;
     CVG_TRY(ensure(ctx, ctx->d_rec, static_cast<size_t>(n) * sizeof(double4)));
-    CVG_TRY(ensure(ctx, ctx->d_lists, static_cast<size_t>(kLists) * n * sizeof(int4)));
+    // (the no-alloc scratch has the degrees by now, and no float maps)
+    const int regions = ctx->arena && ctx->max_deg <= 64 ? kListRegions - 1 : kListRegions;
+    CVG_TRY(ensure(ctx, ctx->d_lists, static_cast<size_t>(regions) * n * sizeof(int4)));
     CVG_TRY(ensure(ctx, ctx->d_acc, static_cast<size_t>(n) * sizeof(unsigned)));
     hipLaunchKernelGGL(k_edge_rec, dim3(blocks_for(n)), dim3(kBlock), 0, ctx->stream, n, as<double>(ctx->d_x),
                        as<double>(ctx->d_y), as<double>(ctx->d_th), as<double4>(ctx->d_rec),
@@ -3768,7 +3770,7 @@ int build_curvelets_generic(cvg_context *ctx, const cvg_params &p)
                            M);
         M.partial += 3 * f.waves;
         hipLaunchKernelGGL(open, dim3(static_cast<unsigned>(open_waves)), dim3(64), slice, st, M);
-        A.list = M.lists + static_cast<size_t>(L_WIDE) * n;
+        A.list = M.lists + entry_place(L_WIDE, 0, n);
         A.list_len = M.list_len + L_WIDE * kBucketStride;
     }
     hipLaunchKernelGGL(k_curvelets_generic<T>, dim3(blocks), dim3(64 * kGenWaves), 0, st, A);

@@ -3537,6 +3537,7 @@ int fused_shape(cvg_context *ctx, int K, FusedShape *f)
 // The launch of k_curvelets_direct on lists of up to 64 NW neighbours.
 struct DirectShape {
     DirectKernel fn;
+    int slots;  // bundle slots in LDS
     unsigned shmem;
     size_t spill;  // bytes per wave
     long long waves;
@@ -3546,10 +3547,17 @@ template <int NW>
 int direct_shape(cvg_context *ctx, int cpl, int kt, DirectShape *f)
 {
     f->fn = direct_kernel<NW>(cpl);
-    f->shmem = static_cast<unsigned>(direct_carve(kDirectSlots, cpl, kt).bytes);
+    // Sixteen waves a CU leave room for eight slots (at one cell per lane).  Maps
+    // with fewer anchors than four a CU take as many as their lists are long, up
+    // to 32 KB: a spill region of 4 MB, allocated for a hundred edges, was 30 us
+    // of a new context's first run.
+    f->slots = kDirectSlots;
+    if (ctx->n <= 4 * ctx->num_cu)
+        f->slots = std::max(kDirectSlots, std::min(static_cast<int>(std::min(ctx->max_deg, 64u * NW)), 32 / cpl));
+    f->shmem = static_cast<unsigned>(direct_carve(f->slots, cpl, kt).bytes);
     int occ = 0;
     CVG_TRY(prepare_launch(ctx, reinterpret_cast<const void *>(f->fn), 64, f->shmem, &occ));
-    f->spill = static_cast<size_t>(std::max(0, static_cast<int>(std::min(ctx->max_deg, 64u * NW)) - kDirectSlots)) *
+    f->spill = static_cast<size_t>(std::max(0, static_cast<int>(std::min(ctx->max_deg, 64u * NW)) - f->slots)) *
                cpl * 64 * sizeof(double2);
     f->waves = std::min({static_cast<long long>(ctx->n), static_cast<long long>(std::max(occ, 1)) * ctx->num_cu,
                          spill_fit(ctx, f->spill)});
@@ -3904,7 +3912,6 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     A.list_len = scal + kBucketBase;
     A.n = n;
     FusedArgs X = A;  // the direct kernel's
-    X.slots = kDirectSlots;
     A.slots = f.slots;
 
     const int ring = static_cast<int>(ctx->fused_runs % cvg_context::kFusedRing);
@@ -3915,6 +3922,7 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     A.spill = as<char>(ctx->d_gbundle) + spill_wide;
     A.spill_stride = f.spill;
     A.partial = as<unsigned>(ctx->d_partial);
+    X.slots = fo.slots;
     X.spill = A.spill;
     X.spill_stride = fo.spill;
     X.partial = A.partial;
@@ -3926,6 +3934,7 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
                            static_cast<int>(L_FIRST), kLists - 1);
     if (wide) {
         CVG_HIP(ctx, hipStreamWaitEvent(ctx->aux, fork, 0));
+        X.slots = fw.slots;
         X.spill = as<char>(ctx->d_gbundle);
         X.spill_stride = fw.spill;
         X.partial = A.partial + 3 * (f.waves + open_waves);
@@ -3934,6 +3943,7 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
         CVG_HIP(ctx, hipEventRecord(ctx->ev_join, ctx->aux));
     }
     if (approximate) {
+        X.slots = fo.slots;
         X.spill = A.spill;
         X.spill_stride = fo.spill;
         X.partial = A.partial + 3 * f.waves;

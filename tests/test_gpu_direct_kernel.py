@@ -52,6 +52,17 @@ def test_run_lengths(both, oracle_cr, run, group):
     same_bits(both, oracle_cr, e, CurveletParams(group_max_sz=group, max_candidates=256))
 
 
+@pytest.mark.parametrize("group", [4, 9])
+@pytest.mark.parametrize("run", [7, 8, 9, 16, 17, 40, 65, 100])
+def test_run_lengths_on_larger_maps(both, oracle_cr, run, group):
+    """More than four anchors a CU: eight slots in LDS, the other bundles in
+    device memory (smaller maps have slots for whole lists)."""
+    e = lines(run, seed=run, rows=2100 // (2 * run + 3))
+    e[:, 2] += FAR
+    assert len(e) > 1900
+    same_bits(both, oracle_cr, e, CurveletParams(group_max_sz=group, max_candidates=256))
+
+
 # kt = 1, 3, 7, 13, 31, 33, 45, 131
 @pytest.mark.parametrize("sx,st", [(0.1, 10.0), (0.1, 0.16), (0.1, 0.08), (0.05, 0.08), (0.05, 0.04), (0.2, 0.0175),
                                    (0.2, 0.016), (0.4, 0.0117), (1.0, 0.004)])

@@ -190,6 +190,23 @@ __device__ __forceinline__ int fix(double v)
     return r;
 }
 
+// One instruction each (fmax and fmin quiet their operands first; bounds are NaN
+// all or none, with max_k).
+__device__ __forceinline__ double larger(double a, double b)
+{
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double smaller(double a, double b)
+{
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ int larger(int a, int b) { return max(a, b); }
+__device__ __forceinline__ int smaller(int a, int b) { return min(a, b); }
+
 __device__ __forceinline__ int sub_sat(int a, int b) { return __builtin_elementwise_sub_sat(a, b); }
 
 __device__ __forceinline__ unsigned long long perm64(int src_lane, unsigned long long v)
@@ -1200,8 +1217,8 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                 u64 T = 0ULL;
 #pragma unroll
                 for (int m = 0; m < CPL; ++m) {
-                    n[m].lo = cur[m].lo < nx[m].lo ? nx[m].lo : cur[m].lo;
-                    n[m].hi = cur[m].hi > nx[m].hi ? nx[m].hi : cur[m].hi;
+                    n[m].lo = larger(cur[m].lo, nx[m].lo);
+                    n[m].hi = smaller(cur[m].hi, nx[m].hi);
                     T |= valid_lanes(n[m]);
                 }
                 const int hn = h + 1 < R ? h + 1 : h;
@@ -1497,13 +1514,15 @@ struct ListCursor {
 // those of 65 to 256 neighbours, or all of a map that k_curvelets' error bound
 // does not cover.  One wave per workgroup; the grid is what stays resident, since
 // on whole-pixel maps most anchors can be open, and waves without an anchor leave
-// at once (k_record adds up the others' sums).  Bound by instruction issue: all
+// at once (k_record adds up the others' sums).  Three waves a SIMD for lists of
+// more than 64, whose masks four leave no registers for: 30,000 edges of 200
+// neighbours each 4.56 ms against 4.80.  Bound by instruction issue: all
 // 207,326 anchors of the 1080p map take 1,090 us, 2,100 vector and 912 scalar
 // instructions each.  (Fourteen waves a CU in place of sixteen, with 80 B records
 // and 112 sines at a time, and the anchor's and pairs' sines in two calls: 1,370.
 // Quotients of one denominator on one refined reciprocal: 1,070.)
 template <int CPL, int NW>
-__global__ __launch_bounds__(64, CPL == 1 ? 4 : 2) void k_curvelets_direct(FusedArgs A, int first, int last)
+__global__ __launch_bounds__(64, CPL == 1 ? (NW == 1 ? 4 : 3) : 2) void k_curvelets_direct(FusedArgs A, int first, int last)
 {
     extern __shared__ double lds[];
     const int lane = threadIdx.x & 63;

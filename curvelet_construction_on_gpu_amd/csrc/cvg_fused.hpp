@@ -282,7 +282,8 @@ struct FusedArgs {
 };
 
 constexpr int kFusedWaves = 4;  // anchor streams (waves) per workgroup
-constexpr int kFusedWavesPerSimd = 5;  // at one cell per lane (double maps)
+// What LDS lets stay resident (double maps at one cell per lane: five).
+__host__ __device__ constexpr int waves_per_simd(int cpl, bool flt) { return cpl == 4 ? 2 : (cpl == 1 && !flt ? 5 : 4); }
 constexpr int kFusedSlots = 12;  // bundle slots at one cell per lane
 // pair records in LDS at a time, as a power of two (with two cells per lane 16
 // of them would cost a resident wave per SIMD)
@@ -502,7 +503,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
     // float maps: the smallest magnitude of a bound or of its first denominator
     // (a zero's sign would be lost: :774 makes it -0)
     float least = A.max_k_f;
-    u64 open = 0ULL;
+    u64 open = 0ULL;  // (not CLASSES) neighbours whose direction class is uncertain
 
     const double *ar = reinterpret_cast<const double *>(A.rec + a);
     const double ax = uload(ar), ay = uload(ar + 1), sa = uload(ar + 2), ca = uload(ar + 3);
@@ -582,7 +583,10 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             n1 += __popcll(__ballot(cls[c] == 1));
             if (CLASSES) n2 += __popcll(__ballot(cls[c] == 2));
         }
-        if (!CLASSES) n2 = deg - n1;
+        if (!CLASSES) {
+            if (open != 0ULL) return true;  // (a neighbour across the anchor's direction)
+            n2 = deg - n1;
+        }
         int b1 = 0, b2 = n1, b0 = n1 + n2;
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
@@ -1287,8 +1291,8 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             nacc += static_cast<unsigned>(__popcll(acc));
         }
     }
-    if (MODE == M_FAST && (open | __builtin_amdgcn_ballot_w64(closest <= 2u * kFixTol)) != 0ULL) return true;
-    if (FLT && (open | __builtin_amdgcn_ballot_w64(bad != 0u || least == 0.0f)) != 0ULL) return true;
+    if (MODE == M_FAST && __builtin_amdgcn_ballot_w64(closest <= 2u * kFixTol) != 0ULL) return true;
+    if (FLT && __builtin_amdgcn_ballot_w64(bad != 0u || least == 0.0f) != 0ULL) return true;
     if (lane == 0) ((mem_ptr<unsigned>)A.acc_count)[a] = nacc;
     vp_sum += vp;
     isect_sum += isect + (lane == 0 ? isect_u : 0u);
@@ -1384,7 +1388,7 @@ __device__ __forceinline__ void load_entry(const int4 *p, int &a, unsigned &base
 // code costs the main loop its registers: 1,272 us against 720 on the 1080p
 // map.)
 template <int CPL, bool FLT>
-__global__ __launch_bounds__(64 * kFusedWaves, CPL == 1 && !FLT ? kFusedWavesPerSimd : 4)
+__global__ __launch_bounds__(64 * kFusedWaves, waves_per_simd(CPL, FLT))
 void k_curvelets(FusedArgs A)
 {
     extern __shared__ double lds[];
@@ -1556,7 +1560,7 @@ __global__ __launch_bounds__(64, CPL == 1 ? (NW == 1 ? 4 : 3) : 2) void k_curvel
 // Float maps: the anchors k_curvelets left open.  Those with a zero bound or
 // denominator join the wide ones, for the general kernel.
 template <int CPL>
-__global__ __launch_bounds__(64, 4) void k_curvelets_float_open(FusedArgs A)
+__global__ __launch_bounds__(64, waves_per_simd(CPL, true)) void k_curvelets_float_open(FusedArgs A)
 {
     extern __shared__ double lds[];
     const int lane = threadIdx.x & 63;

@@ -3496,7 +3496,7 @@ int record_rows(cvg_context *ctx, const cvg_params &p, RecordArgs R, int st_stri
 }
 
 // The launch of k_curvelets: as many waves as stay resident, each looping over
-// its share of the lists.  The slots keep kFusedWavesPerSimd waves per SIMD
+// its share of the lists.  The slots keep waves_per_simd of them per SIMD
 // resident (720p map: 263 us at five, 288 at four, 339 at three); a run's
 // bundles beyond them (under 1% of the runs) go to device memory, `spill`
 // words per wave.

@@ -247,6 +247,7 @@ __host__ __device__ inline unsigned row_meta(int rank, bool fwd, bool wide, int 
 struct FusedArgs {
     const double4 *rec;  // per edge (x, y, sin, cos)
     const double *th;
+    const double2 *compass;  // cosine and sine of the eight neighbours' directions, 3 (sign of y) + sign of x
     ExactGrid exact;
     const int *ids;
     const unsigned *off;  // CSR offsets
@@ -576,8 +577,22 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             } else {
                 // (direction_class's projection and a bound at least as strict)
                 const double p = vx * ca + vy * sa;
-                open |= __ballot(in && !(fabs(p) > (FLT ? 1e-5 : 1e-12) * (fabs(vx) + fabs(vy))));
+                bool unsure = in && !(fabs(p) > (FLT ? 1e-5 : 1e-12) * (fabs(vx) + fabs(vy)));
                 k = p > 0 ? 1 : 2;
+                if constexpr (!FLT) {
+                    // on whole pixels, neighbours along an axis or a diagonal:
+                    // the reference's angle is one of eight, and its dot
+                    // product (:459-461) is formed as it is
+                    if (__builtin_amdgcn_ballot_w64(unsure) != 0ULL) {
+                        if (unsure && (vx == 0.0 || vy == 0.0 || fabs(vx) == fabs(vy))) {
+                            const double2 d = A.compass[4 + 3 * ((vy > 0.0) - (vy < 0.0)) + (vx > 0.0) - (vx < 0.0)];
+                            const double dot = d.x * ca + d.y * sa;
+                            k = dot > 0 ? 1 : 2;
+                            unsure = dot == 0.0;  // (there is no third class here)
+                        }
+                    }
+                }
+                open |= __ballot(unsure);
             }
             cls[c] = in ? k : 3;
             n1 += __popcll(__ballot(cls[c] == 1));

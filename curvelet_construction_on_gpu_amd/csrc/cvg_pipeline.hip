@@ -3834,6 +3834,15 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     const size_t o_rank_elig = put(blob, d.rank_elig);
     const size_t o_off_x = put(blob, d.off_x);
     const size_t o_off_t = put(blob, d.off_t);
+    // direction_class's cosine and sine of the directions (-1..1, -1..1)
+    std::vector<double> compass;
+    for (int y = -1; y <= 1; ++y)
+        for (int x = -1; x <= 1; ++x) {
+            double s, c;
+            cvg::cr_sincos(cvg::wrap_two_pi(cvg::cr_atan2(y, x, cvg::kAtanTableHost)), cvg::kSinCosTableHost, &s, &c);
+            compass.insert(compass.end(), {c, s});
+        }
+    const size_t o_compass = put(blob, compass);
     CVG_TRY(upload_tables(ctx, blob));
     const char *tb = static_cast<const char *>(ctx->d_tables.ptr);
     const double *off_x = reinterpret_cast<const double *>(tb + o_off_x);
@@ -3865,6 +3874,7 @@ int build_curvelets(cvg_context *ctx, const cvg_params &p)
     A.rank_elig = reinterpret_cast<const int *>(tb + o_rank_elig);
     A.rank_cell = reinterpret_cast<const int *>(tb + o_rank_cell);
     A.rank_of_cell0 = d.rank_of_cell0;
+    A.compass = reinterpret_cast<const double2 *>(tb + o_compass);
     A.four_dx = 4.0 * d.dx;
     A.max_k = d.max_k;
     A.sin_dt = std::sin(d.dt);

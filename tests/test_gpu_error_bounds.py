@@ -73,6 +73,19 @@ def test_runs_that_fill_the_slots(ctx, oracle_cr, run, group):
     check(ctx, OracleF32(cr=True).run(f, p), ctx.run_f32(f, p), "fused")
 
 
+@pytest.mark.parametrize("off", [0.0, 1e-16, -2e-16, 1e-15, 3e-13, -2e-12])
+@pytest.mark.parametrize("turns", [0, 7, 600])
+def test_neighbours_across_on_pixels(ctx, oracle_cr, off, turns):
+    """Whole-pixel neighbours along an axis or a diagonal, to within rounding
+    across the anchor's direction, and some at the anchor's own place."""
+    xs, ys = np.meshgrid(np.arange(17) * 1.0, np.arange(13) * 1.0)
+    th = np.random.default_rng(4).integers(-8, 8, xs.size) * (np.pi / 4) + off + 2 * np.pi * turns
+    e = np.stack([xs.ravel(), ys.ravel(), th, np.ones(xs.size)], axis=1)
+    e = np.concatenate([e, e[::11]])
+    for p in (CurveletParams(group_max_sz=5), CurveletParams(group_max_sz=4, dx=0.0), CurveletParams(sx=0.05)):
+        check(ctx, oracle_cr.run(e, p), ctx.run(e, p), "fused")
+
+
 @pytest.mark.parametrize("group", [4, 7])
 def test_noalloc_on_the_general_kernel(group, monkeypatch):
     """Its per-wave buffers are made for device memory; on this map they do not

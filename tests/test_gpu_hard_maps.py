@@ -102,3 +102,11 @@ def test_extreme_max_k(ctx, frame, max_k):
     ordinary = shortest(ctx, frame, CurveletParams(group_max_sz=7), "ms_curvelets")
     assert shortest(ctx, frame, CurveletParams(group_max_sz=7, max_k=max_k), "ms_curvelets") < 3.5 * ordinary
     assert ctx.debug_route() == ("fused" if max_k < 1.0 else "direct")
+
+
+@pytest.mark.parametrize("make", [theta_zero, sixteen_thetas])
+def test_curvelets_on_whole_pixels(ctx, frame, make):
+    """Neighbours exactly across the anchor's direction: with none of their
+    classes settled by the fused kernel, 2.0 and 1.0 times the ordinary time."""
+    ordinary = shortest(ctx, frame, CurveletParams(group_max_sz=7), "ms_curvelets")
+    assert shortest(ctx, make(frame), CurveletParams(group_max_sz=7), "ms_curvelets") < 0.9 * ordinary

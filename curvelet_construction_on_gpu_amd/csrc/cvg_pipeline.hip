@@ -115,30 +115,41 @@ struct GridDesc {
 }  // namespace
 
 // Up to 11 helper threads for the copies out of page-locked blocks (the
-// calling thread is another): started at a context's first such download,
-// parked between downloads, joined with the context.
+// calling thread is another): started at a download, parked between downloads,
+// and gone after a second without one, so that contexts a program only keeps
+// hold no threads.  Joined with the context.
 struct CopyCrew {
+    static constexpr int kHelpers = 11;
+    struct Helper {
+        std::thread th;
+        bool live = false;  // (guarded by mu) its loop is running
+    };
     std::mutex mu;
     std::condition_variable wake, idle;
-    std::vector<std::thread> threads;
+    Helper helpers[kHelpers];
     const std::function<void()> *job = nullptr;
     unsigned long long serial = 0;
     int active = 0;
-    bool started = false, stop = false;
+    bool stop = false;
 
     // The helpers run *fn once each, those that wake before end().
     void begin(const std::function<void()> *fn)
     {
-        if (!started) {
-            started = true;
-            const unsigned hw = std::thread::hardware_concurrency();
-            const int count = static_cast<int>(std::min<unsigned>(hw > 1 ? hw - 1 : 0, 11));
-            for (int w = 0; w < count; ++w) {
-                try {
-                    threads.emplace_back([this] { loop(); });
-                } catch (...) {
-                    break;  // fewer helpers
-                }
+        const unsigned hw = std::thread::hardware_concurrency();
+        const int count = static_cast<int>(std::min<unsigned>(hw > 1 ? hw - 1 : 0, kHelpers));
+        for (int w = 0; w < count; ++w) {
+            Helper &h = helpers[w];
+            {
+                std::lock_guard<std::mutex> lk(mu);
+                if (h.live) continue;
+            }
+            if (h.th.joinable()) h.th.join();  // (it has left its loop)
+            h.live = true;
+            try {
+                h.th = std::thread([this, &h] { loop(h); });
+            } catch (...) {
+                h.live = false;
+                break;  // fewer helpers
             }
         }
         {
@@ -161,17 +172,22 @@ struct CopyCrew {
             stop = true;
         }
         wake.notify_all();
-        for (auto &th : threads) th.join();
+        for (Helper &h : helpers)
+            if (h.th.joinable()) h.th.join();
     }
 
 private:
-    void loop()
+    void loop(Helper &h)
     {
         unsigned long long seen = 0;
         std::unique_lock<std::mutex> lk(mu);
         while (true) {
-            wake.wait(lk, [&] { return stop || (job && serial != seen); });
-            if (stop) return;
+            const bool called = wake.wait_for(lk, std::chrono::seconds(1),
+                                              [&] { return stop || (job && serial != seen); });
+            if (stop || !called) {
+                h.live = false;
+                return;
+            }
             seen = serial;
             const std::function<void()> *fn = job;
             ++active;

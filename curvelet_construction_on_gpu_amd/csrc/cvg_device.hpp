@@ -1,6 +1,7 @@
-// Device-side building blocks shared by the fused curvelet kernel and the
-// diagnostic kernels, so that what the diagnostics check is the arithmetic
-// the pipeline runs.
+// Device-side building blocks shared by the curvelet kernels (k_curvelets_direct,
+// k_curvelets_generic) and the diagnostic kernels, so that what the diagnostics
+// check is the arithmetic those run.  (k_curvelets decides on certified
+// approximations of it; tests compare its rows with these kernels' and the oracle's.)
 #ifndef CVG_DEVICE_HPP
 #define CVG_DEVICE_HPP
 
@@ -9,13 +10,6 @@
 #include "cvg_math.hpp"
 
 namespace cvg {
-
-// Per-(anchor, neighbour) quantities of compute_curve_bundle
-// (cpu_curvelet.hpp:646-656, 730-733) that do not depend on the grid cell.
-struct PairRec {
-    double DX, DY, DX2, DY2;
-    double cT0m_DX, sT0m_DY, cT0p_DX, sT0p_DY;
-};
 
 // Direction class of a neighbour: 1 when dot(To2Pi(atan2(ny-ay, nx-ax)), theta_a)
 // > 0 (forward run), 2 when < 0 (backward run), 0 otherwise
@@ -41,58 +35,36 @@ __device__ inline int direction_class(double ax, double ay, double cos_at, doubl
     return dot > 0 ? 1 : (dot < 0 ? 2 : 0);
 }
 
-// The cell-independent part of one pair.
-__device__ inline PairRec pair_record(double ax, double ay, double nx, double ny, double sT0p, double cT0p,
-                                      double sT0m, double cT0m)
-{
-    PairRec r;
-    r.DX = ax - nx;
-    r.DY = ay - ny;
-    r.DX2 = r.DX * r.DX;
-    r.DY2 = r.DY * r.DY;
-    r.cT0m_DX = r.DX * cT0m;
-    r.sT0m_DY = r.DY * sT0m;
-    r.cT0p_DX = r.DX * cT0p;
-    r.sT0p_DY = r.DY * sT0p;
-    return r;
-}
-
 // One grid cell of the circular-arc bundle transport (Prop. 4),
 // compute_curve_bundle's loop body (cpu_curvelet.hpp:697-751 for branch A,
 // :762-806 for branch B), starting from [-max_k, max_k].  Operand order and
 // rounding points are the reference's; the updates use the reference's
-// compare-and-assign, which ignores NaN candidates.
-//   ox    = delta_x2 of the cell's row i
-//   sT2t, cT2t = sin/cos(theta_a + delta_t2)
-//   sm, sp = sin(T2t - (theta_n - dt)), sin(T2t - (theta_n + dt))
-__device__ inline void bundle_cell(const PairRec &p, bool branch_a, double ox, double sT2t, double cT2t, double sm,
-                                   double sp, double dx, double dx2, double max_k, double &lo, double &hi)
+// compare-and-assign, which ignores NaN candidates.  The branches differ in
+// powers of two on both sides of the curvature fraction, in the sign that an
+// exactly zero denominator gets (:774 negates the sum), and in which of
+// theta_n -+ dt bounds which side (branch A: theta_n - dt the lower).
+//   DX, DY, DX2, DY2     n - a negated, and the squares (:646-649)
+//   ox                   delta_x2 of the cell's row i
+//   s2, c2               sin/cos(T2t), T2t = theta_a + delta_t2
+//   s0, cx0, sy0         the lower constraint's angle T0: sin(T2t - T0), DX cos T0, DY sin T0 (:728-733)
+//   s1, cx1, sy1         the upper's
+__device__ inline void bundle_cell(double DX, double DY, double DX2, double DY2, bool branch_a, double ox, double s2,
+                                   double c2, double s0, double cx0, double sy0, double s1, double cx1, double sy1,
+                                   double dx, double dx2, double max_k, double &lo, double &hi)
 {
-    const double tt = sT2t * p.DX - cT2t * p.DY;
+    const double tt = s2 * DX - c2 * DY;  // :705
     const double ttm = tt - ox;
+    const double u = 2.0 * ox * tt - DX2 - DY2 + dx2 - ox * ox;
+    const double den = branch_a ? 0.0 - u : -u / 2.0;
+    const double f = branch_a ? 2.0 : 1.0;
+    const double kx0 = f * (ttm - dx) / den, kx1 = f * (ttm + dx) / den;
+    const double kt0 = s0 / (-s0 * ox + cx0 + sy0), kt1 = s1 / (-s1 * ox + cx1 + sy1);
     lo = -max_k;
     hi = max_k;
-    if (branch_a) {
-        const double den = -2.0 * ox * tt + p.DX2 + p.DY2 - dx2 + ox * ox;
-        const double kx_min = 2.0 * (ttm - dx) / den;
-        const double kx_max = 2.0 * (ttm + dx) / den;
-        if (lo < kx_min) lo = kx_min;
-        if (hi > kx_max) hi = kx_max;
-        const double kt_min = sm / (-sm * ox + p.cT0m_DX + p.sT0m_DY);
-        const double kt_max = sp / (-sp * ox + p.cT0p_DX + p.sT0p_DY);
-        if (lo < kt_min) lo = kt_min;
-        if (hi > kt_max) hi = kt_max;
-    } else {
-        const double den = -(2.0 * ox * tt - p.DX2 - p.DY2 + dx2 - ox * ox) / 2.0;
-        const double kx_min = (ttm - dx) / den;
-        const double kx_max = (ttm + dx) / den;
-        if (lo < kx_min) lo = kx_min;
-        if (hi > kx_max) hi = kx_max;
-        const double kt_max = sm / (-sm * ox + p.cT0m_DX + p.sT0m_DY);
-        if (hi > kt_max) hi = kt_max;
-        const double kt_min = sp / (-sp * ox + p.cT0p_DX + p.sT0p_DY);
-        if (lo < kt_min) lo = kt_min;
-    }
+    if (lo < kx0) lo = kx0;
+    if (lo < kt0) lo = kt0;
+    if (hi > kx1) hi = kx1;
+    if (hi > kt1) hi = kt1;
 }
 
 }  // namespace cvg

@@ -820,29 +820,14 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
             } else if constexpr (DIRECT) {
                 const double DX = q[0].x, DY = q[0].y, DX2 = DX * DX, DY2 = DY * DY;
                 const double cx0 = q[1].x, sy0 = q[1].y, cx1 = q[2].x, sy1 = q[2].y;
-                // the branches (:711-751, :774-806) differ in powers of two and
-                // in the angles' order
-                const bool branch_a = (DX * ca + DY * sa) < 0;
-                const double fn = branch_a ? 2.0 : 1.0;
+                const bool branch_a = (DX * ca + DY * sa) < 0;  // :690
                 const lds_ptr<double> sn = sines + 2 * A.exact.kt * (p & ((1 << slog) - 1));
                 u64 any = 0ULL;
 #pragma unroll
                 for (int m = 0; m < CPL; ++m) {
-                    const double ox = W.ox[m];
-                    const double tt = sT[m] * DX - cT[m] * DY;  // :705
-                    const double ttm = tt - ox;
-                    // (as exact_bound's)
-                    const double u = 2.0 * ox * tt - DX2 - DY2 + A.exact.dx2 - ox * ox;
-                    const double den = branch_a ? 0.0 - u : -u / 2.0;
-                    const double s0 = sn[W.j[m]], s1 = sn[W.j[m] + A.exact.kt];
-                    const double kx0 = fn * (ttm - A.exact.dx) / den, kx1 = fn * (ttm + A.exact.dx) / den;
-                    const double kt0 = s0 / (-s0 * ox + cx0 + sy0), kt1 = s1 / (-s1 * ox + cx1 + sy1);
-                    // the reference's compare-and-assign, which ignores NaN
-                    double lo = -A.exact.max_k, hi = A.exact.max_k;
-                    lo = lo < kx0 ? kx0 : lo;
-                    lo = lo < kt0 ? kt0 : lo;
-                    hi = hi > kx1 ? kx1 : hi;
-                    hi = hi > kt1 ? kt1 : hi;
+                    double lo, hi;
+                    cvg::bundle_cell(DX, DY, DX2, DY2, branch_a, W.ox[m], sT[m], cT[m], sn[W.j[m]], cx0, sy0,
+                                     sn[W.j[m] + A.exact.kt], cx1, sy1, A.exact.dx, A.exact.dx2, A.exact.max_k, lo, hi);
                     v[m].lo = lo;
                     v[m].hi = hi;
                     any |= __builtin_amdgcn_ballot_w64(hi > lo);

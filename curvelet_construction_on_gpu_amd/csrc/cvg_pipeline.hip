@@ -69,7 +69,6 @@
 #include "cvg_stlsort.hpp"
 
 using cvg::Cand;
-using cvg::PairRec;
 
 __constant__ double c_sincos_tab[CVG_SINCOS_TABLE_SIZE] = CVG_SINCOS_TABLE_INIT;
 __constant__ double c_atan_tab[2 * CVG_ATAN_ROWS] = CVG_ATAN_TABLE_INIT;
@@ -2326,20 +2325,21 @@ struct GenMath<double> {
                                   const double *cT2t, double dt, double dx, double dx2, double close_thr,
                                   double max_k, double *lo, double *hi)
     {
-        double sp0, cp0, sm0, cm0;
-        cvg::cr_sincos(nt + dt, c_sincos_tab, &sp0, &cp0);
-        cvg::cr_sincos(nt - dt, c_sincos_tab, &sm0, &cm0);
-        const PairRec pr = cvg::pair_record(ax, ay, nx, ny, sp0, cp0, sm0, cm0);
-        const bool close = pr.DX2 + pr.DY2 < close_thr;  // :682
-        const bool branch_a = (pr.DX * cat + pr.DY * sat) < 0;  // :690
+        const double DX = ax - nx, DY = ay - ny, DX2 = DX * DX, DY2 = DY * DY;
+        const bool close = DX2 + DY2 < close_thr;  // :682
+        const bool branch_a = (DX * cat + DY * sat) < 0;  // :690
+        const double T0 = branch_a ? nt - dt : nt + dt, T1 = branch_a ? nt + dt : nt - dt;
+        double s0, c0, s1, c1;
+        cvg::cr_sincos(T0, c_sincos_tab, &s0, &c0);
+        cvg::cr_sincos(T1, c_sincos_tab, &s1, &c1);
 #pragma unroll
         for (int m = 0; m < M; ++m) {
             lo[m] = -max_k;
             hi[m] = max_k;
             if (close || !live[m]) continue;
-            const double sin_m = cvg::cr_sin(T2t[m] - (nt - dt), c_sincos_tab);
-            const double sin_p = cvg::cr_sin(T2t[m] - (nt + dt), c_sincos_tab);
-            cvg::bundle_cell(pr, branch_a, ox[m], sT2t[m], cT2t[m], sin_m, sin_p, dx, dx2, max_k, lo[m], hi[m]);
+            cvg::bundle_cell(DX, DY, DX2, DY2, branch_a, ox[m], sT2t[m], cT2t[m], cvg::cr_sin(T2t[m] - T0, c_sincos_tab),
+                             DX * c0, DY * s0, cvg::cr_sin(T2t[m] - T1, c_sincos_tab), DX * c1, DY * s1, dx, dx2, max_k,
+                             lo[m], hi[m]);
         }
         return !close;
     }
@@ -2645,19 +2645,20 @@ __global__ void k_debug_anchor(int a, int n, const double *__restrict__ x, const
     const double nx = x[b], ny = y[b], nt = th[b];
     double sa, ca;
     cvg::cr_sincos(at, c_sincos_tab, &sa, &ca);
-    double sp, cp, sm, cm;
-    cvg::cr_sincos(nt + dt, c_sincos_tab, &sp, &cp);
-    cvg::cr_sincos(nt - dt, c_sincos_tab, &sm, &cm);
-    const PairRec p = cvg::pair_record(ax, ay, nx, ny, sp, cp, sm, cm);
-    const bool close = p.DX2 + p.DY2 < close_thr;
-    const bool branch_a = (p.DX * ca + p.DY * sa) < 0;
+    const double DX = ax - nx, DY = ay - ny, DX2 = DX * DX, DY2 = DY * DY;
+    const bool close = DX2 + DY2 < close_thr;
+    const bool branch_a = (DX * ca + DY * sa) < 0;
+    const double T0 = branch_a ? nt - dt : nt + dt, T1 = branch_a ? nt + dt : nt - dt;
+    double s0, c0, s1, c1;
+    cvg::cr_sincos(T0, c_sincos_tab, &s0, &c0);
+    cvg::cr_sincos(T1, c_sincos_tab, &s1, &c1);
     const double T2t = at + off_t[j];
     double s2, c2;
     cvg::cr_sincos(T2t, c_sincos_tab, &s2, &c2);
-    const double sin_m = cvg::cr_sin(T2t - (nt - dt), c_sincos_tab);
-    const double sin_p = cvg::cr_sin(T2t - (nt + dt), c_sincos_tab);
     double lo = -max_k, hi = max_k;
-    if (!close) cvg::bundle_cell(p, branch_a, off_x[i], s2, c2, sin_m, sin_p, dx, dx2, max_k, lo, hi);
+    if (!close)
+        cvg::bundle_cell(DX, DY, DX2, DY2, branch_a, off_x[i], s2, c2, cvg::cr_sin(T2t - T0, c_sincos_tab), DX * c0,
+                         DY * s0, cvg::cr_sin(T2t - T1, c_sincos_tab), DX * c1, DY * s1, dx, dx2, max_k, lo, hi);
     out[static_cast<size_t>(r) * K + c] = lo;
     out[static_cast<size_t>(deg) * K + static_cast<size_t>(r) * K + c] = hi;
     if (c == 0) {

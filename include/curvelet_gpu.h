@@ -369,7 +369,8 @@ int cvg_synth_generate(const cvg_synth_config *config, unsigned long long seed, 
 /* ---- diagnostics ------------------------------------------------------- */
 
 /* Per-neighbour detail of one anchor of the current graph, computed on the
- * device by the same device functions the fused kernel uses: dir[r] = 1
+ * device by the device functions that the direct and the general curvelet
+ * kernels use: dir[r] = 1
  * (forward run), 2 (backward run), 0 (neither); hyp[r] = bundle valid or
  * close; bmin/bmax = deg x K cells in the reference's cell order
  * (i * Kt + j).  Mirrors compute_curve_bundle (cpu_curvelet.hpp:636-819) and

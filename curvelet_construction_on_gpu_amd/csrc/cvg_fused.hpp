@@ -17,10 +17,9 @@
 //
 // Measured on the 1080p map (207,326 edges, 2.04M pairs, G = 7): 1,000 us for
 // the kernel on exact bounds and 141 us for its sines pass (345 MB) before; now
-// 460 us, and 68 us for the few anchors left open, which is one wave's time for
-// one of them.  The same map at whole pixels and 16 orientations leaves about
-// half of its anchors open: 0.70 ms.  (Their open comparisons alone made on
-// exact bounds, on 256 waves: 1.51 ms, and 4.2 ms with all orientations zero.)
+// 432 us, and 32 us for the four anchors left open, which is one wave's time for
+// one of them.  The same map at whole pixels and 16 orientations leaves 9,162 of
+// 184,425 anchors open: 350 us in all.
 #ifndef CVG_FUSED_HPP
 #define CVG_FUSED_HPP
 
@@ -1382,8 +1381,9 @@ __device__ __forceinline__ void load_entry(const int4 *p, int &a, unsigned &base
 // next anchor, the ids of the one after it and the list entry of the third are
 // in flight while an anchor is worked on.  Bound by instruction issue and
 // latency together: on the 1080p map one to four waves per SIMD take 1,145,
-// 723, 574 and 516 us, five 473 (770 vector, 440 scalar and 90 LDS instructions
-// an anchor).  Anchors with a comparison too close
+// 723, 574 and 516 us, five 473 (432 with bounds clamped as they are formed, in
+// place of two differences a cell; 752 vector, 475 scalar and 90 LDS
+// instructions an anchor).  Anchors with a comparison too close
 // for the approximate bounds go to the open list.  (Done again here, their
 // code costs the main loop its registers: 1,272 us against 720 on the 1080p
 // map.)

@@ -439,7 +439,8 @@ CVG_HD bool sin_of_difference(double a, double b, dd sa, dd ca, dd sb, dd cb, do
 }
 
 // cr_sin(fl(a - b)): the subtraction formula where it settles the rounding,
-// else the direct evaluation.
+// else the direct evaluation.  (No kernel uses the two: they are kept as
+// diagnostics, cvg_math_eval's ops 8 and 9.)
 CVG_HD double sin_difference(double a, double b, dd sa, dd ca, dd sb, dd cb, const double *tab)
 {
     double v;

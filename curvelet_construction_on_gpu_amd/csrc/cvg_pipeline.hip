@@ -225,23 +225,23 @@ struct cvg_context {
     bool timed_run = false;  // the current run records the timing events
     std::string err;
     size_t lds_limit = 65536;
-    // accepted, checked and reported as before (cvg_set_tuning, or
-    // CVG_COOP_MIN_CAP / CVG_COOP_WAVES at creation); no launch depends on them
-    // since every anchor is one wave's
+    // accepted, checked and reported (cvg_set_tuning, or CVG_COOP_MIN_CAP /
+    // CVG_COOP_WAVES at creation); no launch depends on them, since every
+    // anchor is one wave's
     int coop_min_cap = 8;
     int coop_waves = 4;
     int num_cu = 1;
     // lanes per anchor in the neighbour-window scans (8, 16, 32 or 64;
     // cvg_set_tuning, or CVG_FILL_LANES at creation; results never depend on it)
     int fill_lanes = 16;
-    // grid of the light buckets' launches as a percentage of their resident
-    // capacity (5..100), or 0: automatic (cvg_set_tuning, or CVG_GRID_PCT)
+    // grid of k_curvelets as a percentage of its resident capacity (5..100), or
+    // 0: all of it (cvg_set_tuning, or CVG_GRID_PCT)
     int grid_pct = 0;
     // use the sorted-key cell layout even where the dense grid fits
     // (CVG_SPARSE_CELLS=1 at creation; results never depend on it)
     bool force_sparse = false;
-    // run double maps on the general curvelet kernel even where the fused one
-    // applies (CVG_GENERIC_KERNEL=1 at creation; same results)
+    // run maps on the general curvelet kernel even where the fused and the direct
+    // one apply (CVG_GENERIC_KERNEL=1 at creation; same results)
     bool force_generic = false;
 
     unsigned *mailbox = nullptr;  // pinned host scalars read back after syncs
@@ -2274,10 +2274,11 @@ __global__ __launch_bounds__(kBlock) void k_record(RecordArgs R, const int *__re
 }
 
 // ---------------------------------------------------------------------------
-// The general curvelet kernel: the float instantiation (run_curvelet<float>,
-// main.cpp:110 with --float), and double maps outside the fused kernel's range
-// (more than 256 neighbours per anchor, group_max_sz above 64, neighbour lists
-// too long for one workgroup's LDS)
+// The general curvelet kernel: double maps with more than 256 neighbours an
+// anchor or group_max_sz above 64, and of the float instantiation
+// (run_curvelet<float>, main.cpp:110 with --float) those and maps outside
+// float_limits, with group_max_sz below 3 or with cells that cannot be a best
+// one; of other float maps the anchors that the fused kernels pass on.
 // ---------------------------------------------------------------------------
 
 // Direction class of a neighbour in float: dot(To2Pi(atan2f(dy, dx)), theta_a)
@@ -2301,7 +2302,7 @@ __device__ inline int direction_class_f(float ax, float ay, float at, float nx, 
 }
 
 // The arithmetic of one instantiation: T = double (the reference's default,
-// and the same device functions as the fused kernel's pre-passes) or T =
+// and the same device functions as k_curvelets_direct) or T =
 // float (main.cpp includes <math.h>, whose float overloads the unqualified
 // sin and cos calls of cpu_curvelet.hpp resolve to; the double literals of
 // :697-698, 711-715 and 774 promote those expressions to double until they
@@ -3259,10 +3260,10 @@ int queue_setup(cvg_context *ctx)
 }
 
 // Whether the fused kernel's fixed-point bounds can be trusted for this graph
-// and these parameters, and the smallest denominator at which they can (a
-// smaller one is settled by its certain sign, with quotients far beyond
-// max_k, or leaves the cell open); min_prod bounds the product of the three
-// where one is that small.
+// and these parameters, and leave few enough anchors open to pay; and the
+// smallest denominator at which they can be trusted (a smaller one is settled by
+// its certain sign, with quotients far beyond max_k, or leaves the cell open).
+// min_prod bounds the product of the three where one is that small.
 //
 // u = 2^-53; S >= |DX| + |DY| over the window, X = dx + max |delta_x2|,
 // B = S + X.  Angles are below 72 (|theta| <= 64), so theta + delta is rounded

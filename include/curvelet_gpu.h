@@ -198,8 +198,8 @@ int cvg_run_device(cvg_context *ctx, int num_edges, int sz_edge_data, const doub
 
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (tight serving loops, harnesses that forbid hipMalloc): cvg_run_device
- * with every intermediate buffer (cell grid, neighbour graph, pair records and
- * sines, staging rows, counters) carved from the library's static device
+ * with every intermediate buffer (cell grid, neighbour graph, edge records and
+ * anchor lists, staging rows, counters) carved from the library's static device
  * scratch array of CVG_NOALLOC_SCRATCH_MIB MiB instead of the context's pools,
  * and the results written straight to caller device buffers: device_chains
  * (max_rows x (group_max_sz + 1) unsigned, 1-based ids) and device_info

@@ -130,3 +130,22 @@ def test_noalloc(group):
     assert got_v == want_v
     assert np.array_equal(got_c, want_c)
     assert np.array_equal(bits(got_i), bits(want_i))
+
+
+def test_batch():
+    """Each map of a batch that takes the direct kernel equals its lone run."""
+    far = np.array(edges_for("synth:C1:1001"))
+    far[:, 2] += FAR
+    maps = [lines(9, seed=2), far, lines(70, seed=4)]
+    p = CurveletParams(group_max_sz=6, max_candidates=256)
+    with Context(0) as ctx:
+        lone = []
+        for m in maps:
+            ctx.run(m, p)
+            lone.append(ctx.curvelets())
+        ctx.run_batch(maps, p)
+        assert ctx.debug_route() == "direct"
+        for k, (chains, info) in enumerate(lone):
+            got_c, got_i = ctx.batch_curvelets(k)
+            assert np.array_equal(got_c, chains)
+            assert np.array_equal(bits(got_i), bits(info))

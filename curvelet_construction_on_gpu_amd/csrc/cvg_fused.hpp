@@ -891,12 +891,14 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
 
         // the run's bundles, a batch of records at a time
         lds_ptr<Bounds> bp = bun;  // the next slot
+        // (without a positive max_k no cell is valid, and only close pairs count)
+        const bool barren = DIRECT && !(A.exact.max_k > 0.0);
         for (int p = p0; p < p1;) {
-            if ((p >> kLog) != batch) {
+            if (!barren && (p >> kLog) != batch) {
                 batch = p >> kLog;
                 fill_batch(batch);
             }
-            if (DIRECT && (p >> slog) != group) {
+            if (DIRECT && !barren && (p >> slog) != group) {
                 group = p >> slog;
                 fill_sines(group);
             }
@@ -932,7 +934,7 @@ __device__ __forceinline__ bool do_anchor(const FusedArgs &A, const WaveCells<CP
                         v[m].lo = def_lo;
                         v[m].hi = def_hi;
                     }
-                } else if (bundle(p, q, v) == 0ULL) {
+                } else if (barren || bundle(p, q, v) == 0ULL) {
                     continue;
                 }
                 if (CLASSES) ++vp;

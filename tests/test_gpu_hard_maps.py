@@ -110,3 +110,9 @@ def test_curvelets_on_whole_pixels(ctx, frame, make):
     classes settled by the fused kernel, 2.0 and 1.0 times the ordinary time."""
     ordinary = shortest(ctx, frame, CurveletParams(group_max_sz=7), "ms_curvelets")
     assert shortest(ctx, make(frame), CurveletParams(group_max_sz=7), "ms_curvelets") < 0.9 * ordinary
+
+
+def test_no_positive_max_k(ctx, frame):
+    """No curvelet can exist: 1.4 times the ordinary time while bundles were formed."""
+    ordinary = shortest(ctx, frame, CurveletParams(group_max_sz=7), "ms_curvelets")
+    assert shortest(ctx, frame, CurveletParams(group_max_sz=7, max_k=0.0), "ms_curvelets") < ordinary
